@@ -349,8 +349,9 @@ int itexhip_qmatmul_device_range(const itexhip_matmul_params* p, const void* a, 
                                  const void* addend, void* out, void* stream);
 
 /* itexhip_qmatmul on the unpacked TF-layout weight ([K, N], or [N, K] with transpose_b), any K, no
- * prepack and no column-sum buffer: one thread per output element.  For the shapes the MFMA kernels
- * do not take (K not a multiple of 16). */
+ * prepack and no column-sum buffer, no alignment: an MFMA kernel that fetches both operands with unaligned
+ * vector loads and sums the weight's columns on the way.  For the shapes the packed kernels do not take
+ * (K not a multiple of 16). */
 int itexhip_qmatmul_unpacked(const itexhip_matmul_params* p, const void* a, const int8_t* w, int transpose_b,
                              int64_t M, int64_t K, int64_t N, const float* min_b, const float* max_b,
                              int64_t nb, const void* bias, const void* addend, void* out, void* stream);

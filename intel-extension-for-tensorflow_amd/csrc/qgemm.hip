@@ -31,6 +31,10 @@ template <int OUT_T>
 int dispatch_tile_conv(const uint8_t* x, uint32_t a_xor, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
                        void* out, hipStream_t st, const ConvTileArgs& cv);
 
+// the op on operands as TensorFlow stores them, any K (qgemm_unpacked.hip)
+int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
+                    const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who);
+
 namespace {
 
 // ------------------------------------------------------------------------------------------------
@@ -382,37 +386,6 @@ __global__ __launch_bounds__(256) void qgemm_naive_kernel(const uint8_t* __restr
   else if (e.n_scales > 1) v = v * e.scales[n];
   if (e.bias) v = v + static_cast<const float*>(e.bias)[n];
   for (int k = 0; k < e.n_eltwise; ++k) v = apply_eltwise(e.elt[k], v);  // no sum post-op on this path
-  store_output<OUT_T>(out, idx, v);
-}
-
-// The whole op on the unpacked weight, any K: the thread also sums its weight column (the zero-point
-// compensation needs it) and derives the channel's scale and bias like the packed kernels do.
-template <int OUT_T>
-__global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __restrict__ a, int a_is_u8,
-                                                                const int8_t* __restrict__ w, int transpose_b,
-                                                                int M, int K, int N, EpilogueArgs e,
-                                                                void* __restrict__ out) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= static_cast<int64_t>(M) * N) return;
-  const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
-  int acc = 0, wsum = 0;
-  for (int k = 0; k < K; ++k) {
-    const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
-                           : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
-    const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
-    acc += av * wv;
-    wsum += wv;
-  }
-  const int jb = (e.nb == N) ? n : 0;
-  const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
-                                                bias_entry(e.prep, e.bias, n), wsum);
-  float v = static_cast<float>(acc);
-  if (e.n_scales > 0) v = v * c.scale;
-  v = v + c.bias;
-  for (int k = 0; k < e.n_eltwise; ++k) {
-    if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
-    else v = apply_eltwise(e.elt[k], v);
-  }
   store_output<OUT_T>(out, idx, v);
 }
 
@@ -852,8 +825,7 @@ extern "C" int itexhip_qmatmul_unpacked(const itexhip_matmul_params* p, const vo
   ITEXHIP_REQUIRE(out != nullptr && min_b != nullptr && max_b != nullptr, "%s: null buffer", who);
   ITEXHIP_REQUIRE(K == 0 || (a && w), "%s: null operand", who);
   ITEXHIP_REQUIRE((p->add_position != 0) == (addend != nullptr), "%s: the addend goes with \"Add\" in fused_ops", who);
-  EpilogueArgs e = make_args(p->t_in, nullptr, nullptr, bias, &ep);
-  e.comp_mul = 0;  // unsigned activations are multiplied directly
+  EpilogueArgs e = make_args(p->t_in, nullptr, nullptr, bias, &ep);  // the kernel sums the weight's columns itself
   e.fused = 1;
   e.nb = static_cast<int>(nb);
   e.min_b = min_b;
@@ -861,19 +833,5 @@ extern "C" int itexhip_qmatmul_unpacked(const itexhip_matmul_params* p, const vo
   e.prep = make_prep_args(p, ep);
   e.addend = addend;
   e.addend_type = is_float16_type(p->t_out) ? p->t_out : ITEXHIP_FLOAT;  // the addend has the output's type
-  const int a_is_u8 = p->t_in == ITEXHIP_QUINT8;
-  const uint8_t* ap = reinterpret_cast<const uint8_t*>(a);
-  const unsigned grid = static_cast<unsigned>((M * N + 255) / 256);
-  hipStream_t hs = as_stream(stream);
-  const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
-  switch (p->t_out) {
-    case ITEXHIP_FLOAT: qmatmul_unpacked_kernel<ITEXHIP_FLOAT><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-    case ITEXHIP_BFLOAT16: qmatmul_unpacked_kernel<ITEXHIP_BFLOAT16><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-    case ITEXHIP_HALF: qmatmul_unpacked_kernel<ITEXHIP_HALF><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-    case ITEXHIP_QINT32: qmatmul_unpacked_kernel<ITEXHIP_QINT32><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-    case ITEXHIP_QINT8: qmatmul_unpacked_kernel<ITEXHIP_QINT8><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-    default: qmatmul_unpacked_kernel<ITEXHIP_QUINT8><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out); break;
-  }
-  ITEXHIP_CHECK_LAUNCH(who);
-  return ITEXHIP_OK;
+  return launch_unpacked(a, p->t_in, w, transpose_b, M, K, N, e, p->t_out, out, as_stream(stream), who);
 }

@@ -1,0 +1,314 @@
+// Quantized MatMul on operands as TensorFlow stores them: any K, no alignment, nothing prepacked.  It takes the problems
+// whose K is not a multiple of 16 (the packed kernels move whole 16-byte pieces of an activation row).
+//
+// A workgroup owns a 64 x 64 output tile and walks K in steps of 256: per step every thread fetches 64 bytes of the
+// activations and 64 of the weight with 16-byte loads at whatever byte address they fall on (the hardware takes unaligned
+// vector loads; two cache lines instead of one now and then), and puts them k-contiguous into LDS; a [K, N] weight is
+// transposed on the way, 4 (k) x 16 (n) bytes per thread by byte permutes.  The long step is for latency: these problems
+// have few tiles per CU, a step costs one round trip to L2 however long it is, and with 8 loads of 16 bytes per thread in
+// flight during the previous step's MFMAs K = 1001 is 4 round trips.  n stays on the lanes of the accumulators
+// (activation = first MFMA operand), so that stores are runs of 32 elements of an output row at any alignment and a lane
+// needs the parameters of one channel per quadrant.
+//
+// Zero-point compensation needs the weight's column sums; they are dot products with ones of the words on their way into
+// LDS (16 instructions per thread and step), added up across the workgroup once at the end.
+//
+// One thread per output element with byte loads, which this replaces, was bound by its loads (two bytes per
+// multiplication): 1000 x 1001 x 1000 with an fp32 result 399 -> 10.7 us, 37 times.
+#include "qgemm_common.hpp"
+
+namespace itexhip {
+
+namespace {
+
+constexpr int kTileM = 64, kTileN = 64, kStepK = 256;
+constexpr int kRow = kStepK + 16;  // LDS bytes per row: 16-byte fragment reads of 16 rows fall into 16 different bank groups
+
+// 16 bytes at base + off, any alignment.  A piece that would reach past the tensor's `end` is read from the last 16 bytes
+// instead (the load is the same instruction for every lane; end >= 16) and moved into place by settle16, once it has
+// arrived.
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+__device__ __forceinline__ v4i fetch16(const uint8_t* __restrict__ base, int64_t off, int64_t end) {
+  return *reinterpret_cast<const v4i_any*>(base + min(off, end - 16));
+}
+__device__ __forceinline__ v4i settle16(v4i v, int64_t off, int64_t end) {
+  const int64_t over = off - (end - 16);
+  // 0: in place; 16 and more: a piece that lies past the end as a whole, whose bytes are never used
+  const uint32_t shift = over > 0 && over < 16 ? static_cast<uint32_t>(over) : 0;
+  uint64_t lo = static_cast<uint64_t>(static_cast<uint32_t>(v[1])) << 32 | static_cast<uint32_t>(v[0]);
+  uint64_t hi = static_cast<uint64_t>(static_cast<uint32_t>(v[3])) << 32 | static_cast<uint32_t>(v[2]);
+  if (shift & 8) { lo = hi; hi = 0; }
+  const uint32_t bits = (shift & 7) * 8;
+  lo = lo >> bits | (hi << 1) << (63 - bits);
+  hi = hi >> bits;
+  return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
+}
+
+// the first `n` bytes of a piece (n < 16 cuts, n <= 0 clears)
+__device__ __forceinline__ v4i keep_bytes(v4i v, int n) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int left = n - 4 * i;
+    const uint32_t mask = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+    v[i] = static_cast<int>(static_cast<uint32_t>(v[i]) & mask);
+  }
+  return v;
+}
+
+// Where byte k of weight column n lives in LDS.  The four 16-column groups that a wavefront of the transposing writer
+// serves at once would meet in the same banks (16 rows are a multiple of all of them apart): each group keeps its 64-byte
+// quarters of a 256-byte span in another order.
+__device__ __forceinline__ int w_offset(int n, int k) { return n * kRow + (k ^ (((n >> 4) & 3) << 6)); }
+
+template <int ALG>
+__device__ __forceinline__ void apply_all(const itexhip_eltwise& elt, float (&v)[16]) {
+  itexhip_eltwise e = elt;
+  e.alg = ALG;  // known here: apply_eltwise folds to one case
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = apply_eltwise(e, v[i]);
+}
+
+template <int OUT_T, bool TRANS>
+__global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
+                                                                const uint8_t* __restrict__ w, int M, int K, int N,
+                                                                int tiles_n, int tiles, EpilogueArgs e, void* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) uint8_t as[kTileM * kRow];
+  __shared__ __attribute__((aligned(16))) uint8_t ws[kTileN * kRow];
+  __shared__ int colsum[kTileN];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  // consecutive workgroup ids go round the 8 XCDs: give each of them a contiguous run of tiles (n fastest), whose
+  // activation rows its L2 then fetches once
+  const int per_xcd = (tiles + 7) / 8;
+  const int tile = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;  // whole workgroup
+  const int tm = tile / tiles_n;
+  const int m0 = tm * kTileM, n0 = (tile - tm * tiles_n) * kTileN;
+  const int64_t a_end = static_cast<int64_t>(M) * K, w_end = static_cast<int64_t>(K) * N;
+  const bool want_sums = e.comp_mul != 0 || e.prep.input_mode == ITEXHIP_MIN_FIRST;
+  if (t < kTileN) colsum[t] = 0;
+
+  // fetch roles: rows (of the activations, or of an [N, K] weight): row t / 16 + 16 h, piece t % 16
+  //              [K, N] weight: 4 k rows from 4 * (t / 4), 16 columns from 16 * (t % 4)
+  const int frow = t >> 4, fpiece = (t & 15) * 16;
+  const int kb = t >> 2, nb = (t & 3) * 16;
+  v4i fa[4], fw[4];
+  int sums[TRANS ? 4 : 16];
+#pragma unroll
+  for (int i = 0; i < (TRANS ? 4 : 16); ++i) sums[i] = 0;
+
+  auto a_off = [&](int h, int k0) {  // rows past M repeat the last one (their results are not stored)
+    return static_cast<int64_t>(min(m0 + frow + 16 * h, M - 1)) * K + k0 + fpiece;
+  };
+  auto w_off = [&](int h, int k0) {
+    if constexpr (TRANS) return static_cast<int64_t>(min(n0 + frow + 16 * h, N - 1)) * K + k0 + fpiece;
+    else return static_cast<int64_t>(k0 + kb * 4 + h) * N + n0 + nb;
+  };
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) fa[h] = fetch16(a, a_off(h, k0), a_end);
+#pragma unroll
+    for (int h = 0; h < 4; ++h) fw[h] = fetch16(w, w_off(h, k0), w_end);
+  };
+  // What lies past K is whatever follows in the activations and zero in the weight.  Pieces that reach past a tensor's end
+  // only occur in the last rows of the last step: the whole workgroup tests for that once per step.
+  auto put = [&](int k0) {
+    const bool last = k0 + kStepK + 16 > K;
+    if (last) {
+      if (m0 + kTileM + 16 > M) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) fa[h] = settle16(fa[h], a_off(h, k0), a_end);
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        fw[h] = settle16(fw[h], w_off(h, k0), w_end);
+        if constexpr (TRANS) fw[h] = keep_bytes(fw[h], K - k0 - fpiece);
+        else if (k0 + kb * 4 + h >= K) fw[h] = v4i{0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      v4i v = fa[h];
+      v.x ^= a_xor; v.y ^= a_xor; v.z ^= a_xor; v.w ^= a_xor;
+      *reinterpret_cast<v4i*>(as + (frow + 16 * h) * kRow + fpiece) = v;
+    }
+    if constexpr (TRANS) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const v4i v = fw[h];
+        *reinterpret_cast<v4i*>(ws + w_offset(frow + 16 * h, fpiece)) = v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[h] = __builtin_amdgcn_sdot4(v[i], 0x01010101, sums[h], false);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {  // columns nb + 4 c .. + 3: a 4 x 4 byte transpose in two rounds of permutes
+        const uint32_t r0 = fw[0][c], r1 = fw[1][c], r2 = fw[2][c], r3 = fw[3][c];
+        const uint32_t lo01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), hi01 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+        const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+        const uint32_t v[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          *reinterpret_cast<uint32_t*>(ws + w_offset(nb + 4 * c + j, kb * 4)) = v[j];
+          sums[4 * c + j] = __builtin_amdgcn_sdot4(static_cast<int>(v[j]), 0x01010101, sums[4 * c + j], false);
+        }
+      }
+    }
+  };
+
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  v16i acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0;
+  // the channel this lane finishes; its parameters travel under the K loop
+  const int n = n0 + wn + (lane & 31);
+  RawChannel raw = load_raw_channel(e, min(n, N - 1), N);
+  fetch(0);
+  for (int k0 = 0; k0 < K; k0 += kStepK) {
+    put(k0);
+    __syncthreads();
+    if (k0 + kStepK < K) fetch(k0 + kStepK);
+    auto multiply = [&](int kk) {
+      const int k = kk + (lane >> 5) * 16;
+      const v4i x = *reinterpret_cast<const v4i*>(as + (wm + (lane & 31)) * kRow + k);
+      const v4i y = *reinterpret_cast<const v4i*>(ws + w_offset(wn + (lane & 31), k));
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(x, y, acc, 0, 0, 0);
+    };
+    if (k0 + kStepK <= K) {
+#pragma unroll
+      for (int kk = 0; kk < kStepK; kk += 32) multiply(kk);
+    } else {
+      for (int kk = 0; k0 + kk < K; kk += 32) multiply(kk);
+    }
+    __syncthreads();
+  }
+  if (want_sums) {
+    if constexpr (TRANS) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+#pragma unroll
+        for (int d = 1; d < 16; d <<= 1) sums[h] += __shfl_xor(sums[h], d, 64);
+        if ((t & 15) == 0) colsum[frow + 16 * h] = sums[h];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {  // over the 4 lanes of a row of 16 that hold these columns, then across rows and wavefronts
+        sums[i] += __shfl_xor(sums[i], 4, 64);
+        sums[i] += __shfl_xor(sums[i], 8, 64);
+        if ((lane & 12) == 0) atomicAdd(&colsum[nb + i], sums[i]);
+      }
+    }
+    __syncthreads();
+  }
+  if (n >= N) return;
+  raw.colsum = colsum[wn + (lane & 31)];
+  int comp;
+  float scale, bias;
+  finish_channel(e, raw, &comp, &scale, &bias);
+  // accumulator i of a lane: row (i / 4) * 8 + (lane / 32) * 4 + i % 4, column lane % 32 of the quadrant
+  const int mrow = m0 + wm + (lane >> 5) * 4;
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    v[i] = static_cast<float>(acc[i] + comp) * scale;  // scale 1.0f when the node has no output scale (exact)
+    v[i] = v[i] + bias;
+  }
+  for (int k = 0; k < e.n_eltwise; ++k) {
+    const itexhip_eltwise& elt = e.elt[k];
+    switch (elt.alg) {
+      case ITEXHIP_ELT_SUM:
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int m = min(mrow + (i >> 2) * 8 + (i & 3), M - 1);
+          v[i] = v[i] + elt.alpha * load_addend(e, static_cast<int64_t>(m) * N + n);
+        }
+        break;
+      case ITEXHIP_ELT_RELU: apply_all<ITEXHIP_ELT_RELU>(elt, v); break;
+      case ITEXHIP_ELT_CLIP: apply_all<ITEXHIP_ELT_CLIP>(elt, v); break;
+      case ITEXHIP_ELT_LINEAR: apply_all<ITEXHIP_ELT_LINEAR>(elt, v); break;
+      case ITEXHIP_ELT_GELU_TANH: apply_all<ITEXHIP_ELT_GELU_TANH>(elt, v); break;
+      case ITEXHIP_ELT_GELU_ERF: apply_all<ITEXHIP_ELT_GELU_ERF>(elt, v); break;
+      case ITEXHIP_ELT_ELU: apply_all<ITEXHIP_ELT_ELU>(elt, v); break;
+      case ITEXHIP_ELT_LOGISTIC: apply_all<ITEXHIP_ELT_LOGISTIC>(elt, v); break;
+      case ITEXHIP_ELT_TANH: apply_all<ITEXHIP_ELT_TANH>(elt, v); break;
+      case ITEXHIP_ELT_SWISH: apply_all<ITEXHIP_ELT_SWISH>(elt, v); break;
+      case ITEXHIP_ELT_MISH: apply_all<ITEXHIP_ELT_MISH>(elt, v); break;
+      default: break;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int m = mrow + (i >> 2) * 8 + (i & 3);
+    if (m < M) store_output<OUT_T>(out, static_cast<int64_t>(m) * N + n, v[i]);
+  }
+}
+
+// An operand of fewer than 16 bytes in all (K < 16): one thread per output element.
+template <int OUT_T>
+__global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __restrict__ a, int a_is_u8,
+                                                            const int8_t* __restrict__ w, int transpose_b,
+                                                            int M, int K, int N, EpilogueArgs e,
+                                                            void* __restrict__ out) {
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (idx >= static_cast<int64_t>(M) * N) return;
+  const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
+  int acc = 0, wsum = 0;
+  for (int k = 0; k < K; ++k) {
+    const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
+                           : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
+    const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
+    acc += av * wv;
+    wsum += wv;
+  }
+  const int jb = (e.nb == N) ? n : 0;
+  const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
+                                                bias_entry(e.prep, e.bias, n), wsum);
+  float v = static_cast<float>(acc);
+  if (e.n_scales > 0) v = v * c.scale;
+  v = v + c.bias;
+  for (int k = 0; k < e.n_eltwise; ++k) {
+    if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
+    else v = apply_eltwise(e.elt[k], v);
+  }
+  store_output<OUT_T>(out, idx, v);
+}
+
+template <int OUT_T>
+void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
+            const EpilogueArgs& e, void* out, hipStream_t st) {
+  if (static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16) {
+    qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((static_cast<int64_t>(M) * N + 255) / 256), 256, 0, st>>>(
+        a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out);
+    return;
+  }
+  const unsigned grid = static_cast<unsigned>((tiles + 7) / 8 * 8);  // whole runs for the 8 XCDs
+  if (transpose_b) qmatmul_unpacked_kernel<OUT_T, true><<<grid, 256, 0, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
+  else qmatmul_unpacked_kernel<OUT_T, false><<<grid, 256, 0, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
+}
+
+}  // namespace
+
+// M, N > 0; `e` is a fused epilogue (the kernel derives scale and bias of a channel itself) without column sums.
+int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
+                    const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who) {
+  const int64_t tiles_m = (M + kTileM - 1) / kTileM, tiles_n = (N + kTileN - 1) / kTileN;
+  ITEXHIP_REQUIRE(tiles_m * tiles_n < (1LL << 24) - 8, "%s: output too large for one launch", who);  // 2^32 threads
+  const uint8_t* ap = static_cast<const uint8_t*>(a);
+  const uint8_t* wp = reinterpret_cast<const uint8_t*>(w);
+  const uint32_t a_xor = a_type == ITEXHIP_QUINT8 ? 0x80808080u : 0u;
+  const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
+  const int tn = static_cast<int>(tiles_n), tiles = static_cast<int>(tiles_m * tiles_n);
+  switch (out_type) {
+    case ITEXHIP_FLOAT: launch<ITEXHIP_FLOAT>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_BFLOAT16: launch<ITEXHIP_BFLOAT16>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_HALF: launch<ITEXHIP_HALF>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_QINT32: launch<ITEXHIP_QINT32>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_QINT8: launch<ITEXHIP_QINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    default: launch<ITEXHIP_QUINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+  }
+  ITEXHIP_CHECK_LAUNCH(who);
+  return ITEXHIP_OK;
+}
+
+}  // namespace itexhip

@@ -234,7 +234,7 @@ class QuantizedMatMulOp : public OpKernel {
     if (min_b_dev == nullptr || max_b_dev == nullptr) return;
     // ---- product: one launch, the MatMul kernel derives each channel's output scale and compensated
     // bias itself, so a new activation range costs nothing extra.  K a multiple of 16: MFMA kernels on
-    // the prepacked weight; other K: the reference-shaped kernel on the unpacked weight.
+    // the prepacked weight; other K: the MFMA kernel on the unpacked operands.
     // "Add": the addend (of the output's type: float, bfloat16 or half) is input 3 (:352-389 adds it in place into the forwarded output buffer; here the
     // kernel reads it and writes a fresh output, same values)
     const void* addend = nullptr;

@@ -1,0 +1,35 @@
+"""The quantized MatMul on operands as TensorFlow stores them (itexhip_qmatmul_unpacked): any K, both weight layouts,
+against the CPU oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as orc
+from tests.test_gpu_matmul import V1_S32, V2_DEQ, V2_REQ_U8_RELU, make_acts, make_layer, tdt
+
+pytestmark = pytest.mark.gpu
+
+# edges of the 64 x 64 tile and of the 256-long K step, tensors of fewer than 16 bytes, pieces cut by the end of either
+# operand in the last rows, several steps
+SHAPES = [(1, 1, 1), (1, 3, 1000), (5, 15, 3), (2, 8, 70), (3, 17, 16), (64, 256, 64), (65, 257, 63), (63, 255, 65),
+          (130, 1001, 70), (17, 13, 129), (200, 530, 33)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("kw,transpose_b", [(V2_DEQ, False), (V2_REQ_U8_RELU, False), (V1_S32, False),
+                                            (dict(V2_DEQ, input_mode=orc.SCALED), True),
+                                            (dict(V1_S32, input_mode=orc.SCALED), True)])
+def test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b):
+    import torch
+    layer, w, bias = make_layer(hip, dev, K, N, seed=K + N)
+    x, xq, mn, mx = make_acts(M, K, seed=M, mode=kw["input_mode"])
+    r_out = float(np.abs(x @ w + bias).max())
+    ref = layer.oracle(xq, kw, mn, mx, -r_out, r_out)
+    t_in = orc.QUINT8 if xq.dtype == np.uint8 else orc.QINT8
+    p = hip.matmul_params(t_in=t_in, min_a=mn, max_a=mx, min_out=-r_out, max_out=r_out, **kw)
+    w_d = torch.from_numpy(np.ascontiguousarray(layer.wq.T) if transpose_b else layer.wq).to(dev)
+    out = torch.empty((M, N), dtype=tdt(kw["t_out"]), device=dev)
+    out.view(torch.uint8).fill_(0x55)
+    hip.qmatmul_unpacked(p, torch.from_numpy(xq).to(dev), w_d, transpose_b, M, K, N, layer.min_b_d, layer.max_b_d,
+                         layer.min_b.size, layer.bias_d, out)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy(), ref)
