@@ -13,13 +13,10 @@
 #include <type_traits>
 #include <utility>
 
-#include "common.hpp"
+#include "qgemm_common.hpp"
 
 namespace itexhip {
 namespace {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kTile = 64;          // output tile edge and k step
 constexpr int kLdsStride = 80;     // bytes per LDS row: 64 + 16, keeps the 16-byte fragment reads aligned
@@ -28,25 +25,42 @@ constexpr int kBmmThreads = 256;
 struct BmmArgs {
   itexhip_bmm_params p;
   int tiles_m, tiles_n;
-  int vec_x, vec_y;  // operand layouts allow aligned vector loads
-  int grid3;         // launched as (tiles, innermost batch dimension, the other batch dimensions): no division finds them
+  int mode;          // kBytes, kAligned or kAny: how both operands are read
+  int xcd_grid;      // launched as (8, tiles, matrices / 8): see the kernel
+  uint32_t batch;
+  FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
 };
+
+// How an operand is read.  kBytes: K < 16 (or fewer than 4 rows / columns) and unaligned: byte by byte.  kAligned: aligned
+// 16-byte (KCONT) / 4-byte (transposed) loads that never straddle a bound.  kAny: the same loads at whatever byte address
+// they fall on (the hardware takes unaligned vector loads); a load that would cross the end of its row starts at the last
+// place inside it and settle_tile shifts the bytes into place once they have arrived.  P.V over 197 tokens (384 products of
+// 197 x 197 by 197 x 64 to bfloat16): 36.9 us with byte loads (16 per piece), 11.6 us with these.
+enum : int { kBytes = 0, kAligned = 1, kAny = 2 };
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
 
 // One 64 (rows or columns of the output) x 64 (k) byte tile on its way into LDS, k-contiguous there.  The
 // global loads (fetch_tile) and the LDS stores (put_tile) are separate so that the next tile's loads are in
 // flight while the current one is multiplied.
 //   KCONT: the operand is stored [R, K] (k fastest);  else [K, R] (r fastest) and is transposed in put_tile.
-//   VEC:   aligned 16-byte (KCONT) / 4-byte (transposed) global loads are legal and never straddle a bound.
-template <bool KCONT, bool VEC>
+template <bool KCONT, int MODE>
 __device__ __forceinline__ void fetch_tile(const int8_t* __restrict__ g, int64_t R, int64_t K, int64_t r0, int64_t k0,
                                            int t, uint32_t (&w)[4]) {
-  w[0] = w[1] = w[2] = w[3] = 0;
   if constexpr (KCONT) {  // thread: row t / 4, 16 consecutive k
-    const int64_t row = r0 + (t >> 2), k = k0 + (t & 3) * 16;
+    int64_t row = r0 + (t >> 2), k = k0 + (t & 3) * 16;
+    if constexpr (MODE == kAny) {  // rows past R repeat the last one (their results are not stored)
+      row = row < R ? row : R - 1;
+      k = k < K - 16 ? k : K - 16;
+      const v4i v = *reinterpret_cast<const v4i_any*>(g + row * K + k);
+      w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
+      return;
+    }
+    w[0] = w[1] = w[2] = w[3] = 0;
     if (row >= R) return;
     const int8_t* src = g + row * K + k;
-    if constexpr (VEC) {
+    if constexpr (MODE == kAligned) {
       if (k < K) {
         const v4i v = *reinterpret_cast<const v4i*>(src);
         w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
@@ -58,19 +72,61 @@ __device__ __forceinline__ void fetch_tile(const int8_t* __restrict__ g, int64_t
     }
   } else {  // thread: 4 (k) x 4 (r) bytes; kb = t / 16 picks the k rows, cb = t % 16 the r columns; w[i] = k row i
     const int kb = t >> 4, cb = t & 15;
-    const int64_t r = r0 + cb * 4;
+    int64_t r = r0 + cb * 4;
+    if constexpr (MODE == kAny) {
+      r = r < R - 4 ? r : R - 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t k = k0 + kb * 4 + i;
+        w[i] = *reinterpret_cast<const u32_any*>(g + (k < K ? k : K - 1) * R + r);
+      }
+      return;
+    }
+    w[0] = w[1] = w[2] = w[3] = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t k = k0 + kb * 4 + i;
       if (k >= K) continue;
       const int8_t* src = g + k * R + r;
-      if constexpr (VEC) {
+      if constexpr (MODE == kAligned) {
         if (r < R) w[i] = *reinterpret_cast<const uint32_t*>(src);
       } else {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
           if (r + b < R) w[i] |= static_cast<uint32_t>(static_cast<uint8_t>(src[b])) << (8 * b);
       }
+    }
+  }
+}
+
+// kAny: what fetch_tile brought, with the bytes of a piece that crosses a bound moved into place and everything past K
+// cleared.  Only the last k tile and the last columns of the operand have such pieces.
+template <bool KCONT>
+__device__ __forceinline__ void settle_tile(int64_t R, int64_t K, int64_t r0, int64_t k0, int t, uint32_t (&w)[4]) {
+  if constexpr (KCONT) {
+    if (k0 + kTile <= K) return;
+    const int left = static_cast<int>(K - k0) - (t & 3) * 16;  // bytes of this piece inside the row
+    if (left >= 16) return;
+    const uint32_t shift = left > 0 ? 16 - left : 0;           // 1 .. 15
+    uint64_t lo = static_cast<uint64_t>(w[1]) << 32 | w[0], hi = static_cast<uint64_t>(w[3]) << 32 | w[2];
+    if (shift & 8) { lo = hi; hi = 0; }
+    const uint32_t bits = (shift & 7) * 8;
+    lo = lo >> bits | (hi << 1) << (63 - bits);
+    hi = hi >> bits;
+    if (left <= 0) lo = hi = 0;
+    w[0] = static_cast<uint32_t>(lo); w[1] = static_cast<uint32_t>(lo >> 32);
+    w[2] = static_cast<uint32_t>(hi); w[3] = static_cast<uint32_t>(hi >> 32);
+  } else {
+    if (r0 + kTile > R) {
+      const int over = static_cast<int>(r0 - (R - 4)) + (t & 15) * 4;  // how far the load was moved back
+      const uint32_t bits = over > 0 && over < 4 ? over * 8 : 0;       // past the last column: whatever came (not stored)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] >>= bits;
+    }
+    if (k0 + kTile > K) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k0 + (t >> 4) * 4 + i >= K) w[i] = 0;
     }
   }
 }
@@ -141,21 +197,26 @@ __device__ __forceinline__ void fetch_operands(const QuadrantSite& s, int lane, 
   }
 }
 
-// One result on its way out: scale, fused operands in order (each separately rounded), narrowing, store.
-template <int OUT_T, int NB, bool ROWB, int ALG0, int ALG1>
-__device__ __forceinline__ void store_one(int acc, const QuadrantSite& s, int i, uint32_t off,
-                                          const float (&o)[ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16]) {
-  using elem_t = typename std::conditional<OUT_T == ITEXHIP_FLOAT, float, uint16_t>::type;
+// One result: scale, fused operands in order (each separately rounded).
+template <int NB, bool ROWB, int ALG0, int ALG1>
+__device__ __forceinline__ float finish_one(int acc, const QuadrantSite& s, int i,
+                                            const float (&o)[ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16]) {
   float v = static_cast<float>(acc) * s.scale;
   if constexpr (NB > 0) v = ALG0 == ITEXHIP_BIN_MUL ? v * o[0][ROWB ? 0 : i] : v + o[0][ROWB ? 0 : i];
   if constexpr (NB > 1) v = ALG1 == ITEXHIP_BIN_MUL ? v * o[1][ROWB ? 0 : i] : v + o[1][ROWB ? 0 : i];
-  elem_t* dst = reinterpret_cast<elem_t*>(s.out + off);
-  // the output is written back as it goes instead of staying dirty in L2 until the kernel ends: as system-scope
-  // (write-through) stores without fused operands (P.V over 128 sequences: 21.3 -> 18.8 us), as streaming stores
-  // with them (Q.K^T + Mul + Add measured 3 % slower written through)
-  if constexpr (OUT_T == ITEXHIP_FLOAT && NB == 0) __hip_atomic_store(dst, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  else if constexpr (OUT_T == ITEXHIP_FLOAT) __builtin_nontemporal_store(v, dst);
-  else __builtin_nontemporal_store(static_cast<uint16_t>(f32_to_bits16<OUT_T>(v)), dst);
+  return v;
+}
+
+// Its way out.  fp32: the output is written back as it goes instead of staying dirty in L2 until the kernel ends: as
+// system-scope (write-through) stores without fused operands (P.V over 128 sequences: 21.3 -> 18.8 us), as streaming
+// stores with them (Q.K^T + Mul + Add measured 3 % slower written through).  16-bit: plain stores, because a store covers
+// half a cache line at best and L2 puts the lines together (Q.K^T over 197 tokens, rows of 394 bytes: 31.1 us with
+// streaming stores, 19.4 us with plain ones).
+template <int OUT_T, int NB>
+__device__ __forceinline__ void store_one(float v, char* dst) {
+  if constexpr (OUT_T == ITEXHIP_FLOAT && NB == 0) __hip_atomic_store(reinterpret_cast<float*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else if constexpr (OUT_T == ITEXHIP_FLOAT) __builtin_nontemporal_store(v, reinterpret_cast<float*>(dst));
+  else *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(f32_to_bits16<OUT_T>(v));
 }
 
 template <int OUT_T, int NB, bool ROWB, int ALG0, int ALG1>
@@ -163,11 +224,33 @@ __device__ __forceinline__ void store_rows(const v16i& acc, const QuadrantSite& 
                                            const float (&o)[ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16]) {
   using elem_t = typename std::conditional<OUT_T == ITEXHIP_FLOAT, float, uint16_t>::type;
   const uint32_t lrow = (lane >> 5) * 4, lcol = lane & 31;
+  auto result = [&](int i) { return finish_one<NB, ROWB, ALG0, ALG1>(acc[i], s, i, o); };
+  if constexpr (OUT_T != ITEXHIP_FLOAT) {
+    // 16-bit results, all 32 columns exist: two neighbouring lanes trade one of their two rows, so that the even lane
+    // stores two columns of the upper row and the odd lane two of the lower one as a dword (at any 2-byte address: rows
+    // of an odd number of elements).  Half the store instructions; Q.K^T over 197 tokens 19.4 -> 18.4 us together with the
+    // mapping of matrices to XCDs.
+    if (s.cols_left == 32) {
+      const uint32_t odd = lane & 1;
+      const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+      const uint32_t base = (lrow + odd) * s.out_row + (lcol & ~1u) * 2;
+      const bool whole = s.rows_left == 32;
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const uint32_t mine = f32x2_to_bits16<OUT_T>(result(i), result(i + 1));
+        const uint32_t other = __builtin_amdgcn_update_dpp(0u, mine, 0xb1, 0xf, 0xf, true);  // quad_perm 1, 0, 3, 2
+        const uint32_t r = (i >> 2) * 8 + (i & 3);
+        if (whole || static_cast<int>(lrow + odd + r) < s.rows_left)
+          *reinterpret_cast<u32_any*>(s.out + (base + r * s.out_row)) = __builtin_amdgcn_perm(other, mine, sel);
+      }
+      return;
+    }
+  }
   const uint32_t obase = lrow * s.out_row + lcol * static_cast<uint32_t>(sizeof(elem_t));
   if (s.rows_left == 32 && s.cols_left == 32) {  // a whole quadrant (the same answer for the wavefront): nothing to test
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      store_one<OUT_T, NB, ROWB, ALG0, ALG1>(acc[i], s, i, obase + static_cast<uint32_t>((i >> 2) * 8 + (i & 3)) * s.out_row, o);
+      store_one<OUT_T, NB>(result(i), s.out + (obase + static_cast<uint32_t>((i >> 2) * 8 + (i & 3)) * s.out_row));
     return;
   }
   if (static_cast<int>(lcol) >= s.cols_left) return;
@@ -175,7 +258,7 @@ __device__ __forceinline__ void store_rows(const v16i& acc, const QuadrantSite& 
   for (int i = 0; i < 16; ++i) {
     const int r = (i >> 2) * 8 + (i & 3);
     if (static_cast<int>(lrow) + r >= s.rows_left) continue;
-    store_one<OUT_T, NB, ROWB, ALG0, ALG1>(acc[i], s, i, obase + r * s.out_row, o);
+    store_one<OUT_T, NB>(result(i), s.out + (obase + r * s.out_row));
   }
 }
 
@@ -240,7 +323,7 @@ __device__ __forceinline__ QuadrantSite quadrant_site(const itexhip_bmm_params& 
 // The larger tiles amortise what a wavefront spends around its MFMAs (a 64 x 64 tile of K = 64 is two MFMAs and some
 // 450 other instructions per wavefront) and read each operand half as often; they exist for the calls whose fused
 // operands take one register per lane and quadrant column (none, or ROWB).
-template <bool ADJ_X, bool ADJ_Y, bool VEC_X, bool VEC_Y, int NB, int OUT_T, bool ROWB, int RM, int RN>
+template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB, int RM, int RN>
 __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8_t* __restrict__ xb,
                                          const int8_t* __restrict__ yb, const int64_t (&bo)[ITEXHIP_BMM_MAX_BINARY], uint32_t bi,
                                          int m0, int n0, int wm, int wn, int t, int lane, void* __restrict__ out,
@@ -249,9 +332,9 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
   // first tiles and the fused operands: all loads the results depend on are issued before any is needed
   uint32_t wx[RM][4], wy[RN][4];
 #pragma unroll
-  for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, VEC_X>(xb, p.M, p.K, m0 + 64 * h, 0, t, wx[h]);  // x is [M, K] unless adj_x
+  for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE>(xb, p.M, p.K, m0 + 64 * h, 0, t, wx[h]);  // x is [M, K] unless adj_x
 #pragma unroll
-  for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, VEC_Y>(yb, p.N, p.K, n0 + 64 * h, 0, t, wy[h]);   // y is [N, K] only with adj_y
+  for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE>(yb, p.N, p.K, n0 + 64 * h, 0, t, wy[h]);   // y is [N, K] only with adj_y
   // (the quadrants are walked with compile-time indices: what describes a quadrant is the same for the whole
   // wavefront and must stay in scalar registers, which an indexed array of descriptors does not)
   float o[RM * RN][ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16];
@@ -268,6 +351,12 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
   });
 
   for (int64_t k0 = 0; k0 < p.K; k0 += kTile) {
+    if constexpr (MODE == kAny) {
+#pragma unroll
+      for (int h = 0; h < RM; ++h) settle_tile<!ADJ_X>(p.M, p.K, m0 + 64 * h, k0, t, wx[h]);
+#pragma unroll
+      for (int h = 0; h < RN; ++h) settle_tile<ADJ_Y>(p.N, p.K, n0 + 64 * h, k0, t, wy[h]);
+    }
 #pragma unroll
     for (int h = 0; h < RM; ++h) put_tile<!ADJ_X>(xs + h * 64 * kLdsStride, t, wx[h]);
 #pragma unroll
@@ -275,9 +364,9 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
     __syncthreads();
     if (k0 + kTile < p.K) {  // the next tile travels while this one is multiplied
 #pragma unroll
-      for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, VEC_X>(xb, p.M, p.K, m0 + 64 * h, k0 + kTile, t, wx[h]);
+      for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE>(xb, p.M, p.K, m0 + 64 * h, k0 + kTile, t, wx[h]);
 #pragma unroll
-      for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, VEC_Y>(yb, p.N, p.K, n0 + 64 * h, k0 + kTile, t, wy[h]);
+      for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE>(yb, p.N, p.K, n0 + 64 * h, k0 + kTile, t, wy[h]);
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -304,7 +393,7 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
 // One kernel per (layouts, number of fused operands, output type, operands independent of the row): compiled as one
 // kernel with a switch over these, every variant took the registers of the largest (112 - 140, three or four
 // wavefronts per SIMD; P.V over 128 sequences 18.7 -> 16.4 us as a kernel of its own).
-template <bool ADJ_X, bool ADJ_Y, bool VEC_X, bool VEC_Y, int NB, int OUT_T, bool ROWB, int RM = 1, int RN = 1>
+template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB, int RM = 1, int RN = 1>
 __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, const int8_t* __restrict__ x,
                                                            const int8_t* __restrict__ y, void* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) uint8_t xs[RM * kTile * kLdsStride];
@@ -314,65 +403,59 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // the same for the whole wavefront: keep it scalar
   const int wm = wave >> 1, wn = wave & 1;
 
-  // workgroup -> (batch entry, tile); consecutive workgroups walk the tiles of one matrix.  Launched as a 3-d grid
-  // (whenever its extents allow) the innermost batch index and the product of the others come from the workgroup id;
-  // otherwise, and for more than two batch dimensions, divisions find them.  The launch has fewer than 2^31
-  // workgroups, so 32-bit arithmetic covers the decomposition.
-  const uint32_t tile = a.grid3 ? blockIdx.x : blockIdx.x % (static_cast<uint32_t>(a.tiles_m) * static_cast<uint32_t>(a.tiles_n));
+  // Workgroup -> (batch entry, tile).  Consecutive workgroup ids go round the 8 XCDs.  Launched as (8, tiles, matrices / 8)
+  // the XCD takes whole matrices: their operands are read into one L2, and output lines that two tiles share (rows that are
+  // no multiple of a cache line) are put together there instead of leaving two L2s in pieces.  Otherwise consecutive
+  // workgroups walk the tiles of one matrix.  The launch has fewer than 2^31 workgroups: 32-bit arithmetic.
+  uint32_t bi, tile;  // index of the output matrix
+  if (a.xcd_grid) {
+    bi = blockIdx.z * 8 + blockIdx.x;
+    tile = blockIdx.y;
+    if (bi >= a.batch) return;  // whole workgroup
+  } else {
+    const uint32_t tiles = static_cast<uint32_t>(a.tiles_m) * static_cast<uint32_t>(a.tiles_n);
+    bi = blockIdx.x / tiles;
+    tile = blockIdx.x - bi * tiles;
+  }
   const int tm = a.tiles_n == 1 ? static_cast<int>(tile) : static_cast<int>(tile / a.tiles_n);
   const int m0 = tm * (RM * kTile), n0 = static_cast<int>(tile - tm * a.tiles_n) * (RN * kTile);
 
   int64_t xo = 0, yo = 0, bo[ITEXHIP_BMM_MAX_BINARY] = {0, 0};
-  uint32_t bi;  // index of the output matrix
-  {
-    int d = p.n_batch_dims - 1;
-    uint32_t rem;
-    if (a.grid3) {
-      if (d >= 0) {  // the innermost batch dimension: blockIdx.y
-        const int64_t i = blockIdx.y;
-        xo = i * p.x_batch_stride[d];
-        yo = i * p.y_batch_stride[d];
+  uint32_t rem = bi;
+  for (int d = p.n_batch_dims - 1; d >= 0; --d) {
+    // the outermost index needs no division
+    const uint32_t q = d == 0 ? 0 : static_cast<uint32_t>(fast_div(static_cast<int>(rem), a.by_dim[d]));
+    const int64_t i = rem - q * static_cast<uint32_t>(p.batch_dims[d]);
+    rem = q;
+    xo += i * p.x_batch_stride[d];
+    yo += i * p.y_batch_stride[d];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) bo[b] = i * p.binary[b].batch_stride[d];
-        --d;
-      }
-      rem = blockIdx.z;
-      bi = blockIdx.z * gridDim.y + blockIdx.y;
-    } else {
-      bi = blockIdx.x / (static_cast<uint32_t>(a.tiles_m) * static_cast<uint32_t>(a.tiles_n));
-      rem = bi;
-    }
-    for (; d >= 0; --d) {
-      const uint32_t dim = static_cast<uint32_t>(p.batch_dims[d]);
-      const uint32_t q = d == 0 ? 0 : rem / dim;   // the outermost index needs no division
-      const int64_t i = rem - q * dim;
-      rem = q;
-      xo += i * p.x_batch_stride[d];
-      yo += i * p.y_batch_stride[d];
-#pragma unroll
-      for (int b = 0; b < NB; ++b) bo[b] += i * p.binary[b].batch_stride[d];
-    }
+    for (int b = 0; b < NB; ++b) bo[b] += i * p.binary[b].batch_stride[d];
   }
   // accumulator e of a lane is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32 of its quadrant
-  bmm_body<ADJ_X, ADJ_Y, VEC_X, VEC_Y, NB, OUT_T, ROWB, RM, RN>(p, x + xo, y + yo, bo, bi, m0, n0, wm, wn, t, lane, out, xs, ys);
+  bmm_body<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, RM, RN>(p, x + xo, y + yo, bo, bi, m0, n0, wm, wn, t, lane, out, xs, ys);
+}
+
+template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB>
+void launch_tiles(const BmmArgs& a, const int8_t* x, const int8_t* y, void* out, dim3 grid, hipStream_t st) {
+  if constexpr (NB == 0 || ROWB) {  // the larger tiles (chosen by the host)
+    if (a.rm == 2 && a.rn == 2) {
+      qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, 2, 2><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+      return;
+    }
+    if (a.rm == 2 && a.rn == 1) {
+      qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, 2, 1><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+      return;
+    }
+  }
+  qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
 }
 
 template <bool ADJ_X, bool ADJ_Y, int NB, int OUT_T, bool ROWB>
 void launch_vec(const BmmArgs& a, const int8_t* x, const int8_t* y, void* out, dim3 grid, hipStream_t st) {
-  if constexpr (NB == 0 || ROWB) {  // the larger tiles (chosen by the host for aligned operands only)
-    if (a.rm == 2 && a.rn == 2) {
-      qbmm_kernel<ADJ_X, ADJ_Y, true, true, NB, OUT_T, ROWB, 2, 2><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
-      return;
-    }
-    if (a.rm == 2 && a.rn == 1) {
-      qbmm_kernel<ADJ_X, ADJ_Y, true, true, NB, OUT_T, ROWB, 2, 1><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
-      return;
-    }
-  }
-  if (a.vec_x && a.vec_y) qbmm_kernel<ADJ_X, ADJ_Y, true, true, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
-  else if (a.vec_x) qbmm_kernel<ADJ_X, ADJ_Y, true, false, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
-  else if (a.vec_y) qbmm_kernel<ADJ_X, ADJ_Y, false, true, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
-  else qbmm_kernel<ADJ_X, ADJ_Y, false, false, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+  if (a.mode == kAligned) launch_tiles<ADJ_X, ADJ_Y, kAligned, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
+  else if (a.mode == kAny) launch_tiles<ADJ_X, ADJ_Y, kAny, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
+  else qbmm_kernel<ADJ_X, ADJ_Y, kBytes, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
 }
 
 template <bool ADJ_X, bool ADJ_Y, int OUT_T>
@@ -465,8 +548,11 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
     --a.p.n_batch_dims;
   }
   // [R, K] layouts load 16 bytes along k, [K, R] layouts 4 bytes along r
-  a.vec_x = p->adj_x ? vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->M, 4) : vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->K, 16);
-  a.vec_y = p->adj_y ? vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->K, 16) : vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->N, 4);
+  const bool vec_x = p->adj_x ? vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->M, 4) : vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->K, 16);
+  const bool vec_y = p->adj_y ? vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->K, 16) : vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->N, 4);
+  // (the loads of kAny stay inside a row of the operand)
+  const bool any = (p->adj_x ? p->M >= 4 : p->K >= 16) && (p->adj_y ? p->K >= 16 : p->N >= 4);
+  a.mode = vec_x && vec_y ? kAligned : any ? kAny : kBytes;
   // Tiles of 128 rows (and 128 columns) where more than 64 exist, the operands are aligned, the fused operands do not
   // depend on the row, and at least 1024 tiles remain (four per CU); else 64 x 64.  BERT-base attention over 128
   // sequences, 1536 tiles: Q.K^T + Mul + Add 24.6 -> 20.0 us, P.V 16.9 -> 14.2 us; over 32 sequences the 384 larger
@@ -474,7 +560,7 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   bool rowb = true;
   for (int b = 0; b < p->n_binary; ++b) rowb = rowb && p->binary[b].stride_m == 0;
   a.rm = a.rn = 1;
-  if (a.vec_x && a.vec_y && rowb && p->M > kTile) {
+  if (a.mode != kBytes && rowb && p->M > kTile) {
     const int rn = p->N > kTile ? 2 : 1;
     if (batch * ((p->M + 2 * kTile - 1) / (2 * kTile)) * ((p->N + rn * kTile - 1) / (rn * kTile)) >= 1024) {
       a.rm = 2;
@@ -486,12 +572,13 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   const int64_t grid = batch * a.tiles_m * a.tiles_n;
   ITEXHIP_REQUIRE(grid < (1LL << 31), "%s: %lld output tiles exceed one launch", who, static_cast<long long>(grid));
   hipStream_t st = as_stream(stream);
-  // (tiles of a matrix, innermost batch dimension, product of the other batch dimensions) when the extents fit a grid
+  // Whole matrices per XCD where there are enough of them to keep all 8 equally busy.
   const int64_t tiles = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
-  const int64_t inner = a.p.n_batch_dims > 0 ? a.p.batch_dims[a.p.n_batch_dims - 1] : 1;
-  a.grid3 = inner <= 65535 && batch / inner <= 65535 ? 1 : 0;
-  const dim3 g = a.grid3 ? dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(inner), static_cast<unsigned>(batch / inner))
-                         : dim3(static_cast<unsigned>(grid));
+  a.batch = static_cast<uint32_t>(batch);
+  a.xcd_grid = (batch % 8 == 0 || batch >= 64) && tiles <= 65535 && (batch + 7) / 8 <= 65535 ? 1 : 0;
+  for (int d = 0; d < a.p.n_batch_dims; ++d) a.by_dim[d] = make_fast_div(a.p.batch_dims[d]);
+  const dim3 g = a.xcd_grid ? dim3(8, static_cast<unsigned>(tiles), static_cast<unsigned>((batch + 7) / 8))
+                            : dim3(static_cast<unsigned>(grid));
   if (p->adj_x && p->adj_y) launch_layout<true, true>(a, x, y, out, g, st);
   else if (p->adj_x) launch_layout<true, false>(a, x, y, out, g, st);
   else if (p->adj_y) launch_layout<false, true>(a, x, y, out, g, st);

@@ -1,0 +1,41 @@
+"""The quantized BatchMatMul where rows are no multiple of a vector load: loads at any byte address, pieces cut by the end of
+a row, 16-bit results stored in pairs at odd addresses, whole matrices per XCD.  Against the CPU oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as orc
+from tests.test_gpu_bmm import check, to16
+
+pytestmark = pytest.mark.gpu
+
+# the shortest operands that take vector loads (K = 16, 4 columns), remainders of the 64-wide tile and of a 16-byte piece,
+# 128-row tiles, batches around a multiple of 8
+SHAPES = [((3,), 4, 16, 4), ((8,), 5, 17, 7), ((9,), 63, 31, 65), ((64,), 65, 79, 33), ((2, 4), 130, 197, 64), ((70,), 33, 16, 35)]
+
+
+@pytest.mark.parametrize("B,M,K,N", SHAPES)
+@pytest.mark.parametrize("adj_x,adj_y", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("t_out", [orc.FLOAT, orc.BFLOAT16, orc.HALF])
+def test_rows_of_any_length(hip, dev, B, M, K, N, adj_x, adj_y, t_out):
+    import torch
+    rng = np.random.default_rng(M + K * 5 + N)
+    x = rng.integers(-128, 128, B + ((K, M) if adj_x else (M, K))).astype(np.int8)
+    y = rng.integers(-128, 128, B + ((N, K) if adj_y else (K, N))).astype(np.int8)
+    add = rng.standard_normal((1,) * len(B) + (1, N)).astype(np.float32)
+    mul = rng.standard_normal(B + (M, 1)).astype(np.float32)
+    binary = [(orc.BIN_MUL, mul), (orc.BIN_ADD, add)]
+    if t_out != orc.FLOAT:
+        binary = [(alg, to16(torch, v, t_out)) for alg, v in binary]
+    check(hip, dev, x, y, adj_x, adj_y, binary[1:], t_out, x_off=3, y_off=1)   # an operand broadcast over the rows
+    check(hip, dev, x, y, adj_x, adj_y, binary, t_out)
+    check(hip, dev, x, y, adj_x, adj_y, (), t_out, x_off=1)
+
+
+@pytest.mark.parametrize("t_out", [orc.FLOAT, orc.BFLOAT16])
+def test_large_tiles(hip, dev, t_out):
+    """At least 1024 tiles of 128 rows: the larger tiles on unaligned operands."""
+    rng = np.random.default_rng(3)
+    x = rng.integers(-128, 128, (520, 131, 37)).astype(np.int8)
+    for n in (3 * 21, 131):
+        y = rng.integers(-128, 128, (520, 37, n)).astype(np.int8)
+        check(hip, dev, x, y, t_out=t_out, y_off=2)
