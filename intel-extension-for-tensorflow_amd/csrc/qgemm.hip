@@ -31,6 +31,11 @@ template <int OUT_T>
 int dispatch_tile_conv(const uint8_t* x, uint32_t a_xor, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
                        void* out, hipStream_t st, const ConvTileArgs& cv);
 
+// the kernel for a short K, many rows and an 8-bit result (qgemm_stream.hip): 1 launched, 0 not a call for it, < 0 the negated
+// status
+int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e, int out_type,
+               void* out, hipStream_t st, const ConvTileArgs* cv);
+
 // the op on operands as TensorFlow stores them, any K (qgemm_unpacked.hip)
 int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
                     const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who);
@@ -513,13 +518,17 @@ static bool small_m(int64_t M, int64_t K, int64_t N) {
   return ((M + 63) / 64) * ((N + 63) / 64) <= 128;             // the tile kernel would leave half of the CUs idle
 }
 
-int launch_packed(bool gemv, const void* a, int a_type, const int8_t* packed_b, int64_t M, int64_t K, int64_t N,
+enum class Path { kTile, kSmallM, kAny };  // kAny: the tile kernel or the one for a short K
+
+static Path pick_path(int64_t M, int64_t K, int64_t N) { return small_m(M, K, N) ? Path::kSmallM : Path::kAny; }
+
+int launch_packed(Path path, const void* a, int a_type, const int8_t* packed_b, int64_t M, int64_t K, int64_t N,
                   const EpilogueArgs& e, int out_type, void* out, void* stream, const char* who) {
   ITEXHIP_REQUIRE(K % 16 == 0, "%s: K must be a multiple of 16 (got %lld); use itexhip_qgemm_naive", who,
                   static_cast<long long>(K));
   ITEXHIP_REQUIRE(aligned(a, 16) && aligned(packed_b, 16), "%s: operands must be 16-byte aligned", who);
   ITEXHIP_REQUIRE(a_type != ITEXHIP_QUINT8 || e.colsum, "%s: quint8 activations need colsum", who);
-  ITEXHIP_REQUIRE(!gemv || M <= kSmallMaxRows, "%s: M must be <= %d", who, kSmallMaxRows);
+  ITEXHIP_REQUIRE(path != Path::kSmallM || M <= kSmallMaxRows, "%s: M must be <= %d", who, kSmallMaxRows);
   ITEXHIP_REQUIRE(M * K < (1LL << 31), "%s: activation matrix too large (M * K must be < 2^31)", who);
   const uint32_t a_xor = (a_type == ITEXHIP_QUINT8) ? 0x80808080u : 0u;
   const uint8_t* ap = reinterpret_cast<const uint8_t*>(a);
@@ -527,7 +536,15 @@ int launch_packed(bool gemv, const void* a, int a_type, const int8_t* packed_b, 
   hipStream_t hs = as_stream(stream);
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
   int st__ = ITEXHIP_OK;
-  if (gemv) {
+  if (path == Path::kAny) {
+    const int rc = try_stream(ap, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, nullptr);
+    if (rc < 0) return -rc;
+    if (rc > 0) {
+      ITEXHIP_CHECK_LAUNCH(who);
+      return ITEXHIP_OK;
+    }
+  }
+  if (path == Path::kSmallM) {
 #define CALL_GEMV(T) dispatch_gemv<T>(ap, a_xor, bp, Mi, Ki, Ni, e, out, hs)
     ITEXHIP_DISPATCH_OUT(out_type, CALL_GEMV)
 #undef CALL_GEMV
@@ -541,13 +558,13 @@ int launch_packed(bool gemv, const void* a, int a_type, const int8_t* packed_b, 
   return ITEXHIP_OK;
 }
 
-int packed_path(bool gemv, const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
+int packed_path(Path path, const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
                 int64_t M, int64_t K, int64_t N, const float* scales, const float* bias,
                 const itexhip_epilogue* ep, int out_type, void* out, void* stream, const char* who,
                 const void* addend = nullptr, int addend_type = 0) {
   if (int st = check_common(a, a_type, packed_b, M, K, N, scales, ep, out_type, out, who, addend, addend_type)) return st;
   if (M == 0 || N == 0) return ITEXHIP_OK;
-  return launch_packed(gemv, a, a_type, packed_b, M, K, N, make_args(a_type, colsum, scales, bias, ep, addend, addend_type),
+  return launch_packed(path, a, a_type, packed_b, M, K, N, make_args(a_type, colsum, scales, bias, ep, addend, addend_type),
                        out_type, out, stream, who);
 }
 
@@ -583,21 +600,21 @@ extern "C" int itexhip_qgemm_prepack_b(const int8_t* w, int transpose_b, int64_t
 extern "C" int itexhip_qgemm_tile(const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
                                   int64_t M, int64_t K, int64_t N, const float* scales, const float* bias,
                                   const itexhip_epilogue* ep, int out_type, void* out, void* stream) {
-  return packed_path(false, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(Path::kTile, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemm_tile");
 }
 
 extern "C" int itexhip_qgemv(const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
                              int64_t M, int64_t K, int64_t N, const float* scales, const float* bias,
                              const itexhip_epilogue* ep, int out_type, void* out, void* stream) {
-  return packed_path(true, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(Path::kSmallM, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemv");
 }
 
 extern "C" int itexhip_qgemm(const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
                              int64_t M, int64_t K, int64_t N, const float* scales, const float* bias,
                              const itexhip_epilogue* ep, int out_type, void* out, void* stream) {
-  return packed_path(small_m(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(pick_path(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemm");
 }
 
@@ -606,7 +623,7 @@ extern "C" int itexhip_qgemm_sum(const void* a, int a_type, const int8_t* packed
                                  const itexhip_epilogue* ep, const void* addend, int addend_type, int out_type, void* out,
                                  void* stream) {
   ITEXHIP_REQUIRE(addend != nullptr || M == 0 || N == 0, "itexhip_qgemm_sum: null addend");
-  return packed_path(small_m(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(pick_path(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemm_sum", addend, addend_type);
 }
 
@@ -672,7 +689,12 @@ int qconv2d_impl(const char* who, const void* x, int x_type, const itexhip_conv_
   const uint8_t* bp = reinterpret_cast<const uint8_t*>(packed_filter);
   hipStream_t hs = as_stream(stream);
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
-  int st__ = ITEXHIP_OK;
+  int st__ = try_stream(xp, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, &cv);
+  if (st__ < 0) return -st__;
+  if (st__ > 0) {
+    ITEXHIP_CHECK_LAUNCH(who);
+    return ITEXHIP_OK;
+  }
   switch (out_type) {
     case ITEXHIP_FLOAT: st__ = dispatch_tile_conv<ITEXHIP_FLOAT>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
     case ITEXHIP_BFLOAT16: st__ = dispatch_tile_conv<ITEXHIP_BFLOAT16>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
@@ -766,7 +788,7 @@ int qmatmul_impl(const char* who, const itexhip_matmul_params* p, const void* a,
   e.range_a = range_a;
   e.addend = addend;
   e.addend_type = is_float16_type(p->t_out) ? p->t_out : ITEXHIP_FLOAT;  // the addend has the output's type
-  return launch_packed(small_m(M, K, N), a, p->t_in, packed_b, M, K, N, e, p->t_out, out, stream, who);
+  return launch_packed(pick_path(M, K, N), a, p->t_in, packed_b, M, K, N, e, p->t_out, out, stream, who);
 }
 }  // namespace
 

@@ -1,0 +1,366 @@
+// Quantized MatMul and Conv2D with a short K, many rows and an 8-bit result: the 1 x 1 and first convolutions of vision
+// networks, pointwise convolutions, narrow linears.  Such a launch is bound by the bytes of its activations, result and
+// residual, and by the instructions of its epilogue; the tile kernel spends it on three K steps of loads that a K of 64
+// does not have, on barriers and on a transposition of the result through LDS.
+//
+// Here the weight of a workgroup's channels (K x 64 per wavefront column) and their parameters are put into LDS once, and
+// the wavefronts then walk the rows without another barrier.  A wavefront takes 32 rows x 64 channels at a time: its
+// activation fragments come straight from global memory (a lane loads 16 consecutive k of one row; a convolution resolves
+// the window position per 16-byte piece), a group of them ahead of the MFMAs that use them.  The weight is the first MFMA
+// operand and its channels are put into LDS in an order that leaves a lane with 16 consecutive channels of one row: the
+// result is packed in registers and goes out as 16-byte stores, and a residual comes in as 16-byte loads a tile ahead.
+//
+// Measured, tile kernel -> this one, us: 401408 x 32 -> 64 with a clip 18.4 -> 10.9; 100352 x 64 -> 256 with a residual and
+// a ReLU 24.3 -> 15.5; 7 x 7 convolution over 32 x 224 x 224, stride 2, 224 bytes of patch -> 64 channels 30.1 -> 16.0.
+// What bounds it there: about half of the time is vector instructions (9 per result with a residual), the rest the start
+// of the launch (parameters and weight on their way to LDS, 3 us) and the results leaving L2.
+#include "qgemm_common.hpp"
+
+namespace itexhip {
+namespace {
+
+constexpr int kMaxWeightBytes = 72 * 1024;  // of a workgroup: two of them per CU
+constexpr int kForceStream = 16;            // of itexhip_test_force_tile_shape
+constexpr int kBlocks = 2;                  // 32-channel blocks per wavefront (the stores are laid out for two)
+
+struct StreamArgs {
+  int M, K, N;
+  int chunks;       // 32-deep K chunks that hold data
+  int packed_kt;    // K chunks of the packed weight (K padded to a multiple of 64)
+  FastDiv by_chunks;
+  int waves_n;      // wavefronts side by side along N: 1, 2 or 4
+  int tiles;        // row tiles of 32
+  int walkers;      // wavefronts that share them (per wavefront column)
+  uint64_t share;   // 2^24 * tiles / walkers: wavefront w takes the tiles from (w * share) >> 24 on
+  int padded;       // convolution: a window may reach into the padding
+  float lo, hi;     // post-op bounds, see POST
+  float sum_scale;
+};
+
+static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
+
+// What follows scale and bias: nothing (saturation does it), max(v, 0), or min(max(v, lo), hi).
+enum : int { kPostNone = 0, kPostRelu = 1, kPostClip = 2 };
+
+// 4 values -> 4 bytes.  v_cvt_pk_u8_f32 rounds to nearest even, saturates to 0 .. 255 and puts the byte into place in one
+// instruction: for every fp32 value but NaN the byte that clamp, magic-number add and permute give (compared over all 2^32
+// patterns on the device); a value that may be NaN is clamped first, as there.
+template <int OUT_T, int POST>
+__device__ __forceinline__ uint32_t pack_bytes(const float (&v)[4]) {
+  if constexpr (OUT_T == ITEXHIP_QUINT8) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      w = __builtin_amdgcn_cvt_pk_u8_f32(POST == kPostNone ? __builtin_amdgcn_fmed3f(v[i], 0.0f, 255.0f) : v[i], i, w);
+    return w;
+  } else {
+    return static_cast<uint32_t>(epilogue_pack<OUT_T>(v4i{__float_as_int(v[0]), __float_as_int(v[1]), __float_as_int(v[2]), __float_as_int(v[3])}).x);
+  }
+}
+
+template <int OUT_T, int POST, int SUM, int GROUP, bool CONV>
+__global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __restrict__ a, uint32_t amask,
+                                                            const uint8_t* __restrict__ bp, const StreamArgs s, EpilogueArgs e,
+                                                            uint8_t* __restrict__ out, const ConvTileArgs cv) {
+  extern __shared__ __align__(16) uint8_t lds[];  // [waves_n * kBlocks][chunks] fragments, parameters, window table
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lrow = lane & 31, half = lane >> 5;
+  const int channels = s.waves_n * kBlocks * 32;            // of this workgroup
+  const int n_base = blockIdx.y * channels;
+  const int frags = s.waves_n * kBlocks * s.chunks;
+  int* const p_comp = reinterpret_cast<int*>(lds + frags * kChunkBytes);
+  float* const p_scale = reinterpret_cast<float*>(p_comp + channels);
+  float* const p_bias = p_scale + channels;
+  int2* const table = reinterpret_cast<int2*>(p_bias + channels);  // convolution: per 16-byte piece of a patch row
+
+  const int wn = wave % s.waves_n, wm = wave / s.waves_n, waves_m = 4 / s.waves_n;
+  // consecutive workgroup ids go round the 8 XCDs: each of them walks a contiguous range of rows (neighbouring rows of a
+  // convolution read the same input); gridDim.x is a multiple of 8
+  const int wg = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int walker = wg * waves_m + wm;
+  const int t0 = static_cast<int>((walker * s.share) >> 24);
+  const int t1 = walker >= s.walkers ? 0 : walker + 1 == s.walkers ? s.tiles : static_cast<int>(((walker + 1) * s.share) >> 24);
+  const int klast = s.K - 16, plast = (s.K >> 4) - 1;
+
+  // ---- where the lane's row of a tile begins
+  uint32_t row_off;
+  int win_h = 0, win_w = 0;
+  auto locate = [&](int tile) {
+    const int m = min(tile * 32 + lrow, s.M - 1);
+    if constexpr (CONV) {
+      const int t = fast_div(m, cv.by_out_w), ow = m - t * cv.out_w;
+      const int b = fast_div(t, cv.by_out_h), oh = t - b * cv.out_h;
+      win_h = oh * cv.stride_h - cv.pad_top;
+      win_w = ow * cv.stride_w - cv.pad_left;
+      row_off = static_cast<uint32_t>(((b * cv.in_h + win_h) * cv.in_w + win_w) * cv.in_c);
+    } else {
+      row_off = static_cast<uint32_t>(m) * static_cast<uint32_t>(s.K);  // M * K < 2^31 checked by the host
+    }
+  };
+  auto window_piece = [&](int p) {  // {window row << 16 | window column, byte offset from the window's origin}
+    const int k0 = p * 16;
+    const int kk = fast_div(k0, cv.by_in_c), cc = k0 - kk * cv.in_c;
+    const int kh = fast_div(kk, cv.by_k_w), kw = kk - kh * cv.k_w;
+    const int dh = kh * cv.dil_h, dw = kw * cv.dil_w;  // < 2^15 each, checked by the host
+    return make_int2((dh << 16) | dw, (dh * cv.in_w + dw) * cv.in_c + cc);
+  };
+  auto load_piece = [&](const int2 piece) -> v4i {
+    const uint8_t* src = a + (row_off + static_cast<uint32_t>(piece.y));
+    if (s.padded) {  // a position in the padding reads 16 zero bytes
+      const int ih = win_h + (piece.x >> 16), iw = win_w + (piece.x & 0xffff);
+      const bool inside = static_cast<unsigned>(ih) < static_cast<unsigned>(cv.in_h) &&
+                          static_cast<unsigned>(iw) < static_cast<unsigned>(cv.in_w);
+      src = inside ? src : reinterpret_cast<const uint8_t*>(kZeros);
+    }
+    return *reinterpret_cast<const v4i*>(src);
+  };
+  // fragment of chunk c: k beyond K meets zero weights, any bytes of the tensor will do there
+  auto load = [&](int c) -> v4i {
+    if constexpr (CONV) return load_piece(table[min(c * 2 + half, plast)]);
+    else return *reinterpret_cast<const v4i*>(a + (row_off + static_cast<uint32_t>(min(c * 32 + half * 16, klast))));
+  };
+
+  // ---- the first fragments travel while the weight is put into LDS (without the window table, which is not there yet)
+  v4i cur[GROUP], nxt[GROUP];
+  locate(t0);  // (a wavefront without rows reads the last row)
+#pragma unroll
+  for (int u = 0; u < GROUP; ++u) {
+    const int c = min(u, s.chunks - 1);
+    if constexpr (CONV) cur[u] = load_piece(window_piece(min(c * 2 + half, plast)));
+    else cur[u] = load(c);
+  }
+
+  // the residual of a tile: 16 consecutive channels per block of the lane's row
+  typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
+  const int n0 = n_base + wn * (kBlocks * 32);
+  v4i add[kBlocks], add_nxt[kBlocks];
+  auto load_add = [&](int tile, v4i (&d)[kBlocks]) {
+    if constexpr (SUM != 0) {
+      const uint32_t o = static_cast<uint32_t>(min(tile * 32 + lrow, s.M - 1)) * static_cast<uint32_t>(s.N);
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b)  // (channels past N: the row's last 16, not used)
+        d[b] = *reinterpret_cast<const v4i_a4*>(static_cast<const uint8_t*>(e.addend) + (o + min(n0 + b * 32 + half * 16, s.N - 16)));
+    }
+  };
+  load_add(t0, add);
+
+  // ---- the weight: row r of a fragment holds channel (r / 4 % 2) * 16 + (r / 8) * 4 + r % 4 of its block, so that the 16
+  // results of a lane (rows (i / 4) * 8 + half * 4 + i % 4) are channels half * 16 .. half * 16 + 15.  Direct global -> LDS
+  // loads (lane l's 16 bytes land at 16 l): all of them are in flight at once, where a loop over registers waits for each.
+  {
+    const int ch = ((lrow >> 2) & 1) * 16 + (lrow >> 3) * 4 + (lrow & 3);
+    const int last_nt = ((s.N + 31) >> 5) - 1;
+    for (int f = wave; f < frags; f += 4) {
+      const int block = fast_div(f, s.by_chunks), c = f - block * s.chunks;
+      const int nt = min((n_base >> 5) + block, last_nt);  // blocks past N: any weights, their results are not stored
+      const uint8_t* src = bp + (static_cast<int64_t>(nt) * s.packed_kt + c) * kChunkBytes + ((lane & 32) + ch) * 16;
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(lds + f * kChunkBytes), 16, 0, 0);
+    }
+  }
+  for (int i = threadIdx.x; i < channels; i += 256) {
+    int comp;
+    float scale, bias;
+    resolve_channel(e, min(n_base + i, s.N - 1), s.N, &comp, &scale, &bias);
+    p_comp[i] = comp;
+    p_scale[i] = scale;
+    p_bias[i] = bias;
+  }
+  if constexpr (CONV) {
+    for (int p = threadIdx.x; p < (s.K >> 4); p += 256) table[p] = window_piece(p);
+  }
+  wait_vmcnt<0>();  // the direct loads of this wavefront have landed
+  __syncthreads();
+
+  if (n0 >= s.N || t0 >= t1) return;  // whole wavefront; no barrier follows
+  const uint8_t* const wfrag = lds + wn * kBlocks * s.chunks * kChunkBytes + lane * 16;
+  const int groups = (s.chunks + GROUP - 1) / GROUP;
+  // Rows that a wavefront writes whole are contiguous in memory and go out as streaming stores, ahead of the flush of L2 at
+  // the end of the kernel (401408 x 32 -> 64: 12.2 -> 10.9 us); of longer rows it writes 64 bytes here and there, which L2
+  // has to put together first (100352 x 64 -> 256 with the residual: 18.8 us streaming, 15.5 us plain).
+  const bool stream_out = s.N <= kBlocks * 32;
+  for (int tile = t0; tile < t1; ++tile) {
+    if (tile + 1 < t1) load_add(tile + 1, add_nxt);  // a whole tile ahead: these come from memory
+    // the lane's channels in the parameter panels, hidden from the compiler: it would keep all 96 parameters of a lane in
+    // registers across the loop and spill
+    int col0 = wn * kBlocks * 32 + half * 16;
+    asm volatile("" : "+v"(col0));
+    v16i acc[kBlocks];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4i c = *reinterpret_cast<const v4i*>(p_comp + col0 + b * 32 + g * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[b][g * 4 + r] = c[r];
+      }
+    for (int g = 0; g < groups; ++g) {
+      // the next group (of this tile, or the first of the next one) travels under this group's MFMAs
+      if (g + 1 < groups) {
+#pragma unroll
+        for (int u = 0; u < GROUP; ++u) nxt[u] = load(min((g + 1) * GROUP + u, s.chunks - 1));
+      } else if (tile + 1 < t1) {
+        locate(tile + 1);
+#pragma unroll
+        for (int u = 0; u < GROUP; ++u) nxt[u] = load(min(u, s.chunks - 1));
+      }
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) {
+        const int c = g * GROUP + u;
+        if (c < s.chunks) {  // wavefront uniform
+          v4i x = cur[u];
+          x.x ^= amask; x.y ^= amask; x.z ^= amask; x.w ^= amask;
+#pragma unroll
+          for (int b = 0; b < kBlocks; ++b)
+            acc[b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i*>(wfrag + (b * s.chunks + c) * kChunkBytes), x, acc[b], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < GROUP; ++u) cur[u] = nxt[u];
+    }
+    v4i packed[kBlocks];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = col0 + b * 32 + g * 4;
+        const f4 sc = *reinterpret_cast<const f4*>(p_scale + col);
+        const f4 bi = *reinterpret_cast<const f4*>(p_bias + col);
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = static_cast<float>(acc[b][g * 4 + r]) * sc[r];
+          v[r] = v[r] + bi[r];
+          if constexpr (SUM == 1) v[r] = v[r] + s.sum_scale * static_cast<float>((static_cast<uint32_t>(add[b][g]) >> (8 * r)) & 0xffu);
+          if constexpr (SUM == 2) v[r] = v[r] + s.sum_scale * static_cast<float>((add[b][g] << (24 - 8 * r)) >> 24);
+          if constexpr (POST == kPostRelu && OUT_T != ITEXHIP_QUINT8) v[r] = fmaxf(v[r], 0.0f);
+          if constexpr (POST == kPostClip) v[r] = fminf(fmaxf(v[r], s.lo), s.hi);
+        }
+        packed[b][g] = static_cast<int>(pack_bytes<OUT_T, POST>(v));
+      }
+    }
+    // A lane holds pieces (16 channels) `half` and 2 + half of its row.  Rows 16 .. 31 of the first trade places with rows
+    // 0 .. 15 of the second: then a store covers the 64 bytes of 16 rows instead of 32 bytes of 32 rows.
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const auto t = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(packed[0][g]), static_cast<uint32_t>(packed[1][g]), false, false);
+      packed[0][g] = static_cast<int>(t[0]);
+      packed[1][g] = static_cast<int>(t[1]);
+    }
+    const int n = n0 + (half + 2 * (lrow >> 4)) * 16;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int m = tile * 32 + b * 16 + (lrow & 15);
+      v4i* const dst = reinterpret_cast<v4i*>(out + (static_cast<uint32_t>(m) * static_cast<uint32_t>(s.N) + static_cast<uint32_t>(n)));
+      if (m < s.M && n < s.N) {
+        if (stream_out) __builtin_nontemporal_store(packed[b], dst);
+        else *dst = packed[b];
+      }
+    }
+    if constexpr (SUM != 0) {
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) add[b] = add_nxt[b];
+    }
+  }
+}
+
+template <int OUT_T, int POST, int SUM, int GROUP, bool CONV>
+int launch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs& s, const EpilogueArgs& e, uint8_t* out,
+           const ConvTileArgs& cv, dim3 grid, size_t lds, hipStream_t st) {
+  auto kern = qgemm_stream_kernel<OUT_T, POST, SUM, GROUP, CONV>;
+  static unsigned long long attr_done = 0;  // devices on which this instantiation's attribute is set
+  if (!device_bit(&attr_done, false)) {
+    hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qgemm_stream_kernel)");
+    device_bit(&attr_done, true);
+  }
+  kern<<<grid, 256, lds, st>>>(a, amask, bp, s, e, out, cv);
+  return ITEXHIP_OK;
+}
+
+template <int OUT_T, int GROUP, bool CONV>
+int dispatch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs& s, int post, const EpilogueArgs& e, uint8_t* out,
+             const ConvTileArgs& cv, dim3 grid, size_t lds, hipStream_t st) {
+  const int sum = !e.addend ? 0 : e.addend_type == ITEXHIP_QUINT8 ? 1 : 2;
+#define STREAM(P, S) return launch<OUT_T, P, S, GROUP, CONV>(a, amask, bp, s, e, out, cv, grid, lds, st)
+  switch (post * 3 + sum) {
+    case kPostNone * 3: STREAM(kPostNone, 0);
+    case kPostNone * 3 + 1: STREAM(kPostNone, 1);
+    case kPostNone * 3 + 2: STREAM(kPostNone, 2);
+    case kPostRelu * 3: STREAM(kPostRelu, 0);
+    case kPostRelu * 3 + 1: STREAM(kPostRelu, 1);
+    case kPostRelu * 3 + 2: STREAM(kPostRelu, 2);
+    case kPostClip * 3: STREAM(kPostClip, 0);
+    case kPostClip * 3 + 1: STREAM(kPostClip, 1);
+    default: STREAM(kPostClip, 2);
+  }
+#undef STREAM
+}
+
+}  // namespace
+
+// 1: the call was launched here; 0: not a call for this kernel; < 0: an error (the status, negated).
+int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e, int out_type,
+               void* out, hipStream_t st, const ConvTileArgs* cv) {
+  if (out_type != ITEXHIP_QUINT8 && out_type != ITEXHIP_QINT8) return 0;
+  const int forced = __atomic_load_n(&g_forced_tile_shape[cv ? 1 : 0], __ATOMIC_RELAXED);  // tests ask for a tile shape, or
+  if (forced >= 0 && forced != kForceStream) return 0;                                     // for this kernel at any size
+  if (K % 16 != 0 || K < 16 || N % 16 != 0 || (e.bias == nullptr && !e.fused) || !aligned(out, 16) || e.row_min_a) return 0;
+  if (static_cast<int64_t>(M) * N >= (1LL << 31)) return 0;
+  CanonChain c;
+  const int act = canon_chain(e, &c);
+  if (act < 0 || act > 2 || (c.flags & ~(kChainMax0 | kChainClip | kChainSumFirst)) != 0) return 0;
+  if (e.addend && (!(c.flags & kChainSumFirst) || (e.addend_type != ITEXHIP_QUINT8 && e.addend_type != ITEXHIP_QINT8) ||
+                   !aligned(e.addend, 4)))
+    return 0;
+  StreamArgs s{};
+  s.M = M; s.K = K; s.N = N;
+  s.chunks = (K + 31) / 32;
+  s.by_chunks = make_fast_div(s.chunks);
+  s.packed_kt = 2 * ((K + 63) / 64);
+  const int cols = (N + kBlocks * 32 - 1) / (kBlocks * 32);  // wavefront columns
+  s.waves_n = cols >= 4 ? 4 : cols >= 2 ? 2 : 1;
+  while (s.waves_n > 1 && s.waves_n * kBlocks * s.chunks * kChunkBytes > kMaxWeightBytes) s.waves_n >>= 1;
+  const int weight = s.waves_n * kBlocks * s.chunks * kChunkBytes;
+  if (weight > kMaxWeightBytes) return 0;
+  s.tiles = (M + 31) / 32;
+  // Where it is the faster kernel, by what fills the device: `rounds` is how often the 32 x 64 pieces of the result go into
+  // the 4096 wavefronts that run at once (in quarters).  Below one round a launch is its start, and the tile kernel starts
+  // sooner; with a long K the MFMAs and the weight fragments read from LDS for every 32 rows count, and the tile kernel
+  // reads them for 64 - 256.  Tile kernel / this kernel, time, at 0.77, 1.5, 3 and 6 rounds:
+  //   K <= 64                0.86 - 1.24, 1.03 - 1.58, 1.03 - 1.18, 1.39 - 1.43     with a residual 1.36 - 1.73 everywhere
+  //   64 < K <= 512          0.82 - 0.87, 0.75 - 0.89, 0.96 - 1.08, 1.14 - 1.31     K no multiple of 64: 0.89, 1.01 - 1.18, ...
+  //   K = 768, 1024          0.85,        0.68,        -,           0.91 - 1.09
+  //   convolution, K <= 400  1.13 - 1.24, 1.27,        1.29,        -               K = 576: 0.90 - 1.09, K = 1152: 0.87 - 0.94
+  const int64_t quarter_rounds = static_cast<int64_t>(s.tiles) * cols / 1024;
+  const bool small_k = K <= 64 || (e.addend && K <= 128);
+  const int64_t at_least = cv ? (K <= 448 ? 3 : -1) : small_k ? (e.addend ? 3 : 4) : K > 512 ? -1 : K % 64 != 0 ? 6 : 16;
+  if (forced != kForceStream && (at_least < 0 || quarter_rounds < at_least)) return 0;
+  s.padded = cv && (cv->pad_top > 0 || cv->pad_left > 0 ||
+                    (cv->out_h - 1) * cv->stride_h + (K / (cv->k_w * cv->in_c) - 1) * cv->dil_h >= cv->in_h ||
+                    (cv->out_w - 1) * cv->stride_w + (cv->k_w - 1) * cv->dil_w >= cv->in_w);
+  const size_t lds = static_cast<size_t>(weight) + 12 * s.waves_n * kBlocks * 32 + (cv ? (K >> 4) * 8 : 0);
+  const int per_cu = std::min<int>(4, 160 * 1024 / static_cast<int>(lds));  // 128 registers: four wavefronts per SIMD
+  const int groups_n = (cols + s.waves_n - 1) / s.waves_n;
+  const int waves_m = 4 / s.waves_n;
+  s.walkers = std::min(s.tiles, std::max(1, 256 * per_cu / groups_n) * waves_m);
+  s.share = (static_cast<uint64_t>(s.tiles) << 24) / s.walkers;
+  const int wgs = (s.walkers + waves_m - 1) / waves_m;
+  const dim3 grid(static_cast<unsigned>((wgs + 7) / 8 * 8), static_cast<unsigned>(groups_n));
+  s.lo = c.lo; s.hi = c.hi; s.sum_scale = c.sum_scale;
+  const int post = c.flags & kChainClip ? kPostClip : c.flags & kChainMax0 ? kPostRelu : kPostNone;
+  uint8_t* o = static_cast<uint8_t*>(out);
+  int rc;
+  const bool u8 = out_type == ITEXHIP_QUINT8;
+  if (cv) rc = u8 ? dispatch<ITEXHIP_QUINT8, 4, true>(a, amask, bp, s, post, e, o, *cv, grid, lds, st)
+                  : dispatch<ITEXHIP_QINT8, 4, true>(a, amask, bp, s, post, e, o, *cv, grid, lds, st);
+  else if (s.chunks <= 1) rc = u8 ? dispatch<ITEXHIP_QUINT8, 1, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
+                                  : dispatch<ITEXHIP_QINT8, 1, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
+  else if (s.chunks <= 2) rc = u8 ? dispatch<ITEXHIP_QUINT8, 2, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
+                                  : dispatch<ITEXHIP_QINT8, 2, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
+  else rc = u8 ? dispatch<ITEXHIP_QUINT8, 4, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
+               : dispatch<ITEXHIP_QINT8, 4, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
+  return rc == ITEXHIP_OK ? 1 : -rc;
+}
+
+}  // namespace itexhip
