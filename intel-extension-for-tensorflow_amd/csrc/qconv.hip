@@ -1,8 +1,9 @@
 // Device helpers of the quantized Conv2D ops (itex/core/kernels/common/quantized_conv_ops.h): the patch
 // matrix that turns the convolution into the quantized GEMM of qgemm.hip, and the bias scaling.
 #include <algorithm>
+#include <cmath>
 
-#include "common.hpp"
+#include "qgemm_common.hpp"
 
 namespace itexhip {
 namespace {
@@ -218,6 +219,8 @@ struct DepthwiseArgs {
   // uniform branches; a loop over the chain with a switch per value costs more instruction fetch than arithmetic
   int chain;                 // bit 0 max(x, 0), 1 leaky, 2 clip, 3 linear
   float alpha, lo, hi, lin_a, lin_b;
+  int cols, strips;          // 3x3 kernel: column groups of a row, strips of output rows of an image
+  FastDiv by_groups, by_cols, by_strips;
 };
 
 template <int OUT_T>
@@ -276,116 +279,175 @@ __global__ __launch_bounds__(256) void qdwconv_kernel(const DepthwiseArgs a, con
   }
 }
 
-// The common case - 3x3 window, stride 1, dilation 1, multiplier 1, channels a multiple of 4 - with the window
-// unrolled and 32-bit index arithmetic: a thread owns 4 consecutive channels of a column of R = 4 output rows, so it
-// loads each input dword once for up to 3 of its outputs (18 input + 9 filter dwords for 16 outputs), and a wavefront's
-// loads cover 256 contiguous bytes (consecutive lanes = consecutive channel groups, then consecutive columns).
-template <int OUT_T, bool X_SIGNED>
-__global__ __launch_bounds__(256) void qdwconv3x3_kernel(const DepthwiseArgs a, const uint8_t* __restrict__ x,
+// The common case - 3x3 window, stride 1 or 2 in both directions, dilation 1, multiplier 1, channels a multiple of 4.  A
+// thread owns 4 consecutive channels of R = 4 output rows and, with stride 1, two output columns.  The three taps of a window
+// row are one 4-byte dot product: the pixels of an input row (4 with stride 1, 3 with stride 2; a dword of 4 channels each)
+// are transposed to a dword of pixels per channel, 8 or 6 byte permutes, which serves every output row that reads this input
+// row and, with stride 1, both columns (the second with the weights a byte further on).  Unsigned input is fed as x - 128
+// and 128 * (sum of the weights) added back, in the padding too.  A multiply-add per tap and channel on bytes extracted one
+// by one came to 45 vector instructions per output and was bound by them; now 19, still most of the time: 32 x 112 x 112 x 32
+// 17.3 -> 11.4 us; stride 2, which had one thread per output dword and 64-bit divisions, 17.0 -> 6.4 us.
+// BOUNDS: an 8-bit result and a chain that is nothing, a ReLU or a clip, all of them min(max(v, lo), hi) there (no branch per
+// value; a missing bias adds +0, whose sign an integer does not keep).
+template <int OUT_T, bool X_SIGNED, int S, bool BOUNDS>
+__global__ __launch_bounds__(256, 7) void qdwconv3x3_kernel(const DepthwiseArgs a, const uint8_t* __restrict__ x,
                                                          const int8_t* __restrict__ w, const float* __restrict__ scales,
                                                          const float* __restrict__ bias, void* __restrict__ out) {
-  constexpr int R = 4;
-  const uint32_t row_items = static_cast<uint32_t>(a.out_w) * a.groups4;  // (column, channel group) pairs of one output row
-  const uint32_t strips = (a.out_h + R - 1) / R;
-  const uint32_t total = static_cast<uint32_t>(a.total);                  // batch * strips * row_items, < 2^31 (host)
-  const uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const uint32_t t = i / row_items, item = i - t * row_items;
-    const uint32_t b = t / strips, strip = t - b * strips;
-    const int ow = static_cast<int>(item / a.groups4);
-    const int oc0 = static_cast<int>(item - ow * a.groups4) * 4;
-    const int oh0 = static_cast<int>(strip) * R;
-    int acc[R][4];
+  constexpr int R = 4, CW = S == 1 ? 2 : 1, PIX = S == 1 ? 4 : 3, IR = (R - 1) * S + 3;
+  // consecutive workgroup ids go round the 8 XCDs: each takes a contiguous range, neighbours share input rows (the grid is a
+  // multiple of 8)
+  const uint32_t wg = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t i = wg * 256u + threadIdx.x;
+  if (i >= static_cast<uint32_t>(a.total)) return;  // batch * strips * columns / CW * channel groups, < 2^31 (host)
+  const int t0 = fast_div(static_cast<int>(i), a.by_groups), oc0 = (static_cast<int>(i) - t0 * a.groups4) * 4;
+  const int t1 = fast_div(t0, a.by_cols), ow0 = (t0 - t1 * a.cols) * CW;
+  const int b = fast_div(t1, a.by_strips), oh0 = (t1 - b * a.strips) * R;
+  const int ih0 = oh0 * S - a.pad_top, iw0 = ow0 * S - a.pad_left;
+
+  // ---- the input, all loads unconditional from clamped (valid) positions
+  const uint32_t base = static_cast<uint32_t>(b) * static_cast<uint32_t>(a.in_h * a.in_w * a.in_c) + static_cast<uint32_t>(oc0);
+  uint32_t xin[IR][PIX], col_off[PIX];  // input bytes < 2^31 (host)
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+  for (int p = 0; p < PIX; ++p) col_off[p] = base + static_cast<uint32_t>(min(max(iw0 + p, 0), a.in_w - 1) * a.in_c);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[r][c] = 0;
-    const uint8_t* xb = x + static_cast<uint32_t>(b) * static_cast<uint32_t>(a.in_h * a.in_w * a.in_c) + oc0;  // input bytes < 2^31 (host)
-    // All 18 input dwords are loaded unconditionally from clamped (valid) positions and zeroed afterwards where the
-    // position lies in the padding: a branch around each load would make every load wait for the one before it.
-    uint32_t xin[3][R + 2];
+  for (int r = 0; r < IR; ++r) {
+    const uint32_t row_off = static_cast<uint32_t>(min(max(ih0 + r, 0), a.in_h - 1) * a.in_w) * static_cast<uint32_t>(a.in_c);
 #pragma unroll
-    for (int kw = 0; kw < 3; ++kw) {
-      const int iw = ow - a.pad_left + kw;
-      const int iwc = min(max(iw, 0), a.in_w - 1);
+    for (int p = 0; p < PIX; ++p) xin[r][p] = *reinterpret_cast<const uint32_t*>(x + (row_off + col_off[p]));
+  }
+  uint32_t win[9];
 #pragma unroll
-      for (int rr = 0; rr < R + 2; ++rr) {
-        const int ih = oh0 - a.pad_top + rr;
-        const int ihc = min(max(ih, 0), a.in_h - 1);
-        xin[kw][rr] = *reinterpret_cast<const uint32_t*>(xb + (ihc * a.in_w + iwc) * a.in_c);
-      }
+  for (int k = 0; k < 9; ++k) win[k] = *reinterpret_cast<const uint32_t*>(w + k * a.out_c + oc0);
+  float sc[4], bi[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    sc[c] = a.n_scales == 0 ? 1.0f : scales[a.n_scales == 1 ? 0 : oc0 + c];
+    bi[c] = bias ? bias[oc0 + c] : 0.0f;
+  }
+
+  // ---- weights: per window row and channel {w0, w1, w2, 0}
+  uint32_t wt[3][4];
+  int acc[R][CW][4], comp[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int kh = 0; kh < 3; ++kh) {
+    const uint32_t lo = __builtin_amdgcn_perm(win[kh * 3 + 1], win[kh * 3], 0x05010400u);  // w0.b0 w1.b0 w0.b1 w1.b1
+    const uint32_t hi = __builtin_amdgcn_perm(win[kh * 3 + 1], win[kh * 3], 0x07030602u);
+    const uint32_t w2 = win[kh * 3 + 2];
+    wt[kh][0] = __builtin_amdgcn_perm(w2, lo, 0x0c040100u);  // selector 0x0c: a zero byte
+    wt[kh][1] = __builtin_amdgcn_perm(w2, lo, 0x0c050302u);
+    wt[kh][2] = __builtin_amdgcn_perm(w2, hi, 0x0c060100u);
+    wt[kh][3] = __builtin_amdgcn_perm(w2, hi, 0x0c070302u);
+    if constexpr (!X_SIGNED) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) comp[c] = __builtin_amdgcn_sdot4(static_cast<int>(wt[kh][c]), 0x01010101, comp[c], false);
     }
+  }
 #pragma unroll
-    for (int kw = 0; kw < 3; ++kw) {
-      const int iw = ow - a.pad_left + kw;
-      const bool col_ok = iw >= 0 && iw < a.in_w;
-      uint32_t wv[3];
+  for (int c = 0; c < 4; ++c) comp[c] *= 128;
+
+  // ---- zeros where the position lies in the padding (only the wavefronts at the border look)
+  const bool border = ih0 < 0 || iw0 < 0 || ih0 + IR > a.in_h || iw0 + PIX > a.in_w;
+  if (__builtin_amdgcn_ballot_w64(border) != 0) {
 #pragma unroll
-      for (int kh = 0; kh < 3; ++kh) wv[kh] = *reinterpret_cast<const uint32_t*>(w + (kh * 3 + kw) * a.out_c + oc0);
+    for (int r = 0; r < IR; ++r) {
+      const bool row_ok = static_cast<unsigned>(ih0 + r) < static_cast<unsigned>(a.in_h);
 #pragma unroll
-      for (int rr = 0; rr < R + 2; ++rr) {  // input rows oh0 - pad_top + rr feed output rows rr - kh
-        const int ih = oh0 - a.pad_top + rr;
-        const uint32_t xv = (col_ok && ih >= 0 && ih < a.in_h) ? xin[kw][rr] : 0u;
-        int xs[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          xs[c] = X_SIGNED ? (static_cast<int>(xv << (24 - 8 * c)) >> 24) : static_cast<int>((xv >> (8 * c)) & 0xffu);
-#pragma unroll
-        for (int kh = 0; kh < 3; ++kh) {
-          const int r = rr - kh;
-          if (r < 0 || r >= R) continue;
-#pragma unroll
-          for (int c = 0; c < 4; ++c)  // 8-bit factors: the 24-bit multiply-add is exact and full rate (a 32-bit multiply is not)
-            acc[r][c] = __mul24(xs[c], static_cast<int>(wv[kh] << (24 - 8 * c)) >> 24) + acc[r][c];
-        }
-      }
+      for (int p = 0; p < PIX; ++p)
+        if (!row_ok || static_cast<unsigned>(iw0 + p) >= static_cast<unsigned>(a.in_w)) xin[r][p] = 0;
     }
-    float sc[4], bi[4];
+  }
+#pragma unroll
+  for (int r = 0; r < IR; ++r) {
+    uint32_t t[4];
+    const uint32_t lo = __builtin_amdgcn_perm(xin[r][1], xin[r][0], 0x05010400u);
+    const uint32_t hi = __builtin_amdgcn_perm(xin[r][1], xin[r][0], 0x07030602u);
+    if constexpr (PIX == 4) {
+      const uint32_t lo23 = __builtin_amdgcn_perm(xin[r][3], xin[r][2], 0x05010400u);
+      const uint32_t hi23 = __builtin_amdgcn_perm(xin[r][3], xin[r][2], 0x07030602u);
+      t[0] = __builtin_amdgcn_perm(lo23, lo, 0x05040100u);
+      t[1] = __builtin_amdgcn_perm(lo23, lo, 0x07060302u);
+      t[2] = __builtin_amdgcn_perm(hi23, hi, 0x05040100u);
+      t[3] = __builtin_amdgcn_perm(hi23, hi, 0x07060302u);
+    } else {  // the fourth byte meets a zero weight
+      const uint32_t x2 = xin[r][2];
+      t[0] = __builtin_amdgcn_perm(x2, lo, 0x0c040100u);
+      t[1] = __builtin_amdgcn_perm(x2, lo, 0x0c050302u);
+      t[2] = __builtin_amdgcn_perm(x2, hi, 0x0c060100u);
+      t[3] = __builtin_amdgcn_perm(x2, hi, 0x0c070302u);
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      sc[c] = a.n_scales == 0 ? 1.0f : scales[a.n_scales == 1 ? 0 : oc0 + c];
-      bi[c] = bias ? bias[oc0 + c] : 0.0f;
+      if constexpr (!X_SIGNED) t[c] ^= 0x80808080u;
+#pragma unroll
+      for (int kh = 0; kh < 3; ++kh) {  // input row r is window row kh of output row (r - kh) / S
+        if (r - kh < 0 || (r - kh) % S != 0 || (r - kh) / S >= R) continue;
+        int(&o)[CW][4] = acc[(r - kh) / S];
+        // (window row 0 comes first and starts the sum)
+        o[0][c] = __builtin_amdgcn_sdot4(static_cast<int>(t[c]), static_cast<int>(wt[kh][c]), kh == 0 ? comp[c] : o[0][c], false);
+        if constexpr (CW == 2)
+          o[1][c] = __builtin_amdgcn_sdot4(static_cast<int>(t[c]), static_cast<int>(wt[kh][c] << 8), kh == 0 ? comp[c] : o[1][c], false);
+      }
     }
+  }
+
+  constexpr int ESZ = is_float16_type(OUT_T) ? 2 : OUT_T == ITEXHIP_QINT8 || OUT_T == ITEXHIP_QUINT8 ? 1 : 4;
+  char* dst_row = static_cast<char*>(out) + (((static_cast<int64_t>(b) * a.out_h + oh0) * a.out_w + ow0) * a.out_c + oc0) * ESZ;
+  const int64_t row_bytes = static_cast<int64_t>(a.out_w) * a.out_c * ESZ;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int oh = oh0 + r;
-      if (oh >= a.out_h) break;
-      const int64_t o = ((static_cast<int64_t>(b) * a.out_h + oh) * a.out_w + ow) * a.out_c + oc0;
+  for (int r = 0; r < R; ++r, dst_row += row_bytes) {
+    if (oh0 + r >= a.out_h) break;
+#pragma unroll
+    for (int j = 0; j < CW; ++j) {
+      if (ow0 + j >= a.out_w) continue;
+      char* const dst = dst_row + j * a.out_c * ESZ;
       float y[4];
+      if constexpr (BOUNDS) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        float v = static_cast<float>(acc[r][c]);
-        if (a.n_scales != 0) v = v * sc[c];
-        if (bias) v = v + bi[c];
-        y[c] = v;
-      }
-      if (a.chain & 1) {
+        for (int c = 0; c < 4; ++c) {
+          const float v = static_cast<float>(acc[r][j][c]) * sc[c];
+          y[c] = fminf(fmaxf(v + bi[c], a.lo), a.hi);
+        }
+      } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[c] = fmaxf(y[c], 0.0f);
-      }
-      if (a.chain & 2) {
+        for (int c = 0; c < 4; ++c) {
+          float v = static_cast<float>(acc[r][j][c]) * sc[c];  // 1.0f without scales (exact)
+          if (bias) v = v + bi[c];
+          y[c] = v;
+        }
+        if (a.chain & 1) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[c] = y[c] > 0.0f ? y[c] : y[c] * a.alpha;
-      }
-      if (a.chain & 4) {
+          for (int c = 0; c < 4; ++c) y[c] = fmaxf(y[c], 0.0f);
+        }
+        if (a.chain & 2) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[c] = fminf(fmaxf(y[c], a.lo), a.hi);
-      }
-      if (a.chain & 8) {
+          for (int c = 0; c < 4; ++c) y[c] = y[c] > 0.0f ? y[c] : y[c] * a.alpha;
+        }
+        if (a.chain & 4) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) y[c] = a.lin_a * y[c] + a.lin_b;
+          for (int c = 0; c < 4; ++c) y[c] = fminf(fmaxf(y[c], a.lo), a.hi);
+        }
+        if (a.chain & 8) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) y[c] = a.lin_a * y[c] + a.lin_b;
+        }
       }
       // the 4 channels as one store (the host checked the output's alignment)
       if constexpr (OUT_T == ITEXHIP_FLOAT) {
-        *reinterpret_cast<f4*>(static_cast<float*>(out) + o) = f4{y[0], y[1], y[2], y[3]};
+        *reinterpret_cast<f4*>(dst) = f4{y[0], y[1], y[2], y[3]};
       } else if constexpr (is_float16_type(OUT_T)) {
         typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-        *reinterpret_cast<u2*>(static_cast<uint16_t*>(out) + o) = u2{f32x2_to_bits16<OUT_T>(y[0], y[1]), f32x2_to_bits16<OUT_T>(y[2], y[3])};
+        *reinterpret_cast<u2*>(dst) = u2{f32x2_to_bits16<OUT_T>(y[0], y[1]), f32x2_to_bits16<OUT_T>(y[2], y[3])};
       } else if constexpr (OUT_T == ITEXHIP_QINT32) {
-        *reinterpret_cast<i4*>(static_cast<int32_t*>(out) + o) = i4{sat_rne<ITEXHIP_QINT32>(y[0]), sat_rne<ITEXHIP_QINT32>(y[1]),
+        *reinterpret_cast<i4*>(dst) = i4{sat_rne<ITEXHIP_QINT32>(y[0]), sat_rne<ITEXHIP_QINT32>(y[1]),
                                                                     sat_rne<ITEXHIP_QINT32>(y[2]), sat_rne<ITEXHIP_QINT32>(y[3])};
+      } else if constexpr (OUT_T == ITEXHIP_QUINT8) {
+        // rounds to nearest even and saturates to 0 .. 255, NaN to 0, as sat_rne does (compared over all fp32 patterns)
+        uint32_t q = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) q = __builtin_amdgcn_cvt_pk_u8_f32(y[c], c, q);
+        *reinterpret_cast<uint32_t*>(dst) = q;
       } else {
-        *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(out) + o) =
+        *reinterpret_cast<uint32_t*>(dst) =
             pack4(sat_rne<OUT_T>(y[0]), sat_rne<OUT_T>(y[1]), sat_rne<OUT_T>(y[2]), sat_rne<OUT_T>(y[3]));
       }
     }
@@ -439,7 +501,6 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
   a.total = positions * a.groups4;
   const uint8_t* xp = static_cast<const uint8_t*>(x);
   hipStream_t st = as_stream(stream);
-  const int64_t strip_total = g->batch * ((g->out_h + 3) / 4) * g->out_w * a.groups4;
   bool canonical = true;
   {
     int k = 0;
@@ -456,13 +517,34 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
     }
     canonical = k == ep->n_eltwise;
   }
-  if (canonical && a.vec && aligned(out, 16) && g->k_h == 3 && g->k_w == 3 && g->stride_h == 1 && g->stride_w == 1 && g->dil_h == 1 && g->dil_w == 1 &&
-      strip_total < lim && g->batch * g->in_h * g->in_w * g->in_c < lim) {
+  const int step = static_cast<int>(g->stride_h);
+  const int64_t cols = step == 1 ? (g->out_w + 1) / 2 : g->out_w, strips = (g->out_h + 3) / 4;
+  const int64_t strip_total = g->batch * strips * cols * a.groups4;
+  if (canonical && a.vec && aligned(out, 16) && g->k_h == 3 && g->k_w == 3 && (step == 1 || step == 2) && g->stride_w == step &&
+      g->dil_h == 1 && g->dil_w == 1 && strip_total < lim && g->in_h > 0 && g->in_w > 0 && g->batch * g->in_h * g->in_w * g->in_c < lim) {
     a.total = strip_total;
-    const unsigned sblocks = static_cast<unsigned>(std::min<int64_t>((a.total + 255) / 256, 256 * 64));
-#define DW3(T)                                                                                           \
-  if (a.x_signed) qdwconv3x3_kernel<T, true><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out); \
-  else qdwconv3x3_kernel<T, false><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out)
+    a.cols = static_cast<int>(cols);
+    a.strips = static_cast<int>(strips);
+    a.by_groups = make_fast_div(a.groups4);
+    a.by_cols = make_fast_div(cols);
+    a.by_strips = make_fast_div(strips);
+    const unsigned sblocks = static_cast<unsigned>((strip_total + 2047) / 2048 * 8);
+    const bool b8 = (a.chain & ~5) == 0 && (out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8);
+    if (b8 && !(a.chain & 4)) {
+      a.lo = a.chain & 1 ? 0.0f : -INFINITY;
+      a.hi = INFINITY;
+    }
+#define DW3K(T, S, B)                                                                                          \
+  if (a.x_signed) qdwconv3x3_kernel<T, true, S, B><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out); \
+  else qdwconv3x3_kernel<T, false, S, B><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out)
+#define DW3S(T, S)                                                            \
+  if constexpr (T == ITEXHIP_QINT8 || T == ITEXHIP_QUINT8) {                  \
+    if (b8) { DW3K(T, S, true); break; }                                      \
+  }                                                                           \
+  DW3K(T, S, false)
+#define DW3(T)                       \
+  if (step == 1) { DW3S(T, 1); }     \
+  else { DW3S(T, 2); }
     switch (out_type) {
       case ITEXHIP_FLOAT: DW3(ITEXHIP_FLOAT); break;
       case ITEXHIP_BFLOAT16: DW3(ITEXHIP_BFLOAT16); break;
@@ -471,6 +553,8 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
       default: DW3(ITEXHIP_QUINT8); break;
     }
 #undef DW3
+#undef DW3S
+#undef DW3K
     ITEXHIP_CHECK_LAUNCH(who);
     return ITEXHIP_OK;
   }
