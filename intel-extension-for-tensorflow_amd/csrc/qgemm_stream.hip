@@ -342,6 +342,7 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   const size_t lds = static_cast<size_t>(weight) + 12 * s.waves_n * kBlocks * 32 + (cv ? (K >> 4) * 8 : 0);
   const int per_cu = std::min<int>(4, 160 * 1024 / static_cast<int>(lds));  // 128 registers: four wavefronts per SIMD
   const int groups_n = (cols + s.waves_n - 1) / s.waves_n;
+  if (groups_n > 65535) return 0;  // gridDim.y
   const int waves_m = 4 / s.waves_n;
   s.walkers = std::min(s.tiles, std::max(1, 256 * per_cu / groups_n) * waves_m);
   s.share = (static_cast<uint64_t>(s.tiles) << 24) / s.walkers;
