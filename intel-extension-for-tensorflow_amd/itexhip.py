@@ -100,6 +100,29 @@ def _i64(v):
     return C.c_int64(int(v))
 
 
+# The ops a program enqueues per step are called through prototypes: ctypes then converts plain Python numbers in C, and
+# a call builds no c_void_p / c_int64 object per argument.  A launch of a few microseconds is no longer than a dozen of those:
+# host time without the launch 2.0 -> 1.6 us (quantize) and 4.4 -> 3.3 us (qmatmul); QuantizeV2 -> MatMul -> Dequantize of
+# 128 x 1024 x 1024, which the host's calls bound, 15.0 -> 14.3 us.
+_ARG = {"p": C.c_void_p, "i": C.c_int, "l": C.c_int64, "f": C.c_float}
+
+
+def _bind(name, signature):
+    """The entry point with its arguments: p = address or structure, i = int, l = int64_t, f = float."""
+    return C.CFUNCTYPE(C.c_int, *(_ARG[c] for c in signature))((name, _lib))
+
+
+def _addr(x):
+    """The address that _ptr wraps, as a number (prototyped entry points only: elsewhere ctypes would pass 32 bits)."""
+    if x is None or type(x) is int:
+        return x
+    try:
+        f = x.data_ptr
+    except AttributeError:
+        return int(x)
+    return f()
+
+
 def build_info():
     return _lib.itexhip_build_info().decode()
 
@@ -120,9 +143,11 @@ def memcpy_d2d_async(dst, src, nbytes, stream=0):
     _check(_lib.itexhip_memcpy_d2d_async(_ptr(dst), _ptr(src), C.c_size_t(int(nbytes)), _ptr(stream)))
 
 
+_quantize = _bind("itexhip_quantize", "ppliffp")
+
+
 def quantize(x, q, n, dst_type, scale, addend=0.0, stream=0):
-    _check(_lib.itexhip_quantize(_ptr(x), _ptr(q), _i64(n), dst_type, C.c_float(scale),
-                                 C.c_float(addend), _ptr(stream)))
+    _check(_quantize(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
 
 
 def quantize_axis(x, q, outer, slices, inner, dst_type, scales, addends=None, stream=0):
@@ -130,9 +155,11 @@ def quantize_axis(x, q, outer, slices, inner, dst_type, scales, addends=None, st
                                       dst_type, _ptr(scales), _ptr(addends), _ptr(stream)))
 
 
+_quantize_bf16 = _bind("itexhip_quantize_bf16", "ppliffp")
+
+
 def quantize_bf16(x, q, n, dst_type, scale, addend=0.0, stream=0):
-    _check(_lib.itexhip_quantize_bf16(_ptr(x), _ptr(q), _i64(n), dst_type, C.c_float(scale), C.c_float(addend),
-                                      _ptr(stream)))
+    _check(_quantize_bf16(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
 
 
 def quantize_axis_bf16(x, q, outer, slices, inner, dst_type, scales, addends=None, stream=0):
@@ -140,9 +167,11 @@ def quantize_axis_bf16(x, q, outer, slices, inner, dst_type, scales, addends=Non
                                            _ptr(scales), _ptr(addends), _ptr(stream)))
 
 
+_dequantize16 = _bind("itexhip_dequantize16", "ppliifip")
+
+
 def dequantize16(q, y, n, src_type, y_type, scale, zero_point=0, stream=0):
-    _check(_lib.itexhip_dequantize16(_ptr(q), _ptr(y), _i64(n), src_type, y_type, C.c_float(scale),
-                                     C.c_int32(int(zero_point)), _ptr(stream)))
+    _check(_dequantize16(_addr(q), _addr(y), int(n), src_type, y_type, scale, int(zero_point), _addr(stream)))
 
 
 def dequantize_axis16(q, y, outer, slices, inner, src_type, y_type, scales, zero_points=None, stream=0):
@@ -150,9 +179,11 @@ def dequantize_axis16(q, y, outer, slices, inner, src_type, y_type, scales, zero
                                           _ptr(scales), _ptr(zero_points), _ptr(stream)))
 
 
+_dequantize = _bind("itexhip_dequantize", "pplifip")
+
+
 def dequantize(q, y, n, src_type, scale, zero_point=0, stream=0):
-    _check(_lib.itexhip_dequantize(_ptr(q), _ptr(y), _i64(n), src_type, C.c_float(scale),
-                                   C.c_int32(int(zero_point)), _ptr(stream)))
+    _check(_dequantize(_addr(q), _addr(y), int(n), src_type, scale, int(zero_point), _addr(stream)))
 
 
 def dequantize_axis(q, y, outer, slices, inner, src_type, scales, zero_points=None, stream=0):
@@ -160,23 +191,32 @@ def dequantize_axis(q, y, outer, slices, inner, src_type, scales, zero_points=No
                                         src_type, _ptr(scales), _ptr(zero_points), _ptr(stream)))
 
 
+_requantize_per_channel = _bind("itexhip_requantize_per_channel", "ppllipp")
+
+
 def requantize_per_channel(x, q, rows, depth, dst_type, scales, stream=0):
-    _check(_lib.itexhip_requantize_per_channel(_ptr(x), _ptr(q), _i64(rows), _i64(depth), dst_type,
-                                               _ptr(scales), _ptr(stream)))
+    _check(_requantize_per_channel(_addr(x), _addr(q), int(rows), int(depth), dst_type, _addr(scales), _addr(stream)))
+
+
+_requantize = _bind("itexhip_requantize", "pplifp")
 
 
 def requantize(x, q, n, dst_type, scale, stream=0):
-    _check(_lib.itexhip_requantize(_ptr(x), _ptr(q), _i64(n), dst_type, C.c_float(scale),
-                                   _ptr(stream)))
+    _check(_requantize(_addr(x), _addr(q), int(n), dst_type, scale, _addr(stream)))
+
+
+_minmax_i32_per_channel = _bind("itexhip_minmax_i32_per_channel", "pllppp")
 
 
 def minmax_i32_per_channel(x, rows, depth, min_out, max_out, stream=0):
-    _check(_lib.itexhip_minmax_i32_per_channel(_ptr(x), _i64(rows), _i64(depth), _ptr(min_out),
-                                               _ptr(max_out), _ptr(stream)))
+    _check(_minmax_i32_per_channel(_addr(x), int(rows), int(depth), _addr(min_out), _addr(max_out), _addr(stream)))
+
+
+_minmax_f32 = _bind("itexhip_minmax_f32", "plpp")
 
 
 def minmax_f32(x, n, minmax_out, stream=0):
-    _check(_lib.itexhip_minmax_f32(_ptr(x), _i64(n), _ptr(minmax_out), _ptr(stream)))
+    _check(_minmax_f32(_addr(x), int(n), _addr(minmax_out), _addr(stream)))
 
 
 def matmul_params(api=API_V2, t_in=QUINT8, t_out=FLOAT, input_mode=MIN_FIRST, out_min_first=False,
@@ -209,69 +249,96 @@ def qgemm_prepack_b(w, transpose_b, K, N, packed, colsum, stream=0):
 
 
 def _gemm_call(fn, a, a_type, b, colsum, M, K, N, scales, bias, ep, out_type, out, stream):
-    _check(fn(_ptr(a), a_type, _ptr(b), _ptr(colsum), _i64(M), _i64(K), _i64(N), _ptr(scales),
-              _ptr(bias), C.byref(ep), out_type, _ptr(out), _ptr(stream)))
+    _check(fn(_addr(a), a_type, _addr(b), _addr(colsum), int(M), int(K), int(N), _addr(scales),
+              _addr(bias), C.byref(ep), out_type, _addr(out), _addr(stream)))
+
+
+_qgemm = _bind("itexhip_qgemm", "pipplllpppipp")
 
 
 def qgemm(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_lib.itexhip_qgemm, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
+    _gemm_call(_qgemm, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
                out, stream)
+
+
+_qgemm_tile = _bind("itexhip_qgemm_tile", "pipplllpppipp")
 
 
 def qgemm_tile(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_lib.itexhip_qgemm_tile, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep,
+    _gemm_call(_qgemm_tile, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep,
                out_type, out, stream)
 
 
+_qgemv = _bind("itexhip_qgemv", "pipplllpppipp")
+
+
 def qgemv(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_lib.itexhip_qgemv, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
+    _gemm_call(_qgemv, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
                out, stream)
+
+
+_qmatmul = _bind("itexhip_qmatmul", "pppplllpplpppp")
 
 
 def qmatmul(p, a, packed_b, colsum, M, K, N, min_b, max_b, nb, bias, out, stream=0, addend=None):
     """The whole op in one launch (parameters derived inside the MatMul kernel)."""
-    _check(_lib.itexhip_qmatmul(C.byref(p), _ptr(a), _ptr(packed_b), _ptr(colsum), _i64(M), _i64(K), _i64(N),
-                                _ptr(min_b), _ptr(max_b), _i64(nb), _ptr(bias), _ptr(addend), _ptr(out),
-                                _ptr(stream)))
+    _check(_qmatmul(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(min_b),
+                    _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
+
+
+_qmatmul_per_row = _bind("itexhip_qmatmul_per_row", "pppplllpppplpppp")
 
 
 def qmatmul_per_row(p, a, packed_b, colsum, M, K, N, row_min_a, row_max_a, min_b, max_b, nb, bias, out, stream=0,
                     addend=None):
-    _check(_lib.itexhip_qmatmul_per_row(C.byref(p), _ptr(a), _ptr(packed_b), _ptr(colsum), _i64(M), _i64(K), _i64(N),
-                                        _ptr(row_min_a), _ptr(row_max_a), _ptr(min_b), _ptr(max_b), _i64(nb),
-                                        _ptr(bias), _ptr(addend), _ptr(out), _ptr(stream)))
+    _check(_qmatmul_per_row(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
+                            _addr(row_min_a), _addr(row_max_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias),
+                            _addr(addend), _addr(out), _addr(stream)))
+
+
+_qmatmul_device_range = _bind("itexhip_qmatmul_device_range", "pppplllppplpppp")
 
 
 def qmatmul_device_range(p, a, packed_b, colsum, M, K, N, range_a, min_b, max_b, nb, bias, out, stream=0, addend=None):
-    _check(_lib.itexhip_qmatmul_device_range(C.byref(p), _ptr(a), _ptr(packed_b), _ptr(colsum), _i64(M), _i64(K), _i64(N),
-                                             _ptr(range_a), _ptr(min_b), _ptr(max_b), _i64(nb), _ptr(bias),
-                                             _ptr(addend), _ptr(out), _ptr(stream)))
+    _check(_qmatmul_device_range(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
+                                 _addr(range_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend),
+                                 _addr(out), _addr(stream)))
+
+
+_quantize_dynamic = _bind("itexhip_quantize_dynamic", "ppliifpp")
 
 
 def quantize_dynamic(x, q, n, dst_type, mode, ensure_minimum_range, state, stream=0):
-    _check(_lib.itexhip_quantize_dynamic(_ptr(x), _ptr(q), _i64(n), int(dst_type), int(mode),
-                                         C.c_float(ensure_minimum_range), _ptr(state), _ptr(stream)))
+    _check(_quantize_dynamic(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range, _addr(state),
+                             _addr(stream)))
 
 
 def read_probe(src, nbytes, sink, stream=0):
     _check(_lib.itexhip_read_probe(_ptr(src), C.c_size_t(nbytes), _ptr(sink), _ptr(stream)))
 
 
+_quantize_dynamic_static = _bind("itexhip_quantize_dynamic_static", "ppliifpp")
+
+
 def quantize_dynamic_static(x, q, n, dst_type, mode, ensure_minimum_range, range_out, stream=0):
-    _check(_lib.itexhip_quantize_dynamic_static(_ptr(x), _ptr(q), _i64(n), int(dst_type), int(mode),
-                                                C.c_float(ensure_minimum_range), _ptr(range_out), _ptr(stream)))
+    _check(_quantize_dynamic_static(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range,
+                                    _addr(range_out), _addr(stream)))
+
+
+_quantize_dynamic_rows = _bind("itexhip_quantize_dynamic_rows", "pplliifppp")
 
 
 def quantize_dynamic_rows(x, q, rows, cols, dst_type, mode, ensure_minimum_range, row_min_out, row_max_out, stream=0):
-    _check(_lib.itexhip_quantize_dynamic_rows(_ptr(x), _ptr(q), _i64(rows), _i64(cols), int(dst_type), int(mode),
-                                              C.c_float(ensure_minimum_range), _ptr(row_min_out), _ptr(row_max_out),
-                                              _ptr(stream)))
+    _check(_quantize_dynamic_rows(_addr(x), _addr(q), int(rows), int(cols), int(dst_type), int(mode),
+                                  ensure_minimum_range, _addr(row_min_out), _addr(row_max_out), _addr(stream)))
+
+
+_qmatmul_unpacked = _bind("itexhip_qmatmul_unpacked", "pppilllpplpppp")
 
 
 def qmatmul_unpacked(p, a, w, transpose_b, M, K, N, min_b, max_b, nb, bias, out, stream=0, addend=None):
-    _check(_lib.itexhip_qmatmul_unpacked(C.byref(p), _ptr(a), _ptr(w), int(bool(transpose_b)), _i64(M), _i64(K), _i64(N),
-                                         _ptr(min_b), _ptr(max_b), _i64(nb), _ptr(bias), _ptr(addend), _ptr(out),
-                                         _ptr(stream)))
+    _check(_qmatmul_unpacked(C.byref(p), _addr(a), _addr(w), int(bool(transpose_b)), int(M), int(K), int(N),
+                             _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
 
 
 def mfma_probe(workgroups, iters, operands, sink, stream=0):
@@ -352,15 +419,21 @@ def bmm_params(x_shape, y_shape, adj_x, adj_y, out_type, scale, binary=()):
     return p, out_shape
 
 
+_qbatch_matmul = _bind("itexhip_qbatch_matmul", "ppppp")
+
+
 def qbatch_matmul(p, x, y, out, stream=0):
-    _check(_lib.itexhip_qbatch_matmul(C.byref(p), _ptr(x), _ptr(y), _ptr(out), _ptr(stream)))
+    _check(_qbatch_matmul(C.byref(p), _addr(x), _addr(y), _addr(out), _addr(stream)))
+
+
+_transpose = _bind("itexhip_transpose", "ppiippp")
 
 
 def transpose(x, y, elem_size, dims, perm, stream=0):
     rank = len(dims)
     d = (C.c_int64 * max(rank, 1))(*dims)
     pm = (C.c_int32 * max(rank, 1))(*perm)
-    _check(_lib.itexhip_transpose(_ptr(x), _ptr(y), int(elem_size), rank, d, pm, _ptr(stream)))
+    _check(_transpose(_addr(x), _addr(y), int(elem_size), rank, d, pm, _addr(stream)))
 
 
 class ConvGeometry(C.Structure):
@@ -372,35 +445,51 @@ def im2col8(x, geometry, row_bytes, cols, stream=0):
     _check(_lib.itexhip_im2col8(_ptr(x), C.byref(geometry), _i64(row_bytes), _ptr(cols), _ptr(stream)))
 
 
+_pad_nhwc8 = _bind("itexhip_pad_nhwc8", "plllllllllpp")
+
+
 def pad_nhwc8(x, n, h, w, c, lead_h, lead_w, out_h, out_w, out_c, out, stream=0):
-    _check(_lib.itexhip_pad_nhwc8(_ptr(x), _i64(n), _i64(h), _i64(w), _i64(c), _i64(lead_h), _i64(lead_w), _i64(out_h),
-                                  _i64(out_w), _i64(out_c), _ptr(out), _ptr(stream)))
+    _check(_pad_nhwc8(_addr(x), int(n), int(h), int(w), int(c), int(lead_h), int(lead_w), int(out_h), int(out_w),
+                      int(out_c), _addr(out), _addr(stream)))
 
 
 def qconv2d_implicit_ok(geometry, x, out_channels, out_type, out):
     return bool(_lib.itexhip_qconv2d_implicit_ok(C.byref(geometry), _ptr(x), _i64(out_channels), int(out_type), _ptr(out)))
 
 
+_qconv2d = _bind("itexhip_qconv2d", "pippplpppipp")
+
+
 def qconv2d(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, out_type, out, stream=0):
-    _check(_lib.itexhip_qconv2d(_ptr(x), int(x_type), C.byref(geometry), _ptr(packed_filter), _ptr(colsum), _i64(out_channels),
-                                _ptr(scales), _ptr(bias), C.byref(ep), int(out_type), _ptr(out), _ptr(stream)))
+    _check(_qconv2d(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
+                    _addr(scales), _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
+
+
+_qconv2d_sum = _bind("itexhip_qconv2d_sum", "pippplppppiipp")
 
 
 def qconv2d_sum(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, addend, addend_type, out_type, out,
                 stream=0):
-    _check(_lib.itexhip_qconv2d_sum(_ptr(x), int(x_type), C.byref(geometry), _ptr(packed_filter), _ptr(colsum), _i64(out_channels),
-                                    _ptr(scales), _ptr(bias), C.byref(ep), _ptr(addend), int(addend_type), int(out_type),
-                                    _ptr(out), _ptr(stream)))
+    _check(_qconv2d_sum(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
+                        _addr(scales), _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type),
+                        _addr(out), _addr(stream)))
+
+
+_qgemm_sum = _bind("itexhip_qgemm_sum", "pipplllppppiipp")
 
 
 def qgemm_sum(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, addend, addend_type, out_type, out, stream=0):
-    _check(_lib.itexhip_qgemm_sum(_ptr(a), int(a_type), _ptr(packed_b), _ptr(colsum), _i64(M), _i64(K), _i64(N), _ptr(scales),
-                                  _ptr(bias), C.byref(ep), _ptr(addend), int(addend_type), int(out_type), _ptr(out), _ptr(stream)))
+    _check(_qgemm_sum(_addr(a), int(a_type), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(scales),
+                      _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type), _addr(out),
+                      _addr(stream)))
+
+
+_qdepthwise_conv2d = _bind("itexhip_qdepthwise_conv2d", "piplppppipp")
 
 
 def qdepthwise_conv2d(x, x_type, geometry, multiplier, filt, scales, bias, ep, out_type, out, stream=0):
-    _check(_lib.itexhip_qdepthwise_conv2d(_ptr(x), int(x_type), C.byref(geometry), _i64(multiplier), _ptr(filt), _ptr(scales),
-                                          _ptr(bias), C.byref(ep), int(out_type), _ptr(out), _ptr(stream)))
+    _check(_qdepthwise_conv2d(_addr(x), int(x_type), C.byref(geometry), int(multiplier), _addr(filt), _addr(scales),
+                              _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
 
 
 def scale_vector(bias, bias_type, factors, n_factors, n, out, stream=0):
