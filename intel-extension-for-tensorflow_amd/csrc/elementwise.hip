@@ -663,29 +663,41 @@ __global__ __launch_bounds__(kSmallThreads) void quantize_dynamic_small_kernel(c
 }
 
 // Per-row (per-token) form: workgroup m reduces row m, derives its parameters and quantizes it; the rows' output
-// ranges go to two device arrays (what itexhip_qmatmul_per_row takes).
+// ranges go to two device arrays (what itexhip_qmatmul_per_row takes).  Bound by latency: a decode batch is 1 - 16 workgroups.
+// So a thread has its first HELD groups of 4 elements in flight at once and keeps them for the quantization (HELD: 1, 2 or 4,
+// the fewest that hold the row; what lies beyond 16384 columns is read twice), and every wavefront finishes the reduction by
+// itself instead of waiting for one thread's walk over 16 partial results.
+// One row, kernel time: 14336 columns 4.0 -> 3.4 us, 4096 columns 2.5 -> 2.6 us; a decoder's feed-forward step over one token
+// (both of them and two linears) 29.6 -> 28.9 us.
 constexpr int kRowThreads = 1024;
+constexpr int kRowWaves = kRowThreads / 64;
 
-template <int T>
+template <int T, int HELD>  // HELD 0: single elements (odd lengths, unaligned rows)
 __global__ __launch_bounds__(kRowThreads) void quantize_dynamic_rows_kernel(const float* __restrict__ x,
-                                                                            uint8_t* __restrict__ q, int cols, int vec,
+                                                                            uint8_t* __restrict__ q, int cols,
                                                                             float* __restrict__ row_min,
                                                                             float* __restrict__ row_max, int mode,
                                                                             float ensure_minimum_range) {
-  __shared__ float red[2 * (kRowThreads / 64)];
-  __shared__ float params[2];
+  __shared__ float red_min[kRowWaves], red_max[kRowWaves];
   const float* xr = x + static_cast<int64_t>(blockIdx.x) * cols;
   uint8_t* qr = q + static_cast<int64_t>(blockIdx.x) * cols;
+  const f4* x4 = reinterpret_cast<const f4*>(xr);
+  const int n4 = cols / 4, tid = threadIdx.x;
   float mn = __builtin_inff(), mx = -__builtin_inff();
-  if (vec) {
-    const f4* x4 = reinterpret_cast<const f4*>(xr);
-    for (int i = threadIdx.x; i < cols / 4; i += kRowThreads) {
-      const f4 v = x4[i];
-      mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
-      mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
-    }
+  auto reduce = [&](const f4& v) {
+    mn = fminf(fminf(mn, v.x), fminf(v.y, fminf(v.z, v.w)));
+    mx = fmaxf(fmaxf(mx, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
+  };
+  f4 held[HELD > 0 ? HELD : 1];
+  if constexpr (HELD > 0) {
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) held[u] = x4[min(tid + u * kRowThreads, n4 - 1)];  // past the end: the last group again
+#pragma unroll
+    for (int u = 0; u < HELD; ++u) reduce(held[u]);
+    if constexpr (HELD == 4)
+      for (int i = tid + HELD * kRowThreads; i < n4; i += kRowThreads) reduce(x4[i]);
   } else {
-    for (int i = threadIdx.x; i < cols; i += kRowThreads) {
+    for (int i = tid; i < cols; i += kRowThreads) {
       mn = fminf(mn, xr[i]);
       mx = fmaxf(mx, xr[i]);
     }
@@ -695,34 +707,49 @@ __global__ __launch_bounds__(kRowThreads) void quantize_dynamic_rows_kernel(cons
     mn = fminf(mn, __shfl_xor(mn, o, 64));
     mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   }
-  if ((threadIdx.x & 63) == 0) {
-    red[2 * (threadIdx.x >> 6)] = mn;
-    red[2 * (threadIdx.x >> 6) + 1] = mx;
+  if ((tid & 63) == 0) {
+    red_min[tid >> 6] = mn;
+    red_max[tid >> 6] = mx;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kRowThreads / 64; ++w) {
-      mn = fminf(mn, red[2 * w]);
-      mx = fmaxf(mx, red[2 * w + 1]);
-    }
-    const DynamicParams p = dynamic_params(mn, mx, T, mode, ensure_minimum_range);
-    params[0] = p.scale;
-    params[1] = p.addend;
+  mn = red_min[tid & (kRowWaves - 1)];
+  mx = red_max[tid & (kRowWaves - 1)];
+#pragma unroll
+  for (int o = kRowWaves / 2; o > 0; o >>= 1) {
+    mn = fminf(mn, __shfl_xor(mn, o, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  }
+  const DynamicParams p = dynamic_params(mn, mx, T, mode, ensure_minimum_range);
+  if (tid == 0) {
     row_min[blockIdx.x] = p.out_min;
     row_max[blockIdx.x] = p.out_max;
   }
-  __syncthreads();
-  const float scale = params[0], addend = params[1];
-  if (vec) {
-    const f4* x4 = reinterpret_cast<const f4*>(xr);
+  if constexpr (HELD > 0) {
     uint32_t* q4 = reinterpret_cast<uint32_t*>(qr);
-    for (int i = threadIdx.x; i < cols / 4; i += kRowThreads) q4[i] = quantize4<T>(x4[i], scale, addend);
+#pragma unroll
+    for (int u = 0; u < HELD; ++u)
+      if (tid + u * kRowThreads < n4) q4[tid + u * kRowThreads] = quantize4<T>(held[u], p.scale, p.addend);
+    if constexpr (HELD == 4)
+      for (int i = tid + HELD * kRowThreads; i < n4; i += kRowThreads) q4[i] = quantize4<T>(x4[i], p.scale, p.addend);
   } else {
-    for (int i = threadIdx.x; i < cols; i += kRowThreads) {
-      const float t = xr[i] * scale;
-      qr[i] = static_cast<uint8_t>(sat_rne<T>(t + addend));
+    for (int i = tid; i < cols; i += kRowThreads) {
+      const float t = xr[i] * p.scale;
+      qr[i] = static_cast<uint8_t>(sat_rne<T>(t + p.addend));
     }
   }
+}
+
+template <int T>
+void launch_rows(const float* x, uint8_t* q, int64_t rows, int cols, bool vec, float* row_min, float* row_max, int mode,
+                 float ensure_minimum_range, hipStream_t st) {
+  const unsigned grid = static_cast<unsigned>(rows);
+#define LAUNCH_ROWS(HELD) \
+  quantize_dynamic_rows_kernel<T, HELD><<<grid, kRowThreads, 0, st>>>(x, q, cols, row_min, row_max, mode, ensure_minimum_range)
+  if (!vec) LAUNCH_ROWS(0);
+  else if (cols <= 4 * kRowThreads) LAUNCH_ROWS(1);
+  else if (cols <= 8 * kRowThreads) LAUNCH_ROWS(2);
+  else LAUNCH_ROWS(4);
+#undef LAUNCH_ROWS
 }
 
 // Second half of the two-launch form for larger tensors: every workgroup reduces the partial ranges the reduction
@@ -886,14 +913,10 @@ extern "C" int itexhip_quantize_dynamic_rows(const float* x, void* q, int64_t ro
                   "itexhip_quantize_dynamic_rows: bad shape (an empty row has no range)");
   if (rows == 0) return ITEXHIP_OK;
   ITEXHIP_REQUIRE(x && q && row_min_out && row_max_out, "itexhip_quantize_dynamic_rows: null buffer");
-  const int vec = cols % 4 == 0 && aligned(x, 16) && aligned(q, 4);
-  const unsigned grid = static_cast<unsigned>(rows);
-  if (dst_type == ITEXHIP_QINT8)
-    quantize_dynamic_rows_kernel<ITEXHIP_QINT8><<<grid, kRowThreads, 0, as_stream(stream)>>>(
-        x, reinterpret_cast<uint8_t*>(q), static_cast<int>(cols), vec, row_min_out, row_max_out, mode, ensure_minimum_range);
-  else
-    quantize_dynamic_rows_kernel<ITEXHIP_QUINT8><<<grid, kRowThreads, 0, as_stream(stream)>>>(
-        x, reinterpret_cast<uint8_t*>(q), static_cast<int>(cols), vec, row_min_out, row_max_out, mode, ensure_minimum_range);
+  const bool vec = cols % 4 == 0 && aligned(x, 16) && aligned(q, 4);
+  const auto launch = dst_type == ITEXHIP_QINT8 ? launch_rows<ITEXHIP_QINT8> : launch_rows<ITEXHIP_QUINT8>;
+  launch(x, static_cast<uint8_t*>(q), rows, static_cast<int>(cols), vec, row_min_out, row_max_out, mode, ensure_minimum_range,
+         as_stream(stream));
   ITEXHIP_CHECK_LAUNCH("itexhip_quantize_dynamic_rows");
   return ITEXHIP_OK;
 }
