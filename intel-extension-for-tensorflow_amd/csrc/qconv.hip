@@ -77,28 +77,69 @@ __global__ __launch_bounds__(256) void pad_nhwc8_kernel(const Pad4dArgs a, const
   out[i] = v;
 }
 
-// The same for out_c = 4 or 8 and out_w a multiple of 16 / out_c: one thread per 16 output bytes (4 or 2 pixels of one
-// row), so the index decomposition is paid once per 16 bytes (the 4-byte form spent most of its time on it).
-template <int OUT_C>
-__global__ __launch_bounds__(256) void pad_nhwc8_vec_kernel(const Pad4dArgs a, const uint8_t* __restrict__ x, i4* __restrict__ out) {
-  constexpr int PIX = 16 / OUT_C;
+// The same for out_c = 8 and an even out_w: one thread per 16 output bytes (2 pixels of one row), so the index decomposition
+// is paid once per 16 bytes (the 4-byte form spent most of its time on it).
+__global__ __launch_bounds__(256) void pad_nhwc8_to8_kernel(const Pad4dArgs a, const uint8_t* __restrict__ x, i4* __restrict__ out) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;  // vector index
   if (i >= a.total / 4) return;
-  const uint32_t per_row = static_cast<uint32_t>(a.out_w) / PIX;
-  const uint32_t row = i / per_row, ow0 = (i - row * per_row) * PIX;
+  const uint32_t per_row = static_cast<uint32_t>(a.out_w) / 2;
+  const uint32_t row = i / per_row, ow0 = (i - row * per_row) * 2;
   const uint32_t n = row / static_cast<uint32_t>(a.out_h), oh = row - n * static_cast<uint32_t>(a.out_h);
   const int ih = static_cast<int>(oh) - a.lead_h;
   uint32_t v[4] = {0u, 0u, 0u, 0u};
   if (ih >= 0 && ih < a.h) {
     const uint8_t* src_row = x + (static_cast<int64_t>(n) * a.h + ih) * a.w * a.c;
 #pragma unroll
-    for (int p = 0; p < PIX; ++p) {
+    for (int p = 0; p < 2; ++p) {
       const int iw = static_cast<int>(ow0) + p - a.lead_w;
       if (iw < 0 || iw >= a.w) continue;
       const uint8_t* src = src_row + static_cast<int64_t>(iw) * a.c;
 #pragma unroll
-      for (int e = 0; e < OUT_C; ++e)
-        if (e < a.c) v[(p * OUT_C + e) >> 2] |= static_cast<uint32_t>(src[e]) << (8 * (e & 3));
+      for (int e = 0; e < 8; ++e)
+        if (e < a.c) v[(p * 8 + e) >> 2] |= static_cast<uint32_t>(src[e]) << (8 * (e & 3));
+    }
+  }
+  out[i] = i4{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
+}
+
+// The same for out_c = 4, 1 to 4 input channels and out_w a multiple of 4: one thread per 4 pixels of an output row.  Their
+// 4 * C input bytes are contiguous, so one 16-byte load at whatever address they fall on brings them (4 * C byte loads set
+// the pace before); a load that would begin before the tensor or reach past its end (`bytes` >= 16) is moved inside and its
+// bytes shifted back, and pixels outside the row are cleared.
+// 32 x 224 x 224 x 3 into 231 x 232 x 4: 7.6 -> 6.1 us, the first layer of ResNet-50 on it (copy and convolution) 21.3 -> 19.9 us.
+// 11.7 MB: what is left is the launch and one round trip to memory.
+template <int C>
+__global__ __launch_bounds__(256) void pad_nhwc8_to4_kernel(const Pad4dArgs a, const FastDiv by_row, const FastDiv by_out_h, int64_t bytes,
+                                                            const uint8_t* __restrict__ x, i4* __restrict__ out) {
+  typedef uint32_t u4_any __attribute__((ext_vector_type(4), aligned(1)));
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;  // vector index, < 2^29
+  if (i >= a.total / 4) return;
+  const int row = fast_div(static_cast<int>(i), by_row);
+  const int iw0 = (static_cast<int>(i) - row * (a.out_w >> 2)) * 4 - a.lead_w;
+  const int n = fast_div(row, by_out_h), ih = row - n * a.out_h - a.lead_h;
+  uint32_t v[4] = {0u, 0u, 0u, 0u};
+  if (ih >= 0 && ih < a.h && iw0 > -4 && iw0 < a.w) {
+    const int64_t want = ((static_cast<int64_t>(n) * a.h + ih) * a.w + iw0) * C;
+    const int64_t at = want < 0 ? 0 : want > bytes - 16 ? bytes - 16 : want;
+    const u4_any w = *reinterpret_cast<const u4_any*>(x + at);
+    uint64_t lo = static_cast<uint64_t>(w.y) << 32 | w.x, hi = static_cast<uint64_t>(w.w) << 32 | w.z;
+    const int d = static_cast<int>(want - at);  // -12 .. 15: a pixel of the four exists
+    if (d > 0) {
+      const int s = 8 * (d & 7);
+      if (d & 8) { lo = hi; hi = 0; }
+      if (s) { lo = lo >> s | hi << (64 - s); hi >>= s; }
+    } else if (d < 0) {
+      const int s = 8 * (-d & 7);
+      if (-d & 8) { hi = lo; lo = 0; }
+      if (s) { hi = hi << s | lo >> (64 - s); lo <<= s; }
+    }
+    const uint32_t in[5] = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+                            static_cast<uint32_t>(hi >> 32), 0u};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t pixel = static_cast<uint32_t>((static_cast<uint64_t>(in[p * C / 4 + 1]) << 32 | in[p * C / 4]) >> (8 * (p * C % 4)));
+      const bool inside = iw0 + p >= 0 && iw0 + p < a.w;
+      v[p] = inside ? pixel & (0xffffffffu >> (8 * (4 - C))) : 0u;
     }
   }
   out[i] = i4{static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])};
@@ -645,10 +686,13 @@ extern "C" int itexhip_pad_nhwc8(const void* x, int64_t n, int64_t h, int64_t w,
   a.total = static_cast<uint32_t>(total);
   const uint8_t* xb = static_cast<const uint8_t*>(x);
   const unsigned vblocks = static_cast<unsigned>((total / 4 + 255) / 256);
-  if (out_c == 4 && out_w % 4 == 0 && aligned(out, 16))
-    pad_nhwc8_vec_kernel<4><<<vblocks, 256, 0, as_stream(stream)>>>(a, xb, static_cast<i4*>(out));
-  else if (out_c == 8 && out_w % 2 == 0 && aligned(out, 16))
-    pad_nhwc8_vec_kernel<8><<<vblocks, 256, 0, as_stream(stream)>>>(a, xb, static_cast<i4*>(out));
+  const int64_t bytes = n * h * w * c;
+  if (out_c == 4 && c > 0 && bytes >= 16 && out_w % 4 == 0 && aligned(out, 16)) {
+    const FastDiv by_row = make_fast_div(out_w / 4), by_out_h = make_fast_div(out_h);
+    const auto kernel = c == 1 ? pad_nhwc8_to4_kernel<1> : c == 2 ? pad_nhwc8_to4_kernel<2> : c == 3 ? pad_nhwc8_to4_kernel<3> : pad_nhwc8_to4_kernel<4>;
+    kernel<<<vblocks, 256, 0, as_stream(stream)>>>(a, by_row, by_out_h, bytes, xb, static_cast<i4*>(out));
+  } else if (out_c == 8 && out_w % 2 == 0 && aligned(out, 16))
+    pad_nhwc8_to8_kernel<<<vblocks, 256, 0, as_stream(stream)>>>(a, xb, static_cast<i4*>(out));
   else
     pad_nhwc8_kernel<<<static_cast<unsigned>((total + 255) / 256), 256, 0, as_stream(stream)>>>(a, xb, static_cast<uint32_t*>(out));
   ITEXHIP_CHECK_LAUNCH(who);
