@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   }
 }
 
-// An operand of fewer than 16 bytes in all (K < 16): one thread per output element.
+// An operand of fewer than 16 bytes in all (K < 16), or too many tiles for a launch: one thread per output element.
 template <int OUT_T>
 __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __restrict__ a, int a_is_u8,
                                                             const int8_t* __restrict__ w, int transpose_b,
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __rest
 template <int OUT_T>
 void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
             const EpilogueArgs& e, void* out, hipStream_t st) {
-  if (static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16) {
+  if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16) {
     qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((static_cast<int64_t>(M) * N + 255) / 256), 256, 0, st>>>(
         a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out);
     return;
@@ -293,12 +293,15 @@ void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b,
 int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
                     const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who) {
   const int64_t tiles_m = (M + kTileM - 1) / kTileM, tiles_n = (N + kTileN - 1) / kTileN;
-  ITEXHIP_REQUIRE(tiles_m * tiles_n < (1LL << 24) - 8, "%s: output too large for one launch", who);  // 2^32 threads
+  // 2^32 threads at most; a result of more tiles than that allows is long and narrow (2^30 rows or columns and more) and goes
+  // one thread per output element
+  const bool many_tiles = tiles_m * tiles_n >= (1LL << 24) - 8;
+  ITEXHIP_REQUIRE(!many_tiles || (M < (1LL << 32) / N), "%s: output too large for one launch", who);
   const uint8_t* ap = static_cast<const uint8_t*>(a);
   const uint8_t* wp = reinterpret_cast<const uint8_t*>(w);
   const uint32_t a_xor = a_type == ITEXHIP_QUINT8 ? 0x80808080u : 0u;
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
-  const int tn = static_cast<int>(tiles_n), tiles = static_cast<int>(tiles_m * tiles_n);
+  const int tn = static_cast<int>(tiles_n), tiles = many_tiles ? 0 : static_cast<int>(tiles_m * tiles_n);
   switch (out_type) {
     case ITEXHIP_FLOAT: launch<ITEXHIP_FLOAT>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
     case ITEXHIP_BFLOAT16: launch<ITEXHIP_BFLOAT16>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;

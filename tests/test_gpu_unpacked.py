@@ -33,3 +33,20 @@ def test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b):
                          layer.min_b.size, layer.bias_d, out)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(out.cpu().numpy(), ref)
+
+
+def test_more_rows_than_tiles_in_a_launch(hip, dev):
+    """2^30 rows of one value and one column: 2^24 tiles of 64 rows, one more launch than 2^32 threads allow."""
+    import torch
+    M = 1 << 30
+    if torch.cuda.mem_get_info()[0] < 8 * M:
+        pytest.skip("needs 8 GiB")
+    p = hip.matmul_params(t_in=hip.QINT8, t_out=hip.QINT8, input_mode=hip.SCALED, min_a=-127.0, max_a=127.0, has_requantize=True,
+                          min_out=-127.0, max_out=127.0)
+    a = torch.arange(64, dtype=torch.int8, device=dev).repeat(M // 64)
+    w = torch.ones(1, dtype=torch.int8, device=dev)
+    lo, hi = torch.full((1,), -127.0, device=dev), torch.full((1,), 127.0, device=dev)
+    out = torch.full((M,), -1, dtype=torch.int8, device=dev)
+    hip.qmatmul_unpacked(p, a, w, False, M, 1, 1, lo, hi, 1, torch.zeros(1, device=dev), out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, a)
