@@ -13,6 +13,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "qbmm_reads.hpp"
 #include "qgemm_common.hpp"
 
 namespace itexhip {
@@ -49,11 +50,9 @@ template <bool KCONT, int MODE>
 __device__ __forceinline__ void fetch_tile(const int8_t* __restrict__ g, int64_t R, int64_t K, int64_t r0, int64_t k0,
                                            int t, uint32_t (&w)[4]) {
   if constexpr (KCONT) {  // thread: row t / 4, 16 consecutive k
-    int64_t row = r0 + (t >> 2), k = k0 + (t & 3) * 16;
-    if constexpr (MODE == kAny) {  // rows past R repeat the last one (their results are not stored)
-      row = row < R ? row : R - 1;
-      k = k < K - 16 ? k : K - 16;
-      const v4i v = *reinterpret_cast<const v4i_any*>(g + row * K + k);
+    const int64_t row = r0 + (t >> 2), k = k0 + (t & 3) * 16;
+    if constexpr (MODE == kAny) {  // (results of rows past R are not stored)
+      const v4i v = *reinterpret_cast<const v4i_any*>(g + read_offset_k_fastest(row, k, R, K));
       w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
       return;
     }
@@ -72,14 +71,10 @@ __device__ __forceinline__ void fetch_tile(const int8_t* __restrict__ g, int64_t
     }
   } else {  // thread: 4 (k) x 4 (r) bytes; kb = t / 16 picks the k rows, cb = t % 16 the r columns; w[i] = k row i
     const int kb = t >> 4, cb = t & 15;
-    int64_t r = r0 + cb * 4;
+    const int64_t r = r0 + cb * 4;
     if constexpr (MODE == kAny) {
-      r = r < R - 4 ? r : R - 4;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t k = k0 + kb * 4 + i;
-        w[i] = *reinterpret_cast<const u32_any*>(g + (k < K ? k : K - 1) * R + r);
-      }
+      for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const u32_any*>(g + read_offset_r_fastest(r, k0 + kb * 4 + i, R, K));
       return;
     }
     w[0] = w[1] = w[2] = w[3] = 0;
@@ -550,8 +545,7 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   // [R, K] layouts load 16 bytes along k, [K, R] layouts 4 bytes along r
   const bool vec_x = p->adj_x ? vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->M, 4) : vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->K, 16);
   const bool vec_y = p->adj_y ? vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->K, 16) : vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->N, 4);
-  // (the loads of kAny stay inside a row of the operand)
-  const bool any = (p->adj_x ? p->M >= 4 : p->K >= 16) && (p->adj_y ? p->K >= 16 : p->N >= 4);
+  const bool any = vector_reads_fit(!p->adj_x, p->M, p->K) && vector_reads_fit(p->adj_y, p->N, p->K);
   a.mode = vec_x && vec_y ? kAligned : any ? kAny : kBytes;
   // Tiles of 128 rows (and 128 columns) where more than 64 exist, the operands are aligned, the fused operands do not
   // depend on the row, and at least 1024 tiles remain (four per CU); else 64 x 64.  BERT-base attention over 128

@@ -39,3 +39,23 @@ def test_large_tiles(hip, dev, t_out):
     for n in (3 * 21, 131):
         y = rng.integers(-128, 128, (520, 37, n)).astype(np.int8)
         check(hip, dev, x, y, t_out=t_out, y_off=2)
+
+
+@pytest.mark.parametrize("adj_x,adj_y", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N", [(5, 7), (4, 6), (2, 9), (70, 65)])
+@pytest.mark.parametrize("t_out", [orc.FLOAT, orc.BFLOAT16])
+def test_empty_reduction(hip, dev, adj_x, adj_y, M, N, t_out):
+    """K = 0 with the null operands of empty tensors: the empty sum, scaled, and the fused operands."""
+    import torch
+    rng = np.random.default_rng(M + N)
+    x, y = (np.zeros(s, np.int8) for s in ((3, 0, M) if adj_x else (3, M, 0), (3, N, 0) if adj_y else (3, 0, N)))
+    mul, add = rng.standard_normal((3, M, 1)).astype(np.float32), rng.standard_normal((1, 1, N)).astype(np.float32)
+    td = torch.float32 if t_out == orc.FLOAT else torch.bfloat16
+    mul, add = torch.from_numpy(mul).to(dev, td), torch.from_numpy(add).to(dev, td)
+    fused = [(hip.BIN_ADD, add, (1, 1, N)), (hip.BIN_MUL, mul, (3, M, 1))]
+    for binary, want in (((), torch.zeros(3, M, N, dtype=td, device=dev)), (fused[:1], add.expand(3, M, N)), (fused, add * mul)):
+        p, shape = hip.bmm_params(x.shape, y.shape, adj_x, adj_y, t_out, 0.5, binary)
+        out = torch.full(shape, 7.0, dtype=td, device=dev)
+        hip.qbatch_matmul(p, None, None, out)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
