@@ -26,18 +26,18 @@ constexpr int kBmmThreads = 256;
 struct BmmArgs {
   itexhip_bmm_params p;
   int tiles_m, tiles_n;
-  int mode;          // kBytes, kAligned or kAny: how both operands are read
+  int mode_x, mode_y;  // kBytes, kAligned or kAny: how the operands are read
   int xcd_grid;      // launched as (8, tiles, matrices / 8): see the kernel
   uint32_t batch;
   FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
 };
 
-// How an operand is read.  kBytes: K < 16 (or fewer than 4 rows / columns) and unaligned: byte by byte.  kAligned: aligned
-// 16-byte (KCONT) / 4-byte (transposed) loads that never straddle a bound.  kAny: the same loads at whatever byte address
-// they fall on (the hardware takes unaligned vector loads); a load that would cross the end of its row starts at the last
-// place inside it and settle_tile shifts the bytes into place once they have arrived.  P.V over 197 tokens (384 products of
-// 197 x 197 by 197 x 64 to bfloat16): 36.9 us with byte loads (16 per piece), 11.6 us with these.
+// How an operand is read, each by itself.  kBytes: rows too short for a load (and an empty K): byte by byte, every read
+// guarded.  kAligned: aligned 16-byte (KCONT) / 4-byte (transposed) loads that never straddle a bound.  kAny: the same loads
+// at whatever byte address they fall on (the hardware takes unaligned vector loads); a load that would cross the end of its
+// row starts at the last place inside it and settle_tile shifts the bytes into place once they have arrived.  P.V over 197
+// tokens (384 products of 197 x 197 by 197 x 64 to bfloat16): 36.9 us with byte loads (16 per piece), 11.6 us with these.
 enum : int { kBytes = 0, kAligned = 1, kAny = 2 };
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t u32_any __attribute__((aligned(1)));
@@ -318,7 +318,7 @@ __device__ __forceinline__ QuadrantSite quadrant_site(const itexhip_bmm_params& 
 // The larger tiles amortise what a wavefront spends around its MFMAs (a 64 x 64 tile of K = 64 is two MFMAs and some
 // 450 other instructions per wavefront) and read each operand half as often; they exist for the calls whose fused
 // operands take one register per lane and quadrant column (none, or ROWB).
-template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB, int RM, int RN>
+template <bool ADJ_X, bool ADJ_Y, int MODE_X, int MODE_Y, int NB, int OUT_T, bool ROWB, int RM, int RN>
 __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8_t* __restrict__ xb,
                                          const int8_t* __restrict__ yb, const int64_t (&bo)[ITEXHIP_BMM_MAX_BINARY], uint32_t bi,
                                          int m0, int n0, int wm, int wn, int t, int lane, void* __restrict__ out,
@@ -327,9 +327,9 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
   // first tiles and the fused operands: all loads the results depend on are issued before any is needed
   uint32_t wx[RM][4], wy[RN][4];
 #pragma unroll
-  for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE>(xb, p.M, p.K, m0 + 64 * h, 0, t, wx[h]);  // x is [M, K] unless adj_x
+  for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE_X>(xb, p.M, p.K, m0 + 64 * h, 0, t, wx[h]);  // x is [M, K] unless adj_x
 #pragma unroll
-  for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE>(yb, p.N, p.K, n0 + 64 * h, 0, t, wy[h]);   // y is [N, K] only with adj_y
+  for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE_Y>(yb, p.N, p.K, n0 + 64 * h, 0, t, wy[h]);   // y is [N, K] only with adj_y
   // (the quadrants are walked with compile-time indices: what describes a quadrant is the same for the whole
   // wavefront and must stay in scalar registers, which an indexed array of descriptors does not)
   float o[RM * RN][ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16];
@@ -346,9 +346,11 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
   });
 
   for (int64_t k0 = 0; k0 < p.K; k0 += kTile) {
-    if constexpr (MODE == kAny) {
+    if constexpr (MODE_X == kAny) {
 #pragma unroll
       for (int h = 0; h < RM; ++h) settle_tile<!ADJ_X>(p.M, p.K, m0 + 64 * h, k0, t, wx[h]);
+    }
+    if constexpr (MODE_Y == kAny) {
 #pragma unroll
       for (int h = 0; h < RN; ++h) settle_tile<ADJ_Y>(p.N, p.K, n0 + 64 * h, k0, t, wy[h]);
     }
@@ -359,9 +361,9 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
     __syncthreads();
     if (k0 + kTile < p.K) {  // the next tile travels while this one is multiplied
 #pragma unroll
-      for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE>(xb, p.M, p.K, m0 + 64 * h, k0 + kTile, t, wx[h]);
+      for (int h = 0; h < RM; ++h) fetch_tile<!ADJ_X, MODE_X>(xb, p.M, p.K, m0 + 64 * h, k0 + kTile, t, wx[h]);
 #pragma unroll
-      for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE>(yb, p.N, p.K, n0 + 64 * h, k0 + kTile, t, wy[h]);
+      for (int h = 0; h < RN; ++h) fetch_tile<ADJ_Y, MODE_Y>(yb, p.N, p.K, n0 + 64 * h, k0 + kTile, t, wy[h]);
     }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -388,7 +390,7 @@ __device__ __forceinline__ void bmm_body(const itexhip_bmm_params& p, const int8
 // One kernel per (layouts, number of fused operands, output type, operands independent of the row): compiled as one
 // kernel with a switch over these, every variant took the registers of the largest (112 - 140, three or four
 // wavefronts per SIMD; P.V over 128 sequences 18.7 -> 16.4 us as a kernel of its own).
-template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB, int RM = 1, int RN = 1>
+template <bool ADJ_X, bool ADJ_Y, int MODE_X, int MODE_Y, int NB, int OUT_T, bool ROWB, int RM = 1, int RN = 1>
 __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, const int8_t* __restrict__ x,
                                                            const int8_t* __restrict__ y, void* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) uint8_t xs[RM * kTile * kLdsStride];
@@ -428,29 +430,36 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
     for (int b = 0; b < NB; ++b) bo[b] += i * p.binary[b].batch_stride[d];
   }
   // accumulator e of a lane is row (e / 4) * 8 + (lane / 32) * 4 + e % 4, column lane % 32 of its quadrant
-  bmm_body<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, RM, RN>(p, x + xo, y + yo, bo, bi, m0, n0, wm, wn, t, lane, out, xs, ys);
+  bmm_body<ADJ_X, ADJ_Y, MODE_X, MODE_Y, NB, OUT_T, ROWB, RM, RN>(p, x + xo, y + yo, bo, bi, m0, n0, wm, wn, t, lane, out, xs, ys);
 }
 
-template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB>
+template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB>  // both operands read alike
 void launch_tiles(const BmmArgs& a, const int8_t* x, const int8_t* y, void* out, dim3 grid, hipStream_t st) {
   if constexpr (NB == 0 || ROWB) {  // the larger tiles (chosen by the host)
     if (a.rm == 2 && a.rn == 2) {
-      qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, 2, 2><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+      qbmm_kernel<ADJ_X, ADJ_Y, MODE, MODE, NB, OUT_T, ROWB, 2, 2><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
       return;
     }
     if (a.rm == 2 && a.rn == 1) {
-      qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB, 2, 1><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+      qbmm_kernel<ADJ_X, ADJ_Y, MODE, MODE, NB, OUT_T, ROWB, 2, 1><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
       return;
     }
   }
-  qbmm_kernel<ADJ_X, ADJ_Y, MODE, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+  qbmm_kernel<ADJ_X, ADJ_Y, MODE, MODE, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
 }
 
 template <bool ADJ_X, bool ADJ_Y, int NB, int OUT_T, bool ROWB>
 void launch_vec(const BmmArgs& a, const int8_t* x, const int8_t* y, void* out, dim3 grid, hipStream_t st) {
-  if (a.mode == kAligned) launch_tiles<ADJ_X, ADJ_Y, kAligned, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
-  else if (a.mode == kAny) launch_tiles<ADJ_X, ADJ_Y, kAny, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
-  else qbmm_kernel<ADJ_X, ADJ_Y, kBytes, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+  // An operand whose rows are too short for a load does not drag the other one along: matrix times vector, 384 products of
+  // 512 x 512 by 512 x 1, 215 us with byte loads for both, 34 us with byte loads for the vector only.  (kAny takes an aligned
+  // operand as well, its loads are the same; with adj_y alone the operands run along k together and never differ.)
+  if (a.mode_x == kAligned && a.mode_y == kAligned) launch_tiles<ADJ_X, ADJ_Y, kAligned, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
+  else if (a.mode_x != kBytes && a.mode_y != kBytes) launch_tiles<ADJ_X, ADJ_Y, kAny, NB, OUT_T, ROWB>(a, x, y, out, grid, st);
+  else if (a.mode_x == kBytes && a.mode_y == kBytes) qbmm_kernel<ADJ_X, ADJ_Y, kBytes, kBytes, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+  else if constexpr (ADJ_X || !ADJ_Y) {
+    if (a.mode_x == kBytes) qbmm_kernel<ADJ_X, ADJ_Y, kBytes, kAny, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+    else qbmm_kernel<ADJ_X, ADJ_Y, kAny, kBytes, NB, OUT_T, ROWB><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
+  }
 }
 
 template <bool ADJ_X, bool ADJ_Y, int OUT_T>
@@ -545,8 +554,8 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   // [R, K] layouts load 16 bytes along k, [K, R] layouts 4 bytes along r
   const bool vec_x = p->adj_x ? vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->M, 4) : vector_layout(x, p->x_batch_stride, p->n_batch_dims, p->K, 16);
   const bool vec_y = p->adj_y ? vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->K, 16) : vector_layout(y, p->y_batch_stride, p->n_batch_dims, p->N, 4);
-  const bool any = vector_reads_fit(!p->adj_x, p->M, p->K) && vector_reads_fit(p->adj_y, p->N, p->K);
-  a.mode = vec_x && vec_y ? kAligned : any ? kAny : kBytes;
+  a.mode_x = !vector_reads_fit(!p->adj_x, p->M, p->K) ? kBytes : vec_x ? kAligned : kAny;
+  a.mode_y = !vector_reads_fit(p->adj_y, p->N, p->K) ? kBytes : vec_y ? kAligned : kAny;
   // Tiles of 128 rows (and 128 columns) where more than 64 exist, the operands are aligned, the fused operands do not
   // depend on the row, and at least 1024 tiles remain (four per CU); else 64 x 64.  BERT-base attention over 128
   // sequences, 1536 tiles: Q.K^T + Mul + Add 24.6 -> 20.0 us, P.V 16.9 -> 14.2 us; over 32 sequences the 384 larger
@@ -554,7 +563,7 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   bool rowb = true;
   for (int b = 0; b < p->n_binary; ++b) rowb = rowb && p->binary[b].stride_m == 0;
   a.rm = a.rn = 1;
-  if (a.mode != kBytes && rowb && p->M > kTile) {
+  if (a.mode_x != kBytes && a.mode_y != kBytes && rowb && p->M > kTile) {
     const int rn = p->N > kTile ? 2 : 1;
     if (batch * ((p->M + 2 * kTile - 1) / (2 * kTile)) * ((p->N + rn * kTile - 1) / (rn * kTile)) >= 1024) {
       a.rm = 2;

@@ -59,3 +59,22 @@ def test_empty_reduction(hip, dev, adj_x, adj_y, M, N, t_out):
         hip.qbatch_matmul(p, None, None, out)
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+# one operand with rows too short for a vector load beside one with any rows: 1 to 3 columns of y, 1 to 3 columns of an adjoint
+# x, K < 16 on the side that runs along k
+@pytest.mark.parametrize("M,K,N,adj_x,adj_y", [(70, 64, 1, False, False), (66, 130, 3, False, False), (130, 37, 2, True, False),
+                                               (3, 70, 68, True, False), (1, 129, 35, True, False), (2, 16, 131, True, True),
+                                               (68, 9, 40, False, False), (37, 15, 5, True, True), (3, 8, 2, True, False)])
+@pytest.mark.parametrize("t_out", [orc.FLOAT, orc.HALF])
+def test_one_narrow_operand(hip, dev, M, K, N, adj_x, adj_y, t_out):
+    import torch
+    rng = np.random.default_rng(M * 3 + K + N)
+    x = rng.integers(-128, 128, (9,) + ((K, M) if adj_x else (M, K))).astype(np.int8)
+    y = rng.integers(-128, 128, (9,) + ((N, K) if adj_y else (K, N))).astype(np.int8)
+    binary = [(orc.BIN_MUL, rng.standard_normal((1, 1, N)).astype(np.float32)), (orc.BIN_ADD, rng.standard_normal((9, M, 1)).astype(np.float32))]
+    if t_out != orc.FLOAT:
+        binary = [(alg, to16(torch, v, t_out)) for alg, v in binary]
+    for fused in ((), binary[:1], binary):
+        check(hip, dev, x, y, adj_x, adj_y, fused, t_out)
+        check(hip, dev, x, y, adj_x, adj_y, fused, t_out, x_off=1, y_off=3)
