@@ -27,7 +27,7 @@ struct BmmArgs {
   itexhip_bmm_params p;
   int tiles_m, tiles_n;
   int mode_x, mode_y;  // kBytes, kAligned or kAny: how the operands are read
-  int xcd_grid;      // launched as (8, tiles, matrices / 8): see the kernel
+  int xcd_grid;      // launched as (8, tiles, matrices / 8), not (tiles, matrices): see the kernel
   uint32_t batch;
   FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
@@ -402,18 +402,18 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
 
   // Workgroup -> (batch entry, tile).  Consecutive workgroup ids go round the 8 XCDs.  Launched as (8, tiles, matrices / 8)
   // the XCD takes whole matrices: their operands are read into one L2, and output lines that two tiles share (rows that are
-  // no multiple of a cache line) are put together there instead of leaving two L2s in pieces.  Otherwise consecutive
+  // no multiple of a cache line) are put together there instead of leaving two L2s in pieces.  Otherwise the launch is
+  // (tiles, matrices) with the matrices over the last two dimensions (the first one ends at 2^24 workgroups), and consecutive
   // workgroups walk the tiles of one matrix.  The launch has fewer than 2^31 workgroups: 32-bit arithmetic.
   uint32_t bi, tile;  // index of the output matrix
   if (a.xcd_grid) {
     bi = blockIdx.z * 8 + blockIdx.x;
     tile = blockIdx.y;
-    if (bi >= a.batch) return;  // whole workgroup
   } else {
-    const uint32_t tiles = static_cast<uint32_t>(a.tiles_m) * static_cast<uint32_t>(a.tiles_n);
-    bi = blockIdx.x / tiles;
-    tile = blockIdx.x - bi * tiles;
+    bi = blockIdx.z * gridDim.y + blockIdx.y;
+    tile = blockIdx.x;
   }
+  if (bi >= a.batch) return;  // whole workgroup
   const int tm = a.tiles_n == 1 ? static_cast<int>(tile) : static_cast<int>(tile / a.tiles_n);
   const int m0 = tm * (RM * kTile), n0 = static_cast<int>(tile - tm * a.tiles_n) * (RN * kTile);
 
@@ -580,8 +580,9 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   a.batch = static_cast<uint32_t>(batch);
   a.xcd_grid = (batch % 8 == 0 || batch >= 64) && tiles <= 65535 && (batch + 7) / 8 <= 65535 ? 1 : 0;
   for (int d = 0; d < a.p.n_batch_dims; ++d) a.by_dim[d] = make_fast_div(a.p.batch_dims[d]);
+  const int64_t slices = (batch + 65534) / 65535;
   const dim3 g = a.xcd_grid ? dim3(8, static_cast<unsigned>(tiles), static_cast<unsigned>((batch + 7) / 8))
-                            : dim3(static_cast<unsigned>(grid));
+                            : dim3(static_cast<unsigned>(tiles), static_cast<unsigned>((batch + slices - 1) / slices), static_cast<unsigned>(slices));
   if (p->adj_x && p->adj_y) launch_layout<true, true>(a, x, y, out, g, st);
   else if (p->adj_x) launch_layout<true, false>(a, x, y, out, g, st);
   else if (p->adj_y) launch_layout<false, true>(a, x, y, out, g, st);

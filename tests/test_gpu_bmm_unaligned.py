@@ -78,3 +78,18 @@ def test_one_narrow_operand(hip, dev, M, K, N, adj_x, adj_y, t_out):
     for fused in ((), binary[:1], binary):
         check(hip, dev, x, y, adj_x, adj_y, fused, t_out)
         check(hip, dev, x, y, adj_x, adj_y, fused, t_out, x_off=1, y_off=3)
+
+
+@pytest.mark.parametrize("B0,B1,M", [(4096, 4099, 1), (3, 5, 70000 * 64 + 1), (2, 33000, 1)])
+def test_launches_of_any_extent(hip, dev, B0, B1, M):
+    """2^24 matrices and more, more tiles of a matrix than one grid dimension behind the first takes, and both ends of the
+    split of the matrices over two grid dimensions: outer products over a broadcast batch, K = N = 1."""
+    import torch
+    g = torch.Generator(device=dev).manual_seed(M + B1)
+    x = torch.randint(-128, 128, (B0, 1, M, 1), dtype=torch.int8, device=dev, generator=g)
+    y = torch.randint(-128, 128, (1, B1, 1, 1), dtype=torch.int8, device=dev, generator=g)
+    p, shape = hip.bmm_params(tuple(x.shape), tuple(y.shape), False, False, hip.FLOAT, 0.25)
+    out = torch.full(shape, 0.125, device=dev)
+    hip.qbatch_matmul(p, x, y, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, x.float() * y.float() * 0.25)
