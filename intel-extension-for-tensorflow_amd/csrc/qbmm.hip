@@ -28,7 +28,7 @@ struct BmmArgs {
   int tiles_m, tiles_n;
   int mode_x, mode_y;  // kBytes, kAligned or kAny: how the operands are read
   int xcd_grid;      // launched as (8, tiles, matrices / 8), not (tiles, matrices): see the kernel
-  uint32_t batch;
+  uint32_t batch, per_slice;  // matrices; of one index of the grid's third dimension (an argument: reading gridDim costs a load)
   FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
 };
@@ -165,6 +165,7 @@ struct QuadrantSite {
   uint32_t operand_row[ITEXHIP_BMM_MAX_BINARY], operand_col[ITEXHIP_BMM_MAX_BINARY];  // byte strides
   char* out;                                             // address of the quadrant's first output element
   uint32_t out_row;                                      // byte stride between output rows
+  bool whole;                                            // rows are whole 64-byte pieces: see store_one
 };
 
 // Operand values of the lane's 16 results.  Straight-line code: every load is issued whatever the operand's
@@ -204,13 +205,15 @@ __device__ __forceinline__ float finish_one(int acc, const QuadrantSite& s, int 
 
 // Its way out.  fp32: the output is written back as it goes instead of staying dirty in L2 until the kernel ends: as
 // system-scope (write-through) stores without fused operands (P.V over 128 sequences: 21.3 -> 18.8 us), as streaming
-// stores with them (Q.K^T + Mul + Add measured 3 % slower written through).  16-bit: plain stores, because a store covers
-// half a cache line at best and L2 puts the lines together (Q.K^T over 197 tokens, rows of 394 bytes: 31.1 us with
-// streaming stores, 19.4 us with plain ones).
-template <int OUT_T, int NB>
+// stores with them (Q.K^T + Mul + Add measured 3 % slower written through).  16-bit: streaming stores too where the rows are
+// whole 64-byte pieces, which is what a store instruction covers of a row (WHOLE; 128 tokens, 128 sequences: Q.K^T + Mul + Add
+// 15.3 us, plain stores 17.9; P.V 12.5, plain 14.5); on other rows a store covers pieces of lines, which L2 has to put
+// together first (Q.K^T over 197 tokens, 32 sequences: 24.4 us streaming, 16.3 us plain).
+template <int OUT_T, int NB, bool WHOLE>
 __device__ __forceinline__ void store_one(float v, char* dst) {
   if constexpr (OUT_T == ITEXHIP_FLOAT && NB == 0) __hip_atomic_store(reinterpret_cast<float*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   else if constexpr (OUT_T == ITEXHIP_FLOAT) __builtin_nontemporal_store(v, reinterpret_cast<float*>(dst));
+  else if constexpr (WHOLE) __builtin_nontemporal_store(static_cast<uint16_t>(f32_to_bits16<OUT_T>(v)), reinterpret_cast<uint16_t*>(dst));
   else *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(f32_to_bits16<OUT_T>(v));
 }
 
@@ -219,42 +222,28 @@ __device__ __forceinline__ void store_rows(const v16i& acc, const QuadrantSite& 
                                            const float (&o)[ITEXHIP_BMM_MAX_BINARY][ROWB ? 1 : 16]) {
   using elem_t = typename std::conditional<OUT_T == ITEXHIP_FLOAT, float, uint16_t>::type;
   const uint32_t lrow = (lane >> 5) * 4, lcol = lane & 31;
-  auto result = [&](int i) { return finish_one<NB, ROWB, ALG0, ALG1>(acc[i], s, i, o); };
-  if constexpr (OUT_T != ITEXHIP_FLOAT) {
-    // 16-bit results, all 32 columns exist: two neighbouring lanes trade one of their two rows, so that the even lane
-    // stores two columns of the upper row and the odd lane two of the lower one as a dword (at any 2-byte address: rows
-    // of an odd number of elements).  Half the store instructions; Q.K^T over 197 tokens 19.4 -> 18.4 us together with the
-    // mapping of matrices to XCDs.
-    if (s.cols_left == 32) {
-      const uint32_t odd = lane & 1;
-      const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
-      const uint32_t base = (lrow + odd) * s.out_row + (lcol & ~1u) * 2;
-      const bool whole = s.rows_left == 32;
-#pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        const uint32_t mine = f32x2_to_bits16<OUT_T>(result(i), result(i + 1));
-        const uint32_t other = __builtin_amdgcn_update_dpp(0u, mine, 0xb1, 0xf, 0xf, true);  // quad_perm 1, 0, 3, 2
-        const uint32_t r = (i >> 2) * 8 + (i & 3);
-        if (whole || static_cast<int>(lrow + odd + r) < s.rows_left)
-          *reinterpret_cast<u32_any*>(s.out + (base + r * s.out_row)) = __builtin_amdgcn_perm(other, mine, sel);
-      }
-      return;
-    }
-  }
   const uint32_t obase = lrow * s.out_row + lcol * static_cast<uint32_t>(sizeof(elem_t));
+  auto store = [&](auto whole, int i) {
+    store_one<OUT_T, NB, decltype(whole)::value>(finish_one<NB, ROWB, ALG0, ALG1>(acc[i], s, i, o),
+                                                 s.out + (obase + static_cast<uint32_t>((i >> 2) * 8 + (i & 3)) * s.out_row));
+  };
   if (s.rows_left == 32 && s.cols_left == 32) {  // a whole quadrant (the same answer for the wavefront): nothing to test
+    if (OUT_T != ITEXHIP_FLOAT && s.whole) {
+      // (the two statements without instructions keep the compiler from making plain stores of both branches' together)
+      asm volatile("" : : : "memory");
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      store_one<OUT_T, NB>(result(i), s.out + (obase + static_cast<uint32_t>((i >> 2) * 8 + (i & 3)) * s.out_row));
+      for (int i = 0; i < 16; ++i) store(std::true_type{}, i);
+      asm volatile("" : : : "memory");
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) store(std::false_type{}, i);
+    }
     return;
   }
   if (static_cast<int>(lcol) >= s.cols_left) return;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = (i >> 2) * 8 + (i & 3);
-    if (static_cast<int>(lrow) + r >= s.rows_left) continue;
-    store_one<OUT_T, NB>(result(i), s.out + (obase + r * s.out_row));
-  }
+  for (int i = 0; i < 16; ++i)
+    if (static_cast<int>(lrow) + (i >> 2) * 8 + (i & 3) < s.rows_left) store(std::false_type{}, i);
 }
 
 // The operands' algorithms are the same for the whole launch: one copy of the store loop per combination, chosen by
@@ -310,6 +299,7 @@ __device__ __forceinline__ QuadrantSite quadrant_site(const itexhip_bmm_params& 
   }
   s.out = static_cast<char*>(out) + ((static_cast<int64_t>(bi) * p.M + qm) * p.N + qn) * esz;
   s.out_row = static_cast<uint32_t>(p.N) * esz;
+  s.whole = ((reinterpret_cast<uintptr_t>(out) | s.out_row) & 63) == 0;
   return s;
 }
 
@@ -402,17 +392,11 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
 
   // Workgroup -> (batch entry, tile).  Consecutive workgroup ids go round the 8 XCDs.  Launched as (8, tiles, matrices / 8)
   // the XCD takes whole matrices: their operands are read into one L2, and output lines that two tiles share (rows that are
-  // no multiple of a cache line) are put together there instead of leaving two L2s in pieces.  Otherwise the launch is
+  // no whole 64-byte pieces) are put together there instead of leaving two L2s in pieces.  Otherwise the launch is
   // (tiles, matrices) with the matrices over the last two dimensions (the first one ends at 2^24 workgroups), and consecutive
   // workgroups walk the tiles of one matrix.  The launch has fewer than 2^31 workgroups: 32-bit arithmetic.
-  uint32_t bi, tile;  // index of the output matrix
-  if (a.xcd_grid) {
-    bi = blockIdx.z * 8 + blockIdx.x;
-    tile = blockIdx.y;
-  } else {
-    bi = blockIdx.z * gridDim.y + blockIdx.y;
-    tile = blockIdx.x;
-  }
+  const uint32_t bi = blockIdx.z * a.per_slice + (a.xcd_grid ? blockIdx.x : blockIdx.y);  // index of the output matrix
+  const uint32_t tile = a.xcd_grid ? blockIdx.y : blockIdx.x;
   if (bi >= a.batch) return;  // whole workgroup
   const int tm = a.tiles_n == 1 ? static_cast<int>(tile) : static_cast<int>(tile / a.tiles_n);
   const int m0 = tm * (RM * kTile), n0 = static_cast<int>(tile - tm * a.tiles_n) * (RN * kTile);
@@ -575,14 +559,19 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   const int64_t grid = batch * a.tiles_m * a.tiles_n;
   ITEXHIP_REQUIRE(grid < (1LL << 31), "%s: %lld output tiles exceed one launch", who, static_cast<long long>(grid));
   hipStream_t st = as_stream(stream);
-  // Whole matrices per XCD where there are enough of them to keep all 8 equally busy.
+  // Whole matrices per XCD where rows are ragged, in the output or in an operand, and there are enough matrices to keep all 8
+  // equally busy: 32 sequences of 197 tokens, fp32, Q.K^T + Mul + Add 45.7 -> 40.2 us, P.V 10.2 -> 9.1 us (bfloat16: 9.9 -> 9.5).
+  // Tiles of a matrix spread over the XCDs where nothing is ragged: bfloat16, 128 tokens, 32 sequences, Q.K^T 7.0 -> 6.4 us,
+  // 32 heads of 384 tokens 6.2 -> 5.8 us (fp32 differs by 0.1 us either way).
   const int64_t tiles = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
   a.batch = static_cast<uint32_t>(batch);
-  a.xcd_grid = (batch % 8 == 0 || batch >= 64) && tiles <= 65535 && (batch + 7) / 8 <= 65535 ? 1 : 0;
+  const bool ragged = a.mode_x != kAligned || a.mode_y != kAligned || (p->N * (p->out_type == ITEXHIP_FLOAT ? 4 : 2)) % 64 != 0;
+  a.xcd_grid = ragged && (batch % 8 == 0 || batch >= 64) && tiles <= 65535 && (batch + 7) / 8 <= 65535 ? 1 : 0;
   for (int d = 0; d < a.p.n_batch_dims; ++d) a.by_dim[d] = make_fast_div(a.p.batch_dims[d]);
   const int64_t slices = (batch + 65534) / 65535;
+  a.per_slice = static_cast<uint32_t>(a.xcd_grid ? 8 : (batch + slices - 1) / slices);
   const dim3 g = a.xcd_grid ? dim3(8, static_cast<unsigned>(tiles), static_cast<unsigned>((batch + 7) / 8))
-                            : dim3(static_cast<unsigned>(tiles), static_cast<unsigned>((batch + slices - 1) / slices), static_cast<unsigned>(slices));
+                            : dim3(static_cast<unsigned>(tiles), a.per_slice, static_cast<unsigned>(slices));
   if (p->adj_x && p->adj_y) launch_layout<true, true>(a, x, y, out, g, st);
   else if (p->adj_x) launch_layout<true, false>(a, x, y, out, g, st);
   else if (p->adj_y) launch_layout<false, true>(a, x, y, out, g, st);

@@ -93,3 +93,21 @@ def test_launches_of_any_extent(hip, dev, B0, B1, M):
     hip.qbatch_matmul(p, x, y, out)
     torch.cuda.synchronize()
     assert torch.equal(out, x.float() * y.float() * 0.25)
+
+
+@pytest.mark.parametrize("N", [32, 64, 96, 128, 131])
+@pytest.mark.parametrize("off", [0, 1, 16, 32])
+def test_16_bit_rows(hip, dev, N, off):
+    """16-bit results whose rows are whole 64-byte pieces or not, by their length or by the address of the output (elements)."""
+    import torch
+    g = torch.Generator(device=dev).manual_seed(N + off)
+    x = torch.randint(-128, 128, (8, 69, 64), dtype=torch.int8, device=dev, generator=g)
+    y = torch.randint(-128, 128, (8, N, 64), dtype=torch.int8, device=dev, generator=g)
+    p, shape = hip.bmm_params(tuple(x.shape), tuple(y.shape), False, True, hip.BFLOAT16, 0.03125)
+    n = 8 * 69 * N
+    buf = torch.full((n + 128,), 7.0, dtype=torch.bfloat16, device=dev)
+    hip.qbatch_matmul(p, x, y, buf[off:])
+    torch.cuda.synchronize()
+    want = (torch.bmm(x.cpu().float(), y.cpu().float().transpose(1, 2)) * 0.03125).bfloat16()
+    assert torch.equal(buf[off:off + n].cpu().view(shape), want)
+    assert bool((buf[:off] == 7.0).all()) and bool((buf[off + n:] == 7.0).all())
