@@ -244,41 +244,44 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   }
 }
 
-// An operand of fewer than 16 bytes in all (K < 16), or too many tiles for a launch: one thread per output element.
+// An operand of fewer than 16 bytes in all (K < 16), or too many tiles for a launch: one thread per output element, several
+// where there are more outputs than a launch has threads (2^32 in one dimension; a larger grid is cut off without an error).
 template <int OUT_T>
 __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __restrict__ a, int a_is_u8,
                                                             const int8_t* __restrict__ w, int transpose_b,
                                                             int M, int K, int N, EpilogueArgs e,
                                                             void* __restrict__ out) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= static_cast<int64_t>(M) * N) return;
-  const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
-  int acc = 0, wsum = 0;
-  for (int k = 0; k < K; ++k) {
-    const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
-                           : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
-    const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
-    acc += av * wv;
-    wsum += wv;
+  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < static_cast<int64_t>(M) * N;
+       idx += static_cast<int64_t>(gridDim.x) * 256) {
+    const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
+    int acc = 0, wsum = 0;
+    for (int k = 0; k < K; ++k) {
+      const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
+                             : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
+      const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
+      acc += av * wv;
+      wsum += wv;
+    }
+    const int jb = (e.nb == N) ? n : 0;
+    const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
+                                                  bias_entry(e.prep, e.bias, n), wsum);
+    float v = static_cast<float>(acc);
+    if (e.n_scales > 0) v = v * c.scale;
+    v = v + c.bias;
+    for (int k = 0; k < e.n_eltwise; ++k) {
+      if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
+      else v = apply_eltwise(e.elt[k], v);
+    }
+    store_output<OUT_T>(out, idx, v);
   }
-  const int jb = (e.nb == N) ? n : 0;
-  const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
-                                                bias_entry(e.prep, e.bias, n), wsum);
-  float v = static_cast<float>(acc);
-  if (e.n_scales > 0) v = v * c.scale;
-  v = v + c.bias;
-  for (int k = 0; k < e.n_eltwise; ++k) {
-    if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
-    else v = apply_eltwise(e.elt[k], v);
-  }
-  store_output<OUT_T>(out, idx, v);
 }
 
 template <int OUT_T>
 void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
             const EpilogueArgs& e, void* out, hipStream_t st) {
   if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16) {
-    qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((static_cast<int64_t>(M) * N + 255) / 256), 256, 0, st>>>(
+    const int64_t blocks = std::min<int64_t>((static_cast<int64_t>(M) * N + 255) / 256, 1 << 23);
+    qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>(blocks), 256, 0, st>>>(
         a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out);
     return;
   }
@@ -293,10 +296,8 @@ void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b,
 int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
                     const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who) {
   const int64_t tiles_m = (M + kTileM - 1) / kTileM, tiles_n = (N + kTileN - 1) / kTileN;
-  // 2^32 threads at most; a result of more tiles than that allows is long and narrow (2^30 rows or columns and more) and goes
-  // one thread per output element
+  // a launch has fewer than 2^32 threads; a result of more tiles than that allows goes one thread per output element
   const bool many_tiles = tiles_m * tiles_n >= (1LL << 24) - 8;
-  ITEXHIP_REQUIRE(!many_tiles || (M < (1LL << 32) / N), "%s: output too large for one launch", who);
   const uint8_t* ap = static_cast<const uint8_t*>(a);
   const uint8_t* wp = reinterpret_cast<const uint8_t*>(w);
   const uint32_t a_xor = a_type == ITEXHIP_QUINT8 ? 0x80808080u : 0u;

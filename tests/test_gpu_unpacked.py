@@ -50,3 +50,24 @@ def test_more_rows_than_tiles_in_a_launch(hip, dev):
     hip.qmatmul_unpacked(p, a, w, False, M, 1, 1, lo, hi, 1, torch.zeros(1, device=dev), out)
     torch.cuda.synchronize()
     assert torch.equal(out, a)
+
+
+def test_more_outputs_than_threads_in_a_launch(hip, dev):
+    """K * N < 16 with more than 2^32 outputs: one thread per output element, several per thread.  The first 128 rows hold every
+    input value once; every later row must be a copy of one of them."""
+    import torch
+    rows, N = (1 << 32) // 15 // 128 + 1000, 15
+    M = rows * 128
+    if torch.cuda.mem_get_info()[0] < 24 * M:
+        pytest.skip("needs 7 GiB")
+    p = hip.matmul_params(t_in=hip.QINT8, t_out=hip.QINT8, input_mode=hip.SCALED, min_a=-127.0, max_a=127.0, has_requantize=True,
+                          min_out=-127.0, max_out=127.0)
+    a = torch.arange(128, dtype=torch.int8, device=dev).repeat(rows)
+    w = torch.arange(-7, 8, dtype=torch.int8, device=dev)
+    lo, hi = torch.full((1,), -16.0, device=dev), torch.full((1,), 16.0, device=dev)
+    out = torch.full((rows, 128, N), -1, dtype=torch.int8, device=dev)
+    hip.qmatmul_unpacked(p, a, w, False, M, 1, N, lo, hi, 1, torch.zeros(N, device=dev), out)
+    torch.cuda.synchronize()
+    want = (torch.arange(128).view(-1, 1) * torch.arange(-7, 8).view(1, -1) * (16.0 / 127.0))
+    assert float((out[0].cpu().float() - want.round()).abs().max()) <= 1.0   # the sizes are the point here, not the rounding
+    assert bool((out == out[:1]).all())
