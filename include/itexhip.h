@@ -50,7 +50,8 @@ const char* itexhip_last_error(void);
 const char* itexhip_build_info(void);
 /* Test hook (no counterpart in the reference): forces the tile shape of the MatMul tile kernel (0..4 = 256x256,
  * 256x192, 256x128, 128x128, 64x64) and of the implicit-GEMM Conv2D (0..2 = 256x128, 128x128, 64x64), or (16) the kernel for
- * a short K at any size, for every later call of the process; -1 gives the choice back to the library.  Results do not depend on the shape. */
+ * a short K at any size, for every later call of the process; any of them also keeps a MatMul on unpacked operands with its
+ * tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */
 void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape);
 
 /* ------------------------------------------------------------------------------------------
@@ -350,7 +351,8 @@ int itexhip_qmatmul_device_range(const itexhip_matmul_params* p, const void* a, 
 
 /* itexhip_qmatmul on the unpacked TF-layout weight ([K, N], or [N, K] with transpose_b), any K, no
  * prepack and no column-sum buffer, no alignment: an MFMA kernel that fetches both operands with unaligned
- * vector loads and sums the weight's columns on the way.  For the shapes the packed kernels do not take
+ * vector loads and sums the weight's columns on the way, or one thread per output for short dot products of
+ * narrow results.  For the shapes the packed kernels do not take
  * (K not a multiple of 16). */
 int itexhip_qmatmul_unpacked(const itexhip_matmul_params* p, const void* a, const int8_t* w, int transpose_b,
                              int64_t M, int64_t K, int64_t N, const float* min_b, const float* max_b,

@@ -13,8 +13,8 @@
 // Zero-point compensation needs the weight's column sums; they are dot products with ones of the words on their way into
 // LDS (16 instructions per thread and step), added up across the workgroup once at the end.
 //
-// One thread per output element with byte loads, which this replaces, was bound by its loads (two bytes per
-// multiplication): 1000 x 1001 x 1000 with an fp32 result 399 -> 10.7 us, 37 times.
+// One thread per output element with byte loads is bound by its loads (two bytes per multiplication): 1000 x 1001 x 1000 with
+// an fp32 result 399 -> 10.7 us, 37 times.  Short dot products of narrow results still go that way.
 #include "qgemm_common.hpp"
 
 namespace itexhip {
@@ -244,45 +244,61 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   }
 }
 
-// An operand of fewer than 16 bytes in all (K < 16), or too many tiles for a launch: one thread per output element, several
-// where there are more outputs than a launch has threads (2^32 in one dimension; a larger grid is cut off without an error).
+// One thread per output element, from `first` on (a launch has fewer than 2^32 threads in one dimension; a larger grid is cut
+// off without an error.  A loop over the outputs in here costs 20 %).  Takes what the tile kernel cannot (an operand of fewer
+// than 16 bytes in all, too many tiles for a launch) and short dot products of narrow results, see one_output_per_thread.
 template <int OUT_T>
 __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __restrict__ a, int a_is_u8,
                                                             const int8_t* __restrict__ w, int transpose_b,
                                                             int M, int K, int N, EpilogueArgs e,
-                                                            void* __restrict__ out) {
-  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < static_cast<int64_t>(M) * N;
-       idx += static_cast<int64_t>(gridDim.x) * 256) {
-    const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
-    int acc = 0, wsum = 0;
-    for (int k = 0; k < K; ++k) {
-      const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
-                             : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
-      const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
-      acc += av * wv;
-      wsum += wv;
-    }
-    const int jb = (e.nb == N) ? n : 0;
-    const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
-                                                  bias_entry(e.prep, e.bias, n), wsum);
-    float v = static_cast<float>(acc);
-    if (e.n_scales > 0) v = v * c.scale;
-    v = v + c.bias;
-    for (int k = 0; k < e.n_eltwise; ++k) {
-      if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
-      else v = apply_eltwise(e.elt[k], v);
-    }
-    store_output<OUT_T>(out, idx, v);
+                                                            void* __restrict__ out, int64_t first) {
+  const int64_t idx = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (idx >= static_cast<int64_t>(M) * N) return;
+  const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
+  int acc = 0, wsum = 0;
+  for (int k = 0; k < K; ++k) {
+    const int av = a_is_u8 ? static_cast<int>(a[static_cast<int64_t>(m) * K + k])
+                           : static_cast<int>(reinterpret_cast<const int8_t*>(a)[static_cast<int64_t>(m) * K + k]);
+    const int wv = transpose_b ? w[static_cast<int64_t>(n) * K + k] : w[static_cast<int64_t>(k) * N + n];
+    acc += av * wv;
+    wsum += wv;
   }
+  const int jb = (e.nb == N) ? n : 0;
+  const ChannelScaleBias c = channel_scale_bias(e.prep, e.min_b[jb], e.max_b[jb], e.min_b[0], e.max_b[0],
+                                                bias_entry(e.prep, e.bias, n), wsum);
+  float v = static_cast<float>(acc);
+  if (e.n_scales > 0) v = v * c.scale;
+  v = v + c.bias;
+  for (int k = 0; k < e.n_eltwise; ++k) {
+    if (e.elt[k].alg == ITEXHIP_ELT_SUM) v = v + e.elt[k].alpha * load_addend(e, idx);
+    else v = apply_eltwise(e.elt[k], v);
+  }
+  store_output<OUT_T>(out, idx, v);
+}
+
+// Short dot products of narrow results: a tile of the other kernel costs the same whether one of its rows or columns exists
+// or all 64 do, and however much of its first K step.  Times in us as both kernels measured (fp32 results; 554 sizes of 1 to
+// 1 000 000 rows and columns, K of 3 to 129): a thread's dot product 0.075 K (latency) + 1e-6 per output and 3.3 + 0.25 K for
+// up to 64 columns, 0.6 K for more, or, where the rows are far apart, 0.025 K^2 + 3 per row; tiles 2.8 + 0.009 each, 0.0045
+// more and 0.9 in all per further K step.  The faster kernel is chosen to within 10 %, for 4 sizes to within 26 %.
+// Per output / tiles: 100000 x 17 x 1 4.8 / 20.7, 1 x 17 x 100000 5.3 / 20.3, 1000000 x 9 x 16 99 / 143, 8 x 9 x 8 3.6 / 6.0,
+// 1000 x 27 x 8 5.3 / 6.6; 1000 x 49 x 8 7.0 / 6.6, 100000 x 65 x 10 57 / 21, 1000 x 17 x 1000 11.3 / 6.8.
+bool one_output_per_thread(int64_t M, int64_t K, int64_t N, int64_t tiles) {
+  const double k = static_cast<double>(K);
+  const double row = std::max(static_cast<double>(N) * (3.3 + (N <= 64 ? 0.25 : 0.6) * k), 0.025 * k * k + 3.0);
+  const double steps = static_cast<double>((K + kStepK - 1) / kStepK);
+  return 0.075 * k + 1e-6 * static_cast<double>(M) * row < 2.8 + 0.9 * (steps - 1.0) + 0.0045 * (1.0 + steps) * static_cast<double>(tiles);
 }
 
 template <int OUT_T>
 void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
             const EpilogueArgs& e, void* out, hipStream_t st) {
-  if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16) {
-    const int64_t blocks = std::min<int64_t>((static_cast<int64_t>(M) * N + 255) / 256, 1 << 23);
-    qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>(blocks), 256, 0, st>>>(
-        a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out);
+  const bool forced = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0;  // tests ask for the tile kernel
+  if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16 || (!forced && one_output_per_thread(M, K, N, tiles))) {
+    const int64_t outputs = static_cast<int64_t>(M) * N, at_once = 1LL << 31;
+    for (int64_t first = 0; first < outputs; first += at_once)
+      qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((std::min(outputs - first, at_once) + 255) / 256), 256, 0, st>>>(
+          a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out, first);
     return;
   }
   const unsigned grid = static_cast<unsigned>((tiles + 7) / 8 * 8);  // whole runs for the 8 XCDs
