@@ -15,6 +15,7 @@ struct TransposeArgs {
   int64_t in_stride[kMaxRank];  // stride in the input (in units) of output dimension i
   int64_t out_stride[kMaxRank];
   FastDiv by_dim[kMaxRank];     // small tensors: division by out_dims[i]
+  int units;                    // small tensors: units per thread, 1 or 2
   int64_t total;              // number of units
 };
 
@@ -37,19 +38,18 @@ __global__ __launch_bounds__(256) void transpose_kernel(const TransposeArgs a, c
   }
 }
 
-// The same for fewer than 2^31 units (every index fits 32 bits): coordinates by multiply-shift divisions, kUnits loads of a
+// The same for fewer than 2^31 units (every index fits 32 bits): coordinates by multiply-shift divisions, UNITS loads of a
 // thread in flight before it stores, and the dimensions walked in whichever of the two tensors' orders the host found
-// better (see below).  Bound by memory; three head splits and one merge of 128 x 128 x 12 x 64 bytes: 7.8 us each on average
+// better (see walk_order).  Bound by memory; three head splits and one merge of 128 x 128 x 12 x 64 bytes: 7.8 us each on average
 // with 64-bit divisions in the output's order, 7.8 us with these divisions alone, 6.3 us with the order as well.
-constexpr int kUnits = 2;
-template <typename unit_t, int RANK>
+template <typename unit_t, int RANK, int UNITS>
 __global__ __launch_bounds__(256) void transpose_small_kernel(const TransposeArgs a, const unit_t* __restrict__ x,
                                                               unit_t* __restrict__ y) {
-  const uint32_t o0 = blockIdx.x * (256u * kUnits) + threadIdx.x, total = static_cast<uint32_t>(a.total);
-  unit_t v[kUnits];
-  uint32_t dst[kUnits];
+  const uint32_t o0 = blockIdx.x * (256u * UNITS) + threadIdx.x, total = static_cast<uint32_t>(a.total);
+  unit_t v[UNITS];
+  uint32_t dst[UNITS];
 #pragma unroll
-  for (int u = 0; u < kUnits; ++u) {
+  for (int u = 0; u < UNITS; ++u) {
     uint32_t rem = min(o0 + u * 256u, total - 1), src = 0;  // past the end: reads the last unit, stores nothing
     dst[u] = 0;
 #pragma unroll
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void transpose_small_kernel(const TransposeArg
     v[u] = x[src];
   }
 #pragma unroll
-  for (int u = 0; u < kUnits; ++u)
+  for (int u = 0; u < UNITS; ++u)
     if (o0 + u * 256u < total) y[dst[u]] = v[u];
 }
 
@@ -73,13 +73,59 @@ void launch(const TransposeArgs& a, const void* x, void* y, hipStream_t st) {
   const unit_t* xp = static_cast<const unit_t*>(x);
   unit_t* yp = static_cast<unit_t*>(y);
   if (a.total < (1LL << 31)) {
-    const unsigned blocks = static_cast<unsigned>((a.total + 256 * kUnits - 1) / (256 * kUnits));
-    if (a.rank <= 4) transpose_small_kernel<unit_t, 4><<<blocks, 256, 0, st>>>(a, xp, yp);
-    else transpose_small_kernel<unit_t, kMaxRank><<<blocks, 256, 0, st>>>(a, xp, yp);
+    const unsigned blocks = static_cast<unsigned>((a.total + 256 * a.units - 1) / (256 * a.units));
+    if (a.units == 1) {
+      if (a.rank <= 4) transpose_small_kernel<unit_t, 4, 1><<<blocks, 256, 0, st>>>(a, xp, yp);
+      else transpose_small_kernel<unit_t, kMaxRank, 1><<<blocks, 256, 0, st>>>(a, xp, yp);
+    } else {
+      if (a.rank <= 4) transpose_small_kernel<unit_t, 4, 2><<<blocks, 256, 0, st>>>(a, xp, yp);
+      else transpose_small_kernel<unit_t, kMaxRank, 2><<<blocks, 256, 0, st>>>(a, xp, yp);
+    }
     return;
   }
   const int64_t blocks = std::min<int64_t>((a.total + 255) / 256, 256 * 16);
   transpose_kernel<unit_t><<<static_cast<unsigned>(blocks), 256, 0, st>>>(a, xp, yp);
+}
+
+// Order and units per thread of a small tensor.  Both tensors are walked in runs: the innermost dimension where it is
+// contiguous in both, else single units.  Next to the run the output has a dimension of r, the input one of c.
+// Runs of 4 units and more (64 bytes of a 16-byte unit): in the input's order where c < r (the head split: c = 12 heads, r =
+// 128 tokens): a workgroup reads whole lines and writes runs of r instead of touching every line of the input once per head;
+// two units per thread (1000 x 32 x 64 bytes, 32 of them: 24.5 us one unit, output's order; 21.2).
+// Shorter runs: the same, where c is at most half of r, the r destinations of a workgroup's reads are worth a line (c * run
+// up to 64) or do not lie a power of two apart; one unit per thread (its neighbours' units are other lines), or two where the
+// rows of the input share lines.  us, output's / input's order: 1000 x 32 x 16 bytes 11.7 / 6.7, 1000 x 7 x 600 x 16 74 / 58,
+// 4096 x 256 x 16 8.4 / 17.6, 4096 x 1024 x 16 22.8 / 39.9, 12 x 197 x 16 2.4 / 3.1; one / two units: 1024 x 1024 x 16 9.6 /
+// 15.0, 1024 x 4096 x 16 30.6 / 49.9, 300 x 301 x 16 52.7 / 42.7.
+// Bytes: always two but for small tensors (300 x 301 x 302 reversed 205 us, one unit 338; 1024 x 1024 5.9, one unit 4.8).
+void walk_order(TransposeArgs& a, int unit) {
+  int n = a.rank;
+  const bool in_runs = a.in_stride[n - 1] == 1 && a.out_dims[n - 1] > 1;
+  if (n > 1 && a.out_dims[n - 1] == 1) a.rank = --n;  // one unit: no dimension of its own
+  int order[kMaxRank];
+  for (int i = 0; i < n; ++i) order[i] = i;
+  std::sort(order, order + n, [&](int p, int q) { return a.in_stride[p] > a.in_stride[q]; });
+  bool by_input = false;
+  a.units = 2;
+  const int next = in_runs ? n - 2 : n - 1;
+  if (next >= 0) {
+    const int64_t run = in_runs ? a.out_dims[n - 1] : 1, r = a.out_dims[next], c = a.out_dims[order[next]];
+    if (in_runs && (run >= 4 || unit == 1)) {
+      by_input = c < r;
+    } else if (unit > 1) {
+      by_input = 2 * c <= r && r >= 32 && (c * run <= 64 || (r * run * unit) % 4096 != 0);
+      a.units = unit == 16 && !by_input && (c * run * unit) % 128 != 0 ? 2 : 1;
+    } else if (a.total <= 1 << 20) {
+      a.units = 1;
+    }
+  }
+  if (!by_input) return;
+  const TransposeArgs b = a;
+  for (int i = 0; i < n; ++i) {
+    a.out_dims[i] = b.out_dims[order[i]];
+    a.in_stride[i] = b.in_stride[order[i]];
+    a.out_stride[i] = b.out_stride[order[i]];
+  }
 }
 
 }  // namespace
@@ -149,23 +195,8 @@ extern "C" int itexhip_transpose(const void* x, void* y, int elem_size, int rank
   if (a.total < (1LL << 31)) {
     int64_t s = 1;
     for (int i = n - 1; i >= 0; --i) { a.out_stride[i] = s; s *= a.out_dims[i]; }
-    // Both tensors are walked in runs of the innermost dimension.  Where the next dimension is the shorter one in the input
-    // (the head split: 12 heads there, 128 tokens in the output), walking in the input's order lets one workgroup read
-    // whole lines and write runs of the other dimension, instead of touching every line of the input once per head.
-    if (n >= 3 && a.in_stride[n - 1] == 1) {
-      int order[kMaxRank];
-      for (int i = 0; i < n; ++i) order[i] = i;
-      std::sort(order, order + n, [&](int p, int q) { return a.in_stride[p] > a.in_stride[q]; });
-      if (a.out_dims[order[n - 2]] < a.out_dims[n - 2]) {
-        const TransposeArgs b = a;
-        for (int i = 0; i < n; ++i) {
-          a.out_dims[i] = b.out_dims[order[i]];
-          a.in_stride[i] = b.in_stride[order[i]];
-          a.out_stride[i] = b.out_stride[order[i]];
-        }
-      }
-    }
-    for (int i = 0; i < n; ++i) a.by_dim[i] = make_fast_div(a.out_dims[i]);
+    walk_order(a, unit);
+    for (int i = 0; i < a.rank; ++i) a.by_dim[i] = make_fast_div(a.out_dims[i]);
   }
   hipStream_t st = as_stream(stream);
   if (unit == 16) launch<i4>(a, x, y, st);

@@ -15,3 +15,16 @@ pytestmark = pytest.mark.gpu
 def test_walk_order(hip, dev, shape, perm, dtype):
     x = np.random.default_rng(sum(shape)).integers(-128, 128, shape).astype(dtype)
     np.testing.assert_array_equal(run_transpose(hip, dev, x, perm), np.transpose(x, perm))
+
+
+# runs of one unit (16 bytes of int8, one int32) and of a few, in the input's order and in the output's, one and two units per
+# thread: rows that share lines, destinations a power of two apart, remainders of a workgroup, bytes on both sides of 2^20
+@pytest.mark.parametrize("shape,perm", [
+    ((64, 7, 16), (1, 0, 2)), ((1000, 32, 16), (1, 0, 2)), ((32, 1000, 16), (1, 0, 2)), ((256, 128, 16), (1, 0, 2)),
+    ((101, 67, 16), (1, 0, 2)), ((50, 9, 80, 16), (2, 1, 0, 3)), ((100, 20, 32), (1, 0, 2)), ((20, 100, 48), (1, 0, 2)),
+    ((33, 16, 4), (1, 0, 2)), ((200, 3, 70, 4), (2, 0, 1, 3)), ((3, 1, 64, 16), (2, 1, 0, 3)), ((16, 16), (1, 0)),
+    ((1024, 1024), (1, 0)), ((1025, 1024), (1, 0)), ((70, 16, 1), (1, 0, 2))])
+@pytest.mark.parametrize("dtype", [np.int8, np.int32])
+def test_short_runs(hip, dev, shape, perm, dtype):
+    x = np.random.default_rng(sum(shape)).integers(-128, 128, shape).astype(dtype)
+    np.testing.assert_array_equal(run_transpose(hip, dev, x, perm), np.transpose(x, perm))
