@@ -1111,13 +1111,18 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
     } else {
       const bool vec = depth % 4 == 0 && aligned(x, 16);
       const int per = vec ? 4 : 1;
-      const int groups = static_cast<int>(std::min<int64_t>(depth / per, vec ? 64 : kThreads));
-      const int side = kThreads / groups;
-      // At most one workgroup per CU (a row chunk costs an atomic pair per channel; 8192 x 4096: 256 workgroups 23.8 us, 384
-      // and 512 26.8, 1024 29.8), each thread at least two rounds of loads
+      int groups = static_cast<int>(std::min<int64_t>(depth / per, vec ? 64 : kThreads));
       const int64_t col_blocks = (depth / per + groups - 1) / groups;
       ITEXHIP_REQUIRE(col_blocks <= 65535, "itexhip_minmax_i32_per_channel: depth too large");
-      int64_t row_blocks = std::max<int64_t>(1, kChannelBlocks / col_blocks);
+      // 16-byte loads: column blocks of one width (400000 x 260: 87 -> 73 us).  Single ints lose by it (100000 x 257: 28 -> 34).
+      if (vec) groups = static_cast<int>((depth / per + col_blocks - 1) / col_blocks);
+      const int side = kThreads / groups;
+      // At most one workgroup per CU (a row chunk costs an atomic pair per channel; 8192 x 4096: 256 workgroups 23.8 us, 384
+      // and 512 26.8, 1024 29.8), each thread at least two rounds of loads.  Single ints have a quarter of the bytes in flight:
+      // one workgroup per 256 KB, up to 1024 (256 / 512 / 1024 workgroups: 16384 x 197 9.5 / 13.8 / 23.2 us, 100000 x 257 39.6 /
+      // 28.6 / 28.4, 400000 x 257 222 / 126 / 83, 1000000 x 197 284 / 171 / 142).
+      const int64_t budget = vec ? kChannelBlocks : std::min<int64_t>(4 * kChannelBlocks, std::max<int64_t>(kChannelBlocks, rows * depth >> 16));
+      int64_t row_blocks = std::max<int64_t>(1, budget / col_blocks);
       const int64_t rpb = std::max<int64_t>(2 * kRowUnroll * side, (rows + row_blocks - 1) / row_blocks);
       row_blocks = (rows + rpb - 1) / rpb;
       dim3 grid(static_cast<unsigned>(row_blocks), static_cast<unsigned>(col_blocks));
