@@ -663,12 +663,13 @@ __global__ __launch_bounds__(kSmallThreads) void quantize_dynamic_small_kernel(c
 }
 
 // Per-row (per-token) form: workgroup m reduces row m, derives its parameters and quantizes it; the rows' output
-// ranges go to two device arrays (what itexhip_qmatmul_per_row takes).  Bound by latency: a decode batch is 1 - 16 workgroups.
-// So a thread has its first HELD groups of 4 elements in flight at once and keeps them for the quantization (HELD: 1, 2 or 4,
-// the fewest that hold the row; what lies beyond 16384 columns is read twice), and every wavefront finishes the reduction by
-// itself instead of waiting for one thread's walk over 16 partial results.
-// One row, kernel time: 14336 columns 4.0 -> 3.4 us, 4096 columns 2.5 -> 2.6 us; a decoder's feed-forward step over one token
-// (both of them and two linears) 29.6 -> 28.9 us.
+// ranges go to two device arrays (what itexhip_qmatmul_per_row takes).  Bound by latency for a decode batch, 1 - 16
+// workgroups: a thread has its first HELD groups of 4 elements in flight at once and keeps them for the quantization (HELD: 1,
+// 2 or 4, the fewest that hold the row; what lies beyond 16384 columns is read twice), and the first wavefront finishes the
+// reduction with shuffles instead of one thread's walk over 16 partial results.  Many rows are bound by instructions: only
+// that wavefront derives the parameters (a division in double precision among them), and wavefronts past the end of a short
+// row load nothing (both by every wavefront: 100000 x 64 380 us, 20000 x 512 80; 291 and 60 this way).
+// One row, kernel time: 14336 columns 3.9 -> 3.5 us, 4096 columns 3.0 -> 2.9 us.
 constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
 
@@ -678,7 +679,7 @@ __global__ __launch_bounds__(kRowThreads) void quantize_dynamic_rows_kernel(cons
                                                                             float* __restrict__ row_min,
                                                                             float* __restrict__ row_max, int mode,
                                                                             float ensure_minimum_range) {
-  __shared__ float red_min[kRowWaves], red_max[kRowWaves];
+  __shared__ float red_min[kRowWaves], red_max[kRowWaves], params[2];
   const float* xr = x + static_cast<int64_t>(blockIdx.x) * cols;
   uint8_t* qr = q + static_cast<int64_t>(blockIdx.x) * cols;
   const f4* x4 = reinterpret_cast<const f4*>(xr);
@@ -690,10 +691,13 @@ __global__ __launch_bounds__(kRowThreads) void quantize_dynamic_rows_kernel(cons
   };
   f4 held[HELD > 0 ? HELD : 1];
   if constexpr (HELD > 0) {
+    const bool any = HELD > 1 || __builtin_amdgcn_readfirstlane(tid) < n4;  // short row: wavefronts without any of it
+    if (any) {
 #pragma unroll
-    for (int u = 0; u < HELD; ++u) held[u] = x4[min(tid + u * kRowThreads, n4 - 1)];  // past the end: the last group again
+      for (int u = 0; u < HELD; ++u) held[u] = x4[min(tid + u * kRowThreads, n4 - 1)];  // past the end: the last group again
 #pragma unroll
-    for (int u = 0; u < HELD; ++u) reduce(held[u]);
+      for (int u = 0; u < HELD; ++u) reduce(held[u]);
+    }
     if constexpr (HELD == 4)
       for (int i = tid + HELD * kRowThreads; i < n4; i += kRowThreads) reduce(x4[i]);
   } else {
@@ -712,29 +716,35 @@ __global__ __launch_bounds__(kRowThreads) void quantize_dynamic_rows_kernel(cons
     red_max[tid >> 6] = mx;
   }
   __syncthreads();
-  mn = red_min[tid & (kRowWaves - 1)];
-  mx = red_max[tid & (kRowWaves - 1)];
+  if (tid < 64) {
+    mn = red_min[tid & (kRowWaves - 1)];
+    mx = red_max[tid & (kRowWaves - 1)];
 #pragma unroll
-  for (int o = kRowWaves / 2; o > 0; o >>= 1) {
-    mn = fminf(mn, __shfl_xor(mn, o, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    for (int o = kRowWaves / 2; o > 0; o >>= 1) {
+      mn = fminf(mn, __shfl_xor(mn, o, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    }
+    const DynamicParams p = dynamic_params(mn, mx, T, mode, ensure_minimum_range);
+    if (tid == 0) {
+      row_min[blockIdx.x] = p.out_min;
+      row_max[blockIdx.x] = p.out_max;
+      params[0] = p.scale;
+      params[1] = p.addend;
+    }
   }
-  const DynamicParams p = dynamic_params(mn, mx, T, mode, ensure_minimum_range);
-  if (tid == 0) {
-    row_min[blockIdx.x] = p.out_min;
-    row_max[blockIdx.x] = p.out_max;
-  }
+  __syncthreads();
+  const float scale = params[0], addend = params[1];
   if constexpr (HELD > 0) {
     uint32_t* q4 = reinterpret_cast<uint32_t*>(qr);
 #pragma unroll
     for (int u = 0; u < HELD; ++u)
-      if (tid + u * kRowThreads < n4) q4[tid + u * kRowThreads] = quantize4<T>(held[u], p.scale, p.addend);
+      if (tid + u * kRowThreads < n4) q4[tid + u * kRowThreads] = quantize4<T>(held[u], scale, addend);
     if constexpr (HELD == 4)
-      for (int i = tid + HELD * kRowThreads; i < n4; i += kRowThreads) q4[i] = quantize4<T>(x4[i], p.scale, p.addend);
+      for (int i = tid + HELD * kRowThreads; i < n4; i += kRowThreads) q4[i] = quantize4<T>(x4[i], scale, addend);
   } else {
     for (int i = tid; i < cols; i += kRowThreads) {
-      const float t = xr[i] * p.scale;
-      qr[i] = static_cast<uint8_t>(sat_rne<T>(t + p.addend));
+      const float t = xr[i] * scale;
+      qr[i] = static_cast<uint8_t>(sat_rne<T>(t + addend));
     }
   }
 }
