@@ -55,6 +55,14 @@ inline bool device_bit(unsigned long long* mask, bool set) {
   return (__atomic_load_n(mask, __ATOMIC_ACQUIRE) & bit) != 0;
 }
 
+// A grid has fewer than 2^32 threads in one dimension; a larger one is cut off without an error.  Kernels with a thread per
+// element are launched in pieces, f(begin, end) for each, where there are more elements than that.
+constexpr int64_t kElementsPerLaunch = 1LL << 31;
+template <class F>
+inline void in_pieces(int64_t begin, int64_t n, F&& f, int64_t piece = kElementsPerLaunch) {
+  for (; begin < n; begin += piece) f(begin, n - begin < piece ? n : begin + piece);
+}
+
 inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 // Saturation bounds of the destination type, in fp32 (the s32 upper bound is the largest float

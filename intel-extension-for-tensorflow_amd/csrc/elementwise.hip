@@ -78,11 +78,11 @@ __global__ __launch_bounds__(kThreads) void quantize_scalar_kernel(const float* 
 // [outer, slices, inner] with per-slice scale / addend
 template <int T>
 __global__ __launch_bounds__(kThreads) void quantize_axis_kernel(const float* __restrict__ x,
-                                                                 uint8_t* __restrict__ q, int64_t n,
+                                                                 uint8_t* __restrict__ q, int64_t begin, int64_t n,
                                                                  int64_t slices, int64_t inner,
                                                                  const float* __restrict__ scales,
                                                                  const float* __restrict__ addends) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  const int64_t i = begin + static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   if (i < n) {
     const int64_t s = (i / inner) % slices;
     const float t = x[i] * scales[s];
@@ -840,15 +840,15 @@ int launch_quantize(const char* who, const float* x, void* q, int64_t n, int dst
           reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n4, scale, addend, dev_params);
     done = n4 * 4;
   }
-  if (done < n) {
-    const unsigned grid = blocks_for(n - done, kThreads);
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    const unsigned grid = blocks_for(end - begin, kThreads);
     if (dst_type == ITEXHIP_QINT8)
       quantize_scalar_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, st>>>(
-          x, reinterpret_cast<uint8_t*>(q), done, n, scale, addend, dev_params);
+          x, reinterpret_cast<uint8_t*>(q), begin, end, scale, addend, dev_params);
     else
       quantize_scalar_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, st>>>(
-          x, reinterpret_cast<uint8_t*>(q), done, n, scale, addend, dev_params);
-  }
+          x, reinterpret_cast<uint8_t*>(q), begin, end, scale, addend, dev_params);
+  });
   ITEXHIP_CHECK_LAUNCH(who);
   return ITEXHIP_OK;
 }
@@ -925,8 +925,10 @@ extern "C" int itexhip_quantize_dynamic_rows(const float* x, void* q, int64_t ro
   ITEXHIP_REQUIRE(x && q && row_min_out && row_max_out, "itexhip_quantize_dynamic_rows: null buffer");
   const bool vec = cols % 4 == 0 && aligned(x, 16) && aligned(q, 4);
   const auto launch = dst_type == ITEXHIP_QINT8 ? launch_rows<ITEXHIP_QINT8> : launch_rows<ITEXHIP_QUINT8>;
-  launch(x, static_cast<uint8_t*>(q), rows, static_cast<int>(cols), vec, row_min_out, row_max_out, mode, ensure_minimum_range,
-         as_stream(stream));
+  in_pieces(0, rows, [&](int64_t r, int64_t end) {
+    launch(x + r * cols, static_cast<uint8_t*>(q) + r * cols, end - r, static_cast<int>(cols), vec, row_min_out + r, row_max_out + r,
+           mode, ensure_minimum_range, as_stream(stream));
+  }, kElementsPerLaunch / kRowThreads);
   ITEXHIP_CHECK_LAUNCH("itexhip_quantize_dynamic_rows");
   return ITEXHIP_OK;
 }
@@ -958,13 +960,15 @@ extern "C" int itexhip_quantize_axis(const float* x, void* q, int64_t outer, int
     ITEXHIP_CHECK_LAUNCH("itexhip_quantize_axis");
     return ITEXHIP_OK;
   }
-  const unsigned grid = blocks_for(n, kThreads);
-  if (dst_type == ITEXHIP_QINT8)
-    quantize_axis_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
-        x, reinterpret_cast<uint8_t*>(q), n, slices, inner, scales, addends);
-  else
-    quantize_axis_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
-        x, reinterpret_cast<uint8_t*>(q), n, slices, inner, scales, addends);
+  in_pieces(0, n, [&](int64_t begin, int64_t end) {
+    const unsigned grid = blocks_for(end - begin, kThreads);
+    if (dst_type == ITEXHIP_QINT8)
+      quantize_axis_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
+          x, reinterpret_cast<uint8_t*>(q), begin, end, slices, inner, scales, addends);
+    else
+      quantize_axis_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
+          x, reinterpret_cast<uint8_t*>(q), begin, end, slices, inner, scales, addends);
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_quantize_axis");
   return ITEXHIP_OK;
 }
@@ -990,15 +994,15 @@ extern "C" int itexhip_dequantize(const void* q, float* y, int64_t n, int src_ty
           reinterpret_cast<const uint32_t*>(q), reinterpret_cast<f4*>(y), n4, scale, zp);
     done = n4 * 4;
   }
-  if (done < n) {
-    const unsigned grid = blocks_for(n - done, kThreads);
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    const unsigned grid = blocks_for(end - begin, kThreads);
     if (src_type == ITEXHIP_QINT8)
       dequantize_axis_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const uint8_t*>(q), y, done, n, 1, 1, nullptr, nullptr, scale, zp);
+          reinterpret_cast<const uint8_t*>(q), y, begin, end, 1, 1, nullptr, nullptr, scale, zp);
     else
       dequantize_axis_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const uint8_t*>(q), y, done, n, 1, 1, nullptr, nullptr, scale, zp);
-  }
+          reinterpret_cast<const uint8_t*>(q), y, begin, end, 1, 1, nullptr, nullptr, scale, zp);
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_dequantize");
   return ITEXHIP_OK;
 }
@@ -1029,13 +1033,15 @@ extern "C" int itexhip_dequantize_axis(const void* q, float* y, int64_t outer, i
     ITEXHIP_CHECK_LAUNCH("itexhip_dequantize_axis");
     return ITEXHIP_OK;
   }
-  const unsigned grid = blocks_for(n, kThreads);
-  if (src_type == ITEXHIP_QINT8)
-    dequantize_axis_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
-        reinterpret_cast<const uint8_t*>(q), y, 0, n, slices, inner, scales, zero_points, 0.f, 0.f);
-  else
-    dequantize_axis_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
-        reinterpret_cast<const uint8_t*>(q), y, 0, n, slices, inner, scales, zero_points, 0.f, 0.f);
+  in_pieces(0, n, [&](int64_t begin, int64_t end) {
+    const unsigned grid = blocks_for(end - begin, kThreads);
+    if (src_type == ITEXHIP_QINT8)
+      dequantize_axis_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
+          reinterpret_cast<const uint8_t*>(q), y, begin, end, slices, inner, scales, zero_points, 0.f, 0.f);
+    else
+      dequantize_axis_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, as_stream(stream)>>>(
+          reinterpret_cast<const uint8_t*>(q), y, begin, end, slices, inner, scales, zero_points, 0.f, 0.f);
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_dequantize_axis");
   return ITEXHIP_OK;
 }
@@ -1061,10 +1067,10 @@ int requantize_impl(const int32_t* x, void* q, int64_t n, int64_t depth, float s
           reinterpret_cast<const i4*>(x), reinterpret_cast<uint32_t*>(q), n4, 0.f, scales, depth / 4);
     done = n4 * 4;
   }
-  if (done < n) {
-    requantize_scalar_kernel<T><<<blocks_for(n - done, kThreads), kThreads, 0, st>>>(
-        x, reinterpret_cast<uint8_t*>(q), done, n, depth, scale, scales);
-  }
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    requantize_scalar_kernel<T><<<blocks_for(end - begin, kThreads), kThreads, 0, st>>>(
+        x, reinterpret_cast<uint8_t*>(q), begin, end, depth, scale, scales);
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_requantize");
   return ITEXHIP_OK;
 }
@@ -1172,9 +1178,10 @@ extern "C" int itexhip_memcpy_d2d_async(void* dst, const void* src, size_t bytes
         reinterpret_cast<const i4*>(src), reinterpret_cast<i4*>(dst), n16);
     done = n16 * 16;
   }
-  if (done < n)
-    copy_byte_kernel<<<blocks_for(n - done, kThreads), kThreads, 0, st>>>(
-        reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), done, n);
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    copy_byte_kernel<<<blocks_for(end - begin, kThreads), kThreads, 0, st>>>(
+        reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), begin, end);
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_memcpy_d2d_async");
   return ITEXHIP_OK;
 }

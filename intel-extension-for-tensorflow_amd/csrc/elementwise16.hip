@@ -138,9 +138,10 @@ void launch_quantize_bf16(const void* x, void* q, int64_t n, int64_t slices, int
         static_cast<const u4*>(x), static_cast<u2*>(q), n8, scale, addend);
     done = n8 * 8;
   }
-  if (done < n)
-    quantize_bf16_scalar_kernel<T><<<blocks_for(n - done, kThreads), kThreads, 0, st>>>(
-        static_cast<const uint16_t*>(x), static_cast<uint8_t*>(q), done, n, slices, inner, scales, addends, scale, addend);
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    quantize_bf16_scalar_kernel<T><<<blocks_for(end - begin, kThreads), kThreads, 0, st>>>(
+        static_cast<const uint16_t*>(x), static_cast<uint8_t*>(q), begin, end, slices, inner, scales, addends, scale, addend);
+  });
 }
 
 template <int T, int YT>
@@ -153,9 +154,10 @@ void launch_dequantize16(const void* q, void* y, int64_t n, int64_t slices, int6
         static_cast<const u2*>(q), static_cast<u4*>(y), n8, scale, zp);
     done = n8 * 8;
   }
-  if (done < n)
-    dequantize16_scalar_kernel<T, YT><<<blocks_for(n - done, kThreads), kThreads, 0, st>>>(
-        static_cast<const uint8_t*>(q), static_cast<uint16_t*>(y), done, n, slices, inner, scales, zps, scale, zp);
+  in_pieces(done, n, [&](int64_t begin, int64_t end) {
+    dequantize16_scalar_kernel<T, YT><<<blocks_for(end - begin, kThreads), kThreads, 0, st>>>(
+        static_cast<const uint8_t*>(q), static_cast<uint16_t*>(y), begin, end, slices, inner, scales, zps, scale, zp);
+  });
 }
 
 int check_types(const char* who, int q_type, int f_type, bool quantize) {

@@ -375,8 +375,8 @@ template <int OUT_T>
 __global__ __launch_bounds__(256) void qgemm_naive_kernel(const uint8_t* __restrict__ a, int a_is_u8,
                                                            const int8_t* __restrict__ w, int transpose_b,
                                                            int M, int K, int N, EpilogueArgs e,
-                                                           void* __restrict__ out) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+                                                           void* __restrict__ out, int64_t first) {
+  const int64_t idx = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (idx >= static_cast<int64_t>(M) * N) return;
   const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
   int acc = 0;
@@ -731,31 +731,23 @@ extern "C" int itexhip_qgemm_naive(const void* a, int a_type, const int8_t* w, i
   if (M == 0 || N == 0) return ITEXHIP_OK;
   EpilogueArgs e = make_args(a_type, nullptr, scales, bias, ep);
   e.comp_mul = 0;  // the naive kernel multiplies unsigned activations directly
-  const unsigned grid = static_cast<unsigned>((M * N + 255) / 256);
   const uint8_t* ap = reinterpret_cast<const uint8_t*>(a);
   const int a_is_u8 = a_type == ITEXHIP_QUINT8;
   hipStream_t hs = as_stream(stream);
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
-  switch (out_type) {
-    case ITEXHIP_BFLOAT16:
-      qgemm_naive_kernel<ITEXHIP_BFLOAT16><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-    case ITEXHIP_HALF:
-      qgemm_naive_kernel<ITEXHIP_HALF><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-    case ITEXHIP_FLOAT:
-      qgemm_naive_kernel<ITEXHIP_FLOAT><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-    case ITEXHIP_QINT32:
-      qgemm_naive_kernel<ITEXHIP_QINT32><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-    case ITEXHIP_QINT8:
-      qgemm_naive_kernel<ITEXHIP_QINT8><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-    default:
-      qgemm_naive_kernel<ITEXHIP_QUINT8><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out);
-      break;
-  }
+  in_pieces(0, M * N, [&](int64_t first, int64_t end) {
+    const unsigned grid = static_cast<unsigned>((end - first + 255) / 256);
+#define NAIVE(T) qgemm_naive_kernel<T><<<grid, 256, 0, hs>>>(ap, a_is_u8, w, transpose_b, Mi, Ki, Ni, e, out, first)
+    switch (out_type) {
+      case ITEXHIP_BFLOAT16: NAIVE(ITEXHIP_BFLOAT16); break;
+      case ITEXHIP_HALF: NAIVE(ITEXHIP_HALF); break;
+      case ITEXHIP_FLOAT: NAIVE(ITEXHIP_FLOAT); break;
+      case ITEXHIP_QINT32: NAIVE(ITEXHIP_QINT32); break;
+      case ITEXHIP_QINT8: NAIVE(ITEXHIP_QINT8); break;
+      default: NAIVE(ITEXHIP_QUINT8); break;
+    }
+#undef NAIVE
+  });
   ITEXHIP_CHECK_LAUNCH("itexhip_qgemm_naive");
   return ITEXHIP_OK;
 }

@@ -244,8 +244,7 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   }
 }
 
-// One thread per output element, from `first` on (a launch has fewer than 2^32 threads in one dimension; a larger grid is cut
-// off without an error.  A loop over the outputs in here costs 20 %).  Takes what the tile kernel cannot (an operand of fewer
+// One thread per output element, from `first` on (in_pieces; a loop over the outputs in here costs 20 %).  Takes what the tile kernel cannot (an operand of fewer
 // than 16 bytes in all, too many tiles for a launch) and short dot products of narrow results, see one_output_per_thread.
 template <int OUT_T>
 __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __restrict__ a, int a_is_u8,
@@ -295,10 +294,10 @@ void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b,
             const EpilogueArgs& e, void* out, hipStream_t st) {
   const bool forced = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0;  // tests ask for the tile kernel
   if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16 || (!forced && one_output_per_thread(M, K, N, tiles))) {
-    const int64_t outputs = static_cast<int64_t>(M) * N, at_once = 1LL << 31;
-    for (int64_t first = 0; first < outputs; first += at_once)
-      qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((std::min(outputs - first, at_once) + 255) / 256), 256, 0, st>>>(
+    in_pieces(0, static_cast<int64_t>(M) * N, [&](int64_t first, int64_t end) {
+      qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((end - first + 255) / 256), 256, 0, st>>>(
           a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out, first);
+    });
     return;
   }
   const unsigned grid = static_cast<unsigned>((tiles + 7) / 8 * 8);  // whole runs for the 8 XCDs

@@ -23,6 +23,11 @@ __global__ void fill_u8_kernel(uint8_t* p, uint8_t pattern, int64_t begin, int64
   const int64_t i = begin + static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = pattern;
 }
+void fill_u32(uint32_t* p, uint32_t pattern, int64_t n, hipStream_t st) {
+  in_pieces(0, n, [&](int64_t begin, int64_t end) {
+    fill_u32_kernel<<<static_cast<unsigned>((end - begin + 255) / 256), 256, 0, st>>>(p + begin, pattern, end - begin);
+  });
+}
 }  // namespace
 
 extern "C" int itexhip_device_count(int* count) {
@@ -190,11 +195,7 @@ extern "C" int itexhip_memset8_async(void* dst, uint8_t pattern, size_t bytes, v
   if (head > n) head = n;
   const int64_t words = (n - head) / 4;
   if (head > 0) fill_u8_kernel<<<1, 64, 0, st>>>(static_cast<uint8_t*>(dst), pattern, 0, head);
-  if (words > 0) {
-    const uint32_t p32 = 0x01010101u * pattern;
-    fill_u32_kernel<<<static_cast<unsigned>((words + 255) / 256), 256, 0, st>>>(
-        reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(dst) + head), p32, words);
-  }
+  fill_u32(reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(dst) + head), 0x01010101u * pattern, words, st);
   const int64_t done = head + words * 4;
   if (done < n) fill_u8_kernel<<<1, 64, 0, st>>>(static_cast<uint8_t*>(dst), pattern, done, n);
   ITEXHIP_CHECK_LAUNCH("itexhip_memset8_async");
@@ -207,8 +208,7 @@ extern "C" int itexhip_memset32_async(void* dst, uint32_t pattern, size_t bytes,
   ITEXHIP_REQUIRE((bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3) == 0,
                   "itexhip_memset32_async: address and size must be multiples of 4");
   const int64_t words = static_cast<int64_t>(bytes / 4);
-  fill_u32_kernel<<<static_cast<unsigned>((words + 255) / 256), 256, 0, as_stream(stream)>>>(
-      static_cast<uint32_t*>(dst), pattern, words);
+  fill_u32(static_cast<uint32_t*>(dst), pattern, words, as_stream(stream));
   ITEXHIP_CHECK_LAUNCH("itexhip_memset32_async");
   return ITEXHIP_OK;
 }
