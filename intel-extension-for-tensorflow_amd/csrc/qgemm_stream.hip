@@ -58,6 +58,7 @@ __device__ __forceinline__ uint32_t pack_bytes(const float (&v)[4]) {
   }
 }
 
+// (128 registers for four wavefronts per SIMD: enough without spills but for GROUP 4 with a sum, which spills 1 to 7.)
 template <int OUT_T, int POST, int SUM, int GROUP, bool CONV>
 __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __restrict__ a, uint32_t amask,
                                                             const uint8_t* __restrict__ bp, const StreamArgs s, EpilogueArgs e,
@@ -327,15 +328,35 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   // Where it is the faster kernel, by what fills the device: `rounds` is how often the 32 x 64 pieces of the result go into
   // the 4096 wavefronts that run at once (in quarters).  Below one round a launch is its start, and the tile kernel starts
   // sooner; with a long K the MFMAs and the weight fragments read from LDS for every 32 rows count, and the tile kernel
-  // reads them for 64 - 256.  Tile kernel / this kernel, time, at 0.77, 1.5, 3 and 6 rounds:
-  //   K <= 64                0.86 - 1.24, 1.03 - 1.58, 1.03 - 1.18, 1.39 - 1.43     with a residual 1.36 - 1.73 everywhere
-  //   64 < K <= 512          0.82 - 0.87, 0.75 - 0.89, 0.96 - 1.08, 1.14 - 1.31     K no multiple of 64: 0.89, 1.01 - 1.18, ...
-  //   K = 768, 1024          0.85,        0.68,        -,           0.91 - 1.09
-  //   convolution, K <= 400  1.13 - 1.24, 1.27,        1.29,        -               K = 576: 0.90 - 1.09, K = 1152: 0.87 - 0.94
+  // reads them for 64 - 256; past K = 384 the weight of 128 channels leaves room for two workgroups per CU instead of three or
+  // four.  Tile kernel / this kernel, time, over 16 to 1024 channels (convolutions: 32 to 512), at about 0.8, 1, 1.5, 2 and 4
+  // rounds (the tile kernel's own steps, whole tiles per CU, are in it):
+  //   K <= 48                1.1 - 1.4, 1.1 - 1.6, 1.3 - 1.7, 1.3 - 1.9, 1.5 - 2.1   with a residual 1.2 - 2.2 everywhere
+  //   K = 64                 1.1 - 1.4, 0.9 - 1.3, 1.0 - 1.4, 1.0 - 1.8, 1.1 - 1.8   with a residual 1.0 - 2.9
+  //                          (0.9 - 1.0 up to 1.5 rounds: multiples of 128 channels from 256 on)
+  //   K = 80, 96, 112        0.9 - 1.3, 0.9 - 1.4, 1.0 - 1.5, 1.1 - 1.7, 1.3 - 1.9   with a residual 1.0 - 2.0
+  //   K = 128                0.9 - 1.2, 0.8 - 1.2, 0.7 - 1.2, 0.8 - 1.5, 1.0 - 1.5   with a residual 1.0 - 1.8, 0.8 - 1.7, 0.8 -
+  //                          1.5, 0.9 - 2.2, 1.0 - 2.4 (below 1: multiples of 128 channels, from 1 to 2 rounds)
+  //   K = 144, 400           0.8 - 1.2, 0.9 - 1.3, 1.0 - 1.3, 1.0 - 1.6, 1.2 - 1.8   with a residual 0.9 - 1.9
+  //   K = 192 ... 448, 64 n  0.8 - 1.2, 0.7 - 1.2, 0.7 - 1.3, 0.8 - 1.4, 1.0 - 1.6   with a residual 0.7 - 2.4
+  //   K = 464, 480           -, -, 1.0, -, up to 64 channels 0.9, more 1.2 - 1.5
+  //   K = 512                0.7 - 0.9, 0.7 - 1.0, 0.7 - 1.1, 0.7 - 1.0, 0.9 - 1.0 (also at 6 and 8 rounds), 128 channels 1.1 - 1.2;
+  //                          with a residual 1.0 - 1.3, 1.0 - 1.2, 0.9 - 1.2, 1.1 - 1.4, 1.3
+  //   convolution, K <= 384  1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
+  //   convolution, K <= 448  up to 64 channels 1.1, 1.05, 1.15, -, -; more 1.0, 0.9, 1.1, 0.9, 0.9   with a residual
+  //                          1.1 - 1.2, 0.95 - 1.0, 1.3, 0.9 - 1.0, 0.9 - 1.05
+  //   convolution, K = 576   0.9 - 1.1, 1.0, 1.15, -, -                               K = 1152: 0.87 - 0.94
   const int64_t quarter_rounds = static_cast<int64_t>(s.tiles) * cols / 1024;
-  const bool small_k = K <= 64 || (e.addend && K <= 128);
-  const int64_t at_least = cv ? (K <= 448 ? 3 : -1) : small_k ? (e.addend ? 3 : 4) : K > 512 ? -1 : K % 64 != 0 ? 6 : 16;
-  if (forced != kForceStream && (at_least < 0 || quarter_rounds < at_least)) return 0;
+  auto within = [&](int64_t least, int64_t most = INT64_MAX) { return quarter_rounds >= least && quarter_rounds <= most; };
+  const bool wide = N > 64, fits = K % 64 == 0 && N % 128 == 0;  // fits: nothing padded in the tile kernel
+  bool take;
+  if (cv) take = K <= (wide ? 384 : 448) ? within(3) : K <= 448 && (e.addend ? within(3, 7) : within(6, 7));
+  else if (K <= 64) take = within(e.addend ? 3 : fits && N >= 256 ? 7 : 4);
+  else if (K <= 128 && e.addend) take = within(3) && !(fits && within(4, 9));
+  else if (K <= 448) take = within(K % 64 == 0 ? 16 : 6);
+  else if (K < 512) take = wide ? within(6) : within(6, 12);
+  else take = K == 512 && (e.addend || (wide && N <= 128)) && within(16);
+  if (forced != kForceStream && !take) return 0;
   s.padded = cv && (cv->pad_top > 0 || cv->pad_left > 0 ||
                     (cv->out_h - 1) * cv->stride_h + (K / (cv->k_w * cv->in_c) - 1) * cv->dil_h >= cv->in_h ||
                     (cv->out_w - 1) * cv->stride_w + (cv->k_w - 1) * cv->dil_w >= cv->in_w);
