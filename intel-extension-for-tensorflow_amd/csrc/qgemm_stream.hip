@@ -329,33 +329,51 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   // the 4096 wavefronts that run at once (in quarters).  Below one round a launch is its start, and the tile kernel starts
   // sooner; with a long K the MFMAs and the weight fragments read from LDS for every 32 rows count, and the tile kernel
   // reads them for 64 - 256; past K = 384 the weight of 128 channels leaves room for two workgroups per CU instead of three or
-  // four.  Tile kernel / this kernel, time, over 16 to 1024 channels (convolutions: 32 to 512), at about 0.8, 1, 1.5, 2 and 4
+  // four.  Tile kernel / this kernel, time, over 16 to 14336 channels (convolutions: 32 to 512), at about 0.8, 1, 1.5, 2 and 4
   // rounds (the tile kernel's own steps, whole tiles per CU, are in it):
-  //   K <= 48                1.1 - 1.4, 1.1 - 1.6, 1.3 - 1.7, 1.3 - 1.9, 1.5 - 2.1   with a residual 1.2 - 2.2 everywhere
-  //   K = 64                 1.1 - 1.4, 0.9 - 1.3, 1.0 - 1.4, 1.0 - 1.8, 1.1 - 1.8   with a residual 1.0 - 2.9
-  //                          (0.9 - 1.0 up to 1.5 rounds: multiples of 128 channels from 256 on)
-  //   K = 80, 96, 112        0.9 - 1.3, 0.9 - 1.4, 1.0 - 1.5, 1.1 - 1.7, 1.3 - 1.9   with a residual 1.0 - 2.0
-  //   K = 128                0.9 - 1.2, 0.8 - 1.2, 0.7 - 1.2, 0.8 - 1.5, 1.0 - 1.5   with a residual 1.0 - 1.8, 0.8 - 1.7, 0.8 -
-  //                          1.5, 0.9 - 2.2, 1.0 - 2.4 (below 1: multiples of 128 channels, from 1 to 2 rounds)
-  //   K = 144, 400           0.8 - 1.2, 0.9 - 1.3, 1.0 - 1.3, 1.0 - 1.6, 1.2 - 1.8   with a residual 0.9 - 1.9
-  //   K = 192 ... 448, 64 n  0.8 - 1.2, 0.7 - 1.2, 0.7 - 1.3, 0.8 - 1.4, 1.0 - 1.6   with a residual 0.7 - 2.4
-  //   K = 464, 480           -, -, 1.0, -, up to 64 channels 0.9, more 1.2 - 1.5
-  //   K = 512                0.7 - 0.9, 0.7 - 1.0, 0.7 - 1.1, 0.7 - 1.0, 0.9 - 1.0 (also at 6 and 8 rounds), 128 channels 1.1 - 1.2;
-  //                          with a residual 1.0 - 1.3, 1.0 - 1.2, 0.9 - 1.2, 1.1 - 1.4, 1.3
-  //   convolution, K <= 384  1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
-  //   convolution, K <= 448  up to 64 channels 1.1, 1.05, 1.15, -, -; more 1.0, 0.9, 1.1, 0.9, 0.9   with a residual
-  //                          1.1 - 1.2, 0.95 - 1.0, 1.3, 0.9 - 1.0, 0.9 - 1.05
-  //   convolution, K = 576   0.9 - 1.1, 1.0, 1.15, -, -                               K = 1152: 0.87 - 0.94
+  //   K <= 48                 1.0 - 1.4, 1.0 - 1.5, 1.1 - 1.7, 1.3 - 1.9, 1.5 - 2.1   with a residual 1.2 - 2.2 everywhere
+  //   K = 64                  1.0 - 1.4, 0.9 - 1.3, 1.0 - 1.4, 1.0 - 1.6, 1.1 - 2.0   with a residual 1.0 - 2.9
+  //                           (up to 1.0 before 1.75 rounds: multiples of 128 channels from 256 on)
+  //   K = 80, 96, 112         0.9 - 1.4, 0.9 - 1.4, 1.0 - 1.5, 1.1 - 1.7, 1.3 - 2.1   with a residual 0.9 - 1.8, 1.0 - 2.0
+  //   K = 128                 0.8 - 1.2, 0.8 - 1.1, 0.7 - 1.2, 0.8 - 1.3, 1.0 - 1.7   with a residual 0.9 - 1.8, 0.8 - 1.6, 0.8 -
+  //                           1.5, 0.9 - 2.0, 1.0 - 2.5 (below 1: multiples of 128 channels, 1 to 2 rounds, over 1024 to 2.75)
+  //   K = 144, 160            0.8 - 1.3, 0.9 - 1.3, 1.0 - 1.4, 1.0 - 1.6, 1.2 - 1.9   with a residual 0.9 - 2.1, from 1.25 on 1.1
+  //   longer, up to 1024 channels (2048 with a residual)
+  //     K = 192, 256, 320, 448  0.7 - 1.2, 0.7 - 1.1, 0.7 - 1.3, 0.8 - 1.3, 1.0 - 1.7   with a residual 1.0 - 2.9 at 4
+  //     K = 208 ... 480, no 64 n  0.7 - 1.3, 0.8 - 1.4, 0.9 - 1.5, 1.0 - 1.6, 1.1 - 1.9   with a residual 1.0 - 2.0 from 1.5 on
+  //     K = 512                 0.7 - 0.9, 0.7 - 1.1, 0.7 - 1.1, 0.7 - 1.0, 0.9 - 1.1 (also at 6 and 8), 128 channels 1.1 - 1.2;
+  //                             with a residual 1.3 - 1.6 at 4
+  //   longer, more channels (few rows per wavefront, workgroups that do not fill the last pass): 1.5 rounds, 2, 4, 6 and more
+  //     K = 192, 256            0.7 - 0.9, 0.7 - 0.9, 0.8 - 0.9, 0.7 - 1.0   with a residual (192) 1.1 at 4, 1.2 - 1.3; (256) 0.7 - 1.0
+  //     K = 208                 1.0, 1.05, 1.15, 1.0 - 1.3                   with a residual 1.0 - 1.1, 1.0 - 1.2, 1.3, 1.2 - 1.5
+  //     K = 272 ... 480         0.7 - 1.0, 0.8 - 1.0, 0.9 - 1.0, 0.7 - 1.1   with a residual 0.9 - 1.2, 0.9 - 1.3, 1.1 - 1.6, 1.0 - 1.7
+  //   convolution, K <= 384   1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
+  //   convolution, K <= 448   up to 64 channels 1.1, 1.05, 1.15, -, -; more 1.0, 0.9, 1.1, 0.9, 0.9   with a residual
+  //                           1.1 - 1.2, 0.95 - 1.0, 1.3, 0.9 - 1.0, 0.9 - 1.05
+  //   convolution, K = 576    0.9 - 1.1, 1.0, 1.15, -, -                              K = 1152: 0.87 - 0.94
   const int64_t quarter_rounds = static_cast<int64_t>(s.tiles) * cols / 1024;
   auto within = [&](int64_t least, int64_t most = INT64_MAX) { return quarter_rounds >= least && quarter_rounds <= most; };
-  const bool wide = N > 64, fits = K % 64 == 0 && N % 128 == 0;  // fits: nothing padded in the tile kernel
+  const bool sum = e.addend != nullptr, wide = N > 64, very_wide = N > (sum ? 2048 : 1024);
+  const bool whole = K % 64 == 0, fits = whole && N % 128 == 0;  // nothing padded in the tile kernel
   bool take;
-  if (cv) take = K <= (wide ? 384 : 448) ? within(3) : K <= 448 && (e.addend ? within(3, 7) : within(6, 7));
-  else if (K <= 64) take = within(e.addend ? 3 : fits && N >= 256 ? 7 : 4);
-  else if (K <= 128 && e.addend) take = within(3) && !(fits && within(4, 9));
-  else if (K <= 448) take = within(K % 64 == 0 ? 16 : 6);
-  else if (K < 512) take = wide ? within(6) : within(6, 12);
-  else take = K == 512 && (e.addend || (wide && N <= 128)) && within(16);
+  if (cv) {
+    take = K <= (wide ? 384 : 448) ? within(3) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
+  } else if (K <= 64) {
+    take = within(sum ? 3 : fits && N >= 256 ? 7 : 4);
+  } else if (K < 128) {
+    take = within(sum ? 3 : 6);
+  } else if (K == 128) {
+    take = sum ? within(3) && !(fits && within(4, very_wide ? 11 : 9)) : within(16);
+  } else if (K <= 160) {
+    take = within(6);
+  } else if (K <= 512) {
+    take = within(whole ? 16 : very_wide ? (sum && K <= 352 ? 12 : 16) : K <= 288 && !sum && N % 128 == 0 ? 7 : 6);
+    if (very_wide) take = take && (sum ? K != 256 : K <= 224 && !whole);
+    if (K == 512) take = take && (sum || N == 128);
+    else if (K > 448 && !wide) take = take && within(6, 12);
+  } else {
+    take = false;
+  }
   if (forced != kForceStream && !take) return 0;
   s.padded = cv && (cv->pad_top > 0 || cv->pad_left > 0 ||
                     (cv->out_h - 1) * cv->stride_h + (K / (cv->k_w * cv->in_c) - 1) * cv->dil_h >= cv->in_h ||
@@ -365,7 +383,9 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   const int groups_n = (cols + s.waves_n - 1) / s.waves_n;
   if (groups_n > 65535) return 0;  // gridDim.y
   const int waves_m = 4 / s.waves_n;
-  s.walkers = std::min(s.tiles, std::max(1, 256 * per_cu / groups_n) * waves_m);
+  // as many workgroups on every XCD (the kernel gives each a contiguous range of them): 2048 x 400 -> 6144, 10 of 16 with work
+  // and all of it on five XCDs, 24.8 us
+  s.walkers = std::min(s.tiles, 8 * std::max(1, 32 * per_cu / groups_n) * waves_m);
   s.share = (static_cast<uint64_t>(s.tiles) << 24) / s.walkers;
   const int wgs = (s.walkers + waves_m - 1) / waves_m;
   const dim3 grid(static_cast<unsigned>((wgs + 7) / 8 * 8), static_cast<unsigned>(groups_n));
