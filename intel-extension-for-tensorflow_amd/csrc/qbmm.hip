@@ -10,6 +10,7 @@
 // adj_y) is transposed on the way into LDS, four bytes at a time.  The output orientation keeps
 // n on the lanes, so every store instruction writes 128 contiguous bytes per half-wavefront: with fp32
 // outputs the op is bound by that write.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -28,6 +29,7 @@ struct BmmArgs {
   int tiles_m, tiles_n;
   int mode_x, mode_y;  // kBytes, kAligned or kAny: how the operands are read
   int xcd_grid;      // launched as (8, tiles, matrices / 8), not (tiles, matrices): see the kernel
+  uint32_t tile0;    // first tile of this launch (a matrix of more tiles than one grid dimension holds takes several)
   uint32_t batch, per_slice;  // matrices; of one index of the grid's third dimension (an argument: reading gridDim costs a load)
   FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
@@ -393,10 +395,10 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
   // Workgroup -> (batch entry, tile).  Consecutive workgroup ids go round the 8 XCDs.  Launched as (8, tiles, matrices / 8)
   // the XCD takes whole matrices: their operands are read into one L2, and output lines that two tiles share (rows that are
   // no whole 64-byte pieces) are put together there instead of leaving two L2s in pieces.  Otherwise the launch is
-  // (tiles, matrices) with the matrices over the last two dimensions (the first one ends at 2^24 workgroups), and consecutive
+  // (tiles, matrices) with the matrices over the last two dimensions (the first one ends below 2^24 workgroups), and consecutive
   // workgroups walk the tiles of one matrix.  The launch has fewer than 2^31 workgroups: 32-bit arithmetic.
   const uint32_t bi = blockIdx.z * a.per_slice + (a.xcd_grid ? blockIdx.x : blockIdx.y);  // index of the output matrix
-  const uint32_t tile = a.xcd_grid ? blockIdx.y : blockIdx.x;
+  const uint32_t tile = a.tile0 + (a.xcd_grid ? blockIdx.y : blockIdx.x);
   if (bi >= a.batch) return;  // whole workgroup
   const int tm = a.tiles_n == 1 ? static_cast<int>(tile) : static_cast<int>(tile / a.tiles_n);
   const int m0 = tm * (RM * kTile), n0 = static_cast<int>(tile - tm * a.tiles_n) * (RN * kTile);
@@ -570,12 +572,16 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   for (int d = 0; d < a.p.n_batch_dims; ++d) a.by_dim[d] = make_fast_div(a.p.batch_dims[d]);
   const int64_t slices = (batch + 65534) / 65535;
   a.per_slice = static_cast<uint32_t>(a.xcd_grid ? 8 : (batch + slices - 1) / slices);
-  const dim3 g = a.xcd_grid ? dim3(8, static_cast<unsigned>(tiles), static_cast<unsigned>((batch + 7) / 8))
-                            : dim3(static_cast<unsigned>(tiles), a.per_slice, static_cast<unsigned>(slices));
-  if (p->adj_x && p->adj_y) launch_layout<true, true>(a, x, y, out, g, st);
-  else if (p->adj_x) launch_layout<true, false>(a, x, y, out, g, st);
-  else if (p->adj_y) launch_layout<false, true>(a, x, y, out, g, st);
-  else launch_layout<false, false>(a, x, y, out, g, st);
+  constexpr int64_t kTilesPerLaunch = 1LL << 23;
+  for (int64_t t = 0; t < tiles; t += kTilesPerLaunch) {
+    a.tile0 = static_cast<uint32_t>(t);
+    const unsigned n = static_cast<unsigned>(std::min(tiles - t, kTilesPerLaunch));
+    const dim3 g = a.xcd_grid ? dim3(8, n, static_cast<unsigned>((batch + 7) / 8)) : dim3(n, a.per_slice, static_cast<unsigned>(slices));
+    if (p->adj_x && p->adj_y) launch_layout<true, true>(a, x, y, out, g, st);
+    else if (p->adj_x) launch_layout<true, false>(a, x, y, out, g, st);
+    else if (p->adj_y) launch_layout<false, true>(a, x, y, out, g, st);
+    else launch_layout<false, false>(a, x, y, out, g, st);
+  }
   ITEXHIP_CHECK_LAUNCH(who);
   return ITEXHIP_OK;
 }

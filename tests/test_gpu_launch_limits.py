@@ -156,3 +156,17 @@ def test_matmul_per_output(hip, dev):
     assert torch.equal(out[0], small) and bool((out == out[:1]).all())
     want = (torch.arange(P).view(-1, 1) * torch.arange(-16, 17).view(1, -1) / 16.0).round().clamp(-128, 127).to(torch.int8)
     assert torch.equal(small.cpu(), want)
+
+
+def test_batch_matmul_rows_of_one_column(hip, dev):
+    """2^30 rows of one column: 2^24 tiles of one matrix."""
+    import torch
+    need(8)
+    M = (1 << 30) // P * P + 70 * P
+    x = torch.arange(P, dtype=torch.int8, device=dev).repeat(M // P)
+    y = torch.full((1,), 3, dtype=torch.int8, device=dev)
+    p, _ = hip.bmm_params((1, M, 1), (1, 1, 1), False, False, hip.BFLOAT16, 0.25)
+    out = torch.full((M,), 99.0, dtype=torch.bfloat16, device=dev)
+    hip.qbatch_matmul(p, x, y, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:P].float(), (x[:P].float() * 0.75).bfloat16().float()) and repeats(out, M)
