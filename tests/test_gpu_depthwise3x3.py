@@ -3,6 +3,8 @@ sums and the epilogue's separately rounded fp32 steps in numpy, bit for bit."""
 import numpy as np
 import pytest
 
+from tests.test_gpu_stream import awkward_floats, finish
+
 pytestmark = pytest.mark.gpu
 
 
@@ -49,3 +51,26 @@ def test_edges(hip, dev, B, H, W, C, stride, top, left, signed_in):
             got = out.cpu().numpy()
             assert (got[-32:] == 0x55).all()
             np.testing.assert_array_equal(got[:-32].view(dt).reshape(ref.shape), ref)
+
+
+@pytest.mark.parametrize("post", ["none", "relu", "clip"])
+@pytest.mark.parametrize("signed_out", [False, True])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_rounding_and_saturation(hip, dev, post, signed_out, stride):
+    """The conversion instructions of the epilogue on values that come in as biases (scale 0)."""
+    import torch
+    C, O = 16384, 3 // stride
+    bias = awkward_floats(C)
+    inf = float("inf")
+    lo, hi = {"none": (-inf, inf), "relu": (0.0, inf), "clip": (-3.5, 90.0)}[post]
+    ep = hip.Epilogue()
+    ep.n_scales, ep.n_eltwise = 1, 0 if post == "none" else 1
+    ep.elt[0].alg, ep.elt[0].alpha, ep.elt[0].beta = (hip.ELT_RELU, 0.0, 0.0) if post == "relu" else (hip.ELT_CLIP, lo, hi)
+    x = torch.randint(0, 256, (1, 3, 3, C), dtype=torch.uint8, device=dev)
+    w = torch.randint(-127, 128, (3, 3, C, 1), dtype=torch.int8, device=dev)
+    out = torch.full((O * O, C), 0x55, dtype=torch.uint8, device=dev)
+    hip.qdepthwise_conv2d(x, hip.QUINT8, hip.ConvGeometry(1, 3, 3, C, 3, 3, O, O, stride, stride, 1, 1, 1, 1), 1, w,
+                          torch.zeros(1, device=dev), torch.from_numpy(bias).to(dev), ep, hip.QINT8 if signed_out else hip.QUINT8, out)
+    torch.cuda.synchronize()
+    ref = finish(np.zeros((O * O, C)), np.float32(0), bias, None, 0.0, lo, hi, signed_out)
+    np.testing.assert_array_equal(out.cpu().numpy().view(ref.dtype), ref)

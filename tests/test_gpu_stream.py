@@ -3,20 +3,28 @@ and the epilogue's separately rounded fp32 steps in numpy, bit for bit.  Convolu
 import numpy as np
 import pytest
 
+from oracle import pyoracle as orc
 from tests.test_gpu_conv import check_implicit_conv
+from tests.test_gpu_matmul import V2_REQ_S8, V2_REQ_U8_RELU, make_acts, make_layer
+from tests.test_oracle_conv import ref_int_conv
 
 pytestmark = pytest.mark.gpu
 ANY_SIZE = 16   # force_tile_shape: this kernel whatever the size of the call
 
 
 def reference(x, w, scale, bias, addend, sum_scale, lo, hi, signed_out):
+    return finish(x.astype(np.int64) @ w.astype(np.int64), scale, bias, addend, sum_scale, lo, hi, signed_out)
+
+
+def finish(acc, scale, bias, addend, sum_scale, lo, hi, signed_out):
     f = np.float32
-    v = (x.astype(np.int64) @ w.astype(np.int64)).astype(f) * scale
-    v = v + bias
+    with np.errstate(invalid="ignore"):   # signalling NaN
+        v = acc.astype(f) * scale
+        v = v + bias
     if addend is not None:
         v = v + f(sum_scale) * addend.astype(f)
-    v = np.minimum(np.maximum(v, f(lo)), f(hi))
-    v = np.clip(v, f(-128 if signed_out else 0), f(127 if signed_out else 255))
+    v = np.fmin(np.fmax(v, f(lo)), f(hi))   # NaN: the bound
+    v = np.fmin(np.fmax(v, f(-128 if signed_out else 0)), f(127 if signed_out else 255))
     return np.rint(v).astype(np.int8 if signed_out else np.uint8)
 
 
@@ -85,3 +93,142 @@ def test_several_tiles_per_wavefront(hip, dev, M, K, N):
 def test_convolutions(hip, dev, shape, wshape, strides, dil, lead, signed_in):
     hip.force_tile_shape(conv=ANY_SIZE)
     check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, np.random.default_rng(sum(shape) + signed_in))
+
+
+@pytest.mark.parametrize("kw", [V2_REQ_S8, V2_REQ_U8_RELU, dict(V2_REQ_S8, input_mode=orc.SCALED),
+                                dict(V2_REQ_U8_RELU, input_mode=orc.SCALED)], ids=["s8", "u8_relu", "s8_scaled", "u8_relu_scaled"])
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("M,K,N", [(300, 96, 272), (161, 48, 80), (140, 400, 528)])
+def test_parameters_derived_in_the_kernel(hip, dev, kw, per_channel, M, K, N):
+    """itexhip_qmatmul and itexhip_qmatmul_device_range with one weight range and one per channel, against the oracle."""
+    import torch
+    layer, w, bias = make_layer(hip, dev, K, N, seed=K + N, per_channel=per_channel)
+    x, xq, mn, mx = make_acts(M, K, seed=M, mode=kw["input_mode"])
+    r_out = float(np.abs(np.maximum(x @ w + bias, 0) if kw.get("activation") else x @ w + bias).max())
+    lo = 0.0 if kw["t_out"] == orc.QUINT8 else -r_out
+    t_in = orc.QUINT8 if xq.dtype == np.uint8 else orc.QINT8
+    p = hip.matmul_params(t_in=t_in, min_a=mn, max_a=mx, min_out=lo, max_out=r_out, **kw)
+    ep = hip.qmatmul_epilogue_desc(p, layer.min_b.size)
+    # the chains this kernel takes: none, or one ReLU
+    assert [(ep.elt[i].alg, ep.elt[i].alpha) for i in range(ep.n_eltwise)] in ([], [(hip.ELT_RELU, 0.0)])
+    ref = layer.oracle(xq, kw, mn, mx, lo, r_out)
+    hip.force_tile_shape(matmul=ANY_SIZE)
+    np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, lo, r_out, path="fused"), ref)
+    p = hip.matmul_params(t_in=t_in, min_a=77.0, max_a=-3.0, min_out=lo, max_out=r_out, **kw)   # min_a / max_a unused
+    range_a = torch.tensor([mn, mx], dtype=torch.float32, device=dev)
+    out = torch.full((M, N), 0x55, dtype=torch.uint8, device=dev)
+    hip.qmatmul_device_range(p, torch.from_numpy(xq).to(dev), layer.packed, layer.colsum, M, K, N, range_a, layer.min_b_d,
+                             layer.max_b_d, layer.min_b.size, layer.bias_d, out)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy().view(ref.dtype), ref)
+
+
+@pytest.mark.parametrize("post", ["none", "relu", "clip"])
+@pytest.mark.parametrize("signed_add", [False, True])
+@pytest.mark.parametrize("signed_out", [False, True])
+@pytest.mark.parametrize("O", [48, 144])
+def test_convolutions_with_a_residual(hip, dev, post, signed_add, signed_out, O):
+    """Every post-op of a convolution, and of a MatMul on its patch matrix, without an addend, with one and with one that is the
+    output's own buffer."""
+    import torch
+    rng = np.random.default_rng(O + signed_add)
+    B, H, W, C = 3, 11, 10, 32
+    M, K = B * H * W, 9 * C
+    x, w = rng.integers(0, 256, (B, H, W, C)).astype(np.uint8), rng.integers(-127, 128, (3, 3, C, O)).astype(np.int8)
+    acc = ref_int_conv(x, w, (1, 1), (1, 1), ((1, 1), (1, 1))).reshape(M, O)
+    scale = ((rng.random(O) + 0.5) * 8e-4).astype(np.float32)
+    bias = (rng.standard_normal(O) * 20).astype(np.float32)
+    addend = rng.integers(-128, 128, (M, O)).astype(np.int8) if signed_add else rng.integers(0, 256, (M, O)).astype(np.uint8)
+    T_add, T_out = (hip.QINT8 if s else hip.QUINT8 for s in (signed_add, signed_out))
+    inf = float("inf")
+    lo, hi = {"none": (-inf, inf), "relu": (0.0, inf), "clip": (-3.5, 90.0)}[post]
+    d = lambda a: torch.from_numpy(a).to(dev)
+    g = hip.ConvGeometry(B, H, W, C, 3, 3, H, W, 1, 1, 1, 1, 1, 1)
+    packed = torch.empty(hip.qgemm_packed_bytes(K, O), dtype=torch.int8, device=dev)
+    colsum = torch.empty(O, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(d(w.reshape(K, O)), False, K, O, packed, colsum)
+    xd, sc, bi = d(x), d(scale), d(bias)
+    cols = torch.empty((M, K), dtype=torch.uint8, device=dev)
+    hip.im2col8(xd, g, K, cols)
+    hip.force_tile_shape(matmul=ANY_SIZE, conv=ANY_SIZE)
+    for add in (False, True):
+        ep = hip.Epilogue()
+        elts = ([(hip.ELT_SUM, 0.375, 0.0)] if add else []) + {"none": [], "relu": [(hip.ELT_RELU, 0.0, 0.0)], "clip": [(hip.ELT_CLIP, lo, hi)]}[post]
+        ep.n_scales, ep.n_eltwise = O, len(elts)
+        for i, e in enumerate(elts):
+            ep.elt[i].alg, ep.elt[i].alpha, ep.elt[i].beta = e
+        ref = finish(acc, scale, bias, addend if add else None, 0.375, lo, hi, signed_out)
+        for in_place in (False, True) if add else (False,):
+            for conv in (False, True):
+                out = d(addend.view(np.uint8)) if in_place else torch.full((M, O), 0x55, dtype=torch.uint8, device=dev)
+                src = out if in_place else d(addend)
+                if conv and add:
+                    hip.qconv2d_sum(xd, hip.QUINT8, g, packed, colsum, O, sc, bi, ep, src, T_add, T_out, out)
+                elif conv:
+                    hip.qconv2d(xd, hip.QUINT8, g, packed, colsum, O, sc, bi, ep, T_out, out)
+                elif add:
+                    hip.qgemm_sum(cols, hip.QUINT8, packed, colsum, M, K, O, sc, bi, ep, src, T_add, T_out, out)
+                else:
+                    hip.qgemm(cols, hip.QUINT8, packed, colsum, M, K, O, sc, bi, ep, T_out, out)
+                torch.cuda.synchronize()
+                np.testing.assert_array_equal(out.cpu().numpy().view(ref.dtype), ref, err_msg=str((add, in_place, conv)))
+
+
+def test_residual_in_place_several_tiles_per_wavefront(hip, dev):
+    """The addend of a tile is read while the tile before it is stored: one buffer for both, at a size that takes this kernel by
+    itself."""
+    import torch
+    M, K, N = 100003, 64, 256
+    g = torch.Generator(device=dev).manual_seed(5)
+    x, both = (torch.randint(0, 256, (M, n), dtype=torch.uint8, device=dev, generator=g) for n in (K, N))
+    w = torch.randint(-127, 128, (K, N), dtype=torch.int8, device=dev, generator=g)
+    packed = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev)
+    colsum = torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(w, False, K, N, packed, colsum)
+    ep = hip.Epilogue()
+    ep.n_scales, ep.n_eltwise = 1, 2
+    for i, e in enumerate([(hip.ELT_SUM, 0.375, 0.0), (hip.ELT_RELU, 0.0, 0.0)]):
+        ep.elt[i].alg, ep.elt[i].alpha, ep.elt[i].beta = e
+    scale, bias = torch.full((1,), 1e-3, device=dev), torch.full((N,), 20.0, device=dev)
+    v = (x.float() @ w.float()) * scale   # every sum below 2^24: exact in fp32 in any order
+    v = v + bias
+    want = (v + 0.375 * both.float()).clamp(0, 255).round().to(torch.uint8)
+    hip.qgemm_sum(x, hip.QUINT8, packed, colsum, M, K, N, scale, bias, ep, both, hip.QUINT8, hip.QUINT8, both)
+    torch.cuda.synchronize()
+    assert torch.equal(both, want)
+
+
+def awkward_floats(n):
+    """n fp32 values: ties around every 8-bit result with their neighbours, infinities, NaN, denormals, random bit patterns."""
+    f = np.float32
+    ties = np.arange(-131, 259).astype(f) + f(0.5)
+    special = np.array([np.inf, -np.inf, np.nan, -np.nan, 0.0, -0.0, 1e-45, -1e-45, 3.4e38, -3.4e38, 2.0 ** 31, -2.0 ** 31], f)
+    v = np.concatenate([ties, np.nextafter(ties, f(-1e9)), np.nextafter(ties, f(1e9)), special])
+    patterns = np.random.default_rng(9).integers(0, 1 << 32, n - v.size, dtype=np.uint64).astype(np.uint32).view(f)
+    return np.concatenate([v, patterns])
+
+
+@pytest.mark.parametrize("post", ["none", "relu", "clip"])
+@pytest.mark.parametrize("signed_out", [False, True])
+def test_rounding_and_saturation(hip, dev, post, signed_out):
+    """The conversion instructions of the epilogue on values that come in as biases (scale 0)."""
+    import torch
+    M, K, N = 40, 16, 16384
+    bias = awkward_floats(N)
+    ep = hip.Epilogue()
+    ep.n_scales, ep.n_eltwise = 1, 0 if post == "none" else 1
+    inf = float("inf")
+    lo, hi = {"none": (-inf, inf), "relu": (0.0, inf), "clip": (-3.5, 90.0)}[post]
+    ep.elt[0].alg, ep.elt[0].alpha, ep.elt[0].beta = (hip.ELT_RELU, 0.0, 0.0) if post == "relu" else (hip.ELT_CLIP, lo, hi)
+    x = torch.randint(0, 256, (M, K), dtype=torch.uint8, device=dev)
+    w = torch.randint(-127, 128, (K, N), dtype=torch.int8, device=dev)
+    packed = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev)
+    colsum = torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(w, False, K, N, packed, colsum)
+    out = torch.full((M, N), 0x55, dtype=torch.uint8, device=dev)
+    hip.force_tile_shape(matmul=ANY_SIZE)
+    hip.qgemm(x, hip.QUINT8, packed, colsum, M, K, N, torch.zeros(1, device=dev), torch.from_numpy(bias).to(dev), ep,
+              hip.QINT8 if signed_out else hip.QUINT8, out)
+    torch.cuda.synchronize()
+    ref = finish(np.zeros((M, N)), np.float32(0), bias, None, 0.0, lo, hi, signed_out)
+    np.testing.assert_array_equal(out.cpu().numpy().view(ref.dtype), ref)
