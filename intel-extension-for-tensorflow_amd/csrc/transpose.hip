@@ -87,17 +87,39 @@ void launch(const TransposeArgs& a, const void* x, void* y, hipStream_t st) {
   transpose_kernel<unit_t><<<static_cast<unsigned>(blocks), 256, 0, st>>>(a, xp, yp);
 }
 
-// Order and units per thread of a small tensor.  Both tensors are walked in runs: the innermost dimension where it is
-// contiguous in both, else single units.  Next to the run the output has a dimension of r, the input one of c.
-// Runs of 4 units and more (64 bytes of a 16-byte unit): in the input's order where c < r (the head split: c = 12 heads, r =
-// 128 tokens): a workgroup reads whole lines and writes runs of r instead of touching every line of the input once per head;
-// two units per thread (1000 x 32 x 64 bytes, 32 of them: 24.5 us one unit, output's order; 21.2).
-// Shorter runs: the same, where c is at most half of r, the r destinations of a workgroup's reads are worth a line (c * run
-// up to 64) or do not lie a power of two apart; one unit per thread (its neighbours' units are other lines), or two where the
-// rows of the input share lines.  us, output's / input's order: 1000 x 32 x 16 bytes 11.7 / 6.7, 1000 x 7 x 600 x 16 74 / 58,
-// 4096 x 256 x 16 8.4 / 17.6, 4096 x 1024 x 16 22.8 / 39.9, 12 x 197 x 16 2.4 / 3.1; one / two units: 1024 x 1024 x 16 9.6 /
-// 15.0, 1024 x 4096 x 16 30.6 / 49.9, 300 x 301 x 16 52.7 / 42.7.
-// Bytes: always two but for small tensors (300 x 301 x 302 reversed 205 us, one unit 338; 1024 x 1024 5.9, one unit 4.8).
+// How many 128-byte lines of the other tensor a walk fetches (or writes back) per unit, where `cache` bytes of them stay close:
+// the walk's dimensions, innermost first, make a window of units whose lines just fit; beyond it every line comes again.
+struct WalkDim {
+  int64_t extent, stride;  // stride in the other tensor, in units
+};
+double lines_per_unit(const WalkDim* walk, int n, int unit, double cache) {
+  double units = 1.0, rows = 1.0, span = unit;  // of the window: rows of `span` bytes each
+  for (int i = 0; i < n; ++i) {
+    const double extent = static_cast<double>(walk[i].extent), step = static_cast<double>(walk[i].stride) * unit;
+    const bool near = step < 128.0;  // neighbours along this dimension share lines
+    const double lines = rows * std::max(1.0, span / 128.0);
+    const double whole = near ? rows * std::max(1.0, (span + (extent - 1.0) * step) / 128.0) : lines * extent;
+    if (whole * 128.0 > cache) {  // a part of this dimension fills the window
+      const double part = std::max(1.0, std::min(extent, near ? extent * cache / (whole * 128.0) : cache / (lines * 128.0)));
+      return (near ? rows * std::max(1.0, (span + (part - 1.0) * step) / 128.0) : lines * part) / (units * part);
+    }
+    units *= extent;
+    if (near) span += (extent - 1.0) * step;
+    else rows *= extent;
+  }
+  return rows * std::max(1.0, span / 128.0) / units;
+}
+
+// Order and units per thread of a small tensor.  One tensor is walked from end to end, the other one jumps: the order is that of
+// the output unless the input's brings the jumping tensor through an L2 (4 MB of lines) at most half as often, or, where neither
+// does in 8 MB and more, needs at most two thirds of the lines within 8 KB, what two wavefronts have in flight.  Two units per thread overlap
+// two loads; one leaves more threads, from where and for which units below.
+// us, one unit per thread in the output's / the input's order: 36 x 50 x 246 x 16 ints (3, 0, 1, 2) 68.3 / 19.4, 44 x 167 x 306
+// x 5 (2, 1, 3, 0) 48 / 146, 54 x 284 x 122 x 16 (2, 1, 3, 0) 197 / 365, 267 x 133 x 24 x 64 bytes (3, 2, 0, 1) 969 / 251; the
+// head split of 128 x 128 x 12 x 64 bytes 7.8 / 6.3 (the second rule).  Over 15000 shapes of up to 5 dimensions and 64 MB the
+// choice is 3 % above the fastest of the four; rules on the two innermost dimensions alone were 5.4 % above it and up to
+// three times as long as the output's order, walked by threads that return for more, with 64-bit divisions.
+// us, one / two units: 300 x 301 x 302 bytes reversed 338 / 205, 1024 x 1024 4.8 / 5.9.
 void walk_order(TransposeArgs& a, int unit) {
   int n = a.rank;
   const bool in_runs = a.in_stride[n - 1] == 1 && a.out_dims[n - 1] > 1;
@@ -105,20 +127,18 @@ void walk_order(TransposeArgs& a, int unit) {
   int order[kMaxRank];
   for (int i = 0; i < n; ++i) order[i] = i;
   std::sort(order, order + n, [&](int p, int q) { return a.in_stride[p] > a.in_stride[q]; });
-  bool by_input = false;
-  a.units = 2;
-  const int next = in_runs ? n - 2 : n - 1;
-  if (next >= 0) {
-    const int64_t run = in_runs ? a.out_dims[n - 1] : 1, r = a.out_dims[next], c = a.out_dims[order[next]];
-    if (in_runs && (run >= 4 || unit == 1)) {
-      by_input = c < r;
-    } else if (unit > 1) {
-      by_input = 2 * c <= r && r >= 32 && (c * run <= 64 || (r * run * unit) % 4096 != 0);
-      a.units = unit == 16 && !by_input && (c * run * unit) % 128 != 0 ? 2 : 1;
-    } else if (a.total <= 1 << 20) {
-      a.units = 1;
-    }
+  const double bytes = static_cast<double>(a.total) * unit, mb = 1024.0 * 1024.0;
+  a.units = bytes < (unit == 1 ? 0.25 : unit == 4 && in_runs ? 1.0 : 8.0) * mb ? 1 : 2;
+  WalkDim out[kMaxRank], in[kMaxRank];
+  for (int i = 0; i < n; ++i) {
+    const int o = n - 1 - i, p = order[n - 1 - i];
+    out[i] = WalkDim{a.out_dims[o], a.in_stride[o]};
+    in[i] = WalkDim{a.out_dims[p], a.out_stride[p]};
   }
+  const double l2_out = lines_per_unit(out, n, unit, 4.0 * mb), l2_in = lines_per_unit(in, n, unit, 4.0 * mb);
+  bool by_input = 2.0 * l2_in < l2_out;
+  if (!by_input && 2.0 * l2_out >= l2_in && bytes >= 8.0 * mb)
+    by_input = 1.5 * lines_per_unit(in, n, unit, 8192.0) < lines_per_unit(out, n, unit, 8192.0);
   if (!by_input) return;
   const TransposeArgs b = a;
   for (int i = 0; i < n; ++i) {
