@@ -321,7 +321,7 @@ __global__ __launch_bounds__(256) void qdwconv_kernel(const DepthwiseArgs a, con
 }
 
 // The common case - 3x3 window, stride 1 or 2 in both directions, dilation 1, multiplier 1, channels a multiple of 4.  A
-// thread owns 4 consecutive channels of R = 4 output rows and, with stride 1, two output columns.  The three taps of a window
+// thread owns 4 consecutive channels of R = 4 output rows and, with stride 1, CW = 2 output columns.  The three taps of a window
 // row are one 4-byte dot product: the pixels of an input row (4 with stride 1, 3 with stride 2; a dword of 4 channels each)
 // are transposed to a dword of pixels per channel, 8 or 6 byte permutes, which serves every output row that reads this input
 // row and, with stride 1, both columns (the second with the weights a byte further on).  Unsigned input is fed as x - 128
@@ -330,11 +330,12 @@ __global__ __launch_bounds__(256) void qdwconv_kernel(const DepthwiseArgs a, con
 // 17.3 -> 11.4 us; stride 2, which had one thread per output dword and 64-bit divisions, 17.0 -> 6.4 us.
 // BOUNDS: an 8-bit result and a chain that is nothing, a ReLU or a clip, all of them min(max(v, lo), hi) there (no branch per
 // value; a missing bias adds +0, whose sign an integer does not keep).
-template <int OUT_T, bool X_SIGNED, int S, bool BOUNDS>
+// R x CW: a launch of little work waits for one thread's chain of loads and instructions, see the host's choice.
+template <int OUT_T, bool X_SIGNED, int S, bool BOUNDS, int R, int CW>
 __global__ __launch_bounds__(256, 7) void qdwconv3x3_kernel(const DepthwiseArgs a, const uint8_t* __restrict__ x,
                                                          const int8_t* __restrict__ w, const float* __restrict__ scales,
                                                          const float* __restrict__ bias, void* __restrict__ out) {
-  constexpr int R = 4, CW = S == 1 ? 2 : 1, PIX = S == 1 ? 4 : 3, IR = (R - 1) * S + 3;
+  constexpr int PIX = CW == 2 ? 4 : 3, IR = (R - 1) * S + 3;
   // consecutive workgroup ids go round the 8 XCDs: each takes a contiguous range, neighbours share input rows (the grid is a
   // multiple of 8)
   const uint32_t wg = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -559,7 +560,13 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
     canonical = k == ep->n_eltwise;
   }
   const int step = static_cast<int>(g->stride_h);
-  const int64_t cols = step == 1 ? (g->out_w + 1) / 2 : g->out_w, strips = (g->out_h + 3) / 4;
+  // Stride 1: 4 rows x 2 columns per thread share the permutes; below 2^20 (position, 4 channels) pairs 4 x 1 and below 96 Ki
+  // 1 x 1 leave more threads with a shorter chain each.  Times over those of one thread per 4 x 1 without dot products, 7700
+  // sizes, 4 x 2 / 4 x 1 / 1 x 1: up to 96 Ki pairs 0.99 - 1.14 / 0.82 - 0.91 / 0.67 - 0.79, 128 Ki 0.99 - 1.09 / 0.82 - 0.90 /
+  // 0.87 - 0.92, 512 Ki 0.81 - 0.90 / 0.77 - 0.85 / 1.2, 1 Mi 0.71 - 0.84 / 0.73 - 0.84 / 1.3, 2 Mi 0.64 - 0.76 / 0.71 - 0.81.
+  const int64_t pairs = positions * a.groups4;
+  const int shape = step != 1 || pairs >= 1 << 20 ? 0 : pairs >= 96 << 10 ? 1 : 2;
+  const int64_t cols = step == 1 && shape == 0 ? (g->out_w + 1) / 2 : g->out_w, strips = shape == 2 ? g->out_h : (g->out_h + 3) / 4;
   const int64_t strip_total = g->batch * strips * cols * a.groups4;
   if (canonical && a.vec && aligned(out, 16) && g->k_h == 3 && g->k_w == 3 && (step == 1 || step == 2) && g->stride_w == step &&
       g->dil_h == 1 && g->dil_w == 1 && strip_total < lim && g->in_h > 0 && g->in_w > 0 && g->batch * g->in_h * g->in_w * g->in_c < lim) {
@@ -575,9 +582,14 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
       a.lo = a.chain & 1 ? 0.0f : -INFINITY;
       a.hi = INFINITY;
     }
-#define DW3K(T, S, B)                                                                                          \
-  if (a.x_signed) qdwconv3x3_kernel<T, true, S, B><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out); \
-  else qdwconv3x3_kernel<T, false, S, B><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out)
+#define DW3R(T, S, B, R, CW)                                                                                          \
+  if (a.x_signed) qdwconv3x3_kernel<T, true, S, B, R, CW><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out); \
+  else qdwconv3x3_kernel<T, false, S, B, R, CW><<<sblocks, 256, 0, st>>>(a, xp, filter, scales, bias, out)
+#define DW3K(T, S, B)                                   \
+  if constexpr (S == 2) { DW3R(T, S, B, 4, 1); }        \
+  else if (shape == 0) { DW3R(T, S, B, 4, 2); }         \
+  else if (shape == 1) { DW3R(T, S, B, 4, 1); }         \
+  else { DW3R(T, S, B, 1, 1); }
 #define DW3S(T, S)                                                            \
   if constexpr (T == ITEXHIP_QINT8 || T == ITEXHIP_QUINT8) {                  \
     if (b8) { DW3K(T, S, true); break; }                                      \
@@ -596,6 +608,7 @@ extern "C" int itexhip_qdepthwise_conv2d(const void* x, int x_type, const itexhi
 #undef DW3
 #undef DW3S
 #undef DW3K
+#undef DW3R
     ITEXHIP_CHECK_LAUNCH(who);
     return ITEXHIP_OK;
   }

@@ -53,6 +53,13 @@ def test_edges(hip, dev, B, H, W, C, stride, top, left, signed_in):
             np.testing.assert_array_equal(got[:-32].view(dt).reshape(ref.shape), ref)
 
 
+@pytest.mark.parametrize("B,H,W,C", [(3, 57, 59, 40), (5, 111, 113, 68)])
+@pytest.mark.parametrize("signed_in", [False, True])
+def test_more_outputs_per_thread(hip, dev, B, H, W, C, signed_in):
+    """At stride 1 a small launch has one output position per thread; sizes that get 4 rows and 4 rows x 2 columns."""
+    test_edges(hip, dev, B, H, W, C, 1, 1, 1, signed_in)
+
+
 @pytest.mark.parametrize("post", ["none", "relu", "clip"])
 @pytest.mark.parametrize("signed_out", [False, True])
 @pytest.mark.parametrize("stride", [1, 2])
