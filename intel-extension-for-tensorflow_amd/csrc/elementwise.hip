@@ -353,53 +353,69 @@ __global__ __launch_bounds__(kThreads) void minmax_i32_flat_kernel(const i4* __r
 // maxima meet in LDS before one pair of atomics per channel.  Bound by its reads: 8192 x 4096 in 23.8 us, 5.6 TB/s; one int
 // per lane and load, with an atomic pair per channel and 32 rows, took 38 us.  Plain loads, not streaming ones: what fits
 // stays in the last-level cache for the Requantize that follows (23.5 against 27 us for that one).
+// Up to kFewRows rows: one thread per channel (V = 1, one row at a time), whose result goes out as it is: the start and the
+// meeting in LDS cost more than the loads there.
 constexpr int kRowUnroll = 8;
+constexpr int64_t kFewRows = 8;
 constexpr int64_t kChannelBlocks = 256;
 template <int V>
 __global__ __launch_bounds__(kThreads) void minmax_i32_channel_kernel(const int32_t* __restrict__ x, int64_t rows, int64_t depth,
-                                                                      int groups, int64_t rows_per_block,
+                                                                      int groups, int side, int64_t rows_per_block,
                                                                       int32_t* mn_out, int32_t* mx_out) {
   __shared__ int smn[V == 4 ? 256 : kThreads], smx[V == 4 ? 256 : kThreads];
-  const int side = kThreads / groups;  // rows walked side by side
+  // `side` rows are walked side by side
   const int ty = static_cast<int>(threadIdx.x) / groups, tx = static_cast<int>(threadIdx.x) - ty * groups;
   const int64_t c = (static_cast<int64_t>(blockIdx.y) * groups + tx) * V;
-  const bool mine = ty < side && c < depth;
-  smn[threadIdx.x] = INT32_MAX;
-  smx[threadIdx.x] = INT32_MIN;
-  __syncthreads();
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows_per_block, r1 = min(rows, r0 + rows_per_block);
+  const bool mine = ty < side && c < depth && ty < r1 - r0;  // (threads without a row would only queue at the LDS atomics)
+  const bool direct = side == 1;
+  if (!direct) {
+    smn[threadIdx.x] = INT32_MAX;
+    smx[threadIdx.x] = INT32_MIN;
+    __syncthreads();
+  }
   int mn[V], mx[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) { mn[j] = INT32_MAX; mx[j] = INT32_MIN; }
-  const int64_t r1 = min(rows, (static_cast<int64_t>(blockIdx.x) + 1) * rows_per_block);
   if (mine) {
     auto take = [&](const int* v) {
 #pragma unroll
       for (int j = 0; j < V; ++j) { mn[j] = min(mn[j], v[j]); mx[j] = max(mx[j], v[j]); }
     };
-    int64_t r = static_cast<int64_t>(blockIdx.x) * rows_per_block + ty;
+    int64_t r = r0 + ty;
     const int32_t* p = x + r * depth + c;
     const int64_t step = static_cast<int64_t>(side) * depth;
-    for (; r + (kRowUnroll - 1) * side < r1; r += kRowUnroll * side, p += kRowUnroll * step) {
+    auto round = [&](auto row_at) {
       int v[kRowUnroll][V];
 #pragma unroll
       for (int u = 0; u < kRowUnroll; ++u) {
+        const int32_t* at = row_at(u);
         if constexpr (V == 4) {
-          const i4 t = *reinterpret_cast<const i4*>(p + u * step);
+          const i4 t = *reinterpret_cast<const i4*>(at);
           v[u][0] = t.x; v[u][1] = t.y; v[u][2] = t.z; v[u][3] = t.w;
         } else {
-          v[u][0] = p[u * step];
+          v[u][0] = *at;
         }
       }
 #pragma unroll
       for (int u = 0; u < kRowUnroll; ++u) take(v[u]);
-    }
-    for (; r < r1; r += side, p += step) take(p);
+    };
+    for (; r + (kRowUnroll - 1) * side < r1; r += kRowUnroll * side, p += kRowUnroll * step)
+      round([&](int u) { return p + u * step; });
+    if (r < r1)  // the rest: past the end the last row again
+      round([&](int u) { return p + (min(r + u * side, r1 - 1) - r) * depth; });
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      atomicMin(&smn[tx * V + j], mn[j]);
-      atomicMax(&smx[tx * V + j], mx[j]);
+      if (direct) {
+        atomicMin(&mn_out[c + j], mn[j]);
+        atomicMax(&mx_out[c + j], mx[j]);
+      } else {
+        atomicMin(&smn[tx * V + j], mn[j]);
+        atomicMax(&smx[tx * V + j], mx[j]);
+      }
     }
   }
+  if (direct) return;  // the whole workgroup
   __syncthreads();
   const int64_t ch = static_cast<int64_t>(blockIdx.y) * groups * V + threadIdx.x;
   if (static_cast<int>(threadIdx.x) < groups * V && ch < depth) {
@@ -1122,17 +1138,17 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       } else {
         const int64_t rpb = 4096;
         dim3 grid(blocks_for(rows, rpb), 1);
-        minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, 1, 1, rpb, min_out, max_out);
+        minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, 1, 1, kThreads, rpb, min_out, max_out);
       }
     } else {
-      const bool vec = depth % 4 == 0 && aligned(x, 16);
+      const bool few = rows <= kFewRows, vec = !few && depth % 4 == 0 && aligned(x, 16);
       const int per = vec ? 4 : 1;
       int groups = static_cast<int>(std::min<int64_t>(depth / per, vec ? 64 : kThreads));
       const int64_t col_blocks = (depth / per + groups - 1) / groups;
       ITEXHIP_REQUIRE(col_blocks <= 65535, "itexhip_minmax_i32_per_channel: depth too large");
       // 16-byte loads: column blocks of one width (400000 x 260: 87 -> 73 us).  Single ints lose by it (100000 x 257: 28 -> 34).
       if (vec) groups = static_cast<int>((depth / per + col_blocks - 1) / col_blocks);
-      const int side = kThreads / groups;
+      const int side = few ? 1 : kThreads / groups;
       // At most one workgroup per CU (a row chunk costs an atomic pair per channel; 8192 x 4096: 256 workgroups 23.8 us, 384
       // and 512 26.8, 1024 29.8), each thread at least two rounds of loads.  Single ints have a quarter of the bytes in flight:
       // one workgroup per 256 KB, up to 1024 (256 / 512 / 1024 workgroups: 16384 x 197 9.5 / 13.8 / 23.2 us, 100000 x 257 39.6 /
@@ -1142,8 +1158,8 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       const int64_t rpb = std::max<int64_t>(2 * kRowUnroll * side, (rows + row_blocks - 1) / row_blocks);
       row_blocks = (rows + rpb - 1) / rpb;
       dim3 grid(static_cast<unsigned>(row_blocks), static_cast<unsigned>(col_blocks));
-      if (vec) minmax_i32_channel_kernel<4><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, rpb, min_out, max_out);
-      else minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, rpb, min_out, max_out);
+      if (vec) minmax_i32_channel_kernel<4><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, min_out, max_out);
+      else minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, min_out, max_out);
     }
   }
   ITEXHIP_CHECK_LAUNCH("itexhip_minmax_i32_per_channel");

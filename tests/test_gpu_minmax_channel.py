@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,depth,off", [
     (1, 4, 0), (3, 8, 0), (2049, 4, 0), (4096, 252, 0), (4097, 256, 0), (700, 260, 0), (33, 4100, 0), (129, 64, 1),
-    (8193, 12, 0), (5000, 1, 1), (4099, 255, 0), (300, 257, 0), (70000, 197, 0), (513, 1000, 1)])
+    (8193, 12, 0), (5000, 1, 1), (4099, 255, 0), (300, 257, 0), (70000, 197, 0), (513, 1000, 1),
+    (8, 4, 0), (9, 4, 0), (5, 260, 0), (8, 1003, 0), (9, 1003, 1), (257, 4, 0), (264, 4, 0), (7, 1, 1)])
 def test_channel_ranges(hip, dev, rows, depth, off):
     """Groups of 4 channels and single ones, fewer and more than a workgroup's channels, unaligned tensors, chunk edges."""
     import torch
