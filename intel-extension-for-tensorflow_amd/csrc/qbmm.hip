@@ -421,7 +421,7 @@ __global__ __launch_bounds__(kBmmThreads) void qbmm_kernel(const BmmArgs a, cons
 
 template <bool ADJ_X, bool ADJ_Y, int MODE, int NB, int OUT_T, bool ROWB>  // both operands read alike
 void launch_tiles(const BmmArgs& a, const int8_t* x, const int8_t* y, void* out, dim3 grid, hipStream_t st) {
-  if constexpr (NB == 0 || ROWB) {  // the larger tiles (chosen by the host)
+  if constexpr (MODE == kAligned && (NB == 0 || ROWB)) {  // the larger tiles (chosen by the host)
     if (a.rm == 2 && a.rn == 2) {
       qbmm_kernel<ADJ_X, ADJ_Y, MODE, MODE, NB, OUT_T, ROWB, 2, 2><<<grid, kBmmThreads, 0, st>>>(a, x, y, out);
       return;
@@ -545,11 +545,13 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   // Tiles of 128 rows (and 128 columns) where more than 64 exist, the operands are aligned, the fused operands do not
   // depend on the row, and at least 1024 tiles remain (four per CU); else 64 x 64.  BERT-base attention over 128
   // sequences, 1536 tiles: Q.K^T + Mul + Add 24.6 -> 20.0 us, P.V 16.9 -> 14.2 us; over 32 sequences the 384 larger
-  // tiles measured slower than the 1536 small ones (7.4 against 6.5 us).
+  // tiles measured slower than the 1536 small ones (7.4 against 6.5 us).  Operands that take unaligned loads stay with 64 x 64
+  // at any count: P.V over 66 to 385 tokens, 64 / 128 x 64: 0.80 - 1.12, in the mean 0.97; an fp32 result with a row-broadcast
+  // operand, 110 x 277 outputs of 713 matrices, 41 us against 59.
   bool rowb = true;
   for (int b = 0; b < p->n_binary; ++b) rowb = rowb && p->binary[b].stride_m == 0;
   a.rm = a.rn = 1;
-  if (a.mode_x != kBytes && a.mode_y != kBytes && rowb && p->M > kTile) {
+  if (a.mode_x == kAligned && a.mode_y == kAligned && rowb && p->M > kTile) {
     const int rn = p->N > kTile ? 2 : 1;
     if (batch * ((p->M + 2 * kTile - 1) / (2 * kTile)) * ((p->N + rn * kTile - 1) / (rn * kTile)) >= 1024) {
       a.rm = 2;
@@ -561,13 +563,14 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
   const int64_t grid = batch * a.tiles_m * a.tiles_n;
   ITEXHIP_REQUIRE(grid < (1LL << 31), "%s: %lld output tiles exceed one launch", who, static_cast<long long>(grid));
   hipStream_t st = as_stream(stream);
-  // Whole matrices per XCD where rows are ragged, in the output or in an operand, and there are enough matrices to keep all 8
+  // Whole matrices per XCD where rows are ragged, in the output or in an operand of unaligned loads, and there are enough matrices to keep all 8
   // equally busy: 32 sequences of 197 tokens, fp32, Q.K^T + Mul + Add 45.7 -> 40.2 us, P.V 10.2 -> 9.1 us (bfloat16: 9.9 -> 9.5).
   // Tiles of a matrix spread over the XCDs where nothing is ragged: bfloat16, 128 tokens, 32 sequences, Q.K^T 7.0 -> 6.4 us,
-  // 32 heads of 384 tokens 6.2 -> 5.8 us (fp32 differs by 0.1 us either way).
+  // 32 heads of 384 tokens 6.2 -> 5.8 us (fp32 differs by 0.1 us either way).  Byte loads alone do not ask for it: 544 products
+  // of 64 x 1 by 1 x 336 with an operand of the result's size 18.1 us, spread 14.6.
   const int64_t tiles = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
   a.batch = static_cast<uint32_t>(batch);
-  const bool ragged = a.mode_x != kAligned || a.mode_y != kAligned || (p->N * (p->out_type == ITEXHIP_FLOAT ? 4 : 2)) % 64 != 0;
+  const bool ragged = a.mode_x == kAny || a.mode_y == kAny || (p->N * (p->out_type == ITEXHIP_FLOAT ? 4 : 2)) % 64 != 0;
   a.xcd_grid = ragged && (batch % 8 == 0 || batch >= 64) && tiles <= 65535 && (batch + 7) / 8 <= 65535 ? 1 : 0;
   for (int d = 0; d < a.p.n_batch_dims; ++d) a.by_dim[d] = make_fast_div(a.p.batch_dims[d]);
   const int64_t slices = (batch + 65534) / 65535;
