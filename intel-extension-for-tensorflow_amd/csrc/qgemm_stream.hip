@@ -348,6 +348,9 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   //     K = 208                 1.0, 1.05, 1.15, 1.0 - 1.3                   with a residual 1.0 - 1.1, 1.0 - 1.2, 1.3, 1.2 - 1.5
   //     K = 272 ... 480         0.7 - 1.0, 0.8 - 1.0, 0.9 - 1.0, 0.7 - 1.1   with a residual 0.9 - 1.2, 0.9 - 1.3, 1.1 - 1.6, 1.0 - 1.7
   //   convolution, K <= 384   1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
+  //                           over 256 channels and K 192 to 288: 0.8 - 1.2, 0.9 - 1.2, 1.0 - 1.4, 1.0 - 1.6, 1.1 - 2.0, but K = 288
+  //                           with three columns of workgroups (over 256 to 384 channels, the activations gathered three
+  //                           times) 0.7 - 0.9, 0.7 - 0.9, 0.7 - 1.1, 0.7 - 1.1, 0.75 - 1.1, from 6 on 1.05 - 1.2
   //   convolution, K <= 448   up to 64 channels 1.1, 1.05, 1.15, -, -; more 1.0, 0.9, 1.1, 0.9, 0.9   with a residual
   //                           1.1 - 1.2, 0.95 - 1.0, 1.3, 0.9 - 1.0, 0.9 - 1.05
   //   convolution, K = 576    0.9 - 1.1, 1.0, 1.15, -, -                              K = 1152: 0.87 - 0.94
@@ -357,7 +360,8 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   const bool whole = K % 64 == 0, fits = whole && N % 128 == 0;  // nothing padded in the tile kernel
   bool take;
   if (cv) {
-    take = K <= (wide ? 384 : 448) ? within(3) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
+    const int64_t least = sum || K <= 160 || !wide ? 3 : K > 256 && K < 384 && N > 256 && N <= 384 ? 24 : N > 256 || K >= 384 ? 6 : 3;
+    take = K <= (wide ? 384 : 448) ? within(least) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
   } else if (K <= 64) {
     take = within(sum ? 3 : fits && N >= 256 ? 7 : 4);
   } else if (K < 128) {
