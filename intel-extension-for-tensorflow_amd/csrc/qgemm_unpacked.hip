@@ -15,6 +15,9 @@
 //
 // One thread per output element with byte loads is bound by its loads (two bytes per multiplication): 1000 x 1001 x 1000 with
 // an fp32 result 399 -> 10.7 us, 37 times.  Short dot products of narrow results still go that way.
+#include <algorithm>
+#include <cmath>
+
 #include "qgemm_common.hpp"
 
 namespace itexhip {
@@ -275,18 +278,23 @@ __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __rest
   store_output<OUT_T>(out, idx, v);
 }
 
-// Short dot products of narrow results: a tile of the other kernel costs the same whether one of its rows or columns exists
-// or all 64 do, and however much of its first K step.  Times in us as both kernels measured (fp32 results; 554 sizes of 1 to
-// 1 000 000 rows and columns, K of 3 to 129): a thread's dot product 0.075 K (latency) + 1e-6 per output and 3.3 + 0.25 K for
-// up to 64 columns, 0.6 K for more, or, where the rows are far apart, 0.025 K^2 + 3 per row; tiles 2.8 + 0.009 each, 0.0045
-// more and 0.9 in all per further K step.  The faster kernel is chosen to within 10 %, for 4 sizes to within 26 %.
+// Short dot products, and narrow results: a tile of the other kernel costs the same whether one of its rows or columns exists or
+// all 64 do, and however much of its first K step.  Times in us as both kernels measured (17000 sizes of 1 to 200000 rows and
+// columns, K of 1 to 300).  A thread per output: the latency of its dot product, 2.4 + 0.071 K (0.105 K beyond 64 columns), or,
+// where the outputs fill the chip, 2 and 1e-6 of 3.4 + 0.26 K per output, more per k where a wavefront's 64 outputs touch many
+// rows (few columns, rows that share no lines) and where the weight is past 2 MB; in between the two join.  Tiles: 3.4 + 0.011
+// each, at least 5.8, per further K step half of that more and 0.9.  The choice is 0.2 % above the faster kernel in the mean and
+// takes the slower one where it costs more than 10 % for 84 of the sizes (up to twice: 122975 x 107 x 1 45 for 23).
 // Per output / tiles: 100000 x 17 x 1 4.8 / 20.7, 1 x 17 x 100000 5.3 / 20.3, 1000000 x 9 x 16 99 / 143, 8 x 9 x 8 3.6 / 6.0,
-// 1000 x 27 x 8 5.3 / 6.6; 1000 x 49 x 8 7.0 / 6.6, 100000 x 65 x 10 57 / 21, 1000 x 17 x 1000 11.3 / 6.8.
+// 270 x 9 x 1413 4.6 / 6.4, 13 x 19 x 36455 6.6 / 11.2; 100000 x 65 x 10 57 / 21, 84678 x 32 x 11 30 / 15, 1000 x 17 x 1000
+// 11.3 / 6.8.
 bool one_output_per_thread(int64_t M, int64_t K, int64_t N, int64_t tiles) {
-  const double k = static_cast<double>(K);
-  const double row = std::max(static_cast<double>(N) * (3.3 + (N <= 64 ? 0.25 : 0.6) * k), 0.025 * k * k + 3.0);
+  const double k = static_cast<double>(K), n = static_cast<double>(N), outputs = static_cast<double>(M) * n;
+  const double per_k = 0.26 + (K * N > 1 << 21 ? 0.45 : 0.0) + std::min(1.3, k / 24.0) * 2.2 / (n + 1.3);
+  const double latency = 2.4 + (N <= 64 ? 0.071 : 0.105) * k, filled = 2.0 + 1e-6 * outputs * (3.4 + per_k * k);
+  const double threads = std::cbrt(latency * latency * latency + filled * filled * filled);
   const double steps = static_cast<double>((K + kStepK - 1) / kStepK);
-  return 0.075 * k + 1e-6 * static_cast<double>(M) * row < 2.8 + 0.9 * (steps - 1.0) + 0.0045 * (1.0 + steps) * static_cast<double>(tiles);
+  return threads < std::max(5.8, 3.4 + 0.0055 * (1.0 + steps) * static_cast<double>(tiles)) + 0.9 * (steps - 1.0);
 }
 
 template <int OUT_T>
