@@ -112,14 +112,18 @@ double lines_per_unit(const WalkDim* walk, int n, int unit, double cache) {
 
 // Order and units per thread of a small tensor.  One tensor is walked from end to end, the other one jumps: the order is that of
 // the output unless the input's brings the jumping tensor through an L2 (4 MB of lines) at most half as often, or, where neither
-// does in 8 MB and more, needs at most two thirds of the lines within 8 KB, what two wavefronts have in flight.  Two units per thread overlap
-// two loads; one leaves more threads, from where and for which units below.
+// does in 8 MB and more, needs at most two thirds of the lines within 8 KB, what two wavefronts have in flight.  Single units
+// whose neighbours go out a multiple of 4 KB apart meet in the same sets and channels and stay in the output's order (3 x 64 x
+// 768 x 256 bytes (3, 1, 2, 0) 164 us, input's 552).  Two units per thread overlap two loads; one leaves more threads, and more
+// lines close by where the rows of the input are lines of their own.
 // us, one unit per thread in the output's / the input's order: 36 x 50 x 246 x 16 ints (3, 0, 1, 2) 68.3 / 19.4, 44 x 167 x 306
 // x 5 (2, 1, 3, 0) 48 / 146, 54 x 284 x 122 x 16 (2, 1, 3, 0) 197 / 365, 267 x 133 x 24 x 64 bytes (3, 2, 0, 1) 969 / 251; the
 // head split of 128 x 128 x 12 x 64 bytes 7.8 / 6.3 (the second rule).  Over 15000 shapes of up to 5 dimensions and 64 MB the
-// choice is 3 % above the fastest of the four; rules on the two innermost dimensions alone were 5.4 % above it and up to
-// three times as long as the output's order, walked by threads that return for more, with 64-bit divisions.
-// us, one / two units: 300 x 301 x 302 bytes reversed 338 / 205, 1024 x 1024 4.8 / 5.9.
+// choice is 3 % above the fastest of the four, 5 % over 7600 whose extents are powers of two and three times such; rules on the
+// two innermost dimensions alone were 5.4 and 5.8 % above it.  1.6 and 2.5 % of them take longer than in the output's order
+// with threads that return for more and 64-bit divisions (320 x 51 x 680 bytes reversed 65 us, here 150): both tensors jump by
+// whole lines there.
+// us, one / two units: 300 x 301 x 302 bytes reversed 338 / 205, 1024 x 1024 4.8 / 5.9, 1024 x 4096 x 16 (1, 0, 2) 30.6 / 49.9.
 void walk_order(TransposeArgs& a, int unit) {
   int n = a.rank;
   const bool in_runs = a.in_stride[n - 1] == 1 && a.out_dims[n - 1] > 1;
@@ -128,7 +132,6 @@ void walk_order(TransposeArgs& a, int unit) {
   for (int i = 0; i < n; ++i) order[i] = i;
   std::sort(order, order + n, [&](int p, int q) { return a.in_stride[p] > a.in_stride[q]; });
   const double bytes = static_cast<double>(a.total) * unit, mb = 1024.0 * 1024.0;
-  a.units = bytes < (unit == 1 ? 0.25 : unit == 4 && in_runs ? 1.0 : 8.0) * mb ? 1 : 2;
   WalkDim out[kMaxRank], in[kMaxRank];
   for (int i = 0; i < n; ++i) {
     const int o = n - 1 - i, p = order[n - 1 - i];
@@ -139,6 +142,13 @@ void walk_order(TransposeArgs& a, int unit) {
   bool by_input = 2.0 * l2_in < l2_out;
   if (!by_input && 2.0 * l2_out >= l2_in && bytes >= 8.0 * mb)
     by_input = 1.5 * lines_per_unit(in, n, unit, 8192.0) < lines_per_unit(out, n, unit, 8192.0);
+  if (by_input && !in_runs) {
+    int i = 0;
+    while (i < n && in[i].stride * unit < 128) ++i;
+    if (i < n && in[i].extent >= 8 && in[i].stride * unit % 4096 == 0) by_input = false;
+  }
+  const bool own_lines = unit == 16 && !in_runs && a.out_dims[order[n - 1]] % 8 == 0;  // rows of whole lines
+  a.units = bytes <= (unit == 1 ? (in_runs ? 0.25 : 1.0) : unit == 4 && in_runs ? 1.0 : 8.0) * mb || own_lines ? 1 : 2;
   if (!by_input) return;
   const TransposeArgs b = a;
   for (int i = 0; i < n; ++i) {

@@ -28,3 +28,13 @@ def test_walk_order(hip, dev, shape, perm, dtype):
 def test_short_runs(hip, dev, shape, perm, dtype):
     x = np.random.default_rng(sum(shape)).integers(-128, 128, shape).astype(dtype)
     np.testing.assert_array_equal(run_transpose(hip, dev, x, perm), np.transpose(x, perm))
+
+
+# tensors that an L2 does not hold, in the input's order: single bytes, ints and 16-byte units, runs, more than 4 dimensions;
+# and one whose destinations lie a multiple of 4 KB apart, which stays in the output's
+@pytest.mark.parametrize("shape,perm,dtype", [
+    ((267, 133, 24, 64), (3, 2, 0, 1), np.int8), ((36, 50, 246, 16), (3, 0, 1, 2), np.int32), ((146, 408, 38, 16), (2, 0, 1, 3), np.int8),
+    ((128, 128, 12, 64), (0, 2, 1, 3), np.int8), ((10, 83, 21, 12, 38), (4, 1, 2, 0, 3), np.int32), ((3, 64, 768, 256), (3, 1, 2, 0), np.int8)])
+def test_large(hip, dev, shape, perm, dtype):
+    x = np.random.default_rng(sum(shape)).integers(-128, 128, shape, dtype=np.int8).astype(dtype)
+    np.testing.assert_array_equal(run_transpose(hip, dev, x, perm), np.transpose(x, perm))
