@@ -1,5 +1,5 @@
 """The quantized BatchMatMul where rows are no multiple of a vector load: loads at any byte address, pieces cut by the end of
-a row, 16-bit results stored in pairs at odd addresses, whole matrices per XCD.  Against the CPU oracle, bit for bit."""
+a row, 16-bit results on rows of any length, whole matrices per XCD.  Against the CPU oracle, bit for bit."""
 import numpy as np
 import pytest
 
@@ -33,7 +33,7 @@ def test_rows_of_any_length(hip, dev, B, M, K, N, adj_x, adj_y, t_out):
 
 @pytest.mark.parametrize("t_out", [orc.FLOAT, orc.BFLOAT16])
 def test_large_tiles(hip, dev, t_out):
-    """At least 1024 tiles of 128 rows: the larger tiles on unaligned operands."""
+    """At least 1024 tiles of 128 rows, which unaligned operands leave to the 64 x 64 ones."""
     rng = np.random.default_rng(3)
     x = rng.integers(-128, 128, (520, 131, 37)).astype(np.int8)
     for n in (3 * 21, 131):

@@ -1,4 +1,4 @@
-"""The quantized Transpose where the walk follows the input's order instead of the output's."""
+"""The quantized Transpose walked in either tensor's order, one and two units per thread."""
 import numpy as np
 import pytest
 
@@ -17,8 +17,7 @@ def test_walk_order(hip, dev, shape, perm, dtype):
     np.testing.assert_array_equal(run_transpose(hip, dev, x, perm), np.transpose(x, perm))
 
 
-# runs of one unit (16 bytes of int8, one int32) and of a few, in the input's order and in the output's, one and two units per
-# thread: rows that share lines, destinations a power of two apart, remainders of a workgroup, bytes on both sides of 2^20
+# runs of one unit (16 bytes of int8, one int32) and of a few: rows that share lines, destinations a power of two apart, remainders of a workgroup, bytes on both sides of 2^20
 @pytest.mark.parametrize("shape,perm", [
     ((64, 7, 16), (1, 0, 2)), ((1000, 32, 16), (1, 0, 2)), ((32, 1000, 16), (1, 0, 2)), ((256, 128, 16), (1, 0, 2)),
     ((101, 67, 16), (1, 0, 2)), ((50, 9, 80, 16), (2, 1, 0, 3)), ((100, 20, 32), (1, 0, 2)), ((20, 100, 48), (1, 0, 2)),
