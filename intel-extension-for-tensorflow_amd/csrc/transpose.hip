@@ -121,7 +121,7 @@ double lines_per_unit(const WalkDim* walk, int n, int unit, double cache) {
 // head split of 128 x 128 x 12 x 64 bytes 7.8 / 6.3 (the second rule).  Over 15000 shapes of up to 5 dimensions and 64 MB the
 // choice is 3 % above the fastest of the four, 5 % over 7600 whose extents are powers of two and three times such; rules on the
 // two innermost dimensions alone were 5.4 and 5.8 % above it.  1.6 and 2.5 % of them take longer than in the output's order
-// with threads that return for more and 64-bit divisions (320 x 51 x 680 bytes reversed 65 us, here 150): both tensors jump by
+// with threads that return for more and 64-bit divisions (51 x 680 x 320 bytes reversed 65 us, here 150): both tensors jump by
 // whole lines there.
 // us, one / two units: 300 x 301 x 302 bytes reversed 338 / 205, 1024 x 1024 4.8 / 5.9, 1024 x 4096 x 16 (1, 0, 2) 30.6 / 49.9.
 void walk_order(TransposeArgs& a, int unit) {
