@@ -30,7 +30,8 @@ namespace itexhip {
 //   at LDS base + 16 * lane, no VGPRs and no ds_write on the way).  LDS is the busiest unit of this
 //   kernel (128 B/clk shared by fragment reads and staging), so staging must not cost store slots.
 //
-//   Software pipeline over K steps, one barrier per step, ring of 4 LDS stages:
+//   Software pipeline over K steps, one barrier per step, ring of 4 LDS stages (NSTAGE; 8 where a CU has one small tile, see
+//   launch_tile: the loads then run 7 steps ahead instead of 3, everything else is the same):
 //     step k computes from stage k%4 and reads the fragments of step k+1 from stage (k+1)%4; the loads
 //     of step k+3 are issued into stage (k+3)%4; before the barrier that ends step k each wavefront
 //     waits for its loads of step k+2 (issued during step k-1, a full step earlier).
@@ -95,7 +96,7 @@ static __device__ __align__(16) const uint32_t kZeroPiece[4] = {0u, 0u, 0u, 0u};
 // register operand, so the sign flip costs a 4-byte instruction per dword.  KALIGNED: K is a multiple
 // of 64, so activation loads never need a per-lane clamp and use a uniform base that advances by 64
 // bytes per step.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int OUT_T, int ACT, bool KALIGNED, bool CONV = false, bool ELEMENTWISE = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int OUT_T, int ACT, bool KALIGNED, bool CONV = false, bool ELEMENTWISE = false, int NSTAGE = 4>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
     const uint8_t* __restrict__ a, uint32_t amask, const uint8_t* __restrict__ bp, int M, int K, int N,
     int KT, int NT, int num_m, int num_n, int xcd_gm, EpilogueArgs e, void* __restrict__ out,
@@ -111,7 +112,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
   constexpr int A_PER_WAVE = A_LOADS / NW, B_PER_WAVE = B_LOADS / NW;
   constexpr int NLD = A_PER_WAVE + B_PER_WAVE;                 // loads per wavefront per step
   constexpr int NSLICE = 2 * TN;
-  constexpr int NSTAGE = 4;
+  constexpr int AHEAD = NSTAGE - 1;                            // steps that the operand loads run ahead
+  static_assert((NSTAGE & (NSTAGE - 1)) == 0 && NSTAGE >= 4, "the ring is indexed with a mask");
   static_assert(A_LOADS % NW == 0 && B_LOADS % NW == 0, "loads must divide among wavefronts");
   static_assert(NLD < 32, "vmcnt budget");
   static_assert(NSLICE % 2 == 0, "slices come in two halves");
@@ -245,17 +247,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
   // epilogue is free of global loads and of branches on them), then the operand loads of steps 0, 1, 2.  Loads return
   // in the order issued: the parameters are there when only the operand loads are outstanding, and their arithmetic
   // runs while those travel.
-  static_assert(kEarlyChannelLoads + 3 * NLD < 64, "vmcnt budget of the prologue");
+  static_assert(kEarlyChannelLoads + AHEAD * NLD < 64, "vmcnt budget of the prologue");
   const bool panel_thread = threadIdx.x < BN;
   RawChannel raw;
   if (panel_thread) raw = load_raw_channel_early(e, min(n_base + static_cast<int>(threadIdx.x), N - 1), N);
-  {
-    const int2 p0 = conv_piece(0), p1 = conv_piece(min(1, KT - 1)), p2 = conv_piece(min(2, KT - 1));
-    static_for<NLD>([&](auto c) { issue_load(c, 0, 0, p0); });
-    static_for<NLD>([&](auto c) { issue_load(c, min(1, KT - 1), 1, p1); });
-    static_for<NLD>([&](auto c) { issue_load(c, min(2, KT - 1), 2, p2); });
-  }
-  wait_vmcnt<3 * NLD>();
+  static_for<AHEAD>([&](auto k) {
+    const int kt = min(decltype(k)::value, KT - 1);
+    const int2 piece = conv_piece(kt);
+    static_for<NLD>([&](auto c) { issue_load(c, kt, decltype(k)::value, piece); });
+  });
+  wait_vmcnt<AHEAD * NLD>();
   if (panel_thread) {
     settle_raw_channel(raw);
     int comp;
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
     panel_scale[threadIdx.x] = scale;
     panel_bias[threadIdx.x] = bias;
   }
-  wait_vmcnt<NLD>();
+  wait_vmcnt<(AHEAD - 2) * NLD>();
   __syncthreads();
   // the accumulators start from the zero-point compensation of their channel (exact in int32)
   static_for<TN>([&](auto j) {
@@ -300,8 +301,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
   // The two activation fragment sets swap roles from step to step (loop unrolled by two).
   constexpr int FA = 2 * TM;                       // activation fragments per step
   auto step = [&](int kt, const v4i (&fa_cur)[FA], v4i (&fa_nxt)[FA]) {
-    const int st_cur = kt & 3, st_nxt = (kt + 1) & 3, st_fill = (kt + 3) & 3;
-    const int kt_load = min(kt + 3, KT - 1);
+    const int st_cur = kt & (NSTAGE - 1), st_nxt = (kt + 1) & (NSTAGE - 1), st_fill = (kt + AHEAD) & (NSTAGE - 1);
+    const int kt_load = min(kt + AHEAD, KT - 1);
     const int2 piece = conv_piece(kt_load);  // read at the top of the step, used by the load slots
     static_for<NSLICE>([&](auto sl) {
       constexpr int s = decltype(sl)::value;
@@ -344,7 +345,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
         __builtin_amdgcn_sched_barrier(0);
       });
     });
-    wait_vmcnt<NLD>();  // the loads of step kt+2 (issued during step kt-1) have landed
+    wait_vmcnt<(AHEAD - 2) * NLD>();  // the loads of step kt+2 have landed
     __syncthreads();
   };
   int kt = 0;
@@ -674,14 +675,23 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
   }
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int OUT_T, int ACT, bool KALIGNED, bool CONV = false, bool ELEMENTWISE = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int OUT_T, int ACT, bool KALIGNED, bool CONV = false, bool ELEMENTWISE = false, int NSTAGE = 4>
 int launch_tile(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
                 void* out, hipStream_t st, typename conv_args_of<CONV>::type cv = {}) {
   const int KT = (K + 63) / 64, NT = (N + kChunkRows - 1) / kChunkRows;
   const int num_m = (M + BM - 1) / BM, num_n = (N + BN - 1) / BN;
-  constexpr size_t lds_bytes = 4 * (BM / 16 + BN / 16) * kChunkBytes + 12 * BN + (CONV ? kMaxConvPieces * 8 : 0);  // the most
+  // One 64 x 64 tile per CU: nothing else hides the latency of its loads, and three steps (24 KB) in flight per CU are less
+  // than a memory round trip times the rate; a ring of 8 stages (64 KB) has seven steps in flight.  us, operands not in L2,
+  // fp32 results: 64 x 4096 -> 14336 16.8 -> 12.6, 512 x 4096 -> 1024 15.0 -> 11.0, 256 x 2048 -> 4096 9.7 -> 8.2, 200 x 1024 ->
+  // 4000 6.7 -> 5.9, 512 x 512 -> 1024 4.8 -> 4.7.  With two tiles per CU (192 x 512 -> 8192) 5.7 -> 6.1: not there.  128 x 128
+  // tiles gain nothing from it (4096 x 3072 -> 768 18.5 -> 18.6): LDS reads and the matrix cores bound them.
+  if constexpr (BM == 64 && BN == 64 && NSTAGE == 4) {
+    if (static_cast<int64_t>(num_m) * num_n <= 256)
+      return launch_tile<BM, BN, WAVES_M, WAVES_N, OUT_T, ACT, KALIGNED, CONV, ELEMENTWISE, 8>(a, amask, bp, M, K, N, e, out, st, cv);
+  }
+  constexpr size_t lds_bytes = NSTAGE * (BM / 16 + BN / 16) * kChunkBytes + 12 * BN + (CONV ? kMaxConvPieces * 8 : 0);  // the most
   const size_t lds_now = lds_bytes - (CONV ? (kMaxConvPieces - (K >> 4)) * 8 : 0);
-  auto kern = qgemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, OUT_T, ACT, KALIGNED, CONV, ELEMENTWISE>;
+  auto kern = qgemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, OUT_T, ACT, KALIGNED, CONV, ELEMENTWISE, NSTAGE>;
   static unsigned long long attr_done = 0;  // devices on which this instantiation's attribute is set
   if (!device_bit(&attr_done, false)) {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -705,19 +715,30 @@ int launch_tile(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int 
 // up to K = 256, where a launch is little more than its epilogue (100352 x 256 outputs, the last 1 x 1 convolution of a
 // ResNet-50 block, K = 64: 18.7 -> 12.4 us, with the residual Sum 39.5 -> 20.5 us; 4096 x 3072, 16384 x 1024 and
 // 2048 x 14336 outputs, 8-bit and fp32: 5 - 30 % faster at K = 64 - 256, mixed at 384, slower from 512 on).
-inline int pick_tile_shape(int M, int N, bool wide_only, int first = 0, bool long_epilogue_short_k = false) {
+//
+// Between one and two 64 x 64 tiles per CU, a long K: 128 x 64 tiles, one per CU, four wavefronts of 32 x 64 stacked along M
+// and the deep ring.  A CU then loads 192 rows of operands per step instead of 256 for two small tiles, and half of the device
+// no longer does twice the work of the other half.  us, 64 x 64 (or 128 x 128) tiles -> these, fp32 results: 2048 x 2048 ->
+// 1024 12.6 -> 11.2, 4096 x 2048 -> 512 14.8 -> 10.7, 128 x 4096 -> 14336 20.6 -> 18.2, 192 x 2048 -> 8192 11.0 -> 10.4,
+// 2048 x 1024 -> 1024 8.3 -> 7.7, 2500 x 768 -> 768 7.3 -> 7.2; not for K = 512 (2048 -> 1024 6.1 -> 6.4, 4096 -> 512 6.6 ->
+// 6.9), and with an addend, whose rows wait for fewer wavefronts, not for K = 1024 (512 -> 4096 8.9 -> 9.4; K = 4096 21.6 -> 18.9).
+inline int pick_tile_shape(int M, int N, int K, bool sum, bool wide_only, bool long_epilogue_short_k = false) {
   struct Shape { int bm, bn; double penalty; };
   static const Shape shapes[5] = {{256, 256, 1.0}, {256, 192, 1.03}, {256, 128, 1.08}, {128, 128, 1.2}, {64, 64, 1.8}};
   // itexhip_test_force_tile_shape forces a shape (tests exercise every shape on ragged problems with it)
   const int f = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED);
-  if (f >= (wide_only ? 3 : first) && f < 5) return f;
+  if (f >= (wide_only ? 3 : 0) && f < 6) return f;
   if (long_epilogue_short_k) {  // at least two 128 x 128 tiles per CU, at most 15 % of their area outside the output
     const int64_t t128 = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
     if (t128 >= 512 && t128 * (128 * 128) * 100 <= static_cast<int64_t>(M) * N * 115) return 3;
   }
+  if (K >= (sum ? 2048 : 768)) {
+    const int64_t t64 = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64), t128x64 = static_cast<int64_t>((M + 127) / 128) * ((N + 63) / 64);
+    if (t64 > 256 && t128x64 <= 256) return 5;
+  }
   int best = 3;
   double best_cost = 1e300;
-  for (int i = wide_only ? 3 : first; i < 5; ++i) {
+  for (int i = wide_only ? 3 : 0; i < 5; ++i) {
     const double tiles = static_cast<double>((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
     const double rounds = std::ceil(tiles / 256.0);
     const double cost = rounds * shapes[i].bm * shapes[i].bn * shapes[i].penalty;
@@ -729,7 +750,7 @@ inline int pick_tile_shape(int M, int N, bool wide_only, int first = 0, bool lon
 template <int OUT_T, int ACT>
 int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N,
                         const EpilogueArgs& e, void* out, hipStream_t st) {
-  switch (pick_tile_shape(M, N, false, 0, (ACT == 3 && K <= 1536) || K <= 256)) {
+  switch (pick_tile_shape(M, N, K, e.addend != nullptr, false, (ACT == 3 && K <= 1536) || K <= 256)) {
     case 0: return launch_tile<256, 256, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 1: return launch_tile<256, 192, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 2: return launch_tile<256, 128, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
@@ -737,15 +758,27 @@ int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int
     // epilogue - BERT-base 768 -> 768 6.85 -> 6.58 us, 3072 -> 768 with the residual Add 18.9 -> 17.4 us, the K loop of
     // 3072 -> 768 unchanged; the same split of the 256 x 128 tile changed nothing)
     case 3: return launch_tile<128, 128, 4, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
+    case 5: return launch_tile<128, 64, 4, 1, OUT_T, ACT, true, false, false, 8>(a, amask, bp, M, K, N, e, out, st);
     default: return launch_tile<64, 64, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
+  }
+}
+
+// Per-lane clamped activation loads: any K (a multiple of 16), or the element-wise epilogue.
+template <int OUT_T, int ACT, bool ELEMENTWISE>
+int dispatch_clamped(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
+                     void* out, hipStream_t st) {
+  switch (pick_tile_shape(M, N, K, e.addend != nullptr, true)) {
+    case 3: return launch_tile<128, 128, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
+    case 5: return launch_tile<128, 64, 4, 1, OUT_T, ACT, false, false, ELEMENTWISE, 8>(a, amask, bp, M, K, N, e, out, st);
+    default: return launch_tile<64, 64, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
   }
 }
 
 // A bias vector, 16-byte aligned output rows and a post-op chain of the canonical form take the vector epilogue:
 // with K a multiple of 64 the specialised kernels (uniform activation addresses) in every tile shape; other K:
-// per-lane clamped activation loads, two tile shapes.
+// per-lane clamped activation loads, three tile shapes.
 // A missing bias, an addend, other chains or unaligned outputs (rare) go to the element-wise epilogue, a kernel of
-// its own in two shapes.
+// its own in the same three shapes.
 template <int OUT_T>
 int dispatch_tile(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int K, int N,
                   const EpilogueArgs& e_in, void* out, hipStream_t st) {
@@ -758,23 +791,15 @@ int dispatch_tile(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
                                     (e.addend_type == ITEXHIP_FLOAT ? 15 : is_float16_type(e.addend_type) ? 7 : 3)) == 0);
   const bool vec_epilogue = act >= 0 && sum_ok && (e.bias != nullptr || e.fused) &&
                             (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ((static_cast<int64_t>(N) * esz) & 15) == 0;
-  const bool wide = pick_tile_shape(M, N, true) == 3;
   if (vec_epilogue && (K & 63) == 0) {
     if (act == 0) return dispatch_tile_shape<OUT_T, 0>(a, a_xor, bp, M, K, N, e, out, st);
     if (act == 1) return dispatch_tile_shape<OUT_T, 1>(a, a_xor, bp, M, K, N, e, out, st);
     if (act == 2) return dispatch_tile_shape<OUT_T, 2>(a, a_xor, bp, M, K, N, e, out, st);
     return dispatch_tile_shape<OUT_T, 3>(a, a_xor, bp, M, K, N, e, out, st);
   }
-  if (vec_epilogue && act == 3) {
-    if (wide) return launch_tile<128, 128, 2, 2, OUT_T, 3, false>(a, a_xor, bp, M, K, N, e, out, st);
-    return launch_tile<64, 64, 2, 2, OUT_T, 3, false>(a, a_xor, bp, M, K, N, e, out, st);
-  }
-  if (vec_epilogue) {  // the canonical chain covers "none" and "ReLU" too
-    if (wide) return launch_tile<128, 128, 2, 2, OUT_T, 2, false>(a, a_xor, bp, M, K, N, e, out, st);
-    return launch_tile<64, 64, 2, 2, OUT_T, 2, false>(a, a_xor, bp, M, K, N, e, out, st);
-  }
-  if (wide) return launch_tile<128, 128, 2, 2, OUT_T, 2, false, false, true>(a, a_xor, bp, M, K, N, e, out, st);
-  return launch_tile<64, 64, 2, 2, OUT_T, 2, false, false, true>(a, a_xor, bp, M, K, N, e, out, st);
+  if (vec_epilogue && act == 3) return dispatch_clamped<OUT_T, 3, false>(a, a_xor, bp, M, K, N, e, out, st);
+  if (vec_epilogue) return dispatch_clamped<OUT_T, 2, false>(a, a_xor, bp, M, K, N, e, out, st);  // covers "none" and "ReLU" too
+  return dispatch_clamped<OUT_T, 2, true>(a, a_xor, bp, M, K, N, e, out, st);
 }
 
 // Implicit GEMM of a Conv2D: `x` is the NHWC input, M = batch * out_h * out_w, K = k_h * k_w * in_c.  Run-time post-op

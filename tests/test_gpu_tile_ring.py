@@ -1,0 +1,50 @@
+"""The tile kernel with a ring of eight LDS stages (64 x 64 tiles, one per CU) and its 128 x 64 tiles: K loops shorter than the
+ring, as long as it and longer, K a multiple of 64 and not, ragged rows and channels, the vector and the element-wise epilogue
+(N not a multiple of 4); and the sizes at which the choice of a tile shape changes.  Bit-equal to the oracle."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as orc
+from tests.test_gpu_matmul import V2_DEQ, V2_REQ_S8, make_acts, make_layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [4, 5])
+@pytest.mark.parametrize("K", [16, 64, 112, 128, 192, 384, 448, 464, 512, 576, 1088])
+def test_k_loops_around_the_ring(hip, dev, shape, K):
+    hip.force_tile_shape(matmul=shape)
+    for M, N, kw in [(70, 80, V2_DEQ), (130, 132, V2_DEQ), (129, 67, V2_DEQ), (193, 144, V2_REQ_S8)]:
+        layer, w, bias = make_layer(hip, dev, K, N, seed=K + N + shape)
+        x, xq, mn, mx = make_acts(M, K, seed=M + K)
+        r = float(np.abs(x @ w + bias).max())
+        ref = layer.oracle(xq, kw, mn, mx, -r, r)
+        for path in ("tile", "fused"):
+            np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path=path), ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(1024, 512, 1024), (1025, 512, 1024),     # 256 and 272 tiles of 64 x 64
+                                   (2048, 768, 1024), (2049, 768, 1024),     # 256 and 272 tiles of 128 x 64
+                                   (2048, 752, 1024), (2048, 784, 1021)])    # K below the line; clamped loads, element-wise
+def test_where_the_shape_changes(hip, dev, M, K, N):
+    layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
+    _, xq, mn, mx = make_acts(M, K, seed=M + K)
+    np.testing.assert_array_equal(layer.run(xq, V2_DEQ, mn, mx, path="fused"), layer.oracle(xq, V2_DEQ, mn, mx))
+
+
+@pytest.mark.parametrize("K", [448, 2048])
+def test_addend_in_the_ring_kernels(hip, dev, K):
+    """The float addend is staged through the transposition buffer, which lies in the ring."""
+    import torch
+    M, N = 200, 196
+    layer, _, _ = make_layer(hip, dev, K, N, seed=K)
+    _, xq, mn, mx = make_acts(M, K, seed=K)
+    addend = np.random.default_rng(K).standard_normal((M, N)).astype(np.float32)
+    base = layer.oracle(xq, V2_DEQ, mn, mx)
+    p = hip.matmul_params(t_in=orc.QUINT8, min_a=mn, max_a=mx, add_position=1, **V2_DEQ)
+    x_d, a_d = torch.from_numpy(xq).to(dev), torch.from_numpy(addend).to(dev)
+    for shape in (4, 5):
+        hip.force_tile_shape(matmul=shape)
+        out = torch.empty((M, N), dtype=torch.float32, device=dev)
+        hip.qmatmul(p, x_d, layer.packed, layer.colsum, M, K, N, layer.min_b_d, layer.max_b_d, N, layer.bias_d, out, addend=a_d)
+        np.testing.assert_array_equal(out.cpu().numpy(), base + addend)
