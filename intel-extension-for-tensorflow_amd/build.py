@@ -6,6 +6,7 @@ Outputs (next to this file, git-ignored):
     lib/libitexhip.so        HIP kernels + the C ABI declared in include/itexhip.h
     lib/libitex_amd.so       the TensorFlow PluggableDevice kernel plugin (TF_InitKernel), if its
                              sources are present
+    lib/itexhip_call.so      the C extension through which the Python binding calls the library
 """
 import argparse
 import concurrent.futures
@@ -13,6 +14,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -101,7 +103,11 @@ def build(jobs=8, verbose=True):
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", libitexhip] + objs)
     if verbose:
         print("built", os.path.relpath(libitexhip, ROOT))
-    built = [libitexhip]
+    call = os.path.join(LIB, "itexhip_call.so")
+    _run([CXX] + CXX_FLAGS + ["-shared", "-o", call, os.path.join(HERE, "binding", "call.cc"), "-I", sysconfig.get_paths()["include"]])
+    if verbose:
+        print("built", os.path.relpath(call, ROOT))
+    built = [libitexhip, call]
     plugin_srcs = sorted(glob.glob(os.path.join(PLUGIN, "*.cc")))
     if plugin_srcs:
         libplugin = os.path.join(LIB, "libitex_amd.so")

@@ -1,10 +1,12 @@
-"""ctypes binding of lib/libitexhip.so (the C ABI declared in include/itexhip.h).
+"""Binding of lib/libitexhip.so (the C ABI declared in include/itexhip.h).
 
 All buffers are raw device addresses (ints) or objects with a `data_ptr()` method (torch tensors);
 streams are raw hipStream_t handles (ints, 0 = default stream).  Every call checks the status and
 raises ItexHipError with the library's message.
 """
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -100,16 +102,26 @@ def _i64(v):
     return C.c_int64(int(v))
 
 
-# The ops a program enqueues per step are called through prototypes: ctypes then converts plain Python numbers in C, and
-# a call builds no c_void_p / c_int64 object per argument.  A launch of a few microseconds is no longer than a dozen of those:
-# host time without the launch 2.0 -> 1.6 us (quantize) and 4.4 -> 3.3 us (qmatmul); QuantizeV2 -> MatMul -> Dequantize of
-# 128 x 1024 x 1024, which the host's calls bound, 15.0 -> 14.3 us.
+# The ops a program enqueues per step go through lib/itexhip_call.so, a C extension that converts the plain forms of the
+# arguments (binding/call.cc), and where that one does not take an argument through a ctypes prototype, which converts plain
+# Python numbers in C and builds no c_void_p / c_int64 object per argument.
 _ARG = {"p": C.c_void_p, "i": C.c_int, "l": C.c_int64, "f": C.c_float}
 
 
 def _bind(name, signature):
     """The entry point with its arguments: p = address or structure, i = int, l = int64_t, f = float."""
     return C.CFUNCTYPE(C.c_int, *(_ARG[c] for c in signature))((name, _lib))
+
+
+def _load_call():
+    loader = importlib.machinery.ExtensionFileLoader("itexhip_call", os.path.join(_HERE, "lib", "itexhip_call.so"))
+    spec = importlib.util.spec_from_file_location("itexhip_call", loader.path, loader=loader)
+    module = importlib.util.module_from_spec(spec)
+    loader.exec_module(module)
+    return module
+
+
+_call = _load_call()
 
 
 def _addr(x):
@@ -147,7 +159,8 @@ _quantize = _bind("itexhip_quantize", "ppliffp")
 
 
 def quantize(x, q, n, dst_type, scale, addend=0.0, stream=0):
-    _check(_quantize(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
+    if not _call.quantize(x, q, n, dst_type, scale, addend, stream):
+        _check(_quantize(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
 
 
 def quantize_axis(x, q, outer, slices, inner, dst_type, scales, addends=None, stream=0):
@@ -159,7 +172,8 @@ _quantize_bf16 = _bind("itexhip_quantize_bf16", "ppliffp")
 
 
 def quantize_bf16(x, q, n, dst_type, scale, addend=0.0, stream=0):
-    _check(_quantize_bf16(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
+    if not _call.quantize_bf16(x, q, n, dst_type, scale, addend, stream):
+        _check(_quantize_bf16(_addr(x), _addr(q), int(n), dst_type, scale, addend, _addr(stream)))
 
 
 def quantize_axis_bf16(x, q, outer, slices, inner, dst_type, scales, addends=None, stream=0):
@@ -171,7 +185,8 @@ _dequantize16 = _bind("itexhip_dequantize16", "ppliifip")
 
 
 def dequantize16(q, y, n, src_type, y_type, scale, zero_point=0, stream=0):
-    _check(_dequantize16(_addr(q), _addr(y), int(n), src_type, y_type, scale, int(zero_point), _addr(stream)))
+    if not _call.dequantize16(q, y, n, src_type, y_type, scale, zero_point, stream):
+        _check(_dequantize16(_addr(q), _addr(y), int(n), src_type, y_type, scale, int(zero_point), _addr(stream)))
 
 
 def dequantize_axis16(q, y, outer, slices, inner, src_type, y_type, scales, zero_points=None, stream=0):
@@ -183,7 +198,8 @@ _dequantize = _bind("itexhip_dequantize", "pplifip")
 
 
 def dequantize(q, y, n, src_type, scale, zero_point=0, stream=0):
-    _check(_dequantize(_addr(q), _addr(y), int(n), src_type, scale, int(zero_point), _addr(stream)))
+    if not _call.dequantize(q, y, n, src_type, scale, zero_point, stream):
+        _check(_dequantize(_addr(q), _addr(y), int(n), src_type, scale, int(zero_point), _addr(stream)))
 
 
 def dequantize_axis(q, y, outer, slices, inner, src_type, scales, zero_points=None, stream=0):
@@ -195,28 +211,32 @@ _requantize_per_channel = _bind("itexhip_requantize_per_channel", "ppllipp")
 
 
 def requantize_per_channel(x, q, rows, depth, dst_type, scales, stream=0):
-    _check(_requantize_per_channel(_addr(x), _addr(q), int(rows), int(depth), dst_type, _addr(scales), _addr(stream)))
+    if not _call.requantize_per_channel(x, q, rows, depth, dst_type, scales, stream):
+        _check(_requantize_per_channel(_addr(x), _addr(q), int(rows), int(depth), dst_type, _addr(scales), _addr(stream)))
 
 
 _requantize = _bind("itexhip_requantize", "pplifp")
 
 
 def requantize(x, q, n, dst_type, scale, stream=0):
-    _check(_requantize(_addr(x), _addr(q), int(n), dst_type, scale, _addr(stream)))
+    if not _call.requantize(x, q, n, dst_type, scale, stream):
+        _check(_requantize(_addr(x), _addr(q), int(n), dst_type, scale, _addr(stream)))
 
 
 _minmax_i32_per_channel = _bind("itexhip_minmax_i32_per_channel", "pllppp")
 
 
 def minmax_i32_per_channel(x, rows, depth, min_out, max_out, stream=0):
-    _check(_minmax_i32_per_channel(_addr(x), int(rows), int(depth), _addr(min_out), _addr(max_out), _addr(stream)))
+    if not _call.minmax_i32_per_channel(x, rows, depth, min_out, max_out, stream):
+        _check(_minmax_i32_per_channel(_addr(x), int(rows), int(depth), _addr(min_out), _addr(max_out), _addr(stream)))
 
 
 _minmax_f32 = _bind("itexhip_minmax_f32", "plpp")
 
 
 def minmax_f32(x, n, minmax_out, stream=0):
-    _check(_minmax_f32(_addr(x), int(n), _addr(minmax_out), _addr(stream)))
+    if not _call.minmax_f32(x, n, minmax_out, stream):
+        _check(_minmax_f32(_addr(x), int(n), _addr(minmax_out), _addr(stream)))
 
 
 def matmul_params(api=API_V2, t_in=QUINT8, t_out=FLOAT, input_mode=MIN_FIRST, out_min_first=False,
@@ -257,24 +277,27 @@ _qgemm = _bind("itexhip_qgemm", "pipplllpppipp")
 
 
 def qgemm(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_qgemm, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
-               out, stream)
+    if not _call.qgemm(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream):
+        _gemm_call(_qgemm, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
+                   out, stream)
 
 
 _qgemm_tile = _bind("itexhip_qgemm_tile", "pipplllpppipp")
 
 
 def qgemm_tile(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_qgemm_tile, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep,
-               out_type, out, stream)
+    if not _call.qgemm_tile(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream):
+        _gemm_call(_qgemm_tile, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep,
+                   out_type, out, stream)
 
 
 _qgemv = _bind("itexhip_qgemv", "pipplllpppipp")
 
 
 def qgemv(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream=0):
-    _gemm_call(_qgemv, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
-               out, stream)
+    if not _call.qgemv(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream):
+        _gemm_call(_qgemv, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type,
+                   out, stream)
 
 
 _qmatmul = _bind("itexhip_qmatmul", "pppplllpplpppp")
@@ -282,8 +305,9 @@ _qmatmul = _bind("itexhip_qmatmul", "pppplllpplpppp")
 
 def qmatmul(p, a, packed_b, colsum, M, K, N, min_b, max_b, nb, bias, out, stream=0, addend=None):
     """The whole op in one launch (parameters derived inside the MatMul kernel)."""
-    _check(_qmatmul(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(min_b),
-                    _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
+    if not _call.qmatmul(p, a, packed_b, colsum, M, K, N, min_b, max_b, nb, bias, addend, out, stream):
+        _check(_qmatmul(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(min_b),
+                        _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
 
 
 _qmatmul_per_row = _bind("itexhip_qmatmul_per_row", "pppplllpppplpppp")
@@ -291,26 +315,30 @@ _qmatmul_per_row = _bind("itexhip_qmatmul_per_row", "pppplllpppplpppp")
 
 def qmatmul_per_row(p, a, packed_b, colsum, M, K, N, row_min_a, row_max_a, min_b, max_b, nb, bias, out, stream=0,
                     addend=None):
-    _check(_qmatmul_per_row(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
-                            _addr(row_min_a), _addr(row_max_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias),
-                            _addr(addend), _addr(out), _addr(stream)))
+    if not _call.qmatmul_per_row(p, a, packed_b, colsum, M, K, N, row_min_a, row_max_a, min_b, max_b, nb, bias, addend,
+                                 out, stream):
+        _check(_qmatmul_per_row(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
+                                _addr(row_min_a), _addr(row_max_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias),
+                                _addr(addend), _addr(out), _addr(stream)))
 
 
 _qmatmul_device_range = _bind("itexhip_qmatmul_device_range", "pppplllppplpppp")
 
 
 def qmatmul_device_range(p, a, packed_b, colsum, M, K, N, range_a, min_b, max_b, nb, bias, out, stream=0, addend=None):
-    _check(_qmatmul_device_range(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
-                                 _addr(range_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend),
-                                 _addr(out), _addr(stream)))
+    if not _call.qmatmul_device_range(p, a, packed_b, colsum, M, K, N, range_a, min_b, max_b, nb, bias, addend, out, stream):
+        _check(_qmatmul_device_range(C.byref(p), _addr(a), _addr(packed_b), _addr(colsum), int(M), int(K), int(N),
+                                     _addr(range_a), _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend),
+                                     _addr(out), _addr(stream)))
 
 
 _quantize_dynamic = _bind("itexhip_quantize_dynamic", "ppliifpp")
 
 
 def quantize_dynamic(x, q, n, dst_type, mode, ensure_minimum_range, state, stream=0):
-    _check(_quantize_dynamic(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range, _addr(state),
-                             _addr(stream)))
+    if not _call.quantize_dynamic(x, q, n, dst_type, mode, ensure_minimum_range, state, stream):
+        _check(_quantize_dynamic(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range, _addr(state),
+                                 _addr(stream)))
 
 
 def read_probe(src, nbytes, sink, stream=0):
@@ -321,24 +349,28 @@ _quantize_dynamic_static = _bind("itexhip_quantize_dynamic_static", "ppliifpp")
 
 
 def quantize_dynamic_static(x, q, n, dst_type, mode, ensure_minimum_range, range_out, stream=0):
-    _check(_quantize_dynamic_static(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range,
-                                    _addr(range_out), _addr(stream)))
+    if not _call.quantize_dynamic_static(x, q, n, dst_type, mode, ensure_minimum_range, range_out, stream):
+        _check(_quantize_dynamic_static(_addr(x), _addr(q), int(n), int(dst_type), int(mode), ensure_minimum_range,
+                                        _addr(range_out), _addr(stream)))
 
 
 _quantize_dynamic_rows = _bind("itexhip_quantize_dynamic_rows", "pplliifppp")
 
 
 def quantize_dynamic_rows(x, q, rows, cols, dst_type, mode, ensure_minimum_range, row_min_out, row_max_out, stream=0):
-    _check(_quantize_dynamic_rows(_addr(x), _addr(q), int(rows), int(cols), int(dst_type), int(mode),
-                                  ensure_minimum_range, _addr(row_min_out), _addr(row_max_out), _addr(stream)))
+    if not _call.quantize_dynamic_rows(x, q, rows, cols, dst_type, mode, ensure_minimum_range, row_min_out, row_max_out,
+                                       stream):
+        _check(_quantize_dynamic_rows(_addr(x), _addr(q), int(rows), int(cols), int(dst_type), int(mode),
+                                      ensure_minimum_range, _addr(row_min_out), _addr(row_max_out), _addr(stream)))
 
 
 _qmatmul_unpacked = _bind("itexhip_qmatmul_unpacked", "pppilllpplpppp")
 
 
 def qmatmul_unpacked(p, a, w, transpose_b, M, K, N, min_b, max_b, nb, bias, out, stream=0, addend=None):
-    _check(_qmatmul_unpacked(C.byref(p), _addr(a), _addr(w), int(bool(transpose_b)), int(M), int(K), int(N),
-                             _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
+    if not _call.qmatmul_unpacked(p, a, w, int(bool(transpose_b)), M, K, N, min_b, max_b, nb, bias, addend, out, stream):
+        _check(_qmatmul_unpacked(C.byref(p), _addr(a), _addr(w), int(bool(transpose_b)), int(M), int(K), int(N),
+                                 _addr(min_b), _addr(max_b), int(nb), _addr(bias), _addr(addend), _addr(out), _addr(stream)))
 
 
 def mfma_probe(workgroups, iters, operands, sink, stream=0):
@@ -423,13 +455,16 @@ _qbatch_matmul = _bind("itexhip_qbatch_matmul", "ppppp")
 
 
 def qbatch_matmul(p, x, y, out, stream=0):
-    _check(_qbatch_matmul(C.byref(p), _addr(x), _addr(y), _addr(out), _addr(stream)))
+    if not _call.qbatch_matmul(p, x, y, out, stream):
+        _check(_qbatch_matmul(C.byref(p), _addr(x), _addr(y), _addr(out), _addr(stream)))
 
 
 _transpose = _bind("itexhip_transpose", "ppiippp")
 
 
 def transpose(x, y, elem_size, dims, perm, stream=0):
+    if _call.transpose(x, y, elem_size, dims, perm, stream):
+        return
     rank = len(dims)
     d = (C.c_int64 * max(rank, 1))(*dims)
     pm = (C.c_int32 * max(rank, 1))(*perm)
@@ -449,8 +484,9 @@ _pad_nhwc8 = _bind("itexhip_pad_nhwc8", "plllllllllpp")
 
 
 def pad_nhwc8(x, n, h, w, c, lead_h, lead_w, out_h, out_w, out_c, out, stream=0):
-    _check(_pad_nhwc8(_addr(x), int(n), int(h), int(w), int(c), int(lead_h), int(lead_w), int(out_h), int(out_w),
-                      int(out_c), _addr(out), _addr(stream)))
+    if not _call.pad_nhwc8(x, n, h, w, c, lead_h, lead_w, out_h, out_w, out_c, out, stream):
+        _check(_pad_nhwc8(_addr(x), int(n), int(h), int(w), int(c), int(lead_h), int(lead_w), int(out_h), int(out_w),
+                          int(out_c), _addr(out), _addr(stream)))
 
 
 def qconv2d_implicit_ok(geometry, x, out_channels, out_type, out):
@@ -461,8 +497,9 @@ _qconv2d = _bind("itexhip_qconv2d", "pippplpppipp")
 
 
 def qconv2d(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, out_type, out, stream=0):
-    _check(_qconv2d(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
-                    _addr(scales), _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
+    if not _call.qconv2d(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, out_type, out, stream):
+        _check(_qconv2d(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
+                        _addr(scales), _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
 
 
 _qconv2d_sum = _bind("itexhip_qconv2d_sum", "pippplppppiipp")
@@ -470,27 +507,35 @@ _qconv2d_sum = _bind("itexhip_qconv2d_sum", "pippplppppiipp")
 
 def qconv2d_sum(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, addend, addend_type, out_type, out,
                 stream=0):
-    _check(_qconv2d_sum(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
-                        _addr(scales), _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type),
-                        _addr(out), _addr(stream)))
+    if not _call.qconv2d_sum(x, x_type, geometry, packed_filter, colsum, out_channels, scales, bias, ep, addend,
+                             addend_type, out_type, out, stream):
+        _check(_qconv2d_sum(_addr(x), int(x_type), C.byref(geometry), _addr(packed_filter), _addr(colsum), int(out_channels),
+                            _addr(scales), _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type),
+                            _addr(out), _addr(stream)))
 
 
 _qgemm_sum = _bind("itexhip_qgemm_sum", "pipplllppppiipp")
 
 
 def qgemm_sum(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, addend, addend_type, out_type, out, stream=0):
-    _check(_qgemm_sum(_addr(a), int(a_type), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(scales),
-                      _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type), _addr(out),
-                      _addr(stream)))
+    if not _call.qgemm_sum(a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, addend, addend_type, out_type, out,
+                           stream):
+        _check(_qgemm_sum(_addr(a), int(a_type), _addr(packed_b), _addr(colsum), int(M), int(K), int(N), _addr(scales),
+                          _addr(bias), C.byref(ep), _addr(addend), int(addend_type), int(out_type), _addr(out),
+                          _addr(stream)))
 
 
 _qdepthwise_conv2d = _bind("itexhip_qdepthwise_conv2d", "piplppppipp")
 
 
 def qdepthwise_conv2d(x, x_type, geometry, multiplier, filt, scales, bias, ep, out_type, out, stream=0):
-    _check(_qdepthwise_conv2d(_addr(x), int(x_type), C.byref(geometry), int(multiplier), _addr(filt), _addr(scales),
-                              _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
+    if not _call.qdepthwise_conv2d(x, x_type, geometry, multiplier, filt, scales, bias, ep, out_type, out, stream):
+        _check(_qdepthwise_conv2d(_addr(x), int(x_type), C.byref(geometry), int(multiplier), _addr(filt), _addr(scales),
+                                  _addr(bias), C.byref(ep), int(out_type), _addr(out), _addr(stream)))
 
 
 def scale_vector(bias, bias_type, factors, n_factors, n, out, stream=0):
     _check(_lib.itexhip_scale_vector(_ptr(bias), int(bias_type), _ptr(factors), _i64(n_factors), _i64(n), _ptr(out), _ptr(stream)))
+
+
+_call.init(lambda name: C.cast(getattr(_lib, name), C.c_void_p).value, _check, (MatmulParams, Epilogue, BmmParams, ConvGeometry))
