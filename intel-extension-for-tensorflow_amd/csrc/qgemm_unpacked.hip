@@ -1,12 +1,12 @@
 // Quantized MatMul on operands as TensorFlow stores them: any K, no alignment, nothing prepacked.  It takes the problems
 // whose K is not a multiple of 16 (the packed kernels move whole 16-byte pieces of an activation row).
 //
-// A workgroup owns a 64 x 64 output tile and walks K in steps of 256: per step every thread fetches 64 bytes of the
+// A workgroup owns a 64 x 64 output tile, whose K is walked in steps of 256: per step every thread fetches 64 bytes of the
 // activations and 64 of the weight with 16-byte loads at whatever byte address they fall on (the hardware takes unaligned
 // vector loads; two cache lines instead of one now and then), and puts them k-contiguous into LDS; a [K, N] weight is
 // transposed on the way, 4 (k) x 16 (n) bytes per thread by byte permutes.  The long step is for latency: these problems
 // have few tiles per CU, a step costs one round trip to L2 however long it is, and with 8 loads of 16 bytes per thread in
-// flight during the previous step's MFMAs K = 1001 is 4 round trips.  n stays on the lanes of the accumulators
+// flight during the previous step's MFMAs K = 1001 is 4 round trips, 2 where two groups of wavefronts share the steps.  n stays on the lanes of the accumulators
 // (activation = first MFMA operand), so that stores are runs of 32 elements of an output row at any alignment and a lane
 // needs the parameters of one channel per quadrant.
 //
@@ -14,7 +14,7 @@
 // LDS (16 instructions per thread and step), added up across the workgroup once at the end.
 //
 // One thread per output element with byte loads is bound by its loads (two bytes per multiplication): 1000 x 1001 x 1000 with
-// an fp32 result 399 -> 10.7 us, 37 times.  Short dot products of narrow results still go that way.
+// an fp32 result 399 -> 9.7 us, 41 times.  Short dot products of narrow results still go that way.
 #include <algorithm>
 #include <cmath>
 
@@ -26,6 +26,9 @@ namespace {
 
 constexpr int kTileM = 64, kTileN = 64, kStepK = 256;
 constexpr int kRow = kStepK + 16;  // LDS bytes per row: 16-byte fragment reads of 16 rows fall into 16 different bank groups
+
+constexpr int kGroupLds = (kTileM + kTileN) * kRow;  // of a group of four wavefronts (the accumulators meet there as well)
+static_assert(kGroupLds >= kTileM * kTileN * 4, "room for the accumulators");
 
 // 16 bytes at base + off, any alignment.  A piece that would reach past the tensor's `end` is read from the last 16 bytes
 // instead (the load is the same instruction for every lane; end >= 16) and moved into place by settle16, once it has
@@ -63,23 +66,30 @@ __device__ __forceinline__ v4i keep_bytes(v4i v, int n) {
 // quarters of a 256-byte span in another order.
 __device__ __forceinline__ int w_offset(int n, int k) { return n * kRow + (k ^ (((n >> 4) & 3) << 6)); }
 
-template <int ALG>
-__device__ __forceinline__ void apply_all(const itexhip_eltwise& elt, float (&v)[16]) {
+template <int ALG, int COUNT>
+__device__ __forceinline__ void apply_all(const itexhip_eltwise& elt, float (&v)[COUNT]) {
   itexhip_eltwise e = elt;
   e.alg = ALG;  // known here: apply_eltwise folds to one case
 #pragma unroll
-  for (int i = 0; i < 16; ++i) v[i] = apply_eltwise(e, v[i]);
+  for (int i = 0; i < COUNT; ++i) v[i] = apply_eltwise(e, v[i]);
 }
 
-template <int OUT_T, bool TRANS>
-__global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
+// SPLIT groups of four wavefronts share a tile: group g takes the K steps g, g + SPLIT, ... in LDS of its own, so that the
+// first SPLIT steps' loads are all in flight at once, and the groups' accumulators meet in LDS at the end, where each group
+// finishes 16 / SPLIT of a lane's 16 rows.  A launch of few tiles is a chain of latencies (start, one round trip per step,
+// parameters, stores: 6 us without its steps, 1.2 per step), which two groups shorten; four (128 registers, 1024 threads to
+// start) are slower than two up to K = 2000.
+template <int OUT_T, bool TRANS, int SPLIT>
+__global__ __launch_bounds__(256 * SPLIT) void qmatmul_unpacked_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
                                                                 const uint8_t* __restrict__ w, int M, int K, int N,
                                                                 int tiles_n, int tiles, EpilogueArgs e, void* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) uint8_t as[kTileM * kRow];
-  __shared__ __attribute__((aligned(16))) uint8_t ws[kTileN * kRow];
-  __shared__ int colsum[kTileN];
-  const int t = threadIdx.x, lane = t & 63;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // per group its rows and columns, then the column sums
+  const int t = threadIdx.x & 255, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int group = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  uint8_t* const as = lds + group * kGroupLds;
+  uint8_t* const ws = as + kTileM * kRow;
+  int* const colsum = reinterpret_cast<int*>(lds + SPLIT * kGroupLds);
   // consecutive workgroup ids go round the 8 XCDs: give each of them a contiguous run of tiles (n fastest), whose
   // activation rows its L2 then fetches once
   const int per_xcd = (tiles + 7) / 8;
@@ -89,7 +99,7 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   const int m0 = tm * kTileM, n0 = (tile - tm * tiles_n) * kTileN;
   const int64_t a_end = static_cast<int64_t>(M) * K, w_end = static_cast<int64_t>(K) * N;
   const bool want_sums = e.comp_mul != 0 || e.prep.input_mode == ITEXHIP_MIN_FIRST;
-  if (t < kTileN) colsum[t] = 0;
+  if (threadIdx.x < kTileN) colsum[threadIdx.x] = 0;
 
   // fetch roles: rows (of the activations, or of an [N, K] weight): row t / 16 + 16 h, piece t % 16
   //              [K, N] weight: 4 k rows from 4 * (t / 4), 16 columns from 16 * (t % 4)
@@ -167,11 +177,12 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   // the channel this lane finishes; its parameters travel under the K loop
   const int n = n0 + wn + (lane & 31);
   RawChannel raw = load_raw_channel(e, min(n, N - 1), N);
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += kStepK) {
-    put(k0);
+  if (group * kStepK < K) fetch(group * kStepK);
+  for (int round = 0; round < K; round += SPLIT * kStepK) {
+    const int k0 = round + group * kStepK;  // a group may have no step in the last round
+    if (k0 < K) put(k0);
     __syncthreads();
-    if (k0 + kStepK < K) fetch(k0 + kStepK);
+    if (k0 + SPLIT * kStepK < K) fetch(k0 + SPLIT * kStepK);
     auto multiply = [&](int kk) {
       const int k = kk + (lane >> 5) * 16;
       const v4i x = *reinterpret_cast<const v4i*>(as + (wm + (lane & 31)) * kRow + k);
@@ -192,7 +203,10 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
       for (int h = 0; h < 4; ++h) {
 #pragma unroll
         for (int d = 1; d < 16; d <<= 1) sums[h] += __shfl_xor(sums[h], d, 64);
-        if ((t & 15) == 0) colsum[frow + 16 * h] = sums[h];
+        if ((t & 15) == 0) {
+          if constexpr (SPLIT == 1) colsum[frow + 16 * h] = sums[h];
+          else atomicAdd(&colsum[frow + 16 * h], sums[h]);
+        }
       }
     } else {
 #pragma unroll
@@ -202,7 +216,27 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
         if ((lane & 12) == 0) atomicAdd(&colsum[nb + i], sums[i]);
       }
     }
+  }
+  constexpr int kPer = 16 / SPLIT;  // rows of a lane that this group finishes, from `first` on
+  const int first = group * kPer;
+  int sum[kPer];
+  if constexpr (SPLIT == 1) {
+    if (want_sums) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sum[i] = acc[i];
+  } else {
+    // (the loop's last barrier: no wavefront reads its operands any more)
+    int* const mine = reinterpret_cast<int*>(as) + wave * 16 * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mine[i * 64] = acc[i];
     __syncthreads();
+    const int* src = reinterpret_cast<const int*>(lds) + (wave * 16 + first) * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sum[i] = 0;
+#pragma unroll
+    for (int g = 0; g < SPLIT; ++g)
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) sum[i] += src[g * (kGroupLds / 4) + i * 64];
   }
   if (n >= N) return;
   raw.colsum = colsum[wn + (lane & 31)];
@@ -211,10 +245,11 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
   finish_channel(e, raw, &comp, &scale, &bias);
   // accumulator i of a lane: row (i / 4) * 8 + (lane / 32) * 4 + i % 4, column lane % 32 of the quadrant
   const int mrow = m0 + wm + (lane >> 5) * 4;
-  float v[16];
+  auto row_of = [&](int i) { return mrow + ((first + i) >> 2) * 8 + ((first + i) & 3); };
+  float v[kPer];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    v[i] = static_cast<float>(acc[i] + comp) * scale;  // scale 1.0f when the node has no output scale (exact)
+  for (int i = 0; i < kPer; ++i) {
+    v[i] = static_cast<float>(sum[i] + comp) * scale;  // scale 1.0f when the node has no output scale (exact)
     v[i] = v[i] + bias;
   }
   for (int k = 0; k < e.n_eltwise; ++k) {
@@ -222,8 +257,8 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
     switch (elt.alg) {
       case ITEXHIP_ELT_SUM:
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int m = min(mrow + (i >> 2) * 8 + (i & 3), M - 1);
+        for (int i = 0; i < kPer; ++i) {
+          const int m = min(row_of(i), M - 1);
           v[i] = v[i] + elt.alpha * load_addend(e, static_cast<int64_t>(m) * N + n);
         }
         break;
@@ -241,8 +276,8 @@ __global__ __launch_bounds__(256) void qmatmul_unpacked_kernel(const uint8_t* __
     }
   }
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int m = mrow + (i >> 2) * 8 + (i & 3);
+  for (int i = 0; i < kPer; ++i) {
+    const int m = row_of(i);
     if (m < M) store_output<OUT_T>(out, static_cast<int64_t>(m) * N + n, v[i]);
   }
 }
@@ -297,8 +332,23 @@ bool one_output_per_thread(int64_t M, int64_t K, int64_t N, int64_t tiles) {
   return threads < std::max(5.8, 3.4 + 0.0055 * (1.0 + steps) * static_cast<double>(tiles)) + 0.9 * (steps - 1.0);
 }
 
+template <int OUT_T, bool TRANS, int SPLIT>
+int launch_tiles(unsigned grid, const uint8_t* a, uint32_t a_xor, const uint8_t* w, int M, int K, int N, int tiles_n, int tiles,
+                 const EpilogueArgs& e, void* out, hipStream_t st) {
+  auto kern = qmatmul_unpacked_kernel<OUT_T, TRANS, SPLIT>;
+  constexpr int kLds = SPLIT * kGroupLds + 4 * kTileN;
+  static unsigned long long attr_done = 0;  // devices on which this instantiation's attribute is set
+  if (kLds > 64 * 1024 && !device_bit(&attr_done, false)) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qmatmul_unpacked_kernel)");
+    device_bit(&attr_done, true);
+  }
+  kern<<<grid, 256 * SPLIT, kLds, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
+  return ITEXHIP_OK;
+}
+
 template <int OUT_T>
-void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
+int launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, int M, int K, int N, int tiles_n, int tiles,
             const EpilogueArgs& e, void* out, hipStream_t st) {
   const bool forced = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0;  // tests ask for the tile kernel
   if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16 || (!forced && one_output_per_thread(M, K, N, tiles))) {
@@ -306,11 +356,18 @@ void launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b,
       qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((end - first + 255) / 256), 256, 0, st>>>(
           a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out, first);
     });
-    return;
+    return ITEXHIP_OK;
   }
   const unsigned grid = static_cast<unsigned>((tiles + 7) / 8 * 8);  // whole runs for the 8 XCDs
-  if (transpose_b) qmatmul_unpacked_kernel<OUT_T, true><<<grid, 256, 0, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
-  else qmatmul_unpacked_kernel<OUT_T, false><<<grid, 256, 0, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
+  // Two groups per tile as long as every tile has a CU to itself (also with one K step, whose result two groups finish in half
+  // the time); beyond that a CU runs two workgroups of one group and hides one's waits behind the other, where one workgroup of
+  // two groups is all that its registers hold.  One group / two, us: 1000 x 1001 x 1000 (256 tiles) 11.0 / 9.7, 200 x 901 x 1000
+  // 10.2 / 8.9, 300 x 511 x 300 8.1 / 7.3, 90 x 129 x 90 6.7 / 6.4; 2000 x 301 x 1000 (512 tiles) 9.4 / 13.0.
+  const bool split = tiles <= 256;
+#define TILES(S) (transpose_b ? launch_tiles<OUT_T, true, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st) \
+                              : launch_tiles<OUT_T, false, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st))
+  return split ? TILES(2) : TILES(1);
+#undef TILES
 }
 
 }  // namespace
@@ -326,14 +383,16 @@ int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b,
   const uint32_t a_xor = a_type == ITEXHIP_QUINT8 ? 0x80808080u : 0u;
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
   const int tn = static_cast<int>(tiles_n), tiles = many_tiles ? 0 : static_cast<int>(tiles_m * tiles_n);
+  int rc;
   switch (out_type) {
-    case ITEXHIP_FLOAT: launch<ITEXHIP_FLOAT>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
-    case ITEXHIP_BFLOAT16: launch<ITEXHIP_BFLOAT16>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
-    case ITEXHIP_HALF: launch<ITEXHIP_HALF>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
-    case ITEXHIP_QINT32: launch<ITEXHIP_QINT32>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
-    case ITEXHIP_QINT8: launch<ITEXHIP_QINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
-    default: launch<ITEXHIP_QUINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_FLOAT: rc = launch<ITEXHIP_FLOAT>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_BFLOAT16: rc = launch<ITEXHIP_BFLOAT16>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_HALF: rc = launch<ITEXHIP_HALF>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_QINT32: rc = launch<ITEXHIP_QINT32>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    case ITEXHIP_QINT8: rc = launch<ITEXHIP_QINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
+    default: rc = launch<ITEXHIP_QUINT8>(ap, a_xor, wp, transpose_b, Mi, Ki, Ni, tn, tiles, e, out, st); break;
   }
+  if (rc != ITEXHIP_OK) return rc;
   ITEXHIP_CHECK_LAUNCH(who);
   return ITEXHIP_OK;
 }

@@ -35,6 +35,14 @@ def test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b):
     np.testing.assert_array_equal(out.cpu().numpy(), ref)
 
 
+# both sides of the line up to which two groups share a tile's K steps (256 tiles); an odd number of steps and a single one,
+# where the second group has none
+@pytest.mark.parametrize("M,K,N", [(1024, 257, 1024), (1025, 257, 1024), (1020, 513, 1023), (77, 1025, 190), (129, 255, 65), (64, 1281, 64)])
+@pytest.mark.parametrize("kw,transpose_b", [(V2_DEQ, False), (V2_REQ_U8_RELU, False), (dict(V2_DEQ, input_mode=orc.SCALED), True)])
+def test_split_of_k_steps(hip, dev, M, K, N, kw, transpose_b):
+    test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b)
+
+
 # sizes that go one thread per output by themselves, through the tile kernel as well, and sizes on both sides of the line
 @pytest.mark.parametrize("M,K,N", [(5, 15, 3), (2, 8, 70), (3, 17, 16), (17, 13, 129), (1, 17, 200), (200, 33, 1), (65, 9, 66), (300, 36, 8), (300, 39, 8)])
 @pytest.mark.parametrize("kw,transpose_b", [(V2_DEQ, False), (V2_REQ_U8_RELU, False), (dict(V2_DEQ, input_mode=orc.SCALED), True)])
