@@ -10,10 +10,11 @@
 // operand and its channels are put into LDS in an order that leaves a lane with 16 consecutive channels of one row: the
 // result is packed in registers and goes out as 16-byte stores, and a residual comes in as 16-byte loads a tile ahead.
 //
-// Measured, tile kernel -> this one, us: 401408 x 32 -> 64 with a clip 18.4 -> 10.9; 100352 x 64 -> 256 with a residual and
-// a ReLU 24.3 -> 15.5; 7 x 7 convolution over 32 x 224 x 224, stride 2, 224 bytes of patch -> 64 channels 30.1 -> 16.0.
-// What bounds it there: about half of the time is vector instructions (9 per result with a residual), the rest the start
-// of the launch (parameters and weight on their way to LDS, 3 us) and the results leaving L2.
+// Measured, tile kernel -> this one, us: 401408 x 32 -> 64 with a clip 18.4 -> 9.9; 100352 x 64 -> 256 with a residual and
+// a ReLU 24.3 -> 14.4; 7 x 7 convolution over 32 x 224 x 224, stride 2, 224 bytes of patch -> 64 channels 30.1 -> 12.8.
+// What bounds it there: the start of a launch that fills the device (parameters and weight on their way to LDS, first rows,
+// last stores: 5 us), then vector instructions (6 per result with a clip, 7 with a residual) and the results leaving L2
+// (401408 x 32 -> 64: 5 us beyond the start, 7.7 TB/s).
 #include "qgemm_common.hpp"
 
 namespace itexhip {
@@ -58,8 +59,12 @@ __device__ __forceinline__ uint32_t pack_bytes(const float (&v)[4]) {
   }
 }
 
-// (128 registers for four wavefronts per SIMD: enough without spills but for GROUP 4 with a sum, which spills 1 to 7.)
-template <int OUT_T, int POST, int SUM, int GROUP, bool CONV>
+// 128 registers for four wavefronts per SIMD, without spills (scratch costs a launch 1.5 us).
+// HOLD: the K chunks of a tile are exactly GROUP; all are held at once, and each is replaced by the next tile's as soon as its
+// MFMAs are issued: no second set of registers, no copies, and where a lane's pieces lie relative to its row is computed
+// once.  With two sets, copies and 21 instructions per piece the 7 x 7 convolution above took 14.6 us and 401408 x 32 -> 64
+// with a clip 10.9.  Otherwise GROUP chunks are multiplied while the next GROUP travel.
+template <int OUT_T, int POST, int SUM, int GROUP, bool CONV, bool HOLD>
 __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __restrict__ a, uint32_t amask,
                                                             const uint8_t* __restrict__ bp, const StreamArgs s, EpilogueArgs e,
                                                             uint8_t* __restrict__ out, const ConvTileArgs cv) {
@@ -121,13 +126,31 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
     else return *reinterpret_cast<const v4i*>(a + (row_off + static_cast<uint32_t>(min(c * 32 + half * 16, klast))));
   };
 
+  // (convolution: lane p works out piece p, the others read it from there; GROUP <= 8 of 2 pieces)
+  int2 mine = make_int2(0, 0);
+  if constexpr (CONV) mine = window_piece(min(lane, plast));
+  auto piece_of = [&](int c) {
+    const int p = min(c * 2 + half, plast);
+    return make_int2(__shfl(mine.x, p, 64), __shfl(mine.y, p, 64));
+  };
+  uint32_t offset[HOLD ? GROUP : 1];  // HOLD: of the lane's piece of chunk u, from the beginning of its row
+  if constexpr (HOLD) {
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) {
+      if constexpr (CONV) offset[u] = static_cast<uint32_t>(piece_of(u).y);
+      else offset[u] = static_cast<uint32_t>(min(u * 32 + half * 16, klast));
+    }
+  }
+  auto load_held = [&](int u) -> v4i { return *reinterpret_cast<const v4i*>(a + (row_off + offset[u])); };
+
   // ---- the first fragments travel while the weight is put into LDS (without the window table, which is not there yet)
-  v4i cur[GROUP], nxt[GROUP];
+  v4i cur[GROUP], nxt[HOLD ? 1 : GROUP];
   locate(t0);  // (a wavefront without rows reads the last row)
 #pragma unroll
   for (int u = 0; u < GROUP; ++u) {
     const int c = min(u, s.chunks - 1);
-    if constexpr (CONV) cur[u] = load_piece(window_piece(min(c * 2 + half, plast)));
+    if constexpr (HOLD) cur[u] = load_held(u);  // (chunks past the last one have its offsets or the row's last piece)
+    else if constexpr (CONV) cur[u] = load_piece(piece_of(c));
     else cur[u] = load(c);
   }
 
@@ -174,6 +197,7 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
   __syncthreads();
 
   if (n0 >= s.N || t0 >= t1) return;  // whole wavefront; no barrier follows
+  const int chunks = HOLD ? GROUP : s.chunks;
   const uint8_t* const wfrag = lds + wn * kBlocks * s.chunks * kChunkBytes + lane * 16;
   const int groups = (s.chunks + GROUP - 1) / GROUP;
   // Rows that a wavefront writes whole are contiguous in memory and go out as streaming stores, ahead of the flush of L2 at
@@ -195,29 +219,51 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[b][g * 4 + r] = c[r];
       }
-    for (int g = 0; g < groups; ++g) {
-      // the next group (of this tile, or the first of the next one) travels under this group's MFMAs
-      if (g + 1 < groups) {
+    auto weight = [&](int c, v4i (&w)[kBlocks]) {
 #pragma unroll
-        for (int u = 0; u < GROUP; ++u) nxt[u] = load(min((g + 1) * GROUP + u, s.chunks - 1));
-      } else if (tile + 1 < t1) {
-        locate(tile + 1);
+      for (int b = 0; b < kBlocks; ++b) w[b] = *reinterpret_cast<const v4i*>(wfrag + (b * chunks + c) * kChunkBytes);
+    };
+    auto multiply = [&](v4i x, const v4i (&w)[kBlocks]) {
+      x.x ^= amask; x.y ^= amask; x.z ^= amask; x.w ^= amask;
 #pragma unroll
-        for (int u = 0; u < GROUP; ++u) nxt[u] = load(min(u, s.chunks - 1));
-      }
+      for (int b = 0; b < kBlocks; ++b) acc[b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[b], x, acc[b], 0, 0, 0);
+    };
+    if constexpr (HOLD) {
+      // The weight comes from LDS a chunk ahead (with each chunk waiting for its own reads 13.0 us instead of 12.8).  The
+      // branch on `more` stays between the chunks: without it the scheduler reads all of them first and spills.
+      const bool more = tile + 1 < t1;  // wavefront uniform
+      if (more) locate(tile + 1);
+      v4i w[2][kBlocks];
+      weight(0, w[0]);
 #pragma unroll
       for (int u = 0; u < GROUP; ++u) {
-        const int c = g * GROUP + u;
-        if (c < s.chunks) {  // wavefront uniform
-          v4i x = cur[u];
-          x.x ^= amask; x.y ^= amask; x.z ^= amask; x.w ^= amask;
-#pragma unroll
-          for (int b = 0; b < kBlocks; ++b)
-            acc[b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i*>(wfrag + (b * s.chunks + c) * kChunkBytes), x, acc[b], 0, 0, 0);
-        }
+        if (u + 1 < GROUP) weight(u + 1, w[(u + 1) & 1]);
+        multiply(cur[u], w[u & 1]);
+        if (more) cur[u] = load_held(u);
       }
+    } else {
+      for (int g = 0; g < groups; ++g) {
+        // the next group (of this tile, or the first of the next one) travels under this group's MFMAs
+        if (g + 1 < groups) {
 #pragma unroll
-      for (int u = 0; u < GROUP; ++u) cur[u] = nxt[u];
+          for (int u = 0; u < GROUP; ++u) nxt[u] = load(min((g + 1) * GROUP + u, s.chunks - 1));
+        } else if (tile + 1 < t1) {
+          locate(tile + 1);
+#pragma unroll
+          for (int u = 0; u < GROUP; ++u) nxt[u] = load(min(u, s.chunks - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < GROUP; ++u) {
+          const int c = g * GROUP + u;
+          if (c < s.chunks) {  // wavefront uniform
+            v4i w[kBlocks];
+            weight(c, w);
+            multiply(cur[u], w);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < GROUP; ++u) cur[u] = nxt[u];
+      }
     }
     v4i packed[kBlocks];
 #pragma unroll
@@ -235,7 +281,7 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
           if constexpr (SUM == 1) v[r] = v[r] + s.sum_scale * static_cast<float>((static_cast<uint32_t>(add[b][g]) >> (8 * r)) & 0xffu);
           if constexpr (SUM == 2) v[r] = v[r] + s.sum_scale * static_cast<float>((add[b][g] << (24 - 8 * r)) >> 24);
           if constexpr (POST == kPostRelu && OUT_T != ITEXHIP_QUINT8) v[r] = fmaxf(v[r], 0.0f);
-          if constexpr (POST == kPostClip) v[r] = fminf(fmaxf(v[r], s.lo), s.hi);
+          if constexpr (POST == kPostClip) v[r] = __builtin_amdgcn_fmed3f(v[r], s.lo, s.hi);  // lo <= hi; lo for NaN, as min(max()) gives
         }
         packed[b][g] = static_cast<int>(pack_bytes<OUT_T, POST>(v));
       }
@@ -265,10 +311,10 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
   }
 }
 
-template <int OUT_T, int POST, int SUM, int GROUP, bool CONV>
+template <int OUT_T, int POST, int SUM, int GROUP, bool CONV, bool HOLD>
 int launch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs& s, const EpilogueArgs& e, uint8_t* out,
            const ConvTileArgs& cv, dim3 grid, size_t lds, hipStream_t st) {
-  auto kern = qgemm_stream_kernel<OUT_T, POST, SUM, GROUP, CONV>;
+  auto kern = qgemm_stream_kernel<OUT_T, POST, SUM, GROUP, CONV, HOLD>;
   static unsigned long long attr_done = 0;  // devices on which this instantiation's attribute is set
   if (!device_bit(&attr_done, false)) {
     hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -279,21 +325,23 @@ int launch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs
   return ITEXHIP_OK;
 }
 
-template <int OUT_T, int GROUP, bool CONV>
+template <int OUT_T, int GROUP, bool CONV, bool HOLD, bool SUMS>  // SUMS: with a residual
 int dispatch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs& s, int post, const EpilogueArgs& e, uint8_t* out,
              const ConvTileArgs& cv, dim3 grid, size_t lds, hipStream_t st) {
-  const int sum = !e.addend ? 0 : e.addend_type == ITEXHIP_QUINT8 ? 1 : 2;
-#define STREAM(P, S) return launch<OUT_T, P, S, GROUP, CONV>(a, amask, bp, s, e, out, cv, grid, lds, st)
-  switch (post * 3 + sum) {
-    case kPostNone * 3: STREAM(kPostNone, 0);
-    case kPostNone * 3 + 1: STREAM(kPostNone, 1);
-    case kPostNone * 3 + 2: STREAM(kPostNone, 2);
-    case kPostRelu * 3: STREAM(kPostRelu, 0);
-    case kPostRelu * 3 + 1: STREAM(kPostRelu, 1);
-    case kPostRelu * 3 + 2: STREAM(kPostRelu, 2);
-    case kPostClip * 3: STREAM(kPostClip, 0);
-    case kPostClip * 3 + 1: STREAM(kPostClip, 1);
-    default: STREAM(kPostClip, 2);
+#define STREAM(P, S) return launch<OUT_T, P, S, GROUP, CONV, HOLD>(a, amask, bp, s, e, out, cv, grid, lds, st)
+  if constexpr (SUMS) {
+    const bool u8 = e.addend_type == ITEXHIP_QUINT8;
+    switch (post) {
+      case kPostNone: if (u8) STREAM(kPostNone, 1); else STREAM(kPostNone, 2);
+      case kPostRelu: if (u8) STREAM(kPostRelu, 1); else STREAM(kPostRelu, 2);
+      default: if (u8) STREAM(kPostClip, 1); else STREAM(kPostClip, 2);
+    }
+  } else {
+    switch (post) {
+      case kPostNone: STREAM(kPostNone, 0);
+      case kPostRelu: STREAM(kPostRelu, 0);
+      default: STREAM(kPostClip, 0);
+    }
   }
 #undef STREAM
 }
@@ -310,6 +358,7 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   if (static_cast<int64_t>(M) * N >= (1LL << 31)) return 0;
   CanonChain c;
   const int act = canon_chain(e, &c);
+  if ((c.flags & kChainClip) && !(c.lo <= c.hi)) return 0;  // the median of three is no clip then
   if (act < 0 || act > 2 || (c.flags & ~(kChainMax0 | kChainClip | kChainSumFirst)) != 0) return 0;
   if (e.addend && (!(c.flags & kChainSumFirst) || (e.addend_type != ITEXHIP_QUINT8 && e.addend_type != ITEXHIP_QINT8) ||
                    !aligned(e.addend, 4)))
@@ -398,14 +447,43 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   uint8_t* o = static_cast<uint8_t*>(out);
   int rc;
   const bool u8 = out_type == ITEXHIP_QUINT8;
-  if (cv) rc = u8 ? dispatch<ITEXHIP_QUINT8, 4, true>(a, amask, bp, s, post, e, o, *cv, grid, lds, st)
-                  : dispatch<ITEXHIP_QINT8, 4, true>(a, amask, bp, s, post, e, o, *cv, grid, lds, st);
-  else if (s.chunks <= 1) rc = u8 ? dispatch<ITEXHIP_QUINT8, 1, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
-                                  : dispatch<ITEXHIP_QINT8, 1, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
-  else if (s.chunks <= 2) rc = u8 ? dispatch<ITEXHIP_QUINT8, 2, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
-                                  : dispatch<ITEXHIP_QINT8, 2, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
-  else rc = u8 ? dispatch<ITEXHIP_QUINT8, 4, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st)
-               : dispatch<ITEXHIP_QINT8, 4, false>(a, amask, bp, s, post, e, o, ConvTileArgs{}, grid, lds, st);
+#define STREAM(G, CONV, HOLD, SUMS, GEO)                                                                                  \
+  rc = u8 ? dispatch<ITEXHIP_QUINT8, G, CONV, HOLD, SUMS>(a, amask, bp, s, post, e, o, GEO, grid, lds, st)                \
+          : dispatch<ITEXHIP_QINT8, G, CONV, HOLD, SUMS>(a, amask, bp, s, post, e, o, GEO, grid, lds, st)
+  const ConvTileArgs none{};
+#define HELD(CONV, SUMS, GEO)                                  \
+  case 1: STREAM(1, CONV, true, SUMS, GEO); break;             \
+  case 2: STREAM(2, CONV, true, SUMS, GEO); break;             \
+  case 3: STREAM(3, CONV, true, SUMS, GEO); break;             \
+  case 4: STREAM(4, CONV, true, SUMS, GEO); break
+#define HELD_LONG(CONV, GEO)                                   \
+  case 5: STREAM(5, CONV, true, false, GEO); break;            \
+  case 6: STREAM(6, CONV, true, false, GEO); break;            \
+  case 7: STREAM(7, CONV, true, false, GEO); break;            \
+  case 8: STREAM(8, CONV, true, false, GEO); break
+  if (cv && sum) {
+    STREAM(2, true, false, true, *cv);
+  } else if (cv) {
+    switch (s.padded ? 0 : s.chunks) {
+      HELD(true, false, *cv);
+      HELD_LONG(true, *cv);
+      default: STREAM(4, true, false, false, *cv);
+    }
+  } else if (sum) {
+    switch (s.chunks) {
+      HELD(false, true, none);
+      default: STREAM(2, false, false, true, none);
+    }
+  } else {
+    switch (s.chunks) {
+      HELD(false, false, none);
+      HELD_LONG(false, none);
+      default: STREAM(4, false, false, false, none);
+    }
+  }
+#undef HELD_LONG
+#undef HELD
+#undef STREAM
   return rc == ITEXHIP_OK ? 1 : -rc;
 }
 

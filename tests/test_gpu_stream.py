@@ -84,6 +84,32 @@ def test_several_tiles_per_wavefront(hip, dev, M, K, N):
     run(hip, dev, M, K, N, "relu", hip.QUINT8, False, False, 2)
 
 
+# every count of 32-deep chunks that a wavefront holds at once and the first one beyond, several row tiles per wavefront, the
+# last chunk whole or half
+@pytest.mark.parametrize("K", [16, 64, 80, 128, 144, 192, 208, 256, 272])
+@pytest.mark.parametrize("add", [False, True])
+def test_chunk_counts(hip, dev, K, add):
+    hip.force_tile_shape(matmul=ANY_SIZE)
+    run(hip, dev, 133001, K, 16, "clip", hip.QUINT8 if add else None, False, K % 32 != 0, seed=K)
+
+
+def test_clip_with_bounds_the_wrong_way_round(hip, dev):
+    """min(max(v, lo), hi) is hi everywhere then, for this kernel's sizes as for others."""
+    import torch
+    M, K, N = 40000, 32, 64
+    ep = hip.Epilogue()
+    ep.n_scales, ep.n_eltwise = N, 1
+    ep.elt[0].alg, ep.elt[0].alpha, ep.elt[0].beta = hip.ELT_CLIP, 9.0, 4.0
+    packed = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev)
+    colsum = torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(torch.ones(K, N, dtype=torch.int8, device=dev), False, K, N, packed, colsum)
+    x = torch.arange(256, dtype=torch.uint8, device=dev).repeat(M * K // 256)
+    out = torch.zeros(M, N, dtype=torch.uint8, device=dev)
+    hip.qgemm(x, hip.QUINT8, packed, colsum, M, K, N, torch.full((N,), 0.01, device=dev), torch.zeros(N, device=dev), ep, hip.QUINT8, out)
+    torch.cuda.synchronize()
+    assert bool((out == 4).all())
+
+
 @pytest.mark.parametrize("shape,wshape,strides,dil,lead", [
     ((2, 9, 10, 16), (3, 3, 16, 48), (1, 1), (1, 1), None), ((1, 8, 7, 32), (3, 2, 32, 64), (2, 1), (1, 2), None),
     ((2, 6, 6, 48), (2, 2, 48, 112), (1, 1), (1, 1), None), ((3, 13, 11, 16), (5, 5, 16, 80), (2, 2), (1, 1), (3, 1)),
@@ -93,6 +119,15 @@ def test_several_tiles_per_wavefront(hip, dev, M, K, N):
 def test_convolutions(hip, dev, shape, wshape, strides, dil, lead, signed_in):
     hip.force_tile_shape(conv=ANY_SIZE)
     check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, np.random.default_rng(sum(shape) + signed_in))
+
+
+# no padding: every count of chunks that a wavefront holds at once, window rows of 4 channels among them
+@pytest.mark.parametrize("wshape,strides", [((1, 1, 32, 48), (1, 1)), ((2, 2, 16, 64), (1, 1)), ((2, 3, 16, 64), (2, 1)), ((2, 2, 32, 80), (1, 2)),
+                                            ((3, 3, 16, 64), (1, 1)), ((3, 4, 16, 64), (2, 2)), ((7, 8, 4, 64), (2, 2)), ((4, 4, 16, 32), (1, 1)),
+                                            ((3, 3, 32, 64), (1, 1))])
+def test_convolutions_without_padding(hip, dev, wshape, strides):
+    hip.force_tile_shape(conv=ANY_SIZE)
+    check_implicit_conv(hip, dev, (3, 23, 24, wshape[2]), wshape, strides, (1, 1), (0, 0), False, np.random.default_rng(sum(wshape)))
 
 
 @pytest.mark.parametrize("kw", [V2_REQ_S8, V2_REQ_U8_RELU, dict(V2_REQ_S8, input_mode=orc.SCALED),
