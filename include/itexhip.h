@@ -50,7 +50,7 @@ const char* itexhip_last_error(void);
 const char* itexhip_build_info(void);
 /* Test hook (no counterpart in the reference): forces the tile shape of the MatMul tile kernel (0..4 = 256x256,
  * 256x192, 256x128, 128x128, 64x64) and of the implicit-GEMM Conv2D (0..2 = 256x128, 128x128, 64x64), or (16) the kernel for
- * a short K at any size, for every later call of the process; any of them also keeps a MatMul on unpacked operands with its
+ * a short K at any size, or (17) the Conv2D kernel that keeps its input rows in LDS, for every later call of the process; any of them also keeps a MatMul on unpacked operands with its
  * tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */
 void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape);
 

@@ -36,6 +36,10 @@ int dispatch_tile_conv(const uint8_t* x, uint32_t a_xor, const uint8_t* bp, int 
 int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e, int out_type,
                void* out, hipStream_t st, const ConvTileArgs* cv);
 
+// the kernel for 3 x 3 convolutions with 32 to 128 channels and an 8-bit result (qconv_direct.hip): the same
+int try_direct(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e, int out_type,
+               void* out, hipStream_t st, const ConvTileArgs& cv);
+
 // the op on operands as TensorFlow stores them, any K (qgemm_unpacked.hip)
 int launch_unpacked(const void* a, int a_type, const int8_t* w, int transpose_b, int64_t M, int64_t K, int64_t N,
                     const EpilogueArgs& e, int out_type, void* out, hipStream_t st, const char* who);
@@ -689,7 +693,8 @@ int qconv2d_impl(const char* who, const void* x, int x_type, const itexhip_conv_
   const uint8_t* bp = reinterpret_cast<const uint8_t*>(packed_filter);
   hipStream_t hs = as_stream(stream);
   const int Mi = static_cast<int>(M), Ki = static_cast<int>(K), Ni = static_cast<int>(N);
-  int st__ = try_stream(xp, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, &cv);
+  int st__ = try_direct(xp, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, cv);
+  if (st__ == 0) st__ = try_stream(xp, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, &cv);
   if (st__ < 0) return -st__;
   if (st__ > 0) {
     ITEXHIP_CHECK_LAUNCH(who);
