@@ -377,6 +377,12 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   //     K = 192, 256            0.7 - 0.9, 0.7 - 0.9, 0.8 - 0.9, 0.7 - 1.0   with a residual (192) 1.1 at 4, 1.2 - 1.3; (256) 0.7 - 1.0
   //     K = 208                 1.0, 1.05, 1.15, 1.0 - 1.3                   with a residual 1.0 - 1.1, 1.0 - 1.2, 1.3, 1.2 - 1.5
   //     K = 272 ... 480         0.7 - 1.0, 0.8 - 1.0, 0.9 - 1.0, 0.7 - 1.1   with a residual 0.9 - 1.2, 0.9 - 1.3, 1.1 - 1.6, 1.0 - 1.7
+  //   up to 256 deep all K chunks of a tile are held at once; without a residual, 0.75, 1, 1.5, 2.5 and 3.5 rounds (the ranges above were
+  //   measured over more channels, and before the chunks were held):
+  //     up to 64 channels     K = 128 1.0, 1.1 - 1.2, 1.3, 1.4, 1.4;  144, 160 1.2 - 1.3, 1.2, 1.35 - 1.45, 1.4 - 1.5, 1.5;  176 to 256
+  //                           1.05 - 1.15, 1.15 - 1.25, 1.25 - 1.35, 1.3 - 1.5, 1.3 - 1.5 (100352 x 256 -> 64 9.5 -> 8.1 us)
+  //     65 to 1024            K = 128 -, -, 0.85 - 1.0, 0.9 - 1.1 (96 and 192 channels 1.3 - 1.7), 1.07 - 1.8, at 3 rounds 1.05 - 1.6;
+  //                           K = 192 -, 0.8, 1.0 - 1.5 (768 at 1.75 0.9), 1.1 - 1.8, 1.3 - 1.9, at 2 rounds 1.1 - 1.5;  K = 256 0.9 up to 2, 1.0 at 3
   //   convolution, K <= 384   1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
   //                           over 256 channels and K 192 to 288: 0.8 - 1.2, 0.9 - 1.2, 1.0 - 1.4, 1.0 - 1.6, 1.1 - 2.0, but K = 288
   //                           with three columns of workgroups (over 256 to 384 channels, the activations gathered three
@@ -397,9 +403,13 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   } else if (K < 128) {
     take = within(sum ? 3 : 6);
   } else if (K == 128) {
-    take = sum ? within(3) && !(fits && within(4, very_wide ? 11 : 9)) : within(16);
+    take = sum ? within(3) && !(fits && within(4, very_wide ? 11 : 9)) : within(!wide ? 4 : very_wide ? 16 : 12);
   } else if (K <= 160) {
-    take = within(6);
+    take = within(!wide && !sum ? 3 : 6);
+  } else if (K <= 256 && !wide && !sum) {
+    take = within(3);
+  } else if (K == 192 && !very_wide && !sum) {
+    take = within(8);
   } else if (K <= 512) {
     take = within(whole ? 16 : very_wide ? (sum && K <= 352 ? 12 : 16) : K <= 288 && !sum && N % 128 == 0 ? 7 : 6);
     if (very_wide) take = take && (sum ? K != 256 : K <= 224 && !whole);

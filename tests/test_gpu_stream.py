@@ -84,6 +84,12 @@ def test_several_tiles_per_wavefront(hip, dev, M, K, N):
     run(hip, dev, M, K, N, "relu", hip.QUINT8, False, False, 2)
 
 
+@pytest.mark.parametrize("M,K,N", [(98305, 256, 48), (131100, 192, 80), (100001, 144, 64)])
+def test_longer_k_by_itself(hip, dev, M, K, N):
+    """Just inside the lines from which a longer K takes this kernel, a row more than whole tiles."""
+    run(hip, dev, M, K, N, "relu", None, False, False, 3)
+
+
 # every count of 32-deep chunks that a wavefront holds at once and the first one beyond, several row tiles per wavefront, the
 # last chunk whole or half
 @pytest.mark.parametrize("K", [16, 64, 80, 128, 144, 192, 208, 256, 272])
