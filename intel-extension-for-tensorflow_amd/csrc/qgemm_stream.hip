@@ -356,7 +356,7 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   if (weight > kMaxWeightBytes) return 0;
   s.tiles = (M + 31) / 32;
   // Where it is the faster kernel, by what fills the device: `rounds` is how often the 32 x 64 pieces of the result go into
-  // the 4096 wavefronts that run at once (in quarters).  Below one round a launch is its start, and the tile kernel starts
+  // the 4096 wavefronts that run at once (in quarters).  Below one round a launch is its start, and without a residual the tile kernel starts
   // sooner; with a long K the MFMAs and the weight fragments read from LDS for every 32 rows count, and the tile kernel
   // reads them for 64 - 256; past K = 384 the weight of 128 channels leaves room for two workgroups per CU instead of three or
   // four.  Tile kernel / this kernel, time, over 16 to 14336 channels (convolutions: 32 to 512), at about 0.8, 1, 1.5, 2 and 4
@@ -383,6 +383,11 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   //                           1.05 - 1.15, 1.15 - 1.25, 1.25 - 1.35, 1.3 - 1.5, 1.3 - 1.5 (100352 x 256 -> 64 9.5 -> 8.1 us)
   //     65 to 1024            K = 128 -, -, 0.85 - 1.0, 0.9 - 1.1 (96 and 192 channels 1.3 - 1.7), 1.07 - 1.8, at 3 rounds 1.05 - 1.6;
   //                           K = 192 -, 0.8, 1.0 - 1.5 (768 at 1.75 0.9), 1.1 - 1.8, 1.3 - 1.9, at 2 rounds 1.1 - 1.5;  K = 256 0.9 up to 2, 1.0 at 3
+  //   with a residual, small launches: 16 to 4096 channels at 0.15, 0.25, 0.5, 0.75, 1 and 1.25 rounds (a MatMul; 128 x 128 tiles start late there)
+  //     K <= 64               1.0 - 1.1, 1.0 - 1.6, 1.2 - 2.2, 1.2 - 2.0;  80 to 112  0.9 - 1.1, 1.0 - 1.6, 1.0 - 1.4, 1.1 - 1.5
+  //     K = 128               0.9 - 1.1, 0.9 - 1.1, 1.1 - 1.9, 1.1 - 1.7, 1.0 - 1.3, 1.05 - 1.3 (from 1024 channels on 0.9 - 1.0), then 1.0 - 2.5
+  //     K = 160               0.9 - 1.0, 1.0 - 1.4, 1.0 - 1.4, 1.05 - 1.4, 1.0 - 1.5, 1.0 - 1.5
+  //     K = 192; 256          0.8 - 1.0, 0.9 - 1.1, 1.2 - 1.9, 1.1 - 1.7, 1.0 - 1.2, 1.0 - 1.2;  0.8 - 0.9, 0.8 - 0.95, 1.0 - 1.7, 1.05 - 1.5, 0.9 - 1.1, 0.9 - 1.1
   //   convolution, K <= 384   1.0 - 1.3, 1.0 - 1.2, 1.2 - 1.5, 1.1 - 1.5, 1.7         with a residual 1.1 - 1.7
   //                           over 256 channels and K 192 to 288: 0.8 - 1.2, 0.9 - 1.2, 1.0 - 1.4, 1.0 - 1.6, 1.1 - 2.0, but K = 288
   //                           with three columns of workgroups (over 256 to 384 channels, the activations gathered three
@@ -399,13 +404,13 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
     const int64_t least = sum || K <= 160 || !wide ? 3 : K > 256 && K < 384 && N > 256 && N <= 384 ? 24 : N > 256 || K >= 384 ? 6 : 3;
     take = K <= (wide ? 384 : 448) ? within(least) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
   } else if (K <= 64) {
-    take = within(sum ? 3 : fits && N >= 256 ? 7 : 4);
+    take = within(sum ? 1 : fits && N >= 256 ? 7 : 4);
   } else if (K < 128) {
-    take = within(sum ? 3 : 6);
+    take = within(sum ? 1 : 6);
   } else if (K == 128) {
-    take = sum ? within(3) && !(fits && within(4, very_wide ? 11 : 9)) : within(!wide ? 4 : very_wide ? 16 : 12);
+    take = sum ? within(2) && !(fits && N >= 1024 && within(4, 5)) : within(!wide ? 4 : very_wide ? 16 : 12);
   } else if (K <= 160) {
-    take = within(!wide && !sum ? 3 : 6);
+    take = within(sum ? 2 : !wide ? 3 : 6);
   } else if (K <= 256 && !wide && !sum) {
     take = within(3);
   } else if (K == 192 && !very_wide && !sum) {
@@ -413,6 +418,7 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   } else if (K <= 512) {
     take = within(whole ? 16 : very_wide ? (sum && K <= 352 ? 12 : 16) : K <= 288 && !sum && N % 128 == 0 ? 7 : 6);
     if (very_wide) take = take && (sum ? K != 256 : K <= 224 && !whole);
+    if (sum && (K == 192 ? within(2, 5) : K == 256 && within(2, 3))) take = true;
     if (K == 512) take = take && (sum || N == 128);
     else if (K > 448 && !wide) take = take && within(6, 12);
   } else {

@@ -90,6 +90,12 @@ def test_longer_k_by_itself(hip, dev, M, K, N):
     run(hip, dev, M, K, N, "relu", None, False, False, 3)
 
 
+@pytest.mark.parametrize("M,K,N", [(32801, 64, 64), (8225, 112, 192), (16500, 128, 256), (16500, 160, 208), (16500, 192, 256), (16500, 256, 256)])
+def test_small_launches_with_a_residual(hip, dev, M, K, N):
+    """Just inside the lines from which a call with a residual takes this kernel."""
+    run(hip, dev, M, K, N, "relu", hip.QUINT8, False, False, 4)
+
+
 # every count of 32-deep chunks that a wavefront holds at once and the first one beyond, several row tiles per wavefront, the
 # last chunk whole or half
 @pytest.mark.parametrize("K", [16, 64, 80, 128, 144, 192, 208, 256, 272])
