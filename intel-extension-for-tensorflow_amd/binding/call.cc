@@ -9,6 +9,8 @@
 // without having done anything and the caller goes through its ctypes prototype, which converts or refuses as ever.
 //
 // The addresses of the entry points come from the library that the binding has loaded (init), so this module links to none.
+// They belong to the module object, as do the check and the structures: a process may hold several copies of the binding
+// (it has several import names, and ITEXHIP_LIB chooses a library for each), and each has a module object of its own.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -21,9 +23,23 @@
 
 namespace {
 
-PyObject* g_check;         // the binding's _check(status): raises unless it is 0
-PyObject* g_data_ptr;      // "data_ptr"
-PyTypeObject* g_structs[4];  // MatmulParams, Epilogue, BmmParams, ConvGeometry
+#define ENTRY_POINTS(X)                                                                                               \
+  X(quantize) X(quantize_bf16) X(dequantize) X(dequantize16) X(requantize) X(requantize_per_channel)                  \
+  X(minmax_i32_per_channel) X(minmax_f32) X(qgemm) X(qgemm_tile) X(qgemv) X(qgemm_sum) X(qmatmul) X(qmatmul_per_row)  \
+  X(qmatmul_device_range) X(qmatmul_unpacked) X(quantize_dynamic) X(quantize_dynamic_static) X(quantize_dynamic_rows) \
+  X(qbatch_matmul) X(pad_nhwc8) X(qconv2d) X(qconv2d_sum) X(qdepthwise_conv2d)
+
+// All zero until init
+struct State {
+  PyObject* check;           // the binding's _check(status): raises unless it is 0
+  PyObject* data_ptr;        // "data_ptr"
+  PyTypeObject* structs[4];  // MatmulParams, Epilogue, BmmParams, ConvGeometry
+#define POINTER(NAME) decltype(&itexhip_##NAME) NAME;
+  ENTRY_POINTS(POINTER) POINTER(transpose)
+#undef POINTER
+};
+
+State* state_of(PyObject* module) { return static_cast<State*>(PyModule_GetState(module)); }
 
 // How many buffers of ctypes structures a call holds on to: at most two structures
 struct Held {
@@ -42,7 +58,7 @@ template <class T> constexpr int struct_index() {
   return -1;
 }
 
-Result address(PyObject* o, void** out) {
+Result address(const State& st, PyObject* o, void** out) {
   if (o == Py_None) { *out = nullptr; return kOk; }
   if (PyLong_CheckExact(o)) {
     *out = PyLong_AsVoidPtr(o);
@@ -50,7 +66,7 @@ Result address(PyObject* o, void** out) {
     return kOk;
   }
   if (PyFloat_CheckExact(o) || PyUnicode_CheckExact(o)) return kOther;
-  PyObject* r = PyObject_CallMethodNoArgs(o, g_data_ptr);
+  PyObject* r = PyObject_CallMethodNoArgs(o, st.data_ptr);
   if (r == nullptr) {
     if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return kError;
     PyErr_Clear();
@@ -65,11 +81,11 @@ Result address(PyObject* o, void** out) {
 }
 
 template <class T>
-Result convert(PyObject* o, T* out, Held& held) {
+Result convert(const State& st, PyObject* o, T* out, Held& held) {
   if constexpr (std::is_pointer_v<T>) {
     constexpr int s = struct_index<std::remove_cv_t<std::remove_pointer_t<T>>>();
     if constexpr (s >= 0) {
-      if (Py_TYPE(o) != g_structs[s] || held.n == 2) return kOther;
+      if (Py_TYPE(o) != st.structs[s] || held.n == 2) return kOther;
       if (PyObject_GetBuffer(o, &held.view[held.n], PyBUF_SIMPLE) != 0) { PyErr_Clear(); return kOther; }
       const Py_buffer& v = held.view[held.n++];
       if (v.len < static_cast<Py_ssize_t>(sizeof(std::remove_pointer_t<T>))) return kOther;
@@ -77,7 +93,7 @@ Result convert(PyObject* o, T* out, Held& held) {
       return kOk;
     } else {
       void* p;
-      const Result r = address(o, &p);
+      const Result r = address(st, o, &p);
       if (r == kOk) *out = static_cast<T>(p);
       return r;
     }
@@ -98,9 +114,9 @@ Result convert(PyObject* o, T* out, Held& held) {
   }
 }
 
-PyObject* finish(int status) {
+PyObject* finish(const State& st, int status) {
   if (status == ITEXHIP_OK) Py_RETURN_TRUE;
-  PyObject* r = PyObject_CallFunction(g_check, "i", status);
+  PyObject* r = PyObject_CallFunction(st.check, "i", status);
   Py_XDECREF(r);
   if (r == nullptr) return nullptr;
   Py_RETURN_TRUE;
@@ -111,52 +127,46 @@ template <class F> struct Call;
 template <class... A>
 struct Call<int(A...)> {
   template <size_t... I>
-  static PyObject* go(int (*fn)(A...), PyObject* const* args, std::index_sequence<I...>) {
+  static PyObject* go(const State& st, int (*fn)(A...), PyObject* const* args, std::index_sequence<I...>) {
     std::tuple<std::remove_const_t<A>...> v{};
     Held held;
     Result r = kOk;
-    (void)((r = convert(args[I], &std::get<I>(v), held), r == kOk) && ...);
+    (void)((r = convert(st, args[I], &std::get<I>(v), held), r == kOk) && ...);
     if (r == kError) return nullptr;
     if (r == kOther) Py_RETURN_FALSE;
     int status;
     Py_BEGIN_ALLOW_THREADS  // as ctypes does: a launch may wait for room in the queue
     status = fn(std::get<I>(v)...);
     Py_END_ALLOW_THREADS
-    return finish(status);
+    return finish(st, status);
   }
-  static PyObject* run(int (*fn)(A...), PyObject* const* args, Py_ssize_t n) {
+  static PyObject* run(const State& st, int (*fn)(A...), PyObject* const* args, Py_ssize_t n) {
     if (n != static_cast<Py_ssize_t>(sizeof...(A)) || fn == nullptr) Py_RETURN_FALSE;
-    return go(fn, args, std::index_sequence_for<A...>{});
+    return go(st, fn, args, std::index_sequence_for<A...>{});
   }
 };
 
-#define ENTRY_POINTS(X)                                                                                               \
-  X(quantize) X(quantize_bf16) X(dequantize) X(dequantize16) X(requantize) X(requantize_per_channel)                  \
-  X(minmax_i32_per_channel) X(minmax_f32) X(qgemm) X(qgemm_tile) X(qgemv) X(qgemm_sum) X(qmatmul) X(qmatmul_per_row)  \
-  X(qmatmul_device_range) X(qmatmul_unpacked) X(quantize_dynamic) X(quantize_dynamic_static) X(quantize_dynamic_rows) \
-  X(qbatch_matmul) X(pad_nhwc8) X(qconv2d) X(qconv2d_sum) X(qdepthwise_conv2d)
-
-#define DEFINE(NAME)                                                                     \
-  decltype(&itexhip_##NAME) p_##NAME;                                                    \
-  PyObject* f_##NAME(PyObject*, PyObject* const* args, Py_ssize_t n) {                   \
-    return Call<std::remove_pointer_t<decltype(&itexhip_##NAME)>>::run(p_##NAME, args, n); \
+#define DEFINE(NAME)                                                                              \
+  PyObject* f_##NAME(PyObject* self, PyObject* const* args, Py_ssize_t n) {                       \
+    const State& st = *state_of(self);                                                            \
+    return Call<std::remove_pointer_t<decltype(&itexhip_##NAME)>>::run(st, st.NAME, args, n);     \
   }
 ENTRY_POINTS(DEFINE)
 #undef DEFINE
 
 // transpose(x, y, elem_size, dims, perm, stream): the extents and the permutation as tuples of plain ints
-decltype(&itexhip_transpose) p_transpose;
 constexpr Py_ssize_t kMaxRank = 8;
 template <class T>
-bool int_tuple(PyObject* o, T (&out)[kMaxRank]) {
+bool int_tuple(const State& st, PyObject* o, T (&out)[kMaxRank]) {
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(o); ++i) {
     Held none;
-    if (convert(PyTuple_GET_ITEM(o, i), &out[i], none) != kOk) return false;
+    if (convert(st, PyTuple_GET_ITEM(o, i), &out[i], none) != kOk) return false;
   }
   return true;
 }
-PyObject* f_transpose(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 6 || p_transpose == nullptr || !PyTuple_CheckExact(args[3]) || !PyTuple_CheckExact(args[4])) Py_RETURN_FALSE;
+PyObject* f_transpose(PyObject* self, PyObject* const* args, Py_ssize_t n) {
+  const State& st = *state_of(self);
+  if (n != 6 || st.transpose == nullptr || !PyTuple_CheckExact(args[3]) || !PyTuple_CheckExact(args[4])) Py_RETURN_FALSE;
   const Py_ssize_t rank = PyTuple_GET_SIZE(args[3]);
   if (rank > kMaxRank || PyTuple_GET_SIZE(args[4]) != rank) Py_RETURN_FALSE;
   Held none;
@@ -164,24 +174,25 @@ PyObject* f_transpose(PyObject*, PyObject* const* args, Py_ssize_t n) {
   int elem_size;
   int64_t dims[kMaxRank];
   int32_t perm[kMaxRank];
-  const Result rx = address(args[0], &x);
+  const Result rx = address(st, args[0], &x);
   if (rx == kError) return nullptr;
-  const Result ry = address(args[1], &y);
+  const Result ry = address(st, args[1], &y);
   if (ry == kError) return nullptr;
-  const Result rs = address(args[5], &stream);
+  const Result rs = address(st, args[5], &stream);
   if (rs == kError) return nullptr;
-  if (rx != kOk || ry != kOk || rs != kOk || convert(args[2], &elem_size, none) != kOk || !int_tuple(args[3], dims) ||
-      !int_tuple(args[4], perm))
+  if (rx != kOk || ry != kOk || rs != kOk || convert(st, args[2], &elem_size, none) != kOk ||
+      !int_tuple(st, args[3], dims) || !int_tuple(st, args[4], perm))
     Py_RETURN_FALSE;
   int status;
   Py_BEGIN_ALLOW_THREADS
-  status = p_transpose(x, y, elem_size, static_cast<int>(rank), dims, perm, stream);
+  status = st.transpose(x, y, elem_size, static_cast<int>(rank), dims, perm, stream);
   Py_END_ALLOW_THREADS
-  return finish(status);
+  return finish(st, status);
 }
 
 // init(address, check, structures): address(name) gives an entry point's address in the loaded library
-PyObject* init(PyObject*, PyObject* args) {
+PyObject* init(PyObject* self, PyObject* args) {
+  State& st = *state_of(self);
   PyObject *addresses, *check, *s[4];
   if (!PyArg_ParseTuple(args, "OO(OOOO)", &addresses, &check, &s[0], &s[1], &s[2], &s[3])) return nullptr;
   for (PyObject* t : s)
@@ -193,17 +204,16 @@ PyObject* init(PyObject*, PyObject* args) {
     Py_XDECREF(r);
     if (PyErr_Occurred()) ok = false;
   };
-#define SET(NAME) set("itexhip_" #NAME, reinterpret_cast<void**>(&p_##NAME));
-  ENTRY_POINTS(SET)
-  SET(transpose)
+#define SET(NAME) set("itexhip_" #NAME, reinterpret_cast<void**>(&st.NAME));
+  ENTRY_POINTS(SET) SET(transpose)
 #undef SET
   if (!ok) return nullptr;
   Py_INCREF(check);
-  Py_XSETREF(g_check, check);
+  Py_XSETREF(st.check, check);
   for (int i = 0; i < 4; ++i) {
     Py_INCREF(s[i]);
-    PyTypeObject* old = g_structs[i];
-    g_structs[i] = reinterpret_cast<PyTypeObject*>(s[i]);
+    PyTypeObject* old = st.structs[i];
+    st.structs[i] = reinterpret_cast<PyTypeObject*>(s[i]);
     Py_XDECREF(old);
   }
   Py_RETURN_NONE;
@@ -216,11 +226,31 @@ PyMethodDef methods[] = {
     {"init", init, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "itexhip_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+int exec_module(PyObject* module) {
+  State& st = *state_of(module);
+  st.data_ptr = PyUnicode_InternFromString("data_ptr");
+  return st.data_ptr != nullptr ? 0 : -1;
+}
+int traverse(PyObject* module, visitproc visit, void* arg) {
+  if (State* st = state_of(module)) {
+    Py_VISIT(st->check);
+    for (PyTypeObject* t : st->structs) Py_VISIT(t);
+  }
+  return 0;
+}
+int clear(PyObject* module) {
+  if (State* st = state_of(module)) {
+    Py_CLEAR(st->check);
+    Py_CLEAR(st->data_ptr);
+    for (PyTypeObject*& t : st->structs) Py_CLEAR(t);
+  }
+  return 0;
+}
+void free_module(void* module) { clear(static_cast<PyObject*>(module)); }
+
+PyModuleDef_Slot slots[] = {{Py_mod_exec, reinterpret_cast<void*>(exec_module)}, {0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "itexhip_call", nullptr, sizeof(State), methods, slots, traverse, clear, free_module};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_itexhip_call() {
-  g_data_ptr = PyUnicode_InternFromString("data_ptr");
-  return g_data_ptr != nullptr ? PyModule_Create(&module) : nullptr;
-}
+PyMODINIT_FUNC PyInit_itexhip_call() { return PyModuleDef_Init(&module); }
