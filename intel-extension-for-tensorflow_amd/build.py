@@ -6,11 +6,13 @@ Outputs (next to this file, git-ignored):
     lib/libitexhip.so        HIP kernels + the C ABI declared in include/itexhip.h
     lib/libitex_amd.so       the TensorFlow PluggableDevice kernel plugin (TF_InitKernel), if its
                              sources are present
-    lib/itexhip_call.so      the C extension through which the Python binding calls the library
+    lib/itexhip_call.<abi>.so  the C extension through which the Python binding calls the library, for the Python that runs
+                             this file and if its headers are there (without it the binding calls through ctypes)
 """
 import argparse
 import concurrent.futures
 import glob
+import importlib.machinery
 import os
 import subprocess
 import sys
@@ -92,6 +94,20 @@ def check_inline_asm_hazards(asm_files, verbose=True):
         print("inline-assembly hazard check: %d assembly files clean" % len(asm_files))
 
 
+def build_call(verbose=True):
+    """The C extension of the binding; None where Python's headers are not installed."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        if verbose:
+            print("no Python.h in %s: the binding will call through ctypes" % include)
+        return None
+    call = os.path.join(LIB, "itexhip_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
+    _run([CXX] + CXX_FLAGS + ["-shared", "-o", call, os.path.join(HERE, "binding", "call.cc"), "-I", include])
+    if verbose:
+        print("built", os.path.relpath(call, ROOT))
+    return call
+
+
 def build(jobs=8, verbose=True):
     os.makedirs(LIB, exist_ok=True)
     os.makedirs(OBJ, exist_ok=True)
@@ -103,11 +119,7 @@ def build(jobs=8, verbose=True):
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", libitexhip] + objs)
     if verbose:
         print("built", os.path.relpath(libitexhip, ROOT))
-    call = os.path.join(LIB, "itexhip_call.so")
-    _run([CXX] + CXX_FLAGS + ["-shared", "-o", call, os.path.join(HERE, "binding", "call.cc"), "-I", sysconfig.get_paths()["include"]])
-    if verbose:
-        print("built", os.path.relpath(call, ROOT))
-    built = [libitexhip, call]
+    built = [libitexhip]
     plugin_srcs = sorted(glob.glob(os.path.join(PLUGIN, "*.cc")))
     if plugin_srcs:
         libplugin = os.path.join(LIB, "libitex_amd.so")
@@ -117,7 +129,8 @@ def build(jobs=8, verbose=True):
         if verbose:
             print("built", os.path.relpath(libplugin, ROOT))
         built.append(libplugin)
-    return built
+    call = build_call(verbose)
+    return built + ([call] if call else [])
 
 
 if __name__ == "__main__":

@@ -102,9 +102,9 @@ def _i64(v):
     return C.c_int64(int(v))
 
 
-# The ops a program enqueues per step go through lib/itexhip_call.so, a C extension that converts the plain forms of the
-# arguments (binding/call.cc), and where that one does not take an argument through a ctypes prototype, which converts plain
-# Python numbers in C and builds no c_void_p / c_int64 object per argument.
+# The ops a program enqueues per step go through lib/itexhip_call.<abi>.so, a C extension that converts the plain forms of the
+# arguments (binding/call.cc), and where that one does not take an argument, or was not built for this Python, through a
+# ctypes prototype, which converts plain Python numbers in C and builds no c_void_p / c_int64 object per argument.
 _ARG = {"p": C.c_void_p, "i": C.c_int, "l": C.c_int64, "f": C.c_float}
 
 
@@ -113,8 +113,22 @@ def _bind(name, signature):
     return C.CFUNCTYPE(C.c_int, *(_ARG[c] for c in signature))((name, _lib))
 
 
+class _Prototypes:
+    """In the extension's place where there is none: takes no call."""
+
+    def __getattr__(self, name):
+        return self._decline
+
+    @staticmethod
+    def _decline(*args):
+        return False
+
+
 def _load_call():
-    loader = importlib.machinery.ExtensionFileLoader("itexhip_call", os.path.join(_HERE, "lib", "itexhip_call.so"))
+    path = os.path.join(_HERE, "lib", "itexhip_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
+    if not os.path.exists(path):
+        return _Prototypes()
+    loader = importlib.machinery.ExtensionFileLoader("itexhip_call", path)
     spec = importlib.util.spec_from_file_location("itexhip_call", loader.path, loader=loader)
     module = importlib.util.module_from_spec(spec)
     loader.exec_module(module)

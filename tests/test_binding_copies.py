@@ -33,3 +33,27 @@ def test_copies_do_not_share_state(hip, monkeypatch, tmp_path, other_library):
             with pytest.raises(copy.ItexHipError):
                 copy.quantize(None, None, n, copy.QUINT8, 1.0)
         assert b"negative" in first.raw().itexhip_last_error() and b"null" in second.raw().itexhip_last_error()
+
+
+def test_without_the_extension(hip, monkeypatch):
+    """No extension for this Python: the same calls through the ctypes prototypes."""
+    import importlib.machinery
+    monkeypatch.setattr(importlib.machinery, "EXTENSION_SUFFIXES", [".no-such-abi.so"])
+    plain = load_copy(hip, "plain")
+    assert plain._call.quantize(None, None, 0, plain.QUINT8, 1.0, 0.0, 0) is False
+    plain.quantize(None, None, 0, plain.QUINT8, 1.0)
+    plain.qmatmul(plain.matmul_params(), 0, 0, 0, 0, 64, 16, 0, 0, 16, 0, 0)
+    plain.transpose(64, 64, 1, (0, 2), (1, 0))
+    with pytest.raises(plain.ItexHipError, match="negative"):
+        plain.quantize(None, None, -1, plain.QUINT8, 1.0)
+
+
+def test_build_without_python_headers(hip, monkeypatch, tmp_path):
+    import sysconfig
+    import __graft_entry__ as entry
+    build = entry._load_build_module()
+    monkeypatch.setattr(build, "LIB", str(tmp_path))
+    built = build.build_call(verbose=False)
+    assert os.path.basename(built).startswith("itexhip_call.") and os.path.basename(built) != "itexhip_call.so"
+    monkeypatch.setattr(sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build.build_call(verbose=False) is None
