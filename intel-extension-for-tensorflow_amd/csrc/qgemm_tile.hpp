@@ -30,8 +30,8 @@ namespace itexhip {
 //   at LDS base + 16 * lane, no VGPRs and no ds_write on the way).  LDS is the busiest unit of this
 //   kernel (128 B/clk shared by fragment reads and staging), so staging must not cost store slots.
 //
-//   Software pipeline over K steps, one barrier per step, ring of 4 LDS stages (NSTAGE; 8 where a CU has one small tile, see
-//   launch_tile: the loads then run 7 steps ahead instead of 3, everything else is the same):
+//   Software pipeline over K steps, one barrier per step, ring of 4 LDS stages (NSTAGE; 8 where a CU has one small tile and K is long,
+//   see launch_tile: the loads then run 7 steps ahead instead of 3, everything else is the same):
 //     step k computes from stage k%4 and reads the fragments of step k+1 from stage (k+1)%4; the loads
 //     of step k+3 are issued into stage (k+3)%4; before the barrier that ends step k each wavefront
 //     waits for its loads of step k+2 (issued during step k-1, a full step earlier).
@@ -683,10 +683,17 @@ int launch_tile(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int 
   // One 64 x 64 tile per CU: nothing else hides the latency of its loads, and three steps (24 KB) in flight per CU are less
   // than a memory round trip times the rate; a ring of 8 stages (64 KB) has seven steps in flight.  us, operands not in L2,
   // fp32 results: 64 x 4096 -> 14336 16.8 -> 12.6, 512 x 4096 -> 1024 15.0 -> 11.0, 256 x 2048 -> 4096 9.7 -> 8.2, 200 x 1024 ->
-  // 4000 6.7 -> 5.9, 512 x 512 -> 1024 4.8 -> 4.7.  With two tiles per CU (192 x 512 -> 8192) 5.7 -> 6.1: not there.  128 x 128
-  // tiles gain nothing from it (4096 x 3072 -> 768 18.5 -> 18.6): LDS reads and the matrix cores bound them.
-  if constexpr (BM == 64 && BN == 64 && NSTAGE == 4) {
-    if (static_cast<int64_t>(num_m) * num_n <= 256)
+  // 4000 6.7 -> 5.9.  Its start and its end issue four more steps of loads, which costs 0.2 us however short K is.  Ring of 8 /
+  // ring of 4, time, over every result type, post-op and both epilogues (4000 sizes of 1 to 256 tiles), operands not in L2:
+  //   steps of 64        1 - 4          5 - 8          9 - 12         13 - 16        17 - 32        33 - 64        more
+  //   vector epilogue    0.99 - 1.13    0.92 - 1.09    0.85 - 1.08    0.82 - 1.05    0.72 - 0.91    0.65 - 0.86    0.60 - 0.85
+  //   element-wise       0.97 - 1.06    0.94 - 1.08    0.87 - 0.99    0.83 - 0.94    0.76 - 0.93    0.67 - 0.86    0.61 - 0.79
+  // and 1.02 - 1.08 with all operands in L2 up to 16 steps (to 32 with fewer than 64 tiles), which a weight seldom is.
+  // A convolution has its window arithmetic in front of those loads: 1.10 - 1.19 up to 12 steps, 0.9 - 1.1 beyond, not there.
+  // With two tiles per CU (192 x 512 -> 8192) 5.7 -> 6.1: not there.  128 x 128 tiles gain nothing from it (4096 x 3072 -> 768
+  // 18.5 -> 18.6): LDS reads and the matrix cores bound them.
+  if constexpr (BM == 64 && BN == 64 && NSTAGE == 4 && !CONV) {
+    if (KT > 12 && static_cast<int64_t>(num_m) * num_n <= 256)
       return launch_tile<BM, BN, WAVES_M, WAVES_N, OUT_T, ACT, KALIGNED, CONV, ELEMENTWISE, 8>(a, amask, bp, M, K, N, e, out, st, cv);
   }
   constexpr size_t lds_bytes = NSTAGE * (BM / 16 + BN / 16) * kChunkBytes + 12 * BN + (CONV ? kMaxConvPieces * 8 : 0);  // the most

@@ -23,6 +23,17 @@ def test_k_loops_around_the_ring(hip, dev, shape, K):
             np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path=path), ref)
 
 
+@pytest.mark.parametrize("K", [752, 768, 784, 832, 896, 960, 1040])
+def test_k_where_the_ring_of_64x64_tiles_changes(hip, dev, K):
+    """Four stages up to 12 steps of 64, eight beyond."""
+    hip.force_tile_shape(matmul=4)
+    for M, N, kw in [(70, 80, V2_DEQ), (129, 67, V2_DEQ), (193, 144, V2_REQ_S8)]:
+        layer, w, bias = make_layer(hip, dev, K, N, seed=K + N)
+        x, xq, mn, mx = make_acts(M, K, seed=M + K)
+        r = float(np.abs(x @ w + bias).max())
+        np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path="tile"), layer.oracle(xq, kw, mn, mx, -r, r))
+
+
 @pytest.mark.parametrize("M,K,N", [(1024, 512, 1024), (1025, 512, 1024),     # 256 and 272 tiles of 64 x 64
                                    (2048, 768, 1024), (2049, 768, 1024),     # 256 and 272 tiles of 128 x 64
                                    (2048, 752, 1024), (2048, 784, 1021)])    # K below the line; clamped loads, element-wise
