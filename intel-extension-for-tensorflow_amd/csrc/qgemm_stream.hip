@@ -467,9 +467,25 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
       default: STREAM(4, true, false, false, *cv);
     }
   } else if (sum) {
-    switch (s.chunks) {
-      HELD(false, true, none);
-      default: STREAM(2, false, false, true, none);
+    // Held, or groups of 1, 2 or 4 (4 with a residual spills up to 7 registers, which a long K covers).  Held chunks need the
+    // caches: past 256 MB of activations, residual and result, or past 96 MB where rows are no multiple of 64 bytes and pieces
+    // of lines have to meet in them, the groups' earlier loads win.  Time over that of groups of 1 (one chunk), 2 (two) or 4
+    // (more), 3000 sizes:
+    //   chunks 1 - 4   held: below the lines 0.8 - 1.1, between them with ragged rows 0.86 - 1.25 (1.02 in the middle), past
+    //                  both 1.05 - 1.39 (323916 x 112 -> 528 118 -> 169 us); groups of 2 there 0.82 - 1.08
+    //   chunks 5 - 9   groups of 2 0.82 - 1.09 (0.97 in the middle), past 256 MB 1.0 - 1.1
+    //   chunks 10 - 12 groups of 2 0.84 - 1.07 everywhere;  13 - 16  0.98 - 1.25 (368813 x 464 -> 176 113 -> 142 us)
+    const int64_t bytes = static_cast<int64_t>(M) * K + 2 * static_cast<int64_t>(M) * N;
+    const bool cached = bytes <= ((N % 64 == 0 || s.chunks > 4 ? 256 : 96) << 20);
+    if (s.chunks > 12 || (s.chunks > 4 && s.chunks <= 9 && !cached)) {
+      STREAM(4, false, false, true, none);
+    } else if (s.chunks == 1 && !cached) {
+      STREAM(1, false, false, true, none);
+    } else {
+      switch (cached ? s.chunks : 0) {
+        HELD(false, true, none);
+        default: STREAM(2, false, false, true, none);
+      }
     }
   } else {
     switch (s.chunks) {

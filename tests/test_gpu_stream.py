@@ -245,6 +245,32 @@ def test_residual_in_place_several_tiles_per_wavefront(hip, dev):
     assert torch.equal(both, want)
 
 
+@pytest.mark.parametrize("M,K,N", [(133003, 64, 1008), (400003, 16, 144), (139003, 32, 960), (123003, 240, 976), (139003, 272, 912), (1003, 304, 80), (1003, 400, 80)])
+def test_residual_forms(hip, dev, M, K, N):
+    """Past 96 or 256 MB of activations, residual and result, and a K past 384, a residual takes loads in groups instead of held
+    chunks."""
+    import torch
+    hip.force_tile_shape(matmul=ANY_SIZE)
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randint(0, 256, (M, K), dtype=torch.uint8, device=dev, generator=g)
+    add = torch.randint(-128, 128, (M, N), dtype=torch.int8, device=dev, generator=g)
+    w = torch.randint(-127, 128, (K, N), dtype=torch.int8, device=dev, generator=g)
+    packed = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev)
+    colsum = torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(w, False, K, N, packed, colsum)
+    ep = hip.Epilogue()
+    ep.n_scales, ep.n_eltwise = 1, 1
+    ep.elt[0].alg, ep.elt[0].alpha = hip.ELT_SUM, 0.375
+    scale, bias = torch.full((1,), 1e-3, device=dev), torch.full((N,), 20.0, device=dev)
+    v = (x.float() @ w.float()) * scale   # every sum below 2^24: exact in fp32 in any order
+    v = v + bias
+    want = (v + 0.375 * add.float()).clamp(-128, 127).round().to(torch.int8)
+    out = torch.empty((M, N), dtype=torch.int8, device=dev)
+    hip.qgemm_sum(x, hip.QUINT8, packed, colsum, M, K, N, scale, bias, ep, add, hip.QINT8, hip.QINT8, out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 def awkward_floats(n):
     """n fp32 values: ties around every 8-bit result with their neighbours, infinities, NaN, denormals, random bit patterns."""
     f = np.float32
