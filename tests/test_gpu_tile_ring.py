@@ -36,7 +36,8 @@ def test_k_where_the_ring_of_64x64_tiles_changes(hip, dev, K):
 
 @pytest.mark.parametrize("M,K,N", [(1024, 512, 1024), (1025, 512, 1024),     # 256 and 272 tiles of 64 x 64
                                    (2048, 768, 1024), (2049, 768, 1024),     # 256 and 272 tiles of 128 x 64
-                                   (2048, 752, 1024), (2048, 784, 1021)])    # K below the line; clamped loads, element-wise
+                                   (2048, 752, 1024), (2048, 784, 1021),     # K below the line; clamped loads, element-wise
+                                   (1920, 832, 544), (1840, 832, 544)])      # 15 tile rows of 128 against 30 or 29 of 64
 def test_where_the_shape_changes(hip, dev, M, K, N):
     layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
     _, xq, mn, mx = make_acts(M, K, seed=M + K)
