@@ -16,23 +16,17 @@
 // the start of a launch (3.7: input rows and weight on their way, together), then a wavefront's tile after another, MFMAs
 // (18 of 32 cycles with 64 channels) and epilogue in turn.  Fragments two chunks ahead left every pair of MFMAs waiting for LDS (0.25 of
 // 1.0 us per tile with 128 channels); row addresses in scalar arithmetic, a branch per piece, were 0.3 slower than the counters.
+#include "qconv_walk.hpp"
 #include "qgemm_pack.hpp"
 
 namespace itexhip {
 namespace {
 
-constexpr int kLdsPerCu = 160 * 1024;
 constexpr int kForceDirect = 17;  // of itexhip_test_force_tile_shape
 
-struct DirectArgs {
-  int M, N;
-  int in_h, in_w, out_h, out_w;
-  int pad_top, pad_left;
-  int wp, vr;         // input columns, and rows of one image, that windows touch, padding included
-  FastDiv by_out_w, by_out_h, by_row_pieces, by_vr;
-  int step_p, step_h, step_image;  // 256 pieces of 16 bytes on: pieces of a row, rows of an image, images
+struct DirectArgs : DirectGeometry<FastDiv> {
+  int N;
   int waves_n;        // wavefronts side by side along the channels: 1, 2 or 4
-  int tiles, per_wg;  // row tiles of 32; of a workgroup
   int wgs;            // workgroups with tiles
   int panel;          // offset of the channel parameters in LDS
   float lo, hi;       // post-op bounds, see POST
@@ -63,50 +57,26 @@ __global__ __launch_bounds__(256, C32 == 1 ? 4 : C32 == 2 ? 3 : 2) void qconv_di
   if (wg >= s.wgs) return;
   const int t0 = wg * s.per_wg, t1 = min(t0 + s.per_wg, s.tiles);
 
-  // row of the padded images (all of them one below the other) in which the windows of output row g begin
-  auto window_row = [&](int g) {
-    const int b = fast_div(g, s.by_out_h);
-    return b * s.vr + (g - b * s.out_h);
-  };
-  const int v0 = window_row(fast_div(t0 * 32, s.by_out_w));
-  const int v1 = window_row(fast_div(min(t1 * 32, s.M) - 1, s.by_out_w)) + 3;
+  const int v0 = s.first_row(t0), v1 = s.last_row(t1);
   // ---- the channel parameters, the input rows and the weight travel together
   const int channel = n_base + min(static_cast<int>(threadIdx.x), channels - 1);
   const int colsum = s.colsum ? s.colsum[channel] : 0;
   const float scale = s.n_scales > 0 ? s.scales[s.n_scales > 1 ? channel : 0] : 1.0f;
   const float bias = s.bias[channel];
 
-  const int row_pieces = s.wp * PIECES, pieces = (v1 - v0) * row_pieces, row_bytes = s.wp * PITCH;
-  // where the thread's next piece lies: row of an image (-pad_top the first), image, piece of that row
-  int ih, image, p;
-  {
-    const int r = fast_div(static_cast<int>(threadIdx.x), s.by_row_pieces);
-    p = static_cast<int>(threadIdx.x) - r * row_pieces;
-    image = fast_div(v0 + r, s.by_vr);
-    ih = v0 + r - image * s.vr;
-  }
-  auto fetch = [&](int i) -> v4i {
-    const int h = ih - s.pad_top, q = p - s.pad_left * PIECES;
-    const bool inside = i < pieces && static_cast<unsigned>(h) < static_cast<unsigned>(s.in_h) &&  // (behind the last piece: no image)
-                        static_cast<unsigned>(q) < static_cast<unsigned>(s.in_w * PIECES);
-    // (input bytes < 2^31 checked by the host; what is outside reads 16 zero bytes)
-    const uint8_t* src = a + ((image * s.in_h + h) * (s.in_w * PIECES) + q) * 16u;
+  const int pieces = (v1 - v0) * s.wp * PIECES, row_bytes = s.wp * PITCH;
+  InputWalk<PIECES, FastDiv> walk(s, v0, static_cast<int>(threadIdx.x));
+  auto fetch = [&](int i) -> v4i {  // what is outside reads 16 zero bytes
+    uint32_t offset;
+    const bool inside = walk.inside(s, &offset) & (i < pieces);
+    const uint8_t* src = a + offset;  // (before the choice: a branch per piece otherwise)
     src = inside ? src : reinterpret_cast<const uint8_t*>(kZeros);
-    // 256 pieces on
-    p += s.step_p;
-    ih += s.step_h;
-    image += s.step_image;
-    const bool next_row = p >= row_pieces;
-    p -= next_row ? row_pieces : 0;
-    ih += next_row ? 1 : 0;
-    const bool next_image = ih >= s.vr;
-    ih -= next_image ? s.vr : 0;
-    image += next_image ? 1 : 0;
+    walk.advance(s);
     return *reinterpret_cast<const v4i*>(src);
   };
   auto put = [&](int i, v4i x) {
     x.x ^= amask; x.y ^= amask; x.z ^= amask; x.w ^= amask;
-    if (i < pieces) *reinterpret_cast<v4i*>(lds + (i + i / PIECES) * 16) = x;
+    if (i < pieces) *reinterpret_cast<v4i*>(lds + piece_at<PIECES>(i)) = x;
   };
   const int t = threadIdx.x;
   v4i x[BATCH];
@@ -141,9 +111,7 @@ __global__ __launch_bounds__(256, C32 == 1 ? 4 : C32 == 2 ? 3 : 2) void qconv_di
   if (t0 + wm >= t1) return;  // whole wavefront; no barrier follows
   const int channel_off = half * 16;
   auto origin_of = [&](int tile) -> const uint8_t* {  // of the window of the lane's output position
-    const int m = min(tile * 32 + lrow, s.M - 1);
-    const int g = fast_div(m, s.by_out_w);
-    return lds + (window_row(g) - v0) * row_bytes + (m - g * s.out_w) * PITCH + channel_off;
+    return lds + s.window_at(min(tile * 32 + lrow, s.M - 1), v0, row_bytes, PITCH) + channel_off;
   };
   auto fragment = [&](const uint8_t* origin, auto c) -> v4i {
     constexpr int k = decltype(c)::value / C32, kh = k / 3, kw = k % 3;
@@ -230,60 +198,34 @@ int try_direct(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   const int act = canon_chain(e, &c);
   if (act < 0 || act > 2 || (c.flags & ~(kChainMax0 | kChainClip)) != 0) return 0;
   if ((c.flags & kChainClip) && !(c.lo <= c.hi)) return 0;  // the median of three is no clip then
-  DirectArgs s{};
-  s.M = M; s.N = N;
-  s.in_h = cv.in_h; s.in_w = cv.in_w; s.out_h = cv.out_h; s.out_w = cv.out_w;
-  s.pad_top = cv.pad_top; s.pad_left = cv.pad_left;
   const int64_t wp = cv.out_w + 2LL, vr = cv.out_h + 2LL;
-  const int pitch = cv.in_c + 16;  // as the kernel's PITCH
-  if (wp * pitch * 3 > kLdsPerCu || M / cv.out_w / cv.out_h * vr >= (1LL << 31)) return 0;
-  s.wp = static_cast<int>(wp); s.vr = static_cast<int>(vr);
-  s.by_out_w = cv.by_out_w; s.by_out_h = cv.by_out_h;
-  const int row_pieces = s.wp * (cv.in_c / 16), step = 256 / row_pieces;
-  s.by_row_pieces = make_fast_div(row_pieces);
-  s.step_p = 256 % row_pieces; s.step_image = step / s.vr; s.step_h = step % s.vr;
-  s.colsum = e.colsum; s.scales = e.scales; s.bias = static_cast<const float*>(e.bias);
-  s.comp_mul = e.comp_mul; s.n_scales = e.n_scales;
-  s.by_vr = make_fast_div(vr);
-  const int blocks = N / 32;
-  s.waves_n = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1;
-  const int waves_m = 4 / s.waves_n, groups_n = blocks / s.waves_n;
-  const int panel = 12 * 32 * s.waves_n;  // bytes of the channel parameters
-  if (groups_n > 65535) return 0;  // gridDim.y
-  s.tiles = static_cast<int>((static_cast<int64_t>(M) + 31) / 32);
-  // The tiles of a workgroup: the smallest estimate, us, fitted to 20 shapes (56 x 56 x 64 to 112 x 112 x 32, 1 to 64 images,
-  // 64 to 512 results; 1 to 20 tiles per workgroup, measured against one another: 1 % above the best on average, 10 % at most).
-  // A wavefront takes 0.18 + 0.2 per 32 channels for a tile, a CU with one workgroup 1.28 times that, since nothing runs
-  // under its waits, and every set of workgroups that a CU holds at once 3.7 for its start.
-  constexpr int kMaxTiles = 24;
-  const int c32 = cv.in_c / 32, resident = c32 == 1 ? 4 : c32 == 2 ? 3 : 2;  // what the registers allow
-  int64_t lds = 0;
-  double best = 1e30;
-  for (int per = 1; per <= kMaxTiles; ++per) {
-    // 32 * per output positions lie in at most `rows` output rows, which cross `images` borders (two more input rows each)
-    const int64_t rows = (32 * per + cv.out_w - 2) / cv.out_w + 1, images = (rows + cv.out_h - 2) / cv.out_h;
-    const int64_t bytes = (rows + 2 + 2 * images) * wp * pitch + panel;
-    if (bytes > kLdsPerCu) break;
-    const int64_t n = ((s.tiles + per - 1) / per * static_cast<int64_t>(groups_n) + 255) / 256;  // workgroups of the busiest CU
-    const int at_once = std::min<int>(resident, kLdsPerCu / static_cast<int>(bytes));
-    const double us = static_cast<double>(n) * ((per + waves_m - 1) / waves_m) * (0.18 + 0.2 * c32) * (n == 1 || at_once == 1 ? 1.28 : 1.0) +
-                      3.7 * static_cast<double>((n + at_once - 1) / at_once);
-    if (us < best) { best = us; s.per_wg = per; lds = bytes; }
-  }
-  if (s.per_wg == 0) return 0;  // rows too wide for LDS
+  if (wp * direct_pitch(cv.in_c) * 3 > kLdsPerCu || M / cv.out_w / cv.out_h * vr >= (1LL << 31)) return 0;
+  const DirectPlan plan = plan_direct(M, cv.in_c, N, cv.out_h, cv.out_w);
+  if (plan.per_wg == 0 || plan.groups_n > 65535) return 0;  // rows too wide for LDS; gridDim.y
   // Where it is the faster kernel: 0.45 to 0.92 of the other kernels' time over 105 shapes (5 x 5 to 244 x 244, 1 to 64 images, 32 to
   // 512 results), but for rows of which a run needs several times its own (300 x 300 x 64, 9.4 positions put into LDS per
   // result: 10.9 -> 13.6 us; 3 x 231 x 231 x 96, 6.2: 22.4 -> 24.4; 10 x 84 x 300 x 32, 4.1: 22.4 -> 23.2; 7 x 218 x 218 x 64, 2.9: 32.7
   // -> 25.4) and, where the device is full, many single blocks of channels that each put the input there (4 x 81 x 81 x 128 ->
   // 160: 18.5 -> 20.4; 22 x 21 x 21 8.9 -> 8.7; 4 x 62 x 6 7.8 -> 4.7).
-  const int64_t staged = (lds - panel) / pitch, positions = 32LL * std::min(s.per_wg, s.tiles);
+  const int c32 = cv.in_c / 32;
+  const int64_t tiles = (static_cast<int64_t>(M) + 31) / 32;
+  const int64_t staged = plan.panel / direct_pitch(cv.in_c), positions = 32 * std::min<int64_t>(plan.per_wg, tiles);
   const bool halo = cv.out_w > 180 && staged > 4 * positions;
-  const bool repeated = s.waves_n == 1 && groups_n >= 5 && c32 == 4 && static_cast<int64_t>(s.tiles) * groups_n > 1024;
+  const bool repeated = plan.waves_n == 1 && plan.groups_n >= 5 && c32 == 4 && tiles * plan.groups_n > 1024;
   if (forced != kForceDirect && (halo || repeated)) return 0;
-  s.wgs = (s.tiles + s.per_wg - 1) / s.per_wg;
-  s.panel = static_cast<int>(lds) - panel;
+  DirectArgs s{};
+  s.M = M; s.N = N;
+  s.in_h = cv.in_h; s.in_w = cv.in_w; s.out_h = cv.out_h; s.out_w = cv.out_w;
+  s.pad_top = cv.pad_top; s.pad_left = cv.pad_left;
+  s.by_out_w = cv.by_out_w; s.by_out_h = cv.by_out_h;
+  set_walk(s, cv.in_c / 16, make_fast_div);
+  s.tiles = static_cast<int>((static_cast<int64_t>(M) + 31) / 32);
+  s.per_wg = plan.per_wg; s.wgs = plan.wgs; s.waves_n = plan.waves_n; s.panel = plan.panel;
+  s.colsum = e.colsum; s.scales = e.scales; s.bias = static_cast<const float*>(e.bias);
+  s.comp_mul = e.comp_mul; s.n_scales = e.n_scales;
   s.lo = c.lo; s.hi = c.hi;
-  const dim3 grid(static_cast<unsigned>((s.wgs + 7) / 8 * 8), static_cast<unsigned>(groups_n));
+  const int64_t lds = plan.lds;
+  const dim3 grid(static_cast<unsigned>((s.wgs + 7) / 8 * 8), static_cast<unsigned>(plan.groups_n));
   const int post = c.flags & kChainClip ? kPostClip : c.flags & kChainMax0 ? kPostRelu : kPostNone;
   uint8_t* o = static_cast<uint8_t*>(out);
   int rc;

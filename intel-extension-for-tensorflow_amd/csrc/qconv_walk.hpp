@@ -1,0 +1,144 @@
+// Where the 3 x 3 convolution kernel (qconv_direct.hip) puts input rows into LDS and reads them, how many row tiles a workgroup
+// takes.  Plain C++: the CPU test of all of it includes this file.  D is the division by a number
+// fixed per launch, fast_div(n, D).
+#ifndef ITEXHIP_QCONV_WALK_HPP_
+#define ITEXHIP_QCONV_WALK_HPP_
+
+#include <stdint.h>
+
+#include <algorithm>
+
+#ifndef ITEXHIP_HD
+#ifdef __HIP__
+#define ITEXHIP_HD __host__ __device__ inline
+#else
+#define ITEXHIP_HD inline
+#endif
+#endif
+
+namespace itexhip {
+
+constexpr int kLdsPerCu = 160 * 1024;
+constexpr int kDirectThreads = 256;
+constexpr int kDirectMaxTiles = 24;  // of a workgroup
+
+// The output positions stand one after the other, rows of one image after those of the image before it; so do the padded
+// images.  A tile is 32 positions.
+template <class D>
+struct DirectGeometry {
+  int M;
+  int in_h, in_w, out_h, out_w;
+  int pad_top, pad_left;
+  int wp, vr;         // input columns, and rows of one image, that windows touch, padding included
+  D by_out_w, by_out_h, by_row_pieces, by_vr;
+  int step_p, step_h, step_image;  // kDirectThreads pieces of 16 bytes on: pieces of a row, rows of an image, images
+  int tiles, per_wg;  // row tiles of 32; of a workgroup
+
+  // row of the padded images in which the windows of output row g begin
+  ITEXHIP_HD int window_row(int g) const {
+    const int b = fast_div(g, by_out_h);
+    return b * vr + (g - b * out_h);
+  }
+  // rows of the padded images that tiles t0 .. t1 - 1 touch: [first, last)
+  ITEXHIP_HD int first_row(int t0) const { return window_row(fast_div(t0 * 32, by_out_w)); }
+  ITEXHIP_HD int last_row(int t1) const { return window_row(fast_div((t1 * 32 < M ? t1 * 32 : M) - 1, by_out_w)) + 3; }
+  // byte in LDS at which the window of position m begins, v0 being the first row there; bytes of a row and of a pixel
+  ITEXHIP_HD int window_at(int m, int v0, int row_bytes, int pitch) const {
+    const int g = fast_div(m, by_out_w);
+    return (window_row(g) - v0) * row_bytes + (m - g * out_w) * pitch;
+  }
+};
+
+// the members that follow from out_h and out_w; `pieces` of 16 bytes per pixel
+template <class D, class MakeDiv>
+void set_walk(DirectGeometry<D>& s, int pieces, MakeDiv make_div) {
+  s.wp = s.out_w + 2;
+  s.vr = s.out_h + 2;
+  const int row_pieces = s.wp * pieces, step = kDirectThreads / row_pieces;
+  s.by_row_pieces = make_div(row_pieces);
+  s.by_vr = make_div(s.vr);
+  s.step_p = kDirectThreads % row_pieces;
+  s.step_image = step / s.vr;
+  s.step_h = step % s.vr;
+}
+
+// A thread's way through the 16-byte pieces of the padded rows from v0 on, kDirectThreads at a time; PIECES per pixel.  The
+// divisions are paid once, then counters carry over rows and images.
+template <int PIECES, class D>
+struct InputWalk {
+  int ih, image, p;  // row of an image (pad_top of them above it), image, piece of that row
+  ITEXHIP_HD InputWalk(const DirectGeometry<D>& s, int v0, int thread) {
+    const int r = fast_div(thread, s.by_row_pieces);
+    p = thread - r * (s.wp * PIECES);
+    image = fast_div(v0 + r, s.by_vr);
+    ih = v0 + r - image * s.vr;
+  }
+  // Whether the piece lies in the input and not in its padding, and its byte offset then (input bytes < 2^31).  (The caller looks
+  // whether there is a piece: behind the last one there may be no image either.)
+  ITEXHIP_HD bool inside(const DirectGeometry<D>& s, uint32_t* offset) const {
+    const int h = ih - s.pad_top, q = p - s.pad_left * PIECES;
+    *offset = static_cast<uint32_t>((image * s.in_h + h) * (s.in_w * PIECES) + q) * 16u;
+    return (static_cast<unsigned>(h) < static_cast<unsigned>(s.in_h)) &  // (no branch)
+           (static_cast<unsigned>(q) < static_cast<unsigned>(s.in_w * PIECES));
+  }
+  ITEXHIP_HD void advance(const DirectGeometry<D>& s) {
+    p += s.step_p;
+    ih += s.step_h;
+    image += s.step_image;
+    const bool next_row = p >= s.wp * PIECES;
+    p -= next_row ? s.wp * PIECES : 0;
+    ih += next_row ? 1 : 0;
+    const bool next_image = ih >= s.vr;
+    ih -= next_image ? s.vr : 0;
+    image += next_image ? 1 : 0;
+  }
+};
+
+// byte of piece i in LDS: pixels lie an odd number of pieces apart, so that the reads of 16 neighbours fall into different banks
+template <int PIECES>
+ITEXHIP_HD int piece_at(int i) { return (i + i / PIECES) * 16; }
+constexpr int direct_pitch(int in_c) { return in_c + 16; }  // of a pixel in LDS
+
+struct DirectPlan {
+  int waves_n;   // wavefronts side by side along the channels: 1, 2 or 4
+  int groups_n;  // workgroups along them
+  int per_wg;    // tiles of a workgroup; 0: rows too wide for LDS
+  int wgs;       // workgroups along the positions
+  int panel;     // offset in LDS of the channel parameters
+  int lds;       // bytes of LDS of a workgroup
+};
+
+// M > 0, M * N < 2^31, three padded rows fit LDS
+inline DirectPlan plan_direct(int M, int in_c, int N, int out_h, int out_w) {
+  DirectPlan s{};
+  const int blocks = N / 32, c32 = in_c / 32, wp = out_w + 2, pitch = direct_pitch(in_c);
+  s.waves_n = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1;
+  s.groups_n = blocks / s.waves_n;
+  const int waves_m = 4 / s.waves_n, panel = 12 * 32 * s.waves_n;  // bytes of the channel parameters
+  const int tiles = static_cast<int>((static_cast<int64_t>(M) + 31) / 32), resident = c32 == 1 ? 4 : c32 == 2 ? 3 : 2;  // (registers)
+  // The tiles of a workgroup: the smallest estimate, us, fitted to 20 shapes (56 x 56 x 64 to 112 x 112 x 32, 1 to 64 images,
+  // 64 to 512 results; 1 to 20 tiles per workgroup, measured against one another: 1 % above the best on average, 10 % at most).
+  // A wavefront takes 0.18 + 0.2 per 32 channels for a tile, a CU with one workgroup 1.28 times that, since nothing runs
+  // under its waits, and every set of workgroups that a CU holds at once 3.7 for its start.
+  double best = 1e30;
+  for (int per = 1; per <= kDirectMaxTiles; ++per) {
+    // 32 * per output positions lie in at most `rows` output rows, which cross `images` borders (two more input rows each)
+    const int64_t rows = (32 * per + out_w - 2) / out_w + 1, images = (rows + out_h - 2) / out_h;
+    const int64_t bytes = (rows + 2 + 2 * images) * wp * pitch + panel;
+    if (bytes > kLdsPerCu) break;
+    const int wgs = (tiles + per - 1) / per;
+    const int64_t n = (wgs * static_cast<int64_t>(s.groups_n) + 255) / 256;  // workgroups of the busiest CU
+    const int at_once = std::min(resident, kLdsPerCu / static_cast<int>(bytes));
+    const double us = static_cast<double>(n) * ((per + waves_m - 1) / waves_m) * (0.18 + 0.2 * c32) * (n == 1 || at_once == 1 ? 1.28 : 1.0) +
+                      3.7 * static_cast<double>((n + at_once - 1) / at_once);
+    if (us < best) {
+      best = us;
+      s.per_wg = per; s.lds = static_cast<int>(bytes); s.wgs = wgs;
+    }
+  }
+  s.panel = s.lds - panel;
+  return s;
+}
+
+}  // namespace itexhip
+#endif  // ITEXHIP_QCONV_WALK_HPP_

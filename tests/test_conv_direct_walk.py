@@ -1,0 +1,116 @@
+"""The addresses of the 3 x 3 convolution kernel that keeps its input rows in LDS (csrc/qconv_walk.hpp), compiled for the host:
+every load of every thread lies in the input or is taken for padding, what it puts into LDS lies before the channel parameters,
+and every fragment read finds the pixel that its window position has."""
+import os
+import subprocess
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "intel-extension-for-tensorflow_amd", "csrc")
+
+PROGRAM = r"""
+#include <cstdio>
+#include <random>
+#include <vector>
+namespace itexhip {
+@FAST_DIV@
+}
+#include "qconv_walk.hpp"
+using namespace itexhip;
+
+long workgroups = 0, bad = 0;
+void fail(const char* what, int c, int b, int h, int w, int oh, int ow, int n, long at) {
+  if (++bad < 10) std::printf("%s: C %d B %d in %d x %d out %d x %d N %d at %ld\n", what, c, b, h, w, oh, ow, n, at);
+}
+
+template <int PIECES>
+void check(int B, int H, int W, int oh, int ow, int pt, int pl, int N) {
+  const int C = PIECES * 16, pitch = direct_pitch(C), M = B * oh * ow;
+  if ((ow + 2LL) * pitch * 3 > kLdsPerCu) return;
+  const DirectPlan plan = plan_direct(M, C, N, oh, ow);
+  if (plan.per_wg == 0) return;
+  DirectGeometry<FastDiv> s{};
+  s.M = M; s.in_h = H; s.in_w = W; s.out_h = oh; s.out_w = ow; s.pad_top = pt; s.pad_left = pl;
+  s.by_out_w = make_fast_div(ow); s.by_out_h = make_fast_div(oh);
+  set_walk(s, PIECES, make_fast_div);
+  s.tiles = (M + 31) / 32;
+  s.per_wg = plan.per_wg;
+  const long bytes = 1L * B * H * W * C;
+  auto pixel = [&](int b, int h, int w) -> long {  // byte of the pixel, -1: padding
+    return h < 0 || h >= H || w < 0 || w >= W ? -1 : ((1L * b * H + h) * W + w) * C;
+  };
+  auto wrong = [&](const char* what, long at) { fail(what, C, B, H, W, oh, ow, N, at); };
+  if (1L * plan.wgs * plan.per_wg < s.tiles || 1L * (plan.wgs - 1) * plan.per_wg >= s.tiles) wrong("workgroups", plan.wgs);
+  if (plan.panel < 0 || plan.panel % 16 != 0 || plan.lds > kLdsPerCu) wrong("LDS", plan.lds);
+  std::vector<long> lds(plan.panel / 16);
+  const int stride = plan.wgs <= 6 ? 1 : plan.wgs / 5;
+  for (int wg = 0; wg < plan.wgs; wg = wg + stride < plan.wgs || wg == plan.wgs - 1 ? wg + stride : plan.wgs - 1) {
+    ++workgroups;
+    const int t0 = wg * s.per_wg, t1 = std::min(t0 + s.per_wg, s.tiles), v0 = s.first_row(t0), v1 = s.last_row(t1);
+    const int row_pieces = s.wp * PIECES, pieces = (v1 - v0) * row_pieces;
+    lds.assign(lds.size(), -2);
+    for (int t = 0; t < kDirectThreads; ++t) {
+      InputWalk<PIECES, FastDiv> walk(s, v0, t);
+      for (int i0 = 0; i0 == 0 || i0 < pieces; i0 += 8 * kDirectThreads)
+        for (int u = 0; u < 8; ++u, walk.advance(s)) {
+          const int i = i0 + t + u * kDirectThreads;
+          long at = -1;
+          uint32_t offset;
+          if (walk.inside(s, &offset) && i < pieces) at = offset;
+          if (at + 16 > bytes) wrong("read", at);
+          if (i >= pieces) continue;
+          const int v = v0 + i / row_pieces, p = i % row_pieces;
+          const long px = pixel(v / s.vr, v % s.vr - pt, p / PIECES - pl);
+          if (at != (px < 0 ? -1 : px + p % PIECES * 16)) wrong("piece", i);
+          const int slot = piece_at<PIECES>(i) / 16;
+          if (slot >= static_cast<int>(lds.size())) wrong("store", slot);
+          else lds[slot] = at;
+        }
+    }
+    for (int tile = t0; tile < t1; ++tile)
+      for (int l = 0; l < 32; ++l) {
+        const int m = std::min(tile * 32 + l, M - 1), at = s.window_at(m, v0, s.wp * pitch, pitch);
+        for (int k = 0; k < 9; ++k)
+          for (int c = 0; c < PIECES; ++c) {
+            const int slot = at / 16 + (k / 3 * s.wp * pitch + k % 3 * pitch) / 16 + c;
+            const long px = pixel(m / ow / oh, m / ow % oh - pt + k / 3, m % ow - pl + k % 3);
+            if (slot < 0 || slot >= static_cast<int>(lds.size())) wrong("fragment", slot);
+            else if (lds[slot] != (px < 0 ? -1 : px + c * 16)) wrong("fragment's pixel", m);
+          }
+      }
+  }
+}
+
+int main() {
+  std::mt19937 g(1);
+  auto below = [&](int n) { return static_cast<int>(g() % n); };
+  auto size = [&](int most) { const int r = 1 << below(9); return 1 + below(std::min(r, most)); };
+  for (int i = 0; i < 6000; ++i) {
+    const int H = size(256), W = size(256), pt = below(3), pl = below(3);
+    const int oh = std::max(1, H + pt - 2 + below(4)), ow = std::max(1, W + pl - 2 + below(4));
+    int B = 1 + below(40);
+    while (B > 1 && 1L * B * oh * ow > 60000) B /= 2;
+    const int N = 32 * (1 + below(12));
+    switch (i % 4) {
+      case 0: check<2>(B, H, W, oh, ow, pt, pl, N); break;
+      case 1: check<4>(B, H, W, oh, ow, pt, pl, N); break;
+      case 2: check<6>(B, H, W, oh, ow, pt, pl, N); break;
+      default: check<8>(B, H, W, oh, ow, pt, pl, N);
+    }
+  }
+  std::printf("%ld workgroups, %ld wrong\n", workgroups, bad);
+  return bad != 0 || workgroups < 10000;
+}
+"""
+
+
+def fast_div_source():
+    src = open(os.path.join(CSRC, "qgemm_common.hpp")).read()
+    end = src.index("}\n", src.index("__device__ __forceinline__ int fast_div")) + 2
+    return src[src.index("struct FastDiv"):end].replace("__device__ __forceinline__", "inline")
+
+
+def test_every_address(tmp_path):
+    src, exe = tmp_path / "walk.cc", tmp_path / "walk"
+    src.write_text(PROGRAM.replace("@FAST_DIV@", fast_div_source()))
+    subprocess.run(["g++", "-std=c++17", "-O2", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    done = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
+    assert done.returncode == 0, done.stdout
