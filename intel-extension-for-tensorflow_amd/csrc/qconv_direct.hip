@@ -202,17 +202,11 @@ int try_direct(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   if (wp * direct_pitch(cv.in_c) * 3 > kLdsPerCu || M / cv.out_w / cv.out_h * vr >= (1LL << 31)) return 0;
   const DirectPlan plan = plan_direct(M, cv.in_c, N, cv.out_h, cv.out_w);
   if (plan.per_wg == 0 || plan.groups_n > 65535) return 0;  // rows too wide for LDS; gridDim.y
-  // Where it is the faster kernel: 0.45 to 0.92 of the other kernels' time over 105 shapes (5 x 5 to 244 x 244, 1 to 64 images, 32 to
-  // 512 results), but for rows of which a run needs several times its own (300 x 300 x 64, 9.4 positions put into LDS per
-  // result: 10.9 -> 13.6 us; 3 x 231 x 231 x 96, 6.2: 22.4 -> 24.4; 10 x 84 x 300 x 32, 4.1: 22.4 -> 23.2; 7 x 218 x 218 x 64, 2.9: 32.7
-  // -> 25.4) and, where the device is full, many single blocks of channels that each put the input there (4 x 81 x 81 x 128 ->
-  // 160: 18.5 -> 20.4; 22 x 21 x 21 8.9 -> 8.7; 4 x 62 x 6 7.8 -> 4.7).
-  const int c32 = cv.in_c / 32;
-  const int64_t tiles = (static_cast<int64_t>(M) + 31) / 32;
-  const int64_t staged = plan.panel / direct_pitch(cv.in_c), positions = 32 * std::min<int64_t>(plan.per_wg, tiles);
-  const bool halo = cv.out_w > 180 && staged > 4 * positions;
-  const bool repeated = plan.waves_n == 1 && plan.groups_n >= 5 && c32 == 4 && tiles * plan.groups_n > 1024;
-  if (forced != kForceDirect && (halo || repeated)) return 0;
+  // Where it is the faster kernel.  What it loses to is the input it puts into LDS: rows of which a run needs several times its own
+  // (11 x 253 x 253 x 32 -> 96 53 us, 75 here), and channels in many groups of which each puts the input there again (4 x 89 x 89 x
+  // 96 -> 384 20.0, 29.8 here).  Both estimates follow it: over 3500 drawn shapes of 4 x 4 to 300 x 300 with 32 to 512 results
+  // 0.745 of the other kernels' time in the mean, 12 of them more than 5 % longer, 1.16 at most.
+  if (forced != kForceDirect && plan.us >= others_us(M, K, N, cv.pad_top > 0 || cv.pad_left > 0)) return 0;
   DirectArgs s{};
   s.M = M; s.N = N;
   s.in_h = cv.in_h; s.in_w = cv.in_w; s.out_h = cv.out_h; s.out_w = cv.out_w;

@@ -1,5 +1,5 @@
 // Where the 3 x 3 convolution kernel (qconv_direct.hip) puts input rows into LDS and reads them, how many row tiles a workgroup
-// takes.  Plain C++: the CPU test of all of it includes this file.  D is the division by a number
+// takes, and which convolutions are its.  Plain C++: the CPU test of all of it includes this file.  D is the division by a number
 // fixed per launch, fast_div(n, D).
 #ifndef ITEXHIP_QCONV_WALK_HPP_
 #define ITEXHIP_QCONV_WALK_HPP_
@@ -106,6 +106,7 @@ struct DirectPlan {
   int wgs;       // workgroups along the positions
   int panel;     // offset in LDS of the channel parameters
   int lds;       // bytes of LDS of a workgroup
+  double us;     // estimate of the launch
 };
 
 // M > 0, M * N < 2^31, three padded rows fit LDS
@@ -117,27 +118,81 @@ inline DirectPlan plan_direct(int M, int in_c, int N, int out_h, int out_w) {
   const int waves_m = 4 / s.waves_n, panel = 12 * 32 * s.waves_n;  // bytes of the channel parameters
   const int tiles = static_cast<int>((static_cast<int64_t>(M) + 31) / 32), resident = c32 == 1 ? 4 : c32 == 2 ? 3 : 2;  // (registers)
   // The tiles of a workgroup: the smallest estimate, us, fitted to 20 shapes (56 x 56 x 64 to 112 x 112 x 32, 1 to 64 images,
-  // 64 to 512 results; 1 to 20 tiles per workgroup, measured against one another: 1 % above the best on average, 10 % at most).
-  // A wavefront takes 0.18 + 0.2 per 32 channels for a tile, a CU with one workgroup 1.28 times that, since nothing runs
-  // under its waits, and every set of workgroups that a CU holds at once 3.7 for its start.
+  // 64 to 512 results).  A wavefront takes 0.18 + 0.2 per 32 channels for a tile, a CU with one workgroup 1.28 times that, since
+  // nothing runs under its waits, and every set of workgroups that a CU holds at once 3.7 for its start.  Workgroups are counted
+  // on the busiest XCD: 35 x 7 of them are fewer than 256, but five of the 35 go to one XCD, 35 workgroups to its 32 CUs
+  // (4 x 62 x 62 x 128 -> 224: 19.2 us, 12.0 with a shorter run).  Over 2200 shapes of 4 x 4 to 300 x 300 with 13 lengths each the
+  // choice is 0.9 % above the best in the mean, 11 % for one in a hundred, 24 % at most.
   double best = 1e30;
   for (int per = 1; per <= kDirectMaxTiles; ++per) {
-    // 32 * per output positions lie in at most `rows` output rows, which cross `images` borders (two more input rows each)
+    // 32 * per positions lie in at most `rows` output rows, which cross `images` borders (two more input rows each)
     const int64_t rows = (32 * per + out_w - 2) / out_w + 1, images = (rows + out_h - 2) / out_h;
-    const int64_t bytes = (rows + 2 + 2 * images) * wp * pitch + panel;
+    const int64_t staged = (rows + 2 + 2 * images) * wp;  // pixels put into LDS
+    const int64_t bytes = staged * pitch + panel;
     if (bytes > kLdsPerCu) break;
     const int wgs = (tiles + per - 1) / per;
-    const int64_t n = (wgs * static_cast<int64_t>(s.groups_n) + 255) / 256;  // workgroups of the busiest CU
+    const int64_t n = (static_cast<int64_t>((wgs + 7) / 8) * s.groups_n + 31) / 32;  // workgroups of the busiest CU
     const int at_once = std::min(resident, kLdsPerCu / static_cast<int>(bytes));
-    const double us = static_cast<double>(n) * ((per + waves_m - 1) / waves_m) * (0.18 + 0.2 * c32) * (n == 1 || at_once == 1 ? 1.28 : 1.0) +
-                      3.7 * static_cast<double>((n + at_once - 1) / at_once);
+    const int turns = (per + waves_m - 1) / waves_m;  // tiles of a wavefront
+    const double sets = static_cast<double>((n + at_once - 1) / at_once);
+    const double us = static_cast<double>(n) * turns * (0.18 + 0.2 * c32) * (n == 1 || at_once == 1 ? 1.28 : 1.0) + 3.7 * sets;
     if (us < best) {
       best = us;
       s.per_wg = per; s.lds = static_cast<int>(bytes); s.wgs = wgs;
+      // The launch as a whole, for others_us to be compared with: 2.0, and per set its start, 0.99 for every eight loads per
+      // thread that put rows into LDS, and the tiles, 0.86 of whose time adds up for workgroups that share a CU.  Within 10 %
+      // (one standard deviation) of 25900 times.
+      const double pieces = static_cast<double>(staged * (in_c / 16));
+      s.us = 2.0 + sets * (1.06 + 0.99 / (8 * kDirectThreads) * pieces + std::min(turns, (tiles + waves_m - 1) / waves_m) * (0.2 + 0.22 * c32) *
+                                      (1.0 + 0.86 * (static_cast<double>(std::min<int64_t>(n, at_once)) - 1.0)));
     }
   }
   s.panel = s.lds - panel;
   return s;
+}
+
+// ---- the other kernels for a convolution: [M, K] patches, N results
+
+// Tile shape of the implicit GEMM: the one with the smallest estimated time, rounds of workgroups over the 256 CUs x tile area x
+// a penalty for the operand traffic per MFMA of smaller tiles.
+inline int pick_conv_tile(int64_t M, int64_t N) {
+  struct Shape { int bm, bn; double penalty; };
+  static constexpr Shape shapes[3] = {{256, 128, 1.08}, {128, 128, 1.2}, {64, 64, 1.8}};
+  int best = 0;
+  double best_cost = 1e300;
+  for (int i = 0; i < 3; ++i) {
+    const int64_t tiles = ((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
+    const double cost = static_cast<double>((tiles + 255) / 256) * shapes[i].bm * shapes[i].bn * shapes[i].penalty;
+    if (cost < best_cost) { best_cost = cost; best = i; }
+  }
+  return best;
+}
+
+// Whether a convolution goes to the kernel for a short K (qgemm_stream.hip, where the reasons stand): quarter_rounds is how often
+// its 32 x 64 pieces fill a quarter of the device.
+inline bool conv_streams(int64_t K, int64_t N, bool sum, int64_t quarter_rounds) {
+  auto within = [&](int64_t least, int64_t most = INT64_MAX) { return quarter_rounds >= least && quarter_rounds <= most; };
+  const bool wide = N > 64;
+  const int64_t least = sum || K <= 160 || !wide ? 3 : K > 256 && K < 384 && N > 256 && N <= 384 ? 24 : N > 256 || K >= 384 ? 6 : 3;
+  return K <= (wide ? 384 : 448) ? within(least) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
+}
+
+// Time of a 3 x 3 convolution over 32 to 128 channels on the kernel that would take it, us: fitted to 2200 shapes (tile shapes, one
+// standard deviation 4 to 7 %) and 550 (the kernel for a short K, 10 %: 32 x 64 results per wavefront and step, and per 32 rows
+// what its wavefront columns cost, idle ones among them, which is less where no window is padded).
+inline double others_us(int64_t M, int64_t K, int64_t N, bool padded) {
+  const int64_t tiles = (M + 31) / 32, cols = (N + 63) / 64;
+  if (conv_streams(K, N, false, tiles * cols / 1024)) {
+    const double per_rows = (cols == 1 ? 0.2 : cols == 2 ? 1.5 : cols <= 4 ? 6.1 : 26.0) * (padded ? 1.0 : 0.56);
+    return 6.0 + static_cast<double>(tiles) / 4096 * (4.56 * static_cast<double>(cols) + per_rows);
+  }
+  const double steps = static_cast<double>((K + 63) / 64);
+  auto rounds = [&](int bm, int bn) { return static_cast<double>((((M + bm - 1) / bm) * ((N + bn - 1) / bn) + 255) / 256); };
+  switch (pick_conv_tile(M, N)) {
+    case 0: return 1.7 + rounds(256, 128) * (5.8 + 0.66 * steps);
+    case 1: return 4.1 + rounds(128, 128) * (1.4 + 0.324 * steps);
+    default: return 3.7 + rounds(64, 64) * 0.15 * steps;
+  }
 }
 
 }  // namespace itexhip

@@ -15,6 +15,7 @@
 // What bounds it there: the start of a launch that fills the device (parameters and weight on their way to LDS, first rows,
 // last stores: 5 us), then vector instructions (6 per result with a clip, 7 with a residual) and the results leaving L2
 // (401408 x 32 -> 64: 5 us beyond the start, 7.7 TB/s).
+#include "qconv_walk.hpp"
 #include "qgemm_pack.hpp"
 
 namespace itexhip {
@@ -401,8 +402,7 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   const bool whole = K % 64 == 0, fits = whole && N % 128 == 0;  // nothing padded in the tile kernel
   bool take;
   if (cv) {
-    const int64_t least = sum || K <= 160 || !wide ? 3 : K > 256 && K < 384 && N > 256 && N <= 384 ? 24 : N > 256 || K >= 384 ? 6 : 3;
-    take = K <= (wide ? 384 : 448) ? within(least) : K <= 448 && (sum ? within(3, 7) : within(6, 7));
+    take = conv_streams(K, N, sum, quarter_rounds);
   } else if (K <= 64) {
     take = within(sum ? 1 : fits && N >= 256 ? 7 : 4);
   } else if (K < 128) {

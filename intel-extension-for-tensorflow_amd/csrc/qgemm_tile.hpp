@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdlib>
 
+#include "qconv_walk.hpp"
 #include "qgemm_common.hpp"
 
 // Measurement builds only (ablate.py): a bit mask of parts of the kernel that are compiled out, so that time, power
@@ -832,15 +833,7 @@ int dispatch_tile_conv(const uint8_t* x, uint32_t a_xor, const uint8_t* bp, int 
     set_error("itexhip_qconv2d_sum: the summand must be 4-byte (8-bit types) or 16-byte (float) aligned and out_channels a multiple of 4");
     return ITEXHIP_INVALID_ARGUMENT;
   }
-  struct Shape { int bm, bn; double penalty; };
-  static const Shape shapes[3] = {{256, 128, 1.08}, {128, 128, 1.2}, {64, 64, 1.8}};
-  int best = 0;
-  double best_cost = 1e300;
-  for (int i = 0; i < 3; ++i) {
-    const double tiles = static_cast<double>((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
-    const double cost = std::ceil(tiles / 256.0) * shapes[i].bm * shapes[i].bn * shapes[i].penalty;
-    if (cost < best_cost) { best_cost = cost; best = i; }
-  }
+  int best = pick_conv_tile(M, N);
   const int f = __atomic_load_n(&g_forced_tile_shape[1], __ATOMIC_RELAXED);  // tests exercise every shape with it
   if (f >= 0 && f < 3) best = f;
   switch (best) {

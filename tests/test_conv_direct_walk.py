@@ -7,6 +7,7 @@ import subprocess
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "intel-extension-for-tensorflow_amd", "csrc")
 
 PROGRAM = r"""
+#include <cstdint>
 #include <cstdio>
 #include <random>
 #include <vector>
@@ -108,9 +109,49 @@ def fast_div_source():
     return src[src.index("struct FastDiv"):end].replace("__device__ __forceinline__", "inline")
 
 
-def test_every_address(tmp_path):
+def run(tmp_path, program):
     src, exe = tmp_path / "walk.cc", tmp_path / "walk"
-    src.write_text(PROGRAM.replace("@FAST_DIV@", fast_div_source()))
+    src.write_text(program.replace("@FAST_DIV@", fast_div_source()))
     subprocess.run(["g++", "-std=c++17", "-O2", "-I", CSRC, str(src), "-o", str(exe)], check=True)
     done = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
     assert done.returncode == 0, done.stdout
+
+
+def test_every_address(tmp_path):
+    run(tmp_path, PROGRAM)
+
+
+PLANS = r"""
+#include <cstdint>
+#include <cstdio>
+namespace itexhip {
+@FAST_DIV@
+}
+#include "qconv_walk.hpp"
+using namespace itexhip;
+// batch, rows, columns, channels, results, where it measured faster: 1 here, 0 elsewhere
+const int cases[][6] = {{32, 56, 56, 64, 64, 1}, {32, 28, 28, 128, 128, 1}, {32, 112, 112, 32, 32, 1}, {1, 14, 14, 32, 32, 1},
+                        {4, 62, 62, 128, 224, 1}, {17, 12, 131, 128, 96, 1}, {4, 288, 288, 32, 96, 0}, {11, 253, 253, 32, 96, 0},
+                        {3, 195, 195, 96, 224, 0}};
+int main() {
+  int bad = 0;
+  for (const auto& c : cases) {
+    const int M = c[0] * c[1] * c[2];
+    const DirectPlan p = plan_direct(M, c[3], c[4], c[1], c[2]);
+    // workgroups of the busiest XCD's CUs: as many as an even spread gives
+    const int busiest = ((p.wgs + 7) / 8 * p.groups_n + 31) / 32, even = (p.wgs * p.groups_n + 255) / 256;
+    const bool here = p.us < others_us(M, 9 * c[3], c[4], true);
+    if (busiest > even || here != (c[5] == 1)) {
+      ++bad;
+      std::printf("%d x %d x %d x %d -> %d: %d workgroups x %d, here %d\n", c[0], c[1], c[2], c[3], c[4], p.wgs, p.groups_n, here);
+    }
+  }
+  return bad;
+}
+"""
+
+
+def test_run_lengths_and_choice(tmp_path):
+    """No run length leaves one XCD with a round of workgroups more than the others; the calls that measured faster elsewhere go
+    there."""
+    run(tmp_path, PLANS)
