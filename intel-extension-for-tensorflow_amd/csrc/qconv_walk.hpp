@@ -126,19 +126,20 @@ inline DirectPlan plan_direct(int M, int in_c, int N, int out_h, int out_w) {
   double best = 1e30;
   for (int per = 1; per <= kDirectMaxTiles; ++per) {
     // 32 * per positions lie in at most `rows` output rows, which cross `images` borders (two more input rows each)
-    const int64_t rows = (32 * per + out_w - 2) / out_w + 1, images = (rows + out_h - 2) / out_h;
-    const int64_t staged = (rows + 2 + 2 * images) * wp;  // pixels put into LDS
+    const unsigned rows = static_cast<unsigned>(32 * per + out_w - 2) / static_cast<unsigned>(out_w) + 1;
+    const unsigned images = rows < 2 ? 0 : rows <= static_cast<unsigned>(out_h) + 1 ? 1 : (rows - 2) / static_cast<unsigned>(out_h) + 1;
+    const int64_t staged = static_cast<int64_t>(rows + 2 + 2 * images) * wp;  // pixels put into LDS
     const int64_t bytes = staged * pitch + panel;
     if (bytes > kLdsPerCu) break;
-    const int wgs = (tiles + per - 1) / per;
+    const unsigned wgs = static_cast<unsigned>(tiles + per - 1) / static_cast<unsigned>(per);
     const int64_t n = (static_cast<int64_t>((wgs + 7) / 8) * s.groups_n + 31) / 32;  // workgroups of the busiest CU
-    const int at_once = std::min(resident, kLdsPerCu / static_cast<int>(bytes));
+    const int at_once = std::min(resident, static_cast<int>(static_cast<unsigned>(kLdsPerCu) / static_cast<unsigned>(bytes)));
     const int turns = (per + waves_m - 1) / waves_m;  // tiles of a wavefront
-    const double sets = static_cast<double>((n + at_once - 1) / at_once);
+    const double sets = n <= at_once ? 1.0 : static_cast<double>((n + at_once - 1) / at_once);
     const double us = static_cast<double>(n) * turns * (0.18 + 0.2 * c32) * (n == 1 || at_once == 1 ? 1.28 : 1.0) + 3.7 * sets;
     if (us < best) {
       best = us;
-      s.per_wg = per; s.lds = static_cast<int>(bytes); s.wgs = wgs;
+      s.per_wg = per; s.lds = static_cast<int>(bytes); s.wgs = static_cast<int>(wgs);
       // The launch as a whole, for others_us to be compared with: 2.0, and per set its start, 0.99 for every eight loads per
       // thread that put rows into LDS, and the tiles, 0.86 of whose time adds up for workgroups that share a CU.  Within 10 %
       // (one standard deviation) of 25900 times.
@@ -146,6 +147,7 @@ inline DirectPlan plan_direct(int M, int in_c, int N, int out_h, int out_w) {
       s.us = 2.0 + sets * (1.06 + 0.99 / (8 * kDirectThreads) * pieces + std::min(turns, (tiles + waves_m - 1) / waves_m) * (0.2 + 0.22 * c32) *
                                       (1.0 + 0.86 * (static_cast<double>(std::min<int64_t>(n, at_once)) - 1.0)));
     }
+    if (n == 1) break;  // longer runs leave CUs without one
   }
   s.panel = s.lds - panel;
   return s;

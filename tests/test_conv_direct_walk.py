@@ -155,3 +155,49 @@ def test_run_lengths_and_choice(tmp_path):
     """No run length leaves one XCD with a round of workgroups more than the others; the calls that measured faster elsewhere go
     there."""
     run(tmp_path, PLANS)
+
+
+SHORTCUTS = r"""
+#include <cstdint>
+#include <cstdio>
+#include <random>
+namespace itexhip {
+@FAST_DIV@
+}
+#include "qconv_walk.hpp"
+using namespace itexhip;
+int main() {
+  std::mt19937 g(2);
+  auto size = [&](int most) { return 1 + static_cast<int>(g() % (1 + g() % most)); };
+  int bad = 0, runs = 0;
+  for (int i = 0; i < 20000; ++i) {
+    const int B = size(64), oh = size(300), ow = size(300), C = 32 * (1 + static_cast<int>(g() % 4)), N = 32 * size(16);
+    if ((ow + 2LL) * direct_pitch(C) * 3 > kLdsPerCu) continue;
+    const int64_t M = 1LL * B * oh * ow, tiles = (M + 31) / 32, c32 = C / 32, blocks = N / 32;
+    const int64_t waves_n = blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1, groups = blocks / waves_n, waves_m = 4 / waves_n;
+    const int64_t resident = c32 == 1 ? 4 : c32 == 2 ? 3 : 2;
+    double best = 1e30;
+    int64_t per_wg = 0;
+    for (int64_t per = 1; per <= kDirectMaxTiles; ++per) {
+      const int64_t rows = (32 * per + ow - 2) / ow + 1, images = (rows + oh - 2) / oh;
+      const int64_t bytes = (rows + 2 + 2 * images) * (ow + 2) * direct_pitch(C) + 384 * waves_n;
+      if (bytes > kLdsPerCu) break;
+      const int64_t n = (((tiles + per - 1) / per + 7) / 8 * groups + 31) / 32, at_once = std::min(resident, kLdsPerCu / bytes);
+      const double us = static_cast<double>(n) * static_cast<double>((per + waves_m - 1) / waves_m) * (0.18 + 0.2 * static_cast<double>(c32)) *
+                            (n == 1 || at_once == 1 ? 1.28 : 1.0) + 3.7 * static_cast<double>((n + at_once - 1) / at_once);
+      if (us < best) { best = us; per_wg = per; }
+    }
+    const DirectPlan p = plan_direct(static_cast<int>(M), C, N, oh, ow);
+    runs += per_wg > 1;
+    if (p.per_wg != per_wg || (per_wg > 0 && p.wgs != (tiles + per_wg - 1) / per_wg) || p.us < 0) {
+      if (++bad < 5) std::printf("%d x %d x %d x %d -> %d: %d, %ld\n", B, oh, ow, C, N, p.per_wg, static_cast<long>(per_wg));
+    }
+  }
+  return bad != 0 || runs < 1000;
+}
+"""
+
+
+def test_shortcuts_of_the_run_length(tmp_path):
+    """The search that a call pays for finds what the whole one does."""
+    run(tmp_path, SHORTCUTS)
