@@ -83,7 +83,13 @@ template <int OUT_T, bool TRANS, int SPLIT>
 __global__ __launch_bounds__(256 * SPLIT) void qmatmul_unpacked_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
                                                                 const uint8_t* __restrict__ w, int M, int K, int N,
                                                                 int tiles_n, int tiles, EpilogueArgs e, void* __restrict__ out) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // per group its rows and columns, then the column sums
+  // per group its rows and columns, then the column sums (one group: at addresses that the compiler knows)
+  extern __shared__ __attribute__((aligned(16))) uint8_t dynamic_lds[];
+  uint8_t* lds = dynamic_lds;
+  if constexpr (SPLIT == 1) {
+    __shared__ __attribute__((aligned(16))) uint8_t fixed[kGroupLds + 4 * kTileN];
+    lds = fixed;
+  }
   const int t = threadIdx.x & 255, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int group = SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
@@ -318,7 +324,8 @@ __global__ __launch_bounds__(256) void qmatmul_tiny_kernel(const uint8_t* __rest
 // columns, K of 1 to 300).  A thread per output: the latency of its dot product, 2.4 + 0.071 K (0.105 K beyond 64 columns), or,
 // where the outputs fill the chip, 2 and 1e-6 of 3.4 + 0.26 K per output, more per k where a wavefront's 64 outputs touch many
 // rows (few columns, rows that share no lines) and where the weight is past 2 MB; in between the two join.  Tiles: 3.4 + 0.011
-// each, at least 5.8, per further K step half of that more and 0.9.  The choice is 0.2 % above the faster kernel in the mean and
+// each, at least 5.8, per further K step half of that more and 0.9 (one group of wavefronts; two are shorter, but from the second
+// step on a thread's dot product alone takes 20).  The choice is 0.2 % above the faster kernel in the mean and
 // takes the slower one where it costs more than 10 % for 84 of the sizes (up to twice: 122975 x 107 x 1 45 for 23).
 // Per output / tiles: 100000 x 17 x 1 4.8 / 20.7, 1 x 17 x 100000 5.3 / 20.3, 1000000 x 9 x 16 99 / 143, 8 x 9 x 8 3.6 / 6.0,
 // 270 x 9 x 1413 4.6 / 6.4, 13 x 19 x 36455 6.6 / 11.2; 100000 x 65 x 10 57 / 21, 84678 x 32 x 11 30 / 15, 1000 x 17 x 1000
@@ -336,7 +343,7 @@ template <int OUT_T, bool TRANS, int SPLIT>
 int launch_tiles(unsigned grid, const uint8_t* a, uint32_t a_xor, const uint8_t* w, int M, int K, int N, int tiles_n, int tiles,
                  const EpilogueArgs& e, void* out, hipStream_t st) {
   auto kern = qmatmul_unpacked_kernel<OUT_T, TRANS, SPLIT>;
-  constexpr int kLds = SPLIT * kGroupLds + 4 * kTileN;
+  constexpr int kLds = SPLIT == 1 ? 0 : SPLIT * kGroupLds + 4 * kTileN;  // dynamic
   static unsigned long long attr_done = 0;  // devices on which this instantiation's attribute is set
   if (kLds > 64 * 1024 && !device_bit(&attr_done, false)) {
     const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -359,11 +366,12 @@ int launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, 
     return ITEXHIP_OK;
   }
   const unsigned grid = static_cast<unsigned>((tiles + 7) / 8 * 8);  // whole runs for the 8 XCDs
-  // Two groups per tile as long as every tile has a CU to itself (also with one K step, whose result two groups finish in half
-  // the time); beyond that a CU runs two workgroups of one group and hides one's waits behind the other, where one workgroup of
-  // two groups is all that its registers hold.  One group / two, us: 1000 x 1001 x 1000 (256 tiles) 11.0 / 9.7, 200 x 901 x 1000
-  // 10.2 / 8.9, 300 x 511 x 300 8.1 / 7.3, 90 x 129 x 90 6.7 / 6.4; 2000 x 301 x 1000 (512 tiles) 9.4 / 13.0.
-  const bool split = tiles <= 256;
+  // Two groups per tile as long as every tile has a CU to itself, with one K step only where the weight is [N, K] (it is put
+  // into LDS as it is); beyond that a CU runs two workgroups of one group and hides one's waits behind the other, where one
+  // workgroup of two groups is all that its registers hold.  One group / two, us: 1000 x 1001 x 1000 (256 tiles) 11.0 / 9.7,
+  // 200 x 901 x 1000 10.2 / 8.9, 300 x 511 x 300 8.1 / 7.3; 2000 x 301 x 1000 (512 tiles) 9.4 / 13.0.  Two / one over 1500 sizes of
+  // one step: [N, K] 0.93 - 1.07 (0.99 in the middle), [K, N] 0.96 - 1.10 (1.02: 3 x 43 x 68 5.6 / 6.1); of more steps 0.81 - 0.99.
+  const bool split = tiles <= 256 && (transpose_b || K > kStepK);
 #define TILES(S) (transpose_b ? launch_tiles<OUT_T, true, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st) \
                               : launch_tiles<OUT_T, false, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st))
   return split ? TILES(2) : TILES(1);
