@@ -41,7 +41,8 @@ struct StreamArgs {
 
 static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
 
-// 128 registers for four wavefronts per SIMD, without spills (scratch costs a launch 1.5 us).
+// 128 vector registers for four wavefronts per SIMD, without scratch but for groups of 4 with a residual (it costs a launch
+// 1.5 us); up to 26 scalar registers go to lanes of a vector register.
 // HOLD: the K chunks of a tile are exactly GROUP; all are held at once, and each is replaced by the next tile's as soon as its
 // MFMAs are issued: no second set of registers, no copies, and where a lane's pieces lie relative to its row is computed
 // once.  With two sets, copies and 21 instructions per piece the 7 x 7 convolution above took 14.6 us and 401408 x 32 -> 64
@@ -59,7 +60,7 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
   int* const p_comp = reinterpret_cast<int*>(lds + frags * kChunkBytes);
   float* const p_scale = reinterpret_cast<float*>(p_comp + channels);
   float* const p_bias = p_scale + channels;
-  int2* const table = reinterpret_cast<int2*>(p_bias + channels);  // convolution: per 16-byte piece of a patch row
+  int2* const table = reinterpret_cast<int2*>(p_bias + channels);  // convolution, not HOLD: per 16-byte piece of a patch row
 
   const int wn = wave % s.waves_n, wm = wave / s.waves_n, waves_m = 4 / s.waves_n;
   // consecutive workgroup ids go round the 8 XCDs: each of them walks a contiguous range of rows (neighbouring rows of a
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
 #pragma unroll
   for (int u = 0; u < GROUP; ++u) {
     const int c = min(u, s.chunks - 1);
-    if constexpr (HOLD) cur[u] = load_held(u);  // (chunks past the last one have its offsets or the row's last piece)
+    if constexpr (HOLD) cur[u] = load_held(u);
     else if constexpr (CONV) cur[u] = load_piece(piece_of(c));
     else cur[u] = load(c);
   }
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(256, 4) void qgemm_stream_kernel(const uint8_t* __r
     p_scale[i] = scale;
     p_bias[i] = bias;
   }
-  if constexpr (CONV) {
+  if constexpr (CONV && !HOLD) {
     for (int p = threadIdx.x; p < (s.K >> 4); p += 256) table[p] = window_piece(p);
   }
   wait_vmcnt<0>();  // the direct loads of this wavefront have landed
@@ -428,7 +429,8 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   s.padded = cv && (cv->pad_top > 0 || cv->pad_left > 0 ||
                     (cv->out_h - 1) * cv->stride_h + (K / (cv->k_w * cv->in_c) - 1) * cv->dil_h >= cv->in_h ||
                     (cv->out_w - 1) * cv->stride_w + (cv->k_w - 1) * cv->dil_w >= cv->in_w);
-  const size_t lds = static_cast<size_t>(weight) + 12 * s.waves_n * kBlocks * 32 + (cv ? (K >> 4) * 8 : 0);
+  const bool held_conv = cv && !sum && !s.padded && s.chunks <= 8;
+  const size_t lds = static_cast<size_t>(weight) + 12 * s.waves_n * kBlocks * 32 + (cv && !held_conv ? (K >> 4) * 8 : 0);
   const int per_cu = std::min<int>(4, 160 * 1024 / static_cast<int>(lds));  // 128 registers: four wavefronts per SIMD
   const int groups_n = (cols + s.waves_n - 1) / s.waves_n;
   if (groups_n > 65535) return 0;  // gridDim.y
@@ -461,13 +463,13 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   if (cv && sum) {
     STREAM(2, true, false, true, *cv);
   } else if (cv) {
-    switch (s.padded ? 0 : s.chunks) {
+    switch (held_conv ? s.chunks : 0) {
       HELD(true, false, *cv);
       HELD_LONG(true, *cv);
       default: STREAM(4, true, false, false, *cv);
     }
   } else if (sum) {
-    // Held, or groups of 1, 2 or 4 (4 with a residual spills up to 7 registers, which a long K covers).  Held chunks need the
+    // Held, or groups of 1, 2 or 4 (4 with a residual spills up to 4 registers, which a long K covers).  Held chunks need the
     // caches: past 256 MB of activations, residual and result, or past 96 MB where rows are no multiple of 64 bytes and pieces
     // of lines have to meet in them, the groups' earlier loads win.  Time over that of groups of 1 (one chunk), 2 (two) or 4
     // (more), 3000 sizes:
