@@ -48,11 +48,17 @@ enum { ITEXHIP_MIN_COMBINED = 0, ITEXHIP_MIN_FIRST = 1, ITEXHIP_SCALED = 2,
 const char* itexhip_last_error(void);
 /* "gfx950" and the library version; no GPU call. */
 const char* itexhip_build_info(void);
-/* Test hook (no counterpart in the reference): forces the tile shape of the MatMul tile kernel (0..4 = 256x256,
- * 256x192, 256x128, 128x128, 64x64) and of the implicit-GEMM Conv2D (0..2 = 256x128, 128x128, 64x64), or (16) the kernel for
- * a short K at any size, or (17) the Conv2D kernel that keeps its input rows in LDS, for every later call of the process; any of them also keeps a MatMul on unpacked operands with its
- * tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */
+/* Test hook (no counterpart in the reference): forces the tile shape of the MatMul tile kernel (0..5 = 256x256,
+ * 256x192, 256x128, 128x128, 64x64, 128x64; clamped loads and the element-wise epilogue have 3 and 4) and of the implicit-GEMM
+ * Conv2D (0..2 = 256x128, 128x128, 64x64), or (16) the kernel for a short K at any size, or (17) the Conv2D kernel that keeps its
+ * input rows in LDS, for every later call of the process that the forced kernel can take; any of them also keeps a MatMul on
+ * unpacked operands with its tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */
 void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape);
+/* Test hook: the kernel that the calling thread's last MatMul or Conv2D (not depthwise, not batched) was launched on, times
+ * 10^8, plus what was chosen within it: 1 small M, 2 tiles (rows * 10^5 + columns * 100 + LDS stages), 3 short K (chunks per group
+ * * 100 + 1 if all are held), 4 3 x 3 convolution (tiles per workgroup), 5 unpacked operands (groups per tile), 6 one output per
+ * thread.  0: none yet. */
+int itexhip_test_last_kernel(void);
 
 /* ------------------------------------------------------------------------------------------
  * Stream-ordered host-to-device copy of small parameter vectors (per-channel ranges, per-axis

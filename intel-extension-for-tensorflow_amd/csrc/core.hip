@@ -6,9 +6,12 @@
 namespace itexhip {
 namespace {
 thread_local char g_error[512] = "";
+thread_local int g_last_kernel = 0;
 }
 
 int g_forced_tile_shape[2] = {-1, -1};
+
+void note_kernel(LastKernel kernel, int detail) { g_last_kernel = kernel * 100000000 + detail; }
 
 void set_error(const char* fmt, ...) {
   va_list ap;
@@ -24,6 +27,8 @@ extern "C" void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape) 
   __atomic_store_n(&itexhip::g_forced_tile_shape[0], matmul_shape, __ATOMIC_RELAXED);
   __atomic_store_n(&itexhip::g_forced_tile_shape[1], conv_shape, __ATOMIC_RELAXED);
 }
+
+extern "C" int itexhip_test_last_kernel(void) { return itexhip::g_last_kernel; }
 
 extern "C" const char* itexhip_build_info(void) { return "itexhip 0.1 gfx950"; }
 

@@ -168,6 +168,7 @@ int launch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const DirectArgs
     if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qconv_direct_kernel)");
     device_bit(&attr_done, true);
   }
+  note_kernel(kLastDirect, s.per_wg);
   kern<<<grid, 256, lds, st>>>(a, amask, bp, s, out);
   return ITEXHIP_OK;
 }

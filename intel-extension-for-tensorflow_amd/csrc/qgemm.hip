@@ -549,6 +549,7 @@ int launch_packed(Path path, const void* a, int a_type, const int8_t* packed_b, 
     }
   }
   if (path == Path::kSmallM) {
+    note_kernel(kLastSmallM, 0);
 #define CALL_GEMV(T) dispatch_gemv<T>(ap, a_xor, bp, Mi, Ki, Ni, e, out, hs)
     ITEXHIP_DISPATCH_OUT(out_type, CALL_GEMV)
 #undef CALL_GEMV

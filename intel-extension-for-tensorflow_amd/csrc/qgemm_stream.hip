@@ -304,6 +304,7 @@ int launch(const uint8_t* a, uint32_t amask, const uint8_t* bp, const StreamArgs
     if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qgemm_stream_kernel)");
     device_bit(&attr_done, true);
   }
+  note_kernel(kLastShortK, GROUP * 100 + HOLD);
   kern<<<grid, 256, lds, st>>>(a, amask, bp, s, e, out, cv);
   return ITEXHIP_OK;
 }

@@ -707,6 +707,7 @@ int launch_tile(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int 
     if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qgemm_tile_kernel)");
     device_bit(&attr_done, true);
   }
+  note_kernel(kLastTile, BM * 100000 + BN * 100 + NSTAGE);
   kern<<<dim3(static_cast<unsigned>(num_m * num_n)), dim3(64 * WAVES_M * WAVES_N), lds_now, st>>>(
       a, amask, bp, M, K, N, KT, NT, num_m, num_n, xcd_rectangles(num_m, num_n, BM, BN, K), e, out, cv);
   return ITEXHIP_OK;

@@ -350,6 +350,7 @@ int launch_tiles(unsigned grid, const uint8_t* a, uint32_t a_xor, const uint8_t*
     if (err != hipSuccess) return hip_fail(err, "hipFuncSetAttribute(qmatmul_unpacked_kernel)");
     device_bit(&attr_done, true);
   }
+  note_kernel(kLastUnpacked, SPLIT);
   kern<<<grid, 256 * SPLIT, kLds, st>>>(a, a_xor, w, M, K, N, tiles_n, tiles, e, out);
   return ITEXHIP_OK;
 }
@@ -359,6 +360,7 @@ int launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, 
             const EpilogueArgs& e, void* out, hipStream_t st) {
   const bool forced = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0;  // tests ask for the tile kernel
   if (tiles == 0 || static_cast<int64_t>(M) * K < 16 || static_cast<int64_t>(K) * N < 16 || (!forced && one_output_per_thread(M, K, N, tiles))) {
+    note_kernel(kLastPerOutput, 0);
     in_pieces(0, static_cast<int64_t>(M) * N, [&](int64_t first, int64_t end) {
       qmatmul_tiny_kernel<OUT_T><<<static_cast<unsigned>((end - first + 255) / 256), 256, 0, st>>>(
           a, a_xor != 0, reinterpret_cast<const int8_t*>(w), transpose_b, M, K, N, e, out, first);

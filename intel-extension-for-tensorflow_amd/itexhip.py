@@ -28,7 +28,7 @@ EXPORTS = [
     "itexhip_stream_query", "itexhip_event_create", "itexhip_event_destroy", "itexhip_event_record",
     "itexhip_event_query", "itexhip_event_synchronize", "itexhip_stream_wait_event", "itexhip_device_synchronize",
     "itexhip_memcpy_d2h_async", "itexhip_memset8_async", "itexhip_memset32_async", "itexhip_launch_host_func",
-    "itexhip_last_error", "itexhip_build_info", "itexhip_test_force_tile_shape", "itexhip_memcpy_h2d_async", "itexhip_memcpy_d2h", "itexhip_memcpy_d2d_async", "itexhip_stream_synchronize", "itexhip_quantize", "itexhip_quantize_axis",
+    "itexhip_last_error", "itexhip_build_info", "itexhip_test_force_tile_shape", "itexhip_test_last_kernel", "itexhip_memcpy_h2d_async", "itexhip_memcpy_d2h", "itexhip_memcpy_d2d_async", "itexhip_stream_synchronize", "itexhip_quantize", "itexhip_quantize_axis",
     "itexhip_dequantize", "itexhip_dequantize_axis", "itexhip_quantize_bf16", "itexhip_quantize_axis_bf16",
     "itexhip_dequantize16", "itexhip_dequantize_axis16", "itexhip_requantize_per_channel",
     "itexhip_requantize", "itexhip_minmax_i32_per_channel", "itexhip_minmax_f32",
@@ -158,6 +158,16 @@ def force_tile_shape(matmul=-1, conv=-1):
     library chooses)."""
     _lib.itexhip_test_force_tile_shape.restype = None
     _lib.itexhip_test_force_tile_shape(C.c_int(int(matmul)), C.c_int(int(conv)))
+
+
+def last_kernel():
+    """Test hook: the kernel of this thread's last MatMul or Conv2D and what was chosen within it, ("tile", 128, 64, 8) for tiles of
+    128 x 64 on eight LDS stages."""
+    kernel, detail = divmod(int(_lib.itexhip_test_last_kernel()), 10 ** 8)
+    name = (None, "small_m", "tile", "short_k", "direct", "unpacked", "per_output")[kernel]
+    if name == "tile":
+        return name, detail // 100000, detail // 100 % 1000, detail % 100
+    return (name, detail // 100, bool(detail % 100)) if name == "short_k" else (name, detail)
 
 
 def memcpy_d2h(host_array, src, nbytes, stream=0):

@@ -63,7 +63,7 @@ def test_arguments_are_those_of_the_wrapper(hip):
     import inspect
     for name in ENTRIES:
         if name in ("transpose", "qgemm", "qgemm_tile", "qgemv"):
-            continue
+            continue   # (the last three below)
         src = " ".join(inspect.getsource(getattr(hip, name)).split())
         fast = re.search(r"_call\.%s\((.*?)\): _check" % name, src).group(1)
         slow = re.search(r"_check\(_%s\((.*)\)\)$" % name, src).group(1)
@@ -71,5 +71,9 @@ def test_arguments_are_those_of_the_wrapper(hip):
         while re.search(r"(?<![\w])\((\w+)\)", plain):
             plain = re.sub(r"(?<![\w])\((\w+)\)", r"\1", plain)
         assert fast == plain, name
-    params = inspect.signature(hip.qgemm).parameters
-    assert ", ".join(params) in " ".join(inspect.getsource(hip.qgemm).split("_call.qgemm(")[1].split())
+    for name in ("qgemm", "qgemm_tile", "qgemv"):
+        wrapper = getattr(hip, name)
+        src = " ".join(inspect.getsource(wrapper).split())
+        params = ", ".join(inspect.signature(wrapper).parameters)
+        assert re.search(r"_call\.%s\((.*?)\): _gemm_call" % name, src).group(1) == params
+        assert re.search(r"_gemm_call\((.*)\)$", src).group(1) == "_%s, %s" % (name, params)

@@ -212,7 +212,8 @@ def test_implicit_gemm_conv_random_geometries(hip, dev, monkeypatch, seed):
         done += 1
 
 
-def check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, rng):
+def check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, rng, kernel=None):
+    """kernel: what an 8-bit result has to be launched on."""
     import torch
     from tests.test_oracle_conv import ref_int_conv
     B, H, W, Cin = shape
@@ -260,6 +261,7 @@ def check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, 
         a.view(torch.uint8).fill_(0x55)          # different fillers: an element neither path writes shows up
         b_.view(torch.uint8).fill_(0xAA)
         hip.qconv2d(xd, T_in, g, packed, colsum, O, scales, bias, ep, T, a)
+        assert kernel is None or T not in (hip.QINT8, hip.QUINT8) or hip.last_kernel()[0] == kernel
         hip.qgemm(cols, T_in, packed, colsum, M, K, O, scales, bias, ep, T, b_)
         torch.cuda.synchronize()
         assert torch.equal(a.view(torch.uint8), b_.view(torch.uint8)), T

@@ -3,14 +3,14 @@ int64 sums and the epilogue's separately rounded fp32 steps in numpy, bit for bi
 import numpy as np
 import pytest
 
-from tests.test_gpu_stream import finish
+from tests.test_gpu_stream import awkward_floats, finish
 from tests.test_oracle_conv import ref_int_conv
 
 pytestmark = pytest.mark.gpu
 DIRECT = 17   # force_tile_shape: this kernel wherever it can take the call
 
 
-def run(hip, dev, shape, O, pad, out_hw, post, signed_in, signed_out, seed, scalar_scale=False):
+def run(hip, dev, shape, O, pad, out_hw, post, signed_in, signed_out, seed, scalar_scale=False, kernel="direct", scale=None, bias=None):
     import torch
     rng = np.random.default_rng(seed)
     B, H, W, C = shape
@@ -19,8 +19,10 @@ def run(hip, dev, shape, O, pad, out_hw, post, signed_in, signed_out, seed, scal
     w = rng.integers(-127, 128, (3, 3, C, O)).astype(np.int8)
     trailing = max(oh + 2 - H - pt, 0), max(ow + 2 - W - pl, 0)
     acc = ref_int_conv(x, w, (1, 1), (1, 1), ((pt, trailing[0]), (pl, trailing[1])))[:, :oh, :ow].reshape(B * oh * ow, O)
-    scale = ((rng.random(1 if scalar_scale else O) + 0.5) * 60.0 / (74.0 * 74.0 * np.sqrt(9 * C))).astype(np.float32)
-    bias = (rng.standard_normal(O) * 20).astype(np.float32)
+    if scale is None:
+        scale = ((rng.random(1 if scalar_scale else O) + 0.5) * 60.0 / (74.0 * 74.0 * np.sqrt(9 * C))).astype(np.float32)
+    if bias is None:
+        bias = (rng.standard_normal(O) * 20).astype(np.float32)
     inf = float("inf")
     lo, hi = {"none": (-inf, inf), "relu": (0.0, inf), "clip": (-3.5, 90.0)}[post]
     ep = hip.Epilogue()
@@ -36,6 +38,7 @@ def run(hip, dev, shape, O, pad, out_hw, post, signed_in, signed_out, seed, scal
     g = hip.ConvGeometry(B, H, W, C, 3, 3, oh, ow, 1, 1, 1, 1, pt, pl)
     hip.qconv2d(d(x), hip.QINT8 if signed_in else hip.QUINT8, g, packed, colsum, O, d(scale), d(bias), ep,
                 hip.QINT8 if signed_out else hip.QUINT8, out)
+    assert hip.last_kernel()[0] == kernel
     torch.cuda.synchronize()
     got = out.cpu().numpy()
     assert (got[n:] == 0x55).all()
@@ -73,7 +76,21 @@ def test_post_ops(hip, dev, post, signed_out, C):
     run(hip, dev, (2, 13, 14, C), 64, *same(13, 14), post, False, signed_out, C, scalar_scale=signed_out)
 
 
-@pytest.mark.parametrize("shape,O", [((13, 56, 56, 64), 64), ((13, 28, 28, 128), 128), ((1, 190, 190, 64), 64), ((4, 64, 64, 128), 160)])
-def test_without_force(hip, dev, shape, O):
+@pytest.mark.parametrize("post", ["none", "relu", "clip"])
+@pytest.mark.parametrize("signed_out", [False, True])
+@pytest.mark.parametrize("where", ["bias", "scale"])
+def test_infinities_and_nan(hip, dev, post, signed_out, where):
+    """Ties, infinities, NaN and random bit patterns as biases (scale 0) and as scales (sums of either sign and 0)."""
+    O = 4096
+    v = awkward_floats(O)
+    hip.force_tile_shape(conv=DIRECT)
+    run(hip, dev, (1, 5, 7, 32), O, *same(5, 7), post, where == "scale", signed_out, 3,
+        **(dict(bias=v, scale=np.zeros(1, np.float32)) if where == "bias" else dict(scale=v, bias=np.zeros(O, np.float32))))
+
+
+@pytest.mark.parametrize("shape,O,kernel", [((13, 56, 56, 64), 64, "direct"), ((13, 28, 28, 128), 128, "direct"), ((1, 190, 190, 64), 64, "direct"),
+                                            ((4, 64, 64, 128), 160, "direct"), ((1, 300, 300, 64), 64, "tile"), ((1, 177, 177, 96), 96, "tile"),
+                                            ((4, 288, 288, 32), 96, "short_k")])
+def test_without_force(hip, dev, shape, O, kernel):
     """Several runs per CU, and the calls on either side of the lines to the other kernels."""
-    run(hip, dev, shape, O, *same(shape[1], shape[2]), "relu", False, False, 9)
+    run(hip, dev, shape, O, *same(shape[1], shape[2]), "relu", False, False, 9, kernel=kernel)

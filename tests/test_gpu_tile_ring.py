@@ -19,8 +19,15 @@ def test_k_loops_around_the_ring(hip, dev, shape, K):
         x, xq, mn, mx = make_acts(M, K, seed=M + K)
         r = float(np.abs(x @ w + bias).max())
         ref = layer.oracle(xq, kw, mn, mx, -r, r)
+        vector = N % 4 == 0   # every row a multiple of 16 bytes
         for path in ("tile", "fused"):
             np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path=path), ref)
+            if path == "fused" and M <= 128:
+                assert hip.last_kernel()[0] == "small_m"
+            elif shape == 5 and vector and K % 64 == 0:
+                assert hip.last_kernel() == ("tile", 128, 64, 8)
+            else:   # K not a multiple of 64 and the element-wise epilogue have no 128 x 64 tiles
+                assert hip.last_kernel() == ("tile", 64, 64, 8 if K > 768 else 4)
 
 
 @pytest.mark.parametrize("K", [752, 768, 784, 832, 896, 960, 1040])
@@ -32,16 +39,19 @@ def test_k_where_the_ring_of_64x64_tiles_changes(hip, dev, K):
         x, xq, mn, mx = make_acts(M, K, seed=M + K)
         r = float(np.abs(x @ w + bias).max())
         np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path="tile"), layer.oracle(xq, kw, mn, mx, -r, r))
+        assert hip.last_kernel() == ("tile", 64, 64, 8 if K > 768 else 4)
 
 
-@pytest.mark.parametrize("M,K,N", [(1024, 512, 1024), (1025, 512, 1024),     # 256 and 272 tiles of 64 x 64
-                                   (2048, 768, 1024), (2049, 768, 1024),     # 256 and 272 tiles of 128 x 64
-                                   (2048, 752, 1024), (2048, 784, 1021),     # K below the line; clamped loads, element-wise
-                                   (1920, 832, 544), (1840, 832, 544)])      # 15 tile rows of 128 against 30 or 29 of 64
-def test_where_the_shape_changes(hip, dev, M, K, N):
+@pytest.mark.parametrize("M,K,N,tile", [(1024, 512, 1024, (64, 64, 4)), (1025, 512, 1024, (64, 64, 4)),       # 256 and 272 tiles of 64 x 64
+                                        (1024, 896, 1024, (64, 64, 8)), (1025, 896, 1024, (128, 64, 8)),
+                                        (2048, 768, 1024, (128, 64, 8)), (2049, 768, 1024, (128, 128, 4)),    # 256 and 272 of 128 x 64
+                                        (2048, 752, 1024, (64, 64, 4)), (2048, 784, 1021, (64, 64, 4)),       # clamped loads, element-wise
+                                        (1920, 832, 544, (64, 64, 4)), (1840, 832, 544, (128, 64, 8))])       # 15 tile rows against 30 or 29
+def test_where_the_shape_changes(hip, dev, M, K, N, tile):
     layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
     _, xq, mn, mx = make_acts(M, K, seed=M + K)
     np.testing.assert_array_equal(layer.run(xq, V2_DEQ, mn, mx, path="fused"), layer.oracle(xq, V2_DEQ, mn, mx))
+    assert hip.last_kernel() == ("tile", *tile)
 
 
 @pytest.mark.parametrize("K", [448, 2048])

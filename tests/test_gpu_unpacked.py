@@ -41,15 +41,18 @@ def test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b):
 @pytest.mark.parametrize("kw,transpose_b", [(V2_DEQ, False), (V2_REQ_U8_RELU, False), (dict(V2_DEQ, input_mode=orc.SCALED), True)])
 def test_split_of_k_steps(hip, dev, M, K, N, kw, transpose_b):
     test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b)
+    tiles = -(-M // 64) * -(-N // 64)
+    assert hip.last_kernel() == ("unpacked", 2 if tiles <= 256 and (transpose_b or K > 256) else 1)
 
 
 # sizes that go one thread per output by themselves, through the tile kernel as well, and sizes on both sides of the line
-@pytest.mark.parametrize("M,K,N", [(5, 15, 3), (2, 8, 70), (3, 17, 16), (17, 13, 129), (1, 17, 200), (200, 33, 1), (65, 9, 66), (300, 36, 8), (300, 39, 8)])
+@pytest.mark.parametrize("M,K,N", [(5, 15, 3), (2, 8, 70), (3, 17, 16), (17, 13, 129), (1, 17, 200), (200, 33, 1), (65, 9, 66), (300, 36, 8), (300, 39, 8), (300, 46, 8), (300, 47, 8)])
 @pytest.mark.parametrize("kw,transpose_b", [(V2_DEQ, False), (V2_REQ_U8_RELU, False), (dict(V2_DEQ, input_mode=orc.SCALED), True)])
 @pytest.mark.parametrize("shape", [-1, 0])
 def test_both_kernels(hip, dev, M, K, N, kw, transpose_b, shape):
     hip.force_tile_shape(matmul=shape)
     test_unpacked_matmul_vs_oracle(hip, dev, M, K, N, kw, transpose_b)
+    assert hip.last_kernel()[0] == ("unpacked" if shape == 0 or K == 47 else "per_output")
 
 
 def test_more_rows_than_tiles_in_a_launch(hip, dev):
