@@ -49,7 +49,7 @@ const char* itexhip_last_error(void);
 /* "gfx950" and the library version; no GPU call. */
 const char* itexhip_build_info(void);
 /* Test hook (no counterpart in the reference): forces the tile shape of the MatMul tile kernel (0..5 = 256x256,
- * 256x192, 256x128, 128x128, 64x64, 128x64; clamped loads and the element-wise epilogue have 3 and 4) and of the implicit-GEMM
+ * 256x192, 256x128, 128x128, 64x64, 128x64; clamped loads have 3, 4 and 5, the element-wise epilogue 3 and 4) and of the implicit-GEMM
  * Conv2D (0..2 = 256x128, 128x128, 64x64), or (16) the kernel for a short K at any size, or (17) the Conv2D kernel that keeps its
  * input rows in LDS, for every later call of the process that the forced kernel can take; any of them also keeps a MatMul on
  * unpacked operands with its tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */

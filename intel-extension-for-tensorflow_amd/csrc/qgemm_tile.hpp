@@ -725,37 +725,49 @@ int launch_tile(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int 
 // ResNet-50 block, K = 64: 18.7 -> 12.4 us, with the residual Sum 39.5 -> 20.5 us; 4096 x 3072, 16384 x 1024 and
 // 2048 x 14336 outputs, 8-bit and fp32: 5 - 30 % faster at K = 64 - 256, mixed at 384, slower from 512 on).
 //
-// Between one and two 64 x 64 tiles per CU, a K of 768 and more that is a multiple of 64: 128 x 64 tiles, one per CU, four
-// wavefronts of 32 x 64 stacked along M and the deep ring.  A CU then loads 192 rows of operands per step instead of 256 for two
-// small tiles, and half of the device no longer does twice the work of the other half.  us, 64 x 64 (or 128 x 128) tiles ->
-// these, fp32 results: 2048 x 2048 -> 1024 12.6 -> 11.2, 4096 x 2048 -> 512 14.8 -> 10.7, 128 x 4096 -> 14336 20.6 -> 18.2, 192 x
-// 2048 -> 8192 11.0 -> 10.4, 2048 x 1024 -> 1024 8.3 -> 7.7; not for K = 512 (2048 -> 1024 6.1 -> 6.4, 4096 -> 512 6.6 -> 6.9),
-// and with an addend, whose rows wait for fewer wavefronts, not for K = 1024 (512 -> 4096 8.9 -> 9.4; K = 4096 21.6 -> 18.9).
-// Over 1850 sizes, every result type and post-op, 0.60 - 1.25 of the other shapes' time; the long ones lose what an XCD's tiles
-// share: unless the tiles divide by 8 (every XCD then has a contiguous range), it gets the tile rows of one residue modulo
-// gcd(tile rows, 8), and twice as many rows of half the height often have the larger divisor (3927 x 4480 -> 416, 31 against 62
-// tile rows: 19.7 -> 24.6).  Where it does not, or the tiles divide by 8, 0.60 - 1.08, 0.89 in the mean.
-// With clamped loads (other K) the same sizes are 0.62 - 1.25 and no such rule holds; the element-wise epilogue, whose registers go
-// to scratch in tiles above 64 x 64, takes 1.0 - 2.6 times as long: neither has this shape.
-inline int pick_tile_shape(int M, int N, int K, bool sum, bool wide_only, bool long_epilogue_short_k = false) {
+// Between one and two 64 x 64 tiles per CU, a K of 768 and more: 128 x 64 tiles, one per CU, four wavefronts of 32 x 64 stacked
+// along M and the deep ring.  A CU then loads 192 rows of operands per step instead of 256 for two small tiles, and half of the
+// device no longer does twice the work of the other half.  us, 64 x 64 (or 128 x 128) tiles -> these, fp32 results: 2048 x 2048 ->
+// 1024 12.6 -> 11.2, 4096 x 2048 -> 512 14.8 -> 10.7, 128 x 4096 -> 14336 20.6 -> 18.2, 192 x 2048 -> 8192 11.0 -> 10.4, 2048 x 1024
+// -> 1024 8.3 -> 7.7; not for K = 512 (2048 -> 1024 6.1 -> 6.4, 4096 -> 512 6.6 -> 6.9), and with an addend, whose rows wait for
+// fewer wavefronts, not for K = 1024 (512 -> 4096 8.9 -> 9.4; K = 4096 21.6 -> 18.9).
+// What they lose to is what an XCD's tiles share.  Unless the tiles divide by 8 (every XCD then has a contiguous range), it gets
+// the tile rows of one residue modulo gcd(tile rows, 8), and twice as many rows of half the height often have the larger divisor
+// (3927 x 4480 -> 416, 31 against 62 tile rows: 19.7 -> 24.6).  Their time over that of the other shapes, 2640 sizes of every
+// result type and post-op:
+//   K a multiple of 64   no divisor lost 0.60 - 1.08 (0.89);  one lost, N >= M and K from 1536 on 0.62 - 1.07 (0.87);  up to 128 rows,
+//                        one tile row either way 0.60 - 1.00 (0.80);  other sizes 0.66 - 1.25 (0.99): not there
+//   clamped loads        up to 128 rows 0.60 - 1.07 (0.82);  no divisor lost, M > 4 N and K from 1536 on 0.62 - 1.02 (0.87);  other
+//                        sizes 0.62 - 1.25 (0.96): not there
+//   element-wise         0.84 - 2.64, its registers go to scratch in tiles above 64 x 64: not there
+enum class Loads { kUniform, kClamped, kElementwise };
+inline bool tall_tiles(int M, int N, int K, Loads loads, bool sum) {
+  if (loads == Loads::kElementwise || K < (sum ? 2048 : 768)) return false;
+  const int m64 = (M + 63) / 64, m128 = (M + 127) / 128, n64 = (N + 63) / 64;
+  const int64_t t64 = static_cast<int64_t>(m64) * n64, t128x64 = static_cast<int64_t>(m128) * n64;
+  if (t64 <= 256 || t128x64 > 256) return false;
+  if (m128 == 1) return true;
+  auto residues = [](int rows) { return std::min(8, rows & -rows); };  // gcd(rows, 8)
+  const bool shared = t128x64 % 8 == 0 || residues(m128) >= residues(m64);
+  if (loads == Loads::kUniform) return shared || (N >= M && K >= 1536);
+  return shared && M > 4 * static_cast<int64_t>(N) && K >= 1536;
+}
+
+inline int pick_tile_shape(int M, int N, int K, bool sum, Loads loads, bool long_epilogue_short_k = false) {
   struct Shape { int bm, bn; double penalty; };
   static const Shape shapes[5] = {{256, 256, 1.0}, {256, 192, 1.03}, {256, 128, 1.08}, {128, 128, 1.2}, {64, 64, 1.8}};
   // itexhip_test_force_tile_shape forces a shape (tests exercise every shape on ragged problems with it)
   const int f = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED);
-  if (f >= (wide_only ? 3 : 0) && f < (wide_only ? 5 : 6)) return f;
+  const int first = loads == Loads::kUniform ? 0 : 3;  // the others have 128 x 128 and 64 x 64 (and 128 x 64)
+  if (f >= first && f < (loads == Loads::kElementwise ? 5 : 6)) return f;
   if (long_epilogue_short_k) {  // at least two 128 x 128 tiles per CU, at most 15 % of their area outside the output
     const int64_t t128 = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
     if (t128 >= 512 && t128 * (128 * 128) * 100 <= static_cast<int64_t>(M) * N * 115) return 3;
   }
-  if (!wide_only && K >= (sum ? 2048 : 768)) {
-    const int m64 = (M + 63) / 64, m128 = (M + 127) / 128, n64 = (N + 63) / 64;
-    const int64_t t64 = static_cast<int64_t>(m64) * n64, t128x64 = static_cast<int64_t>(m128) * n64;
-    auto residues = [](int rows) { return std::min(8, rows & -rows); };  // gcd(rows, 8)
-    if (t64 > 256 && t128x64 <= 256 && (t128x64 % 8 == 0 || residues(m128) >= residues(m64))) return 5;
-  }
+  if (tall_tiles(M, N, K, loads, sum)) return 5;
   int best = 3;
   double best_cost = 1e300;
-  for (int i = wide_only ? 3 : 0; i < 5; ++i) {
+  for (int i = first; i < 5; ++i) {
     const double tiles = static_cast<double>((M + shapes[i].bm - 1) / shapes[i].bm) * ((N + shapes[i].bn - 1) / shapes[i].bn);
     const double rounds = std::ceil(tiles / 256.0);
     const double cost = rounds * shapes[i].bm * shapes[i].bn * shapes[i].penalty;
@@ -767,7 +779,7 @@ inline int pick_tile_shape(int M, int N, int K, bool sum, bool wide_only, bool l
 template <int OUT_T, int ACT>
 int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N,
                         const EpilogueArgs& e, void* out, hipStream_t st) {
-  switch (pick_tile_shape(M, N, K, e.addend != nullptr, false, (ACT == 3 && K <= 1536) || K <= 256)) {
+  switch (pick_tile_shape(M, N, K, e.addend != nullptr, Loads::kUniform, (ACT == 3 && K <= 1536) || K <= 256)) {
     case 0: return launch_tile<256, 256, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 1: return launch_tile<256, 192, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 2: return launch_tile<256, 128, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
@@ -784,16 +796,19 @@ int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int
 template <int OUT_T, int ACT, bool ELEMENTWISE>
 int dispatch_clamped(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
                      void* out, hipStream_t st) {
-  if (pick_tile_shape(M, N, K, e.addend != nullptr, true) == 3)
-    return launch_tile<128, 128, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
+  const int shape = pick_tile_shape(M, N, K, e.addend != nullptr, ELEMENTWISE ? Loads::kElementwise : Loads::kClamped);
+  if (shape == 3) return launch_tile<128, 128, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
+  if constexpr (!ELEMENTWISE) {
+    if (shape == 5) return launch_tile<128, 64, 4, 1, OUT_T, ACT, false, false, false, 8>(a, amask, bp, M, K, N, e, out, st);
+  }
   return launch_tile<64, 64, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
 }
 
 // A bias vector, 16-byte aligned output rows and a post-op chain of the canonical form take the vector epilogue:
 // with K a multiple of 64 the specialised kernels (uniform activation addresses) in every tile shape; other K:
-// per-lane clamped activation loads, two tile shapes.
+// per-lane clamped activation loads, three tile shapes.
 // A missing bias, an addend, other chains or unaligned outputs (rare) go to the element-wise epilogue, a kernel of
-// its own in the same two shapes.
+// its own in 128 x 128 and 64 x 64 tiles.
 template <int OUT_T>
 int dispatch_tile(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int K, int N,
                   const EpilogueArgs& e_in, void* out, hipStream_t st) {

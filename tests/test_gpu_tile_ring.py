@@ -24,9 +24,9 @@ def test_k_loops_around_the_ring(hip, dev, shape, K):
             np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path=path), ref)
             if path == "fused" and M <= 128:
                 assert hip.last_kernel()[0] == "small_m"
-            elif shape == 5 and vector and K % 64 == 0:
+            elif shape == 5 and vector:
                 assert hip.last_kernel() == ("tile", 128, 64, 8)
-            else:   # K not a multiple of 64 and the element-wise epilogue have no 128 x 64 tiles
+            else:   # (the element-wise epilogue has no 128 x 64 tiles)
                 assert hip.last_kernel() == ("tile", 64, 64, 8 if K > 768 else 4)
 
 
@@ -46,7 +46,10 @@ def test_k_where_the_ring_of_64x64_tiles_changes(hip, dev, K):
                                         (1024, 896, 1024, (64, 64, 8)), (1025, 896, 1024, (128, 64, 8)),
                                         (2048, 768, 1024, (128, 64, 8)), (2049, 768, 1024, (128, 128, 4)),    # 256 and 272 of 128 x 64
                                         (2048, 752, 1024, (64, 64, 4)), (2048, 784, 1021, (64, 64, 4)),       # clamped loads, element-wise
-                                        (1920, 832, 544, (64, 64, 4)), (1840, 832, 544, (128, 64, 8))])       # 15 tile rows against 30 or 29
+                                        (1920, 832, 544, (64, 64, 4)), (1840, 832, 544, (128, 64, 8)),        # 15 tile rows against 30 or 29
+                                        (4224, 1552, 256, (64, 64, 4)), (4160, 1552, 256, (128, 64, 8)),      # clamped loads, 33 against 66 or 65
+                                        (384, 1536, 2880, (128, 64, 8)), (384, 1472, 2880, (64, 64, 4)),      # 3 against 6, N >= M
+                                        (120, 1040, 8224, (128, 64, 8))])                                      # one tile row
 def test_where_the_shape_changes(hip, dev, M, K, N, tile):
     layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
     _, xq, mn, mx = make_acts(M, K, seed=M + K)
