@@ -509,22 +509,35 @@ int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
     default: st__ = CALL(ITEXHIP_QUINT8); break;                              \
   }
 
-// Which packed kernel takes a call.  The small-M kernel (a strip of channels x 16 rows x all of K per workgroup)
-// streams the weight once per block of 16 rows; the tile kernel needs enough 64 x 64 tiles to fill the device.
-// Measured on 4096 x 14336 / 14336 x 4096 weights (us, small-M against tile kernel): M = 32: 15 / 17 against 23 / 67;
-// M = 64: 23 / 21 against 23 / 68; M = 128: 28 / 34 against 28 / 67; on a 1024 x 1024 weight the small-M kernel takes
-// 3.6 against 4.8 up to M = 128.  Both kernels accumulate exactly and share the epilogue: the same bytes either way.
+enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or the one for a short K; kAuto: as small_m says
+
+// Which packed kernel takes a call.  The small-M kernel (a strip of channels x 16 or 32 rows x all of K per workgroup)
+// streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  us, small-M against
+// tile kernel, weights out of L2: 4096 -> 14336 (224 tiles, from 65 rows on 448) M = 32 14.4 / 11.3, 64 21.3 / 11.8, 128 39.1 / 15.8;
+// 14336 -> 4096 (64 tiles, from 65 rows on 128) M = 32 16.6 / 27.4, 64 20.4 / 27.6, 128 35.2 / 28.1; 4096 -> 4096 M = 32 8.4 / 10.3, 64
+// 9.9 / 10.3; 1024 -> 1024 4.8 to 5.3 / 4.8 to 5.0.  Tile / small-M, time, with the vector epilogue (4600 sizes, median in brackets; 9 of 1400 that change sides take over 5 % longer):
+//   up to 128 tiles       0.6 - 1.8 (1.0): by weight, and by tiles that leave half of the CUs idle
+//   33 to 128 rows        129 - 160 tiles 0.73 - 1.13 (0.9), 161 - 256 0.66 - 1.09 (0.85), more 0.29 - 0.95 (0.6)
+//   17 to 32 rows         K < 256 0.57 - 1.0 (0.8);  256 to 767, 129 - 256 tiles 0.87 - 1.11 (0.97: not there), more 0.66 - 1.16
+//                         (0.85);  from 768 on, 129 - 256 tiles, one per CU on the deep ring, 0.75 - 1.10 (0.86), 257 - 512, a
+//                         second round for some of the CUs, 0.87 - 1.34 (1.1: not there)
+// With the element-wise epilogue, which the tile kernel has in a form of its own, 0.5 to 1.2 up to 128 tiles and 0.7 to 2.6 beyond:
+// the line by weight and tiles there.  Both kernels accumulate exactly and share the epilogue: the same bytes either way.
 constexpr int kSmallMaxRows = 128;
-static bool small_m(int64_t M, int64_t K, int64_t N) {
-  if (M <= 32) return true;
+static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int out_type, const void* out) {
+  if (M <= 16) return true;
   if (M > kSmallMaxRows) return false;
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (tiles > 128 && K >= 64 && (M > 32 || K < 256 || (K < 768) == (tiles > 256)) && e.addend == nullptr) {
+    CanonChain c;
+    const int act = canon_chain(e, &c);
+    const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
+    if (vector_epilogue(e, act, c, N, esz, out)) return false;
+  }
+  if (M <= 32) return true;
   if (K * N <= (8LL << 20)) return true;                       // the weight stays in L2: launch-bound either way
-  return ((M + 63) / 64) * ((N + 63) / 64) <= 128;             // the tile kernel would leave half of the CUs idle
+  return tiles <= 128;                                         // the tile kernel would leave half of the CUs idle
 }
-
-enum class Path { kTile, kSmallM, kAny };  // kAny: the tile kernel or the one for a short K
-
-static Path pick_path(int64_t M, int64_t K, int64_t N) { return small_m(M, K, N) ? Path::kSmallM : Path::kAny; }
 
 int launch_packed(Path path, const void* a, int a_type, const int8_t* packed_b, int64_t M, int64_t K, int64_t N,
                   const EpilogueArgs& e, int out_type, void* out, void* stream, const char* who) {
@@ -532,6 +545,7 @@ int launch_packed(Path path, const void* a, int a_type, const int8_t* packed_b, 
                   static_cast<long long>(K));
   ITEXHIP_REQUIRE(aligned(a, 16) && aligned(packed_b, 16), "%s: operands must be 16-byte aligned", who);
   ITEXHIP_REQUIRE(a_type != ITEXHIP_QUINT8 || e.colsum, "%s: quint8 activations need colsum", who);
+  if (path == Path::kAuto) path = small_m(M, K, N, e, out_type, out) ? Path::kSmallM : Path::kAny;
   ITEXHIP_REQUIRE(path != Path::kSmallM || M <= kSmallMaxRows, "%s: M must be <= %d", who, kSmallMaxRows);
   ITEXHIP_REQUIRE(M * K < (1LL << 31), "%s: activation matrix too large (M * K must be < 2^31)", who);
   const uint32_t a_xor = (a_type == ITEXHIP_QUINT8) ? 0x80808080u : 0u;
@@ -619,7 +633,7 @@ extern "C" int itexhip_qgemv(const void* a, int a_type, const int8_t* packed_b, 
 extern "C" int itexhip_qgemm(const void* a, int a_type, const int8_t* packed_b, const int32_t* colsum,
                              int64_t M, int64_t K, int64_t N, const float* scales, const float* bias,
                              const itexhip_epilogue* ep, int out_type, void* out, void* stream) {
-  return packed_path(pick_path(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(Path::kAuto, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemm");
 }
 
@@ -628,7 +642,7 @@ extern "C" int itexhip_qgemm_sum(const void* a, int a_type, const int8_t* packed
                                  const itexhip_epilogue* ep, const void* addend, int addend_type, int out_type, void* out,
                                  void* stream) {
   ITEXHIP_REQUIRE(addend != nullptr || M == 0 || N == 0, "itexhip_qgemm_sum: null addend");
-  return packed_path(pick_path(M, K, N), a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
+  return packed_path(Path::kAuto, a, a_type, packed_b, colsum, M, K, N, scales, bias, ep, out_type, out, stream,
                      "itexhip_qgemm_sum", addend, addend_type);
 }
 
@@ -786,7 +800,7 @@ int qmatmul_impl(const char* who, const itexhip_matmul_params* p, const void* a,
   e.range_a = range_a;
   e.addend = addend;
   e.addend_type = is_float16_type(p->t_out) ? p->t_out : ITEXHIP_FLOAT;  // the addend has the output's type
-  return launch_packed(pick_path(M, K, N), a, p->t_in, packed_b, M, K, N, e, p->t_out, out, stream, who);
+  return launch_packed(Path::kAuto, a, p->t_in, packed_b, M, K, N, e, p->t_out, out, stream, who);
 }
 }  // namespace
 

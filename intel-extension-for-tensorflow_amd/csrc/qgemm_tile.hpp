@@ -815,12 +815,7 @@ int dispatch_tile(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
   constexpr int esz = (OUT_T == ITEXHIP_QINT8 || OUT_T == ITEXHIP_QUINT8) ? 1 : is_float16_type(OUT_T) ? 2 : 4;
   EpilogueArgs e = e_in;
   const int act = canon_chain(e, &e.canon);
-  const bool has_sum = (e.canon.flags & (kChainSumFirst | kChainSumLast)) != 0;
-  const bool sum_ok = !has_sum || (e.addend != nullptr && (N & 3) == 0 &&
-                                   (reinterpret_cast<uintptr_t>(e.addend) &
-                                    (e.addend_type == ITEXHIP_FLOAT ? 15 : is_float16_type(e.addend_type) ? 7 : 3)) == 0);
-  const bool vec_epilogue = act >= 0 && sum_ok && (e.bias != nullptr || e.fused) &&
-                            (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ((static_cast<int64_t>(N) * esz) & 15) == 0;
+  const bool vec_epilogue = vector_epilogue(e, act, e.canon, N, esz, out);
   if (vec_epilogue && (K & 63) == 0) {
     if (act == 0) return dispatch_tile_shape<OUT_T, 0>(a, a_xor, bp, M, K, N, e, out, st);
     if (act == 1) return dispatch_tile_shape<OUT_T, 1>(a, a_xor, bp, M, K, N, e, out, st);

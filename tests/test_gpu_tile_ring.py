@@ -57,6 +57,21 @@ def test_where_the_shape_changes(hip, dev, M, K, N, tile):
     assert hip.last_kernel() == ("tile", *tile)
 
 
+@pytest.mark.parametrize("M,K,N,kernel", [(16, 64, 8256, "small_m"), (17, 64, 8192, "small_m"), (17, 64, 8256, "tile"),       # 128 and 129 tiles
+                                          (32, 48, 8256, "small_m"), (32, 64, 8257, "small_m"),                              # element-wise
+                                          (32, 240, 16384, "tile"), (32, 256, 16384, "small_m"), (32, 256, 16448, "tile"),   # 256 and 257
+                                          (32, 752, 16448, "tile"), (32, 768, 16448, "small_m"), (32, 768, 16384, "tile"),
+                                          (33, 64, 8192, "small_m"), (33, 64, 8256, "tile"), (65, 64, 4096, "small_m"),
+                                          (65, 64, 4160, "tile"), (128, 1040, 4160, "tile"), (128, 64, 4161, "small_m"),
+                                          (128, 2032, 4161, "tile"), (128, 2000, 4161, "small_m"),                           # element-wise, 8 MB
+                                          (129, 64, 64, "tile")])
+def test_line_between_the_small_m_and_the_tile_kernel(hip, dev, M, K, N, kernel):
+    layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
+    _, xq, mn, mx = make_acts(M, K, seed=M + K)
+    np.testing.assert_array_equal(layer.run(xq, V2_DEQ, mn, mx, path="fused"), layer.oracle(xq, V2_DEQ, mn, mx))
+    assert hip.last_kernel()[0] == kernel
+
+
 @pytest.mark.parametrize("K", [448, 2048])
 def test_addend_in_the_ring_kernels(hip, dev, K):
     """The float addend is staged through the transposition buffer, which lies in the ring."""
