@@ -515,7 +515,8 @@ enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or th
 // streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  us, small-M against
 // tile kernel, weights out of L2: 4096 -> 14336 (224 tiles, from 65 rows on 448) M = 32 14.4 / 11.3, 64 21.3 / 11.8, 128 39.1 / 15.8;
 // 14336 -> 4096 (64 tiles, from 65 rows on 128) M = 32 16.6 / 27.4, 64 20.4 / 27.6, 128 35.2 / 28.1; 4096 -> 4096 M = 32 8.4 / 10.3, 64
-// 9.9 / 10.3; 1024 -> 1024 4.8 to 5.3 / 4.8 to 5.0.  Tile / small-M, time, with the vector epilogue (4600 sizes, median in brackets; 9 of 1400 that change sides take over 5 % longer):
+// 9.9 / 10.3; 1024 -> 1024 4.8 to 5.3 / 4.8 to 5.0.  Tile / small-M, time, with the vector epilogue (4600 sizes, median in brackets;
+// of 1400 beyond the lines 9 take over 5 % longer than on the other kernel):
 //   up to 128 tiles       0.6 - 1.8 (1.0): by weight, and by tiles that leave half of the CUs idle
 //   33 to 128 rows        129 - 160 tiles 0.73 - 1.13 (0.9), 161 - 256 0.66 - 1.09 (0.85), more 0.29 - 0.95 (0.6)
 //   17 to 32 rows         K < 256 0.57 - 1.0 (0.8);  256 to 767, 129 - 256 tiles 0.87 - 1.11 (0.97: not there), more 0.66 - 1.16
