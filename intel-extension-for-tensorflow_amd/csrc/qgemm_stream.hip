@@ -430,7 +430,12 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   s.padded = cv && (cv->pad_top > 0 || cv->pad_left > 0 ||
                     (cv->out_h - 1) * cv->stride_h + (K / (cv->k_w * cv->in_c) - 1) * cv->dil_h >= cv->in_h ||
                     (cv->out_w - 1) * cv->stride_w + (cv->k_w - 1) * cv->dil_w >= cv->in_w);
-  const bool held_conv = cv && !sum && !s.padded && s.chunks <= 8;
+  // (Input and result past 384 MB: not held where three columns of wavefronts leave every fourth one idle, 0.67 - 1.02 of the time
+  // held (0.80 in the middle), nor with up to 4 chunks over more than 768 channels, 0.75 - 1.04 (0.86); below, and elsewhere,
+  // held chunks are 1.1 times as fast in the mean.  700 sizes.)
+  const int64_t conv_bytes = cv ? static_cast<int64_t>(M) * N + static_cast<int64_t>(M / cv->out_w / cv->out_h) * cv->in_h * cv->in_w * cv->in_c : 0;
+  const bool conv_early = conv_bytes > (384 << 20) && (cols == 3 || (s.chunks <= 4 && cols > 12));
+  const bool held_conv = cv && !sum && !s.padded && s.chunks <= 8 && !conv_early;
   const size_t lds = static_cast<size_t>(weight) + 12 * s.waves_n * kBlocks * 32 + (cv && !held_conv ? (K >> 4) * 8 : 0);
   const int per_cu = std::min<int>(4, 160 * 1024 / static_cast<int>(lds));  // 128 registers: four wavefronts per SIMD
   const int groups_n = (cols + s.waves_n - 1) / s.waves_n;
@@ -491,10 +496,29 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
       }
     }
   } else {
-    switch (s.chunks) {
-      HELD(false, false, none);
-      HELD_LONG(false, none);
-      default: STREAM(4, false, false, false, none);
+    // Held chunks need the caches here too: past `line` MB of activations and result the groups' earlier loads win, but not for
+    // one column of wavefronts, nor everywhere for a longer K.  Groups of 1, 2 or 4 over held chunks, time, 2800 sizes (the
+    // middle in brackets):
+    //   chunks 1 - 4   past 384 MB over 65 to 128 channels 0.74 - 1.01 (0.88), over 193 and more 0.68 - 1.16 (0.82: 94214 x 48 -> 7024
+    //                  275 -> 191 us); over 129 to 192, two workgroups abreast and a column of the second idle, 1.0 - 1.27 (1.17) up
+    //                  to 448 MB, 0.67 - 1.15 (0.94) past them; over more than 448 channels one chunk from 320 MB on 0.85 - 1.05
+    //                  (0.96), two chunks from 128 to 180 MB 0.82 - 0.95 (0.93) and up to 384 MB 0.75 - 1.1 (0.99)
+    //                  else, up to the lines, 0.81 - 1.4 (1.02)
+    //   chunks 5 - 8   up to 384 MB 0.69 - 1.40 (1.12);  past them over 65 to 192 channels 0.61 - 0.96 (0.89), more 0.79 - 1.53
+    //                  (1.05: not there)
+    const int64_t bytes = static_cast<int64_t>(M) * (K + N);
+    const int64_t line = s.chunks > 4 ? 384 : cols == 3 ? 448 : cols >= 8 && s.chunks == 1 ? 320 : cols >= 8 && s.chunks == 2 ? 128 : 384;
+    const bool early = bytes > (line << 20) && cols >= 2 && (s.chunks <= 4 || cols <= 3);
+    if (early && s.chunks == 1) {
+      STREAM(1, false, false, false, none);
+    } else if (early && s.chunks == 2) {
+      STREAM(2, false, false, false, none);
+    } else {
+      switch (early ? 0 : s.chunks) {
+        HELD(false, false, none);
+        HELD_LONG(false, none);
+        default: STREAM(4, false, false, false, none);
+      }
     }
   }
 #undef HELD_LONG

@@ -277,6 +277,43 @@ def test_residual_forms(hip, dev, M, K, N, group):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("image,K,N,form", [((3000007,), 16, 128, (1, False)), ((2000003,), 48, 272, (2, False)), ((2000003,), 112, 256, (4, False)),
+                                            ((1700003,), 144, 128, (4, False)), ((1700003,), 240, 160, (4, False)),
+                                            ((2200003,), 48, 128, (2, True)), ((2200003,), 48, 160, (2, True)),     # below the line, three columns
+                                            ((2300003,), 48, 160, (2, False)), ((1500007,), 16, 240, (1, True)),    # past theirs, four columns
+                                            ((260009,), 64, 480, (2, False)), ((260009,), 64, 448, (2, True)),      # two chunks over 8 columns, 7
+                                            ((700001,), 16, 480, (1, False)), ((700001,), 16, 448, (1, True)),      # one
+                                            ((1200007,), 176, 208, (6, True)), ((5000011,), 32, 64, (1, True)),     # a longer K, one column
+                                            ((1000, 53, 51), 80, 160, (4, False)), ((1000, 53, 51), 80, 128, (3, True)),
+                                            ((540, 29, 31), 16, 832, (4, False)), ((500, 29, 31), 16, 832, (1, True))])
+def test_results_past_the_caches(hip, dev, image, K, N, form):
+    """From 128 to 448 MB of activations and result on, some sizes take loads in groups instead of held chunks; a MatMul, or a 1 x 1
+    convolution."""
+    import torch
+    M = int(np.prod(image))
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.randint(0, 256, (M, K), dtype=torch.uint8, device=dev, generator=g)
+    w = torch.randint(-127, 128, (K, N), dtype=torch.int8, device=dev, generator=g)
+    packed = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev)
+    colsum = torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(w, False, K, N, packed, colsum)
+    ep = hip.Epilogue()
+    ep.n_scales = 1
+    scale, bias = torch.full((1,), 1e-3, device=dev), torch.full((N,), 20.0, device=dev)
+    v = (x.float() @ w.float()) * scale   # every sum below 2^24: exact in fp32 in any order
+    want = (v + bias).clamp(-128, 127).round().to(torch.int8)
+    out = torch.empty((M, N), dtype=torch.int8, device=dev)
+    if len(image) == 1:
+        hip.qgemm(x, hip.QUINT8, packed, colsum, M, K, N, scale, bias, ep, hip.QINT8, out)
+    else:
+        B, H, W = image
+        geometry = hip.ConvGeometry(B, H, W, K, 1, 1, H, W, 1, 1, 1, 1, 0, 0)
+        hip.qconv2d(x, hip.QUINT8, geometry, packed, colsum, N, scale, bias, ep, hip.QINT8, out)
+    assert hip.last_kernel() == ("short_k", *form)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 def awkward_floats(n):
     """n fp32 values: ties around every 8-bit result with their neighbours, infinities, NaN, denormals, random bit patterns."""
     f = np.float32
