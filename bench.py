@@ -752,7 +752,7 @@ def main():
     ap.add_argument("--only", type=str, default="", help="comma list of: headline, c1, prefill, bert, bmm, conv, gemv, elementwise, copy, power")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--tile-shape", type=int, default=-1,
-                    help="force the tile shape of the MatMul tile kernel (0..4) for this run; results do not depend on it")
+                    help="force the tile shape of the MatMul tile kernel (0..5) for this run; results do not depend on it")
     ap.add_argument("--cpu-rows", type=int, default=2048, help="rows of the headline workload the CPU oracle runs")
     args = ap.parse_args()
     if args.gpus != 1:

@@ -37,7 +37,7 @@ struct DirectArgs : DirectGeometry<FastDiv> {
 
 static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
 
-// Registers: 126 with 32 channels, four wavefronts per SIMD; 154 with 64 (72 of weight), three; 202 and 226 (144 of weight), two.
+// Registers: 126 with 32 channels, four wavefronts per SIMD; 152 with 64 (72 of weight), three; 200 and 224 (144 of weight), two.
 template <int OUT_T, int POST, int C32>
 __global__ __launch_bounds__(256, C32 == 1 ? 4 : C32 == 2 ? 3 : 2) void qconv_direct_kernel(
     const uint8_t* __restrict__ a, uint32_t amask, const uint8_t* __restrict__ bp, const DirectArgs s,

@@ -383,7 +383,8 @@ int try_stream(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K
   //   up to 256 deep all K chunks of a tile are held at once; without a residual, 0.75, 1, 1.5, 2.5 and 3.5 rounds (the ranges above were
   //   measured over more channels, and before the chunks were held):
   //     up to 64 channels     K = 128 1.0, 1.1 - 1.2, 1.3, 1.4, 1.4;  144, 160 1.2 - 1.3, 1.2, 1.35 - 1.45, 1.4 - 1.5, 1.5;  176 to 256
-  //                           1.05 - 1.15, 1.15 - 1.25, 1.25 - 1.35, 1.3 - 1.5, 1.3 - 1.5 (100352 x 256 -> 64 9.5 -> 8.1 us)
+  //                           1.05 - 1.15, 1.15 - 1.25, 1.25 - 1.35, 1.3 - 1.5, 1.3 - 1.5 (100352 x 256 -> 64 9.5 -> 8.1 us;
+  //                           only with both tensors in L2, launch after launch, one column is 0.9 - 1.2: 6.8 -> 7.9)
   //     65 to 1024            K = 128 -, -, 0.85 - 1.0, 0.9 - 1.1 (96 and 192 channels 1.3 - 1.7), 1.07 - 1.8, at 3 rounds 1.05 - 1.6;
   //                           K = 192 -, 0.8, 1.0 - 1.5 (768 at 1.75 0.9), 1.1 - 1.8, 1.3 - 1.9, at 2 rounds 1.1 - 1.5;  K = 256 0.9 up to 2, 1.0 at 3
   //   with a residual, small launches: 16 to 4096 channels at 0.15, 0.25, 0.5, 0.75, 1 and 1.25 rounds (a MatMul; 128 x 128 tiles start late there)

@@ -21,7 +21,7 @@ def golden():
 
 @pytest.fixture(scope="session")
 def hip():
-    """The ctypes binding of the native library; importing it fails if the library is not built."""
+    """The binding of the native library; importing it fails if the library is not built."""
     import __graft_entry__ as entry
     return entry.load_package().itexhip
 
