@@ -54,10 +54,10 @@ const char* itexhip_build_info(void);
  * input rows in LDS, for every later call of the process that the forced kernel can take; any of them also keeps a MatMul on
  * unpacked operands with its tile kernel.  -1 gives the choice back to the library.  Results do not depend on the shape. */
 void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape);
-/* Test hook: the kernel that the calling thread's last MatMul or Conv2D (not depthwise, not batched) was launched on, times
+/* Test hook: the kernel that the calling thread's last MatMul, BatchMatMul or Conv2D (not depthwise) was launched on, times
  * 10^8, plus what was chosen within it: 1 small M, 2 tiles (rows * 10^5 + columns * 100 + LDS stages), 3 short K (chunks per group
  * * 100 + 1 if all are held), 4 3 x 3 convolution (tiles per workgroup), 5 unpacked operands (groups per tile), 6 one output per
- * thread.  0: none yet. */
+ * thread, 7 bands of 16 rows (parts that a row is cut into), 8 BatchMatMul tiles (rows / 64 * 10 + columns / 64).  0: none yet. */
 int itexhip_test_last_kernel(void);
 
 /* ------------------------------------------------------------------------------------------
@@ -408,7 +408,8 @@ typedef struct {
 /* x, y, out: device memory.  Any M, K, N >= 0 and any alignment; 16-byte-aligned operands with K (and, for
  * the transposed layouts, the row length) a multiple of 16 take the vector-load path.  MFMA 32x32x32 i8,
  * tiles of 64 x 64 outputs per workgroup, 128 x 128 / 128 x 64 for calls with at least 1024 such tiles, aligned
- * operands and fused operands that do not depend on the row. */
+ * operands and fused operands that do not depend on the row; of those, and of products over many k, most run bands of 16 rows
+ * (MFMA 16x16x64). */
 int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* x, const int8_t* y, void* out, void* stream);
 
 /* ---- quantized Transpose ------------------------------------------------------------------------

@@ -22,7 +22,7 @@ void set_error(const char* fmt, ...);
 // Tile shape forced by itexhip_test_force_tile_shape (-1: chosen from the problem size); [0] MatMul, [1] Conv2D.
 extern int g_forced_tile_shape[2];
 // What itexhip_test_last_kernel reports: the kernel, and what is chosen within it
-enum LastKernel : int { kLastSmallM = 1, kLastTile, kLastShortK, kLastDirect, kLastUnpacked, kLastPerOutput };
+enum LastKernel : int { kLastSmallM = 1, kLastTile, kLastShortK, kLastDirect, kLastUnpacked, kLastPerOutput, kLastBands, kLastBmmTiles };
 void note_kernel(LastKernel kernel, int detail);
 
 inline int hip_fail(hipError_t e, const char* what) {

@@ -14,15 +14,10 @@
 #include <type_traits>
 #include <utility>
 
-#include "qbmm_reads.hpp"
-#include "qgemm_common.hpp"
+#include "qbmm_stage.hpp"
 
 namespace itexhip {
 namespace {
-
-constexpr int kTile = 64;          // output tile edge and k step
-constexpr int kLdsStride = 80;     // bytes per LDS row: 64 + 16, keeps the 16-byte fragment reads aligned
-constexpr int kBmmThreads = 256;
 
 struct BmmArgs {
   itexhip_bmm_params p;
@@ -34,126 +29,6 @@ struct BmmArgs {
   FastDiv by_dim[ITEXHIP_BMM_MAX_BATCH_DIMS];
   int rm, rn;        // the tile is (64 rm) x (64 rn)
 };
-
-// How an operand is read, each by itself.  kBytes: rows too short for a load (and an empty K): byte by byte, every read
-// guarded.  kAligned: aligned 16-byte (KCONT) / 4-byte (transposed) loads that never straddle a bound.  kAny: the same loads
-// at whatever byte address they fall on (the hardware takes unaligned vector loads); a load that would cross the end of its
-// row starts at the last place inside it and settle_tile shifts the bytes into place once they have arrived.  P.V over 197
-// tokens (384 products of 197 x 197 by 197 x 64 to bfloat16): 36.9 us with byte loads (16 per piece), 11.6 us with these.
-enum : int { kBytes = 0, kAligned = 1, kAny = 2 };
-typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
-typedef uint32_t u32_any __attribute__((aligned(1)));
-
-// One 64 (rows or columns of the output) x 64 (k) byte tile on its way into LDS, k-contiguous there.  The
-// global loads (fetch_tile) and the LDS stores (put_tile) are separate so that the next tile's loads are in
-// flight while the current one is multiplied.
-//   KCONT: the operand is stored [R, K] (k fastest);  else [K, R] (r fastest) and is transposed in put_tile.
-template <bool KCONT, int MODE>
-__device__ __forceinline__ void fetch_tile(const int8_t* __restrict__ g, int64_t R, int64_t K, int64_t r0, int64_t k0,
-                                           int t, uint32_t (&w)[4]) {
-  if constexpr (KCONT) {  // thread: row t / 4, 16 consecutive k
-    const int64_t row = r0 + (t >> 2), k = k0 + (t & 3) * 16;
-    if constexpr (MODE == kAny) {  // (results of rows past R are not stored)
-      const v4i v = *reinterpret_cast<const v4i_any*>(g + read_offset_k_fastest(row, k, R, K));
-      w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
-      return;
-    }
-    w[0] = w[1] = w[2] = w[3] = 0;
-    if (row >= R) return;
-    const int8_t* src = g + row * K + k;
-    if constexpr (MODE == kAligned) {
-      if (k < K) {
-        const v4i v = *reinterpret_cast<const v4i*>(src);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
-      }
-    } else {
-#pragma unroll
-      for (int b = 0; b < 16; ++b)
-        if (k + b < K) w[b >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(src[b])) << (8 * (b & 3));
-    }
-  } else {  // thread: 4 (k) x 4 (r) bytes; kb = t / 16 picks the k rows, cb = t % 16 the r columns; w[i] = k row i
-    const int kb = t >> 4, cb = t & 15;
-    const int64_t r = r0 + cb * 4;
-    if constexpr (MODE == kAny) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const u32_any*>(g + read_offset_r_fastest(r, k0 + kb * 4 + i, R, K));
-      return;
-    }
-    w[0] = w[1] = w[2] = w[3] = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t k = k0 + kb * 4 + i;
-      if (k >= K) continue;
-      const int8_t* src = g + k * R + r;
-      if constexpr (MODE == kAligned) {
-        if (r < R) w[i] = *reinterpret_cast<const uint32_t*>(src);
-      } else {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          if (r + b < R) w[i] |= static_cast<uint32_t>(static_cast<uint8_t>(src[b])) << (8 * b);
-      }
-    }
-  }
-}
-
-// kAny: what fetch_tile brought, with the bytes of a piece that crosses a bound moved into place and everything past K
-// cleared.  Only the last k tile and the last columns of the operand have such pieces.
-template <bool KCONT>
-__device__ __forceinline__ void settle_tile(int64_t R, int64_t K, int64_t r0, int64_t k0, int t, uint32_t (&w)[4]) {
-  if constexpr (KCONT) {
-    if (k0 + kTile <= K) return;
-    const int left = static_cast<int>(K - k0) - (t & 3) * 16;  // bytes of this piece inside the row
-    if (left >= 16) return;
-    const uint32_t shift = left > 0 ? 16 - left : 0;           // 1 .. 15
-    uint64_t lo = static_cast<uint64_t>(w[1]) << 32 | w[0], hi = static_cast<uint64_t>(w[3]) << 32 | w[2];
-    if (shift & 8) { lo = hi; hi = 0; }
-    const uint32_t bits = (shift & 7) * 8;
-    lo = lo >> bits | (hi << 1) << (63 - bits);
-    hi = hi >> bits;
-    if (left <= 0) lo = hi = 0;
-    w[0] = static_cast<uint32_t>(lo); w[1] = static_cast<uint32_t>(lo >> 32);
-    w[2] = static_cast<uint32_t>(hi); w[3] = static_cast<uint32_t>(hi >> 32);
-  } else {
-    if (r0 + kTile > R) {
-      const int over = static_cast<int>(r0 - (R - 4)) + (t & 15) * 4;  // how far the load was moved back
-      const uint32_t bits = over > 0 && over < 4 ? over * 8 : 0;       // past the last column: whatever came (not stored)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] >>= bits;
-    }
-    if (k0 + kTile > K) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (k0 + (t >> 4) * 4 + i >= K) w[i] = 0;
-    }
-  }
-}
-
-template <bool KCONT>
-__device__ __forceinline__ void put_tile(uint8_t* __restrict__ lds, int t, const uint32_t (&w)[4]) {
-  if constexpr (KCONT) {
-    *reinterpret_cast<v4i*>(lds + (t >> 2) * kLdsStride + (t & 3) * 16) =
-        v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
-  } else {
-    const int kb = t >> 4, cb = t & 15;
-    // 4 x 4 byte transpose in two rounds of byte permutes: byte j of the four k rows -> four consecutive k of column
-    // cb * 4 + j  (v_perm_b32 numbers the bytes of its second operand 0..3 and of its first 4..7)
-    const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);  // w0.b0 w1.b0 w0.b1 w1.b1
-    const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);  // w0.b2 w1.b2 w0.b3 w1.b3
-    const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-    const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-    const uint32_t v[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                           __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(lds + (cb * 4 + j) * kLdsStride + kb * 4) = v[j];
-  }
-}
-
-template <int T>
-__device__ __forceinline__ float widen(float v) { return v; }
-template <int T>
-__device__ __forceinline__ float widen(uint16_t bits) {
-  return T == ITEXHIP_BFLOAT16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
-}
 
 // Where one wavefront's 32 x 32 quadrant goes.  Everything that is the same for the whole wavefront is a
 // 64-bit base address; what differs between lanes and rows is a 32-bit byte offset (the host bounds N and
@@ -558,6 +433,11 @@ extern "C" int itexhip_qbatch_matmul(const itexhip_bmm_params* p, const int8_t* 
       a.rn = rn;
     }
   }
+  if (qbmm_band(a.p, batch, a.mode_x, a.mode_y, a.rm == 2, x, y, out, as_stream(stream))) {
+    ITEXHIP_CHECK_LAUNCH(who);
+    return ITEXHIP_OK;
+  }
+  note_kernel(kLastBmmTiles, a.rm * 10 + a.rn);
   a.tiles_m = static_cast<int>((p->M + a.rm * kTile - 1) / (a.rm * kTile));
   a.tiles_n = static_cast<int>((p->N + a.rn * kTile - 1) / (a.rn * kTile));
   const int64_t grid = batch * a.tiles_m * a.tiles_n;

@@ -161,10 +161,10 @@ def force_tile_shape(matmul=-1, conv=-1):
 
 
 def last_kernel():
-    """Test hook: the kernel of this thread's last MatMul or Conv2D and what was chosen within it, ("tile", 128, 64, 8) for tiles of
+    """Test hook: the kernel of this thread's last MatMul, BatchMatMul or Conv2D and what was chosen within it, ("tile", 128, 64, 8) for tiles of
     128 x 64 on eight LDS stages."""
     kernel, detail = divmod(int(_lib.itexhip_test_last_kernel()), 10 ** 8)
-    name = (None, "small_m", "tile", "short_k", "direct", "unpacked", "per_output")[kernel]
+    name = (None, "small_m", "tile", "short_k", "direct", "unpacked", "per_output", "bmm_bands", "bmm_tiles")[kernel]
     if name == "tile":
         return name, detail // 100000, detail // 100 % 1000, detail % 100
     return (name, detail // 100, bool(detail % 100)) if name == "short_k" else (name, detail)

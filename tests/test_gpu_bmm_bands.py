@@ -1,0 +1,77 @@
+"""The quantized BatchMatMul by bands of 16 output rows: remainders of a band, of a 16-column tile, of a k tile and of a 16-byte
+vector, rows cut into parts, operands and results at odd addresses, broadcast batches.  Against the CPU oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as orc
+from tests.test_gpu_bmm import check, run, to16
+
+pytestmark = pytest.mark.gpu
+ALL = [orc.FLOAT, orc.BFLOAT16, orc.HALF]
+
+
+def operands(torch, rng, N, t_out, B=1):
+    mul, add = np.float32([0.375]), rng.standard_normal((B, 1, 1, N)).astype(np.float32)
+    binary = [(orc.BIN_MUL, mul), (orc.BIN_ADD, add)]
+    return binary if t_out == orc.FLOAT else [(alg, to16(torch, v, t_out)) for alg, v in binary]
+
+
+# P.V over more than 192 k: one row to several bands per wavefront, the first and last columns of a tile, one to six k tiles
+@pytest.mark.parametrize("M", [1, 15, 17, 70, 200])
+@pytest.mark.parametrize("K,N", [(193, 16), (200, 17), (208, 20), (240, 31), (256, 48), (257, 50), (320, 64), (383, 64), (384, 20), (193, 79)])
+@pytest.mark.parametrize("t_out", ALL)
+def test_products_over_many_k(hip, dev, M, K, N, t_out):
+    import torch
+    rng = np.random.default_rng(M * 7 + K + N)
+    x, y = rng.integers(-128, 128, (2, 3, M, K)).astype(np.int8), rng.integers(-128, 128, (2, 3, K, N)).astype(np.int8)
+    check(hip, dev, x, y, t_out=t_out)
+    assert hip.last_kernel()[0] == "bmm_bands"
+    check(hip, dev, x, y, binary=operands(torch, rng, N, t_out, 2)[::-1], t_out=t_out, x_off=3, y_off=1)
+    check(hip, dev, x, y[:1], binary=operands(torch, rng, N, t_out)[1:], t_out=t_out, x_off=16)
+    assert hip.last_kernel()[0] == "bmm_bands"
+
+
+# Q.K^T of at least 1024 tiles of 128 rows: rows of whole vectors and others, one to eleven column tiles, D of one and two k tiles
+@pytest.mark.parametrize("M,K,N", [(65, 64, 16), (66, 16, 17), (80, 32, 20), (81, 64, 33), (65, 80, 47), (70, 48, 64), (129, 64, 99), (65, 32, 161)])
+@pytest.mark.parametrize("t_out", ALL)
+def test_many_matrices(hip, dev, M, K, N, t_out):
+    import torch
+    rng = np.random.default_rng(M * 7 + K + N)
+    x, y = rng.integers(-128, 128, (129, 8, M, K)).astype(np.int8), rng.integers(-128, 128, (129, 8, N, K)).astype(np.int8)
+    check(hip, dev, x, y, adj_y=True, binary=operands(torch, rng, N, t_out, 129), t_out=t_out)
+    assert hip.last_kernel() == ("bmm_bands", 1)
+    check(hip, dev, x, y[:, :1], adj_y=True, binary=operands(torch, rng, N, t_out)[:1] if N == 20 else (), t_out=t_out)
+    assert hip.last_kernel() == ("bmm_bands", 1)
+
+
+@pytest.mark.parametrize("K,N,parts,t_out", [(64, 288, 2, orc.HALF), (32, 320, 2, orc.BFLOAT16), (200, 160, 2, orc.FLOAT), (193, 144, 2, orc.FLOAT)])
+def test_rows_in_parts(hip, dev, K, N, parts, t_out):
+    """Rows of whole 64-byte pieces above 512 bytes, the last part shorter than the others."""
+    import torch
+    rng = np.random.default_rng(N)
+    adj_y = t_out != orc.FLOAT
+    x = rng.integers(-128, 128, ((400, 70, K) if adj_y else (9, 70, K))).astype(np.int8)
+    y = rng.integers(-128, 128, ((400, N, K) if adj_y else (9, K, N))).astype(np.int8)
+    check(hip, dev, x, y, adj_y=adj_y, binary=[(alg, v.reshape(v.shape[1:] if v.ndim > 1 else v.shape)) for alg, v in operands(torch, rng, N, t_out)],
+          t_out=t_out)
+    assert hip.last_kernel() == ("bmm_bands", parts)
+
+
+@pytest.mark.parametrize("t_out", ALL)
+@pytest.mark.parametrize("N", [64, 67])
+def test_results_at_any_address(hip, dev, t_out, N):
+    """A result that starts off a 16-byte boundary, with the elements around it untouched."""
+    import torch
+    rng = np.random.default_rng(N)
+    x, y = rng.integers(-128, 128, (5, 37, 200)).astype(np.int8), rng.integers(-128, 128, (5, 200, N)).astype(np.int8)
+    want = run(hip, dev, x, y, 2.0, 3.0, t_out=t_out)
+    xd, yd = torch.from_numpy(x).to(dev), torch.from_numpy(y).to(dev)
+    p, _ = hip.bmm_params(x.shape, y.shape, False, False, t_out, float(np.float32(6.0) / np.float32(127 * 127)))
+    dt = torch.float32 if t_out == orc.FLOAT else torch.int16
+    for off in range(1, 16 // dt.itemsize):
+        out = torch.full((want.size + 16,), -77, dtype=dt, device=dev)
+        hip.qbatch_matmul(p, xd, yd, out[off:])
+        assert hip.last_kernel()[0] == "bmm_bands"
+        got = out.cpu().numpy()
+        assert (got[:off] == -77).all() and (got[off + want.size:] == -77).all()
+        np.testing.assert_array_equal(got[off:off + want.size].view(want.dtype), want.ravel())
