@@ -312,7 +312,7 @@ __device__ __forceinline__ void block_minmax_commit(V mn, V mx, Less less, Commi
 
 __global__ __launch_bounds__(kThreads) void minmax_i32_flat_kernel(const i4* __restrict__ x, int64_t n4,
                                                                    const int32_t* __restrict__ tail,
-                                                                   int ntail, int32_t* mn_out,
+                                                                   int ntail, int alone, int32_t* mn_out,
                                                                    int32_t* mx_out) {
   int mn = INT32_MAX, mx = INT32_MIN;
   const int64_t round = static_cast<int64_t>(gridDim.x) * (kThreads * kReduceUnroll);
@@ -342,6 +342,11 @@ __global__ __launch_bounds__(kThreads) void minmax_i32_flat_kernel(const i4* __r
   block_minmax_commit(
       mn, mx, [](int p, int q) { return p < q; },
       [&](int lo, int hi) {
+        if (alone) {  // the only workgroup: nothing was initialised
+          *mn_out = lo;
+          *mx_out = hi;
+          return;
+        }
         atomicMin(mn_out, lo);
         atomicMax(mx_out, hi);
       });
@@ -355,12 +360,14 @@ __global__ __launch_bounds__(kThreads) void minmax_i32_flat_kernel(const i4* __r
 // stays in the last-level cache for the Requantize that follows (23.5 against 27 us for that one).
 // Up to kFewRows rows: one thread per channel (V = 1, one row at a time), whose result goes out as it is: the start and the
 // meeting in LDS cost more than the loads there.
+// `alone`: one workgroup has all rows of its channels and stores what it found; nothing is initialised, a launch less.
 constexpr int kRowUnroll = 8;
 constexpr int64_t kFewRows = 8;
 constexpr int64_t kChannelBlocks = 256;
+constexpr int64_t kFewRounds = 3;  // of 32 KB that one workgroup reads by itself rather than have its result initialised
 template <int V>
 __global__ __launch_bounds__(kThreads) void minmax_i32_channel_kernel(const int32_t* __restrict__ x, int64_t rows, int64_t depth,
-                                                                      int groups, int side, int64_t rows_per_block,
+                                                                      int groups, int side, int64_t rows_per_block, int alone,
                                                                       int32_t* mn_out, int32_t* mx_out) {
   __shared__ int smn[V == 4 ? 256 : kThreads], smx[V == 4 ? 256 : kThreads];
   // `side` rows are walked side by side
@@ -406,7 +413,10 @@ __global__ __launch_bounds__(kThreads) void minmax_i32_channel_kernel(const int3
       round([&](int u) { return p + (min(r + u * side, r1 - 1) - r) * depth; });
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      if (direct) {
+      if (direct && alone) {
+        mn_out[c + j] = mn[j];
+        mx_out[c + j] = mx[j];
+      } else if (direct) {
         atomicMin(&mn_out[c + j], mn[j]);
         atomicMax(&mx_out[c + j], mx[j]);
       } else {
@@ -419,8 +429,13 @@ __global__ __launch_bounds__(kThreads) void minmax_i32_channel_kernel(const int3
   __syncthreads();
   const int64_t ch = static_cast<int64_t>(blockIdx.y) * groups * V + threadIdx.x;
   if (static_cast<int>(threadIdx.x) < groups * V && ch < depth) {
-    atomicMin(&mn_out[ch], smn[threadIdx.x]);
-    atomicMax(&mx_out[ch], smx[threadIdx.x]);
+    if (alone) {
+      mn_out[ch] = smn[threadIdx.x];
+      mx_out[ch] = smx[threadIdx.x];
+    } else {
+      atomicMin(&mn_out[ch], smn[threadIdx.x]);
+      atomicMax(&mx_out[ch], smx[threadIdx.x]);
+    }
   }
 }
 
@@ -1123,7 +1138,8 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
   if (depth == 0) return ITEXHIP_OK;
   ITEXHIP_REQUIRE(min_out && max_out, "itexhip_minmax_i32_per_channel: null output");
   hipStream_t st = as_stream(stream);
-  fill_minmax_i32_kernel<<<blocks_for(depth, 256), 256, 0, st>>>(min_out, max_out, depth);
+  auto initialise = [&] { fill_minmax_i32_kernel<<<blocks_for(depth, 256), 256, 0, st>>>(min_out, max_out, depth); };
+  if (rows == 0) initialise();
   if (rows > 0) {
     ITEXHIP_REQUIRE(x, "itexhip_minmax_i32_per_channel: null input");
     if (depth == 1) {
@@ -1133,21 +1149,35 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       if (vec) {
         const unsigned grid = static_cast<unsigned>(std::min<int64_t>(
             kReduceBlocks, std::max<int64_t>(1, (n4 + kThreads * kReduceUnroll - 1) / (kThreads * kReduceUnroll))));
-        minmax_i32_flat_kernel<<<grid, kThreads, 0, st>>>(reinterpret_cast<const i4*>(x), n4,
-                                                          x + n4 * 4, ntail, min_out, max_out);
+        const bool alone = grid <= kFewRounds;
+        if (!alone) initialise();
+        minmax_i32_flat_kernel<<<alone ? 1 : grid, kThreads, 0, st>>>(reinterpret_cast<const i4*>(x), n4, x + n4 * 4, ntail, alone,
+                                                                      min_out, max_out);
       } else {
         const int64_t rpb = 4096;
+        initialise();
         dim3 grid(blocks_for(rows, rpb), 1);
-        minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, 1, 1, kThreads, rpb, min_out, max_out);
+        minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, 1, 1, kThreads, rpb, 0, min_out, max_out);
       }
     } else {
       const bool few = rows <= kFewRows, vec = !few && depth % 4 == 0 && aligned(x, 16);
       const int per = vec ? 4 : 1;
       int groups = static_cast<int>(std::min<int64_t>(depth / per, vec ? 64 : kThreads));
-      const int64_t col_blocks = (depth / per + groups - 1) / groups;
+      int64_t col_blocks = (depth / per + groups - 1) / groups;
       ITEXHIP_REQUIRE(col_blocks <= 65535, "itexhip_minmax_i32_per_channel: depth too large");
       // 16-byte loads: column blocks of one width (400000 x 260: 87 -> 73 us).  Single ints lose by it (100000 x 257: 28 -> 34).
       if (vec) groups = static_cast<int>((depth / per + col_blocks - 1) / col_blocks);
+      // Few rounds of loads: narrow column blocks (128 bytes, single ints 64) whose workgroup takes all rows; the launch that
+      // initialises costs more than what is lost in parallel reads (us, initialised / alone: 256 x 4096 5.0 / 3.0, 200 x 1000 5.0 / 3.3,
+      // 500 x 64 5.1 / 3.6, 1000 x 1000 5.0 / 5.6), and with a workgroup on every other CU some more rows (1024 x 4096 7.1 / 5.7,
+      // 4096 x 4096 14.5 / 13.6, 8192 x 4096 27 / 37: rows 16 KB apart meet in the same channels).
+      const int narrow = vec ? 8 : 16;
+      const int64_t narrow_blocks = (depth / per + narrow - 1) / narrow, rounds = (rows + kRowUnroll * (kThreads / narrow) - 1) / (kRowUnroll * (kThreads / narrow));
+      const bool alone = !few && narrow_blocks <= 65535 && (rounds <= 2 || (vec && narrow_blocks >= 128 && rounds <= 16));
+      if (alone) {
+        groups = static_cast<int>(std::min<int64_t>(narrow, depth / per));
+        col_blocks = narrow_blocks;
+      }
       const int side = few ? 1 : kThreads / groups;
       // At most one workgroup per CU (a row chunk costs an atomic pair per channel; 8192 x 4096: 256 workgroups 23.8 us, 384
       // and 512 26.8, 1024 29.8), each thread at least two rounds of loads.  Single ints have a quarter of the bytes in flight:
@@ -1155,11 +1185,12 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       // 28.6 / 28.4, 400000 x 257 222 / 126 / 83, 1000000 x 197 284 / 171 / 142).
       const int64_t budget = vec ? kChannelBlocks : std::min<int64_t>(4 * kChannelBlocks, std::max<int64_t>(kChannelBlocks, rows * depth >> 16));
       int64_t row_blocks = std::max<int64_t>(1, budget / col_blocks);
-      const int64_t rpb = std::max<int64_t>(2 * kRowUnroll * side, (rows + row_blocks - 1) / row_blocks);
-      row_blocks = (rows + rpb - 1) / rpb;
+      const int64_t rpb = alone ? rows : std::max<int64_t>(2 * kRowUnroll * side, (rows + row_blocks - 1) / row_blocks);
+      row_blocks = alone ? 1 : (rows + rpb - 1) / rpb;
+      if (row_blocks > 1) initialise();
       dim3 grid(static_cast<unsigned>(row_blocks), static_cast<unsigned>(col_blocks));
-      if (vec) minmax_i32_channel_kernel<4><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, min_out, max_out);
-      else minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, min_out, max_out);
+      if (vec) minmax_i32_channel_kernel<4><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, row_blocks == 1, min_out, max_out);
+      else minmax_i32_channel_kernel<1><<<grid, kThreads, 0, st>>>(x, rows, depth, groups, side, rpb, row_blocks == 1, min_out, max_out);
     }
   }
   ITEXHIP_CHECK_LAUNCH("itexhip_minmax_i32_per_channel");
