@@ -533,7 +533,7 @@ static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int 
     CanonChain c;
     const int act = canon_chain(e, &c);
     const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
-    if (vector_epilogue(e, act, c, N, esz, out)) return false;
+    if (vector_chain(e, act, c, N) && N * esz % 16 == 0 && aligned(out, 16)) return false;
   }
   if (M <= 32) return true;
   if (K * N <= (8LL << 20)) return true;                       // the weight stays in L2: launch-bound either way

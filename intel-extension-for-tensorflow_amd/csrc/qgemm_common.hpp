@@ -110,14 +110,14 @@ inline int canon_chain(const EpilogueArgs& e, CanonChain* c) {
   return (c->flags & (kChainGeluTanh | kChainGeluErf | kChainOther)) ? 3 : 2;
 }
 
-// Whether the tile kernel's vector epilogue can finish a call: a bias vector, 16-byte aligned output rows of `esz` bytes per
-// result, a chain of the canonical form (`act`, what canon_chain says) whose sum, if any, reads 4 aligned channels at a time.
-inline bool vector_epilogue(const EpilogueArgs& e, int act, const CanonChain& c, int64_t N, int esz, const void* out) {
+// Whether the tile kernel's vector epilogue can finish a call: a bias vector and a chain of the canonical form (`act`, what
+// canon_chain says) whose sum, if any, reads 4 aligned channels at a time.
+inline bool vector_chain(const EpilogueArgs& e, int act, const CanonChain& c, int64_t N) {
   const bool has_sum = (c.flags & (kChainSumFirst | kChainSumLast)) != 0;
   const bool sum_ok = !has_sum || (e.addend != nullptr && (N & 3) == 0 &&
                                    (reinterpret_cast<uintptr_t>(e.addend) &
                                     (e.addend_type == ITEXHIP_FLOAT ? 15 : is_float16_type(e.addend_type) ? 7 : 3)) == 0);
-  return act >= 0 && sum_ok && (e.bias != nullptr || e.fused) && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && ((N * esz) & 15) == 0;
+  return act >= 0 && sum_ok && (e.bias != nullptr || e.fused);
 }
 
 // Scale, bias and zero-point compensation of channel n (n < N), however the call supplied them, in two

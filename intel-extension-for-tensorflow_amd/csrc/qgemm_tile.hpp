@@ -387,6 +387,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
   static_assert(NW * WM * PITCH <= NSTAGE * STAGE_BYTES, "epilogue buffer must fit in the ring");
   if constexpr (!GENERAL) {
     uint8_t* ebuf = lds + wave * (WM * PITCH);
+    const bool whole_rows = ((static_cast<uint32_t>(N) * ESZ | static_cast<uint32_t>(reinterpret_cast<uintptr_t>(out))) & 15) == 0;
     const int f_row = lane / LPR, f_piece = lane % LPR;
     // Post-op chain in canonical form (ACT == 2: cheap activation, ACT == 3: GELU or another transcendental one; then
     // an optional linear map),
@@ -623,23 +624,52 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
       });
       // flush: lane -> (row, 16-byte piece); LDS operations of one wavefront complete in order
       const int n_col = n_base + (wn * TN + decltype(jb)::value * JB) * 32 + f_piece * (16 / ESZ);
+      auto flush = [&](auto store) {
 #pragma unroll
-      for (int pass = 0; pass < PASSES; ++pass) {
-        const int row = min(pass * RPP + f_row, WM - 1);
-        const v4i v = *reinterpret_cast<const v4i*>(ebuf + row * PITCH + f_piece * 16);
-        const int m = m_base + wm * WM + row;
-        const bool mine = (64 % LPR == 0 || f_row < RPP) && (WM % RPP == 0 || pass * RPP + f_row < WM);
-        if (mine && m < M && n_col < N) {  // N * ESZ is a multiple of 16, so a piece is entirely inside or outside
-          // Neither form leaves the output dirty in L2 until the flush at the end of the kernel.  32-bit outputs (the
-          // store-bound epilogues: BERT-base 768 -> 3072 + ReLU 19.5 -> 17.6 us) go out as system-scope stores, written
-          // through; 8- and 16-bit outputs, and the GELU epilogue whose stores trickle out between long runs of
-          // arithmetic, measured 1-8 % faster as streaming (nontemporal) stores.
-          uint8_t* const dst = reinterpret_cast<uint8_t*>(out) + (static_cast<int64_t>(m) * N + n_col) * ESZ;
-          // (the s_nop: a store of more than 8 bytes reads its data registers for a cycle or two after it issues, and the
-          // compiler, which cannot see a store inside the assembly, may let the next vector instruction overwrite them)
+        for (int pass = 0; pass < PASSES; ++pass) {
+          const int row = min(pass * RPP + f_row, WM - 1);
+          const uint8_t* const src = ebuf + row * PITCH + f_piece * 16;
+          const v4i v = *reinterpret_cast<const v4i*>(src);
+          const int m = m_base + wm * WM + row;
+          const bool mine = (64 % LPR == 0 || f_row < RPP) && (WM % RPP == 0 || pass * RPP + f_row < WM);
+          if (mine && m < M && n_col < N) store(reinterpret_cast<uint8_t*>(out) + (static_cast<int64_t>(m) * N + n_col) * ESZ, v, src);
+        }
+      };
+      // Neither form leaves the output dirty in L2 until the flush at the end of the kernel.  32-bit outputs (the
+      // store-bound epilogues: BERT-base 768 -> 3072 + ReLU 19.5 -> 17.6 us) go out as system-scope stores, written
+      // through; 8- and 16-bit outputs, and the GELU epilogue whose stores trickle out between long runs of
+      // arithmetic, measured 1-8 % faster as streaming (nontemporal) stores.
+      // (the s_nop: a store of more than 8 bytes reads its data registers for a cycle or two after it issues, and the
+      // compiler, which cannot see a store inside the assembly, may let the next vector instruction overwrite them)
+      if (CONV || whole_rows) {  // N * ESZ is a multiple of 16, so a piece is entirely inside or outside
+        flush([&](uint8_t* dst, const v4i& v, const uint8_t*) {
           if constexpr (ESZ == 4 && ACT != 3) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
           else __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(dst));
-        }
+        });
+      } else {
+        // Rows of any length and address: pieces wherever they fall (plain stores, L2 puts the lines together; streaming ones 1 - 15 %
+        // slower), the last one of a row in parts.  As the element-wise epilogue, a store per value, such rows took (8-bit, us,
+        // element-wise / this): 1034 x 144 -> 1976 45 / 6.1, 592 x 1024 -> 3747 51 / 10.4, 1000 x 512 -> 1004 8.1 / 4.5.
+        const int bytes = (N - n_col) * ESZ;
+        flush([&](uint8_t* dst, const v4i& v, const uint8_t* src) {
+          typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+          typedef uint32_t u32_any __attribute__((aligned(1)));
+          if (bytes >= 16) {
+            if constexpr (ESZ == 4 && ACT != 3) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
+            else *reinterpret_cast<v4i_any*>(dst) = v;
+            return;
+          }
+          int done = 0;
+#pragma unroll 1
+          for (; done + 4 <= bytes; done += 4) *reinterpret_cast<u32_any*>(dst + done) = *reinterpret_cast<const uint32_t*>(src + done);
+          if constexpr (ESZ < 4) {
+#pragma unroll 1
+            for (; done < bytes; done += ESZ) {
+              if constexpr (ESZ == 2) *reinterpret_cast<uint16_t*>(dst + done) = *reinterpret_cast<const uint16_t*>(src + done);
+              else dst[done] = src[done];
+            }
+          }
+        });
       }
     });
   } else {
@@ -754,18 +784,19 @@ inline bool tall_tiles(int M, int N, int K, Loads loads, bool sum) {
   return shared && M > 4 * static_cast<int64_t>(N) && K >= 1536;
 }
 
-inline int pick_tile_shape(int M, int N, int K, bool sum, Loads loads, bool long_epilogue_short_k = false) {
+// `whole_rows`: of 16-byte vectors; other rows leave 128 x 64 tiles alone.
+inline int pick_tile_shape(int M, int N, int K, bool sum, Loads loads, bool whole_rows, bool long_epilogue_short_k = false) {
   struct Shape { int bm, bn; double penalty; };
   static const Shape shapes[5] = {{256, 256, 1.0}, {256, 192, 1.03}, {256, 128, 1.08}, {128, 128, 1.2}, {64, 64, 1.8}};
   // itexhip_test_force_tile_shape forces a shape (tests exercise every shape on ragged problems with it)
   const int f = __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED);
   const int first = loads == Loads::kUniform ? 0 : 3;  // the others have 128 x 128 and 64 x 64 (and 128 x 64)
-  if (f >= first && f < (loads == Loads::kElementwise ? 5 : 6)) return f;
+  if (f >= first && f < (loads == Loads::kElementwise || !whole_rows ? 5 : 6)) return f;
   if (long_epilogue_short_k) {  // at least two 128 x 128 tiles per CU, at most 15 % of their area outside the output
     const int64_t t128 = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
     if (t128 >= 512 && t128 * (128 * 128) * 100 <= static_cast<int64_t>(M) * N * 115) return 3;
   }
-  if (tall_tiles(M, N, K, loads, sum)) return 5;
+  if (whole_rows && tall_tiles(M, N, K, loads, sum)) return 5;
   int best = 3;
   double best_cost = 1e300;
   for (int i = first; i < 5; ++i) {
@@ -777,10 +808,16 @@ inline int pick_tile_shape(int M, int N, int K, bool sum, Loads loads, bool long
   return best;
 }
 
+template <int OUT_T>
+bool whole_rows(int N, const void* out) {
+  constexpr int esz = (OUT_T == ITEXHIP_QINT8 || OUT_T == ITEXHIP_QUINT8) ? 1 : is_float16_type(OUT_T) ? 2 : 4;
+  return ((static_cast<uint32_t>(N) * esz | static_cast<uint32_t>(reinterpret_cast<uintptr_t>(out))) & 15) == 0;
+}
+
 template <int OUT_T, int ACT>
 int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N,
                         const EpilogueArgs& e, void* out, hipStream_t st) {
-  switch (pick_tile_shape(M, N, K, e.addend != nullptr, Loads::kUniform, (ACT == 3 && K <= 1536) || K <= 256)) {
+  switch (pick_tile_shape(M, N, K, e.addend != nullptr, Loads::kUniform, whole_rows<OUT_T>(N, out), (ACT == 3 && K <= 1536) || K <= 256)) {
     case 0: return launch_tile<256, 256, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 1: return launch_tile<256, 192, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
     case 2: return launch_tile<256, 128, 2, 2, OUT_T, ACT, true>(a, amask, bp, M, K, N, e, out, st);
@@ -797,7 +834,7 @@ int dispatch_tile_shape(const uint8_t* a, uint32_t amask, const uint8_t* bp, int
 template <int OUT_T, int ACT, bool ELEMENTWISE>
 int dispatch_clamped(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M, int K, int N, const EpilogueArgs& e,
                      void* out, hipStream_t st) {
-  const int shape = pick_tile_shape(M, N, K, e.addend != nullptr, ELEMENTWISE ? Loads::kElementwise : Loads::kClamped);
+  const int shape = pick_tile_shape(M, N, K, e.addend != nullptr, ELEMENTWISE ? Loads::kElementwise : Loads::kClamped, whole_rows<OUT_T>(N, out));
   if (shape == 3) return launch_tile<128, 128, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
   if constexpr (!ELEMENTWISE) {
     if (shape == 5) return launch_tile<128, 64, 4, 1, OUT_T, ACT, false, false, false, 8>(a, amask, bp, M, K, N, e, out, st);
@@ -805,27 +842,24 @@ int dispatch_clamped(const uint8_t* a, uint32_t amask, const uint8_t* bp, int M,
   return launch_tile<64, 64, 2, 2, OUT_T, ACT, false, false, ELEMENTWISE>(a, amask, bp, M, K, N, e, out, st);
 }
 
-// A bias vector, 16-byte aligned output rows and a post-op chain of the canonical form take the vector epilogue:
-// with K a multiple of 64 the specialised kernels (uniform activation addresses) in every tile shape; other K:
-// per-lane clamped activation loads, three tile shapes.
-// A missing bias, an addend, other chains or unaligned outputs (rare) go to the element-wise epilogue, a kernel of
-// its own in 128 x 128 and 64 x 64 tiles.
+// A bias vector and a post-op chain of the canonical form take the vector epilogue: with K a multiple of 64 the specialised
+// kernels (uniform activation addresses) in every tile shape; other K: per-lane clamped activation loads, three tile shapes.
+// A missing bias, a sum that no vector load reads and other chains (rare) go to the element-wise epilogue, a kernel of its own in
+// 128 x 128 and 64 x 64 tiles.
 template <int OUT_T>
 int dispatch_tile(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int K, int N,
                   const EpilogueArgs& e_in, void* out, hipStream_t st) {
-  constexpr int esz = (OUT_T == ITEXHIP_QINT8 || OUT_T == ITEXHIP_QUINT8) ? 1 : is_float16_type(OUT_T) ? 2 : 4;
   EpilogueArgs e = e_in;
   const int act = canon_chain(e, &e.canon);
-  const bool vec_epilogue = vector_epilogue(e, act, e.canon, N, esz, out);
-  if (vec_epilogue && (K & 63) == 0) {
+  if (!vector_chain(e, act, e.canon, N)) return dispatch_clamped<OUT_T, 2, true>(a, a_xor, bp, M, K, N, e, out, st);
+  if ((K & 63) == 0) {
     if (act == 0) return dispatch_tile_shape<OUT_T, 0>(a, a_xor, bp, M, K, N, e, out, st);
     if (act == 1) return dispatch_tile_shape<OUT_T, 1>(a, a_xor, bp, M, K, N, e, out, st);
     if (act == 2) return dispatch_tile_shape<OUT_T, 2>(a, a_xor, bp, M, K, N, e, out, st);
     return dispatch_tile_shape<OUT_T, 3>(a, a_xor, bp, M, K, N, e, out, st);
   }
-  if (vec_epilogue && act == 3) return dispatch_clamped<OUT_T, 3, false>(a, a_xor, bp, M, K, N, e, out, st);
-  if (vec_epilogue) return dispatch_clamped<OUT_T, 2, false>(a, a_xor, bp, M, K, N, e, out, st);  // covers "none" and "ReLU" too
-  return dispatch_clamped<OUT_T, 2, true>(a, a_xor, bp, M, K, N, e, out, st);
+  if (act == 3) return dispatch_clamped<OUT_T, 3, false>(a, a_xor, bp, M, K, N, e, out, st);
+  return dispatch_clamped<OUT_T, 2, false>(a, a_xor, bp, M, K, N, e, out, st);  // covers "none" and "ReLU" too
 }
 
 // Implicit GEMM of a Conv2D: `x` is the NHWC input, M = batch * out_h * out_w, K = k_h * k_w * in_c.  Run-time post-op

@@ -1,0 +1,44 @@
+"""The tile kernel's vector epilogue on output rows that are no whole 16-byte vectors or start off a 16-byte boundary: every
+result type and tile shape, the last piece of a row in parts.  Against int64 sums and the epilogue's separately rounded fp32
+steps, bit for bit, with the bytes around the result untouched."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def convert(torch, hip, v, T):
+    if T == hip.FLOAT:
+        return v.view(np.uint8)
+    if T in (hip.BFLOAT16, hip.HALF):
+        return torch.from_numpy(v).to(torch.bfloat16 if T == hip.BFLOAT16 else torch.float16).view(torch.uint8).numpy()
+    lo, hi, dt = {hip.QINT8: (-128, 127, np.int8), hip.QUINT8: (0, 255, np.uint8)}[T]
+    return np.rint(np.clip(v, np.float32(lo), np.float32(hi))).astype(dt).view(np.uint8)
+
+
+@pytest.mark.parametrize("M,K,N", [(130, 64, 1), (129, 48, 15), (200, 64, 17), (257, 112, 63), (131, 192, 66), (300, 80, 100), (260, 128, 391), (513, 64, 259)])
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 4, 5])
+def test_rows_of_any_length(hip, dev, M, K, N, shape):
+    import torch
+    f = np.float32
+    rng = np.random.default_rng(M + K + N)
+    x, w = rng.integers(0, 256, (M, K)).astype(np.uint8), rng.integers(-128, 128, (K, N)).astype(np.int8)
+    scale, bias = (rng.random(N).astype(f) + f(0.5)) * f(0.003), (rng.standard_normal(N) * 9).astype(f)
+    v0 = (x.astype(np.int64) @ w.astype(np.int64)).astype(f) * scale + bias
+    packed, colsum = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev), torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(torch.from_numpy(w).to(dev), False, K, N, packed, colsum)
+    d = [torch.from_numpy(a).to(dev) for a in (x, scale, bias)]
+    hip.force_tile_shape(matmul=shape)
+    for T, esz in ((hip.FLOAT, 4), (hip.BFLOAT16, 2), (hip.HALF, 2), (hip.QINT8, 1), (hip.QUINT8, 1)):
+        for elts, v in (((), v0), (((hip.ELT_RELU, 0.0, 0.0),), np.maximum(v0, f(0))), (((hip.ELT_CLIP, -7.5, 50.0),), np.clip(v0, f(-7.5), f(50)))):
+            ep = hip.Epilogue()
+            ep.n_scales, ep.n_eltwise = N, len(elts)
+            for i, e in enumerate(elts):
+                ep.elt[i].alg, ep.elt[i].alpha, ep.elt[i].beta = e
+            off = (M + len(elts)) % 5 * esz
+            out = torch.full((M * N * esz + 64,), 0x5a, dtype=torch.uint8, device=dev)
+            hip.qgemm_tile(d[0], hip.QUINT8, packed, colsum, M, K, N, d[1], d[2], ep, T, out[off:])
+            assert hip.last_kernel()[0] == "tile"
+            got = out.cpu().numpy()
+            assert (got[:off] == 0x5a).all() and (got[off + M * N * esz:] == 0x5a).all()
+            np.testing.assert_array_equal(got[off:off + M * N * esz], convert(torch, hip, np.ascontiguousarray(v), T).ravel())
