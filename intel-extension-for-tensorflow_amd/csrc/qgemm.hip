@@ -478,22 +478,24 @@ int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
                   const EpilogueArgs& e, void* out, hipStream_t st) {
   const int KC = 2 * ((K + 63) / 64), KP = KC / 2;
   // 32-channel strips when they give every CU a workgroup, else 16-channel strips; a strip is finished by one
-  // wavefront per 16-channel tile, so never fewer wavefronts than that.  Wavefronts per strip, at most 8, measured on
-  // 4096 x 14336 and 14336 x 4096 with every count from 2 to 8, both strip widths and both batch sizes: up to 4 rows
-  // about 8 chunk pairs (four batches of 2) each (4096 -> 14336 at M = 1 / 4: 11.3 -> 10.95 us with 8 instead of 4);
-  // 5 to 16 rows about 16 pairs each (4096 -> 14336 at M = 16: 4 wavefronts 11.7 us, 8 over 11.8 us; 14336 -> 4096: 8
-  // wavefronts 12.7 us, 4 wavefronts 15.2 us); prefer a count that divides K into whole batches.
+  // wavefront per 16-channel tile, so never fewer wavefronts than that.  Wavefronts per strip, at most 8: about 8 chunk pairs each,
+  // so that a launch that does not fill the device is a short chain of round trips (500 sizes of up to 128 rows, K and N up to
+  // 14336, every count; against 16 pairs each for 5 to 16 rows and 32 beyond: 0.95 and 0.89 of the time, 1.04 at most: 128 x 1024 -> 1024
+  // 5.2 -> 4.5 us, 16 x 1024 -> 1024 5.8 -> 4.4, 48 x 2992 -> 333 10.8 -> 6.3, 33 x 4096 -> 4096 10.9 -> 8.4); prefer a count that
+  // divides K into whole batches.
   // (blocks of 32 rows count as workgroups of their own: 14336 -> 4096 at M = 64 28.1 -> 20.0 us with 32-channel strips,
   // 256 workgroups instead of 512 that read the activations twice as often)
   const int row_blocks = M > 16 ? (M + 31) / 32 : 1;
   const int nt = ((N + 31) / 32) * row_blocks >= 256 ? 2 : 1;
-  const int per_wave = M <= 4 ? 8 : 16;
+  // From 65 rows on with more than one workgroup per CU: half as many wavefronts with runs four times as long, fewer rings, so that
+  // workgroups share a CU (8 pairs each 1.02 of that, 1.18 at most).
+  const int64_t wgs = static_cast<int64_t>((N + 16 * nt - 1) / (16 * nt)) * row_blocks;
+  const bool paired = M > 64 && wgs > 256;
+  const int per_wave = paired ? 16 : 8;
   int waves = std::max(nt, std::min(8, (KP + per_wave - 1) / per_wave));
   for (int w = waves; w >= std::max(nt, waves / 2 + 1); --w)
     if (KP % (gemv_batch(M) * w) == 0) { waves = w; break; }
-  // Blocks of 32 rows (batches of 4): half as many wavefronts with runs twice as long, fewer partial tiles to reduce
-  // and fewer rings.
-  if (M > 16) waves = std::max(nt, waves / 2);
+  if (paired) waves = std::max(nt, waves / 2);
   const int cnt = (KP + waves - 1) / waves;
   if (nt == 2) return launch_gemv<2, OUT_T>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st);
   return launch_gemv<1, OUT_T>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st);
@@ -512,28 +514,40 @@ int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
 enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or the one for a short K; kAuto: as small_m says
 
 // Which packed kernel takes a call.  The small-M kernel (a strip of channels x 16 or 32 rows x all of K per workgroup)
-// streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  us, small-M against
-// tile kernel, weights out of L2: 4096 -> 14336 (224 tiles, from 65 rows on 448) M = 32 14.4 / 11.3, 64 21.3 / 11.8, 128 39.1 / 15.8;
-// 14336 -> 4096 (64 tiles, from 65 rows on 128) M = 32 16.6 / 27.4, 64 20.4 / 27.6, 128 35.2 / 28.1; 4096 -> 4096 M = 32 8.4 / 10.3, 64
-// 9.9 / 10.3; 1024 -> 1024 4.8 to 5.3 / 4.8 to 5.0.  Tile / small-M, time, with the vector epilogue (4600 sizes, median in brackets;
-// of 1400 beyond the lines 9 take over 5 % longer than on the other kernel):
-//   up to 128 tiles       0.6 - 1.8 (1.0): by weight, and by tiles that leave half of the CUs idle
-//   33 to 128 rows        129 - 160 tiles 0.73 - 1.13 (0.9), 161 - 256 0.66 - 1.09 (0.85), more 0.29 - 0.95 (0.6)
-//   17 to 32 rows         K < 256 0.57 - 1.0 (0.8);  256 to 767, 129 - 256 tiles 0.87 - 1.11 (0.97: not there), more 0.66 - 1.16
-//                         (0.85);  from 768 on, 129 - 256 tiles, one per CU on the deep ring, 0.75 - 1.10 (0.86), 257 - 512, a
-//                         second round for some of the CUs, 0.87 - 1.34 (1.1: not there)
-// With the element-wise epilogue, which the tile kernel has in a form of its own, 0.5 to 1.2 up to 128 tiles and 0.7 to 2.6 beyond:
-// the line by weight and tiles there.  Both kernels accumulate exactly and share the epilogue: the same bytes either way.
-constexpr int kSmallMaxRows = 128;
+// streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  Small-M / tile kernel, time,
+// with a chain that the tile kernel's vector epilogue finishes (2500 sizes of up to 2048 rows, K up to 4096, 64 x 64 tiles; 400 of them with
+// operands out of the caches, which changes no line):
+//   33 to 128 rows        up to 16 tiles 0.5 - 1.27 (K <= 256 1.03, 257 - 1024 0.9, more 0.69), 17 - 64 0.53 - 1.3 (0.96);  65 - 128 tiles
+//                         K <= 1536, or up to 64 rows, 0.94 - 1.66 (1.2: not there), else 0.79 - 1.4 (1.05), more tiles 1.0 - 2.4.  Rows that
+//                         are no whole 16-byte vectors differ by 0.1 at most; with a K of one step, or K > 1536 and few more than
+//                         128 tiles, either kernel does.
+//   129 to 512 rows       up to 16 tiles K <= 256 0.78 - 1.27 (1.02: not there), 257 - 512 0.92, 513 - 1024 0.82, more 0.66;  17 - 32 tiles
+//                         K > 512 0.58 - 1.03 (0.78);  33 - 64 tiles 0.7 - 1.3 (1.0: not there), more 1.0 - 4
+//   513 to 2048 rows      up to 16 tiles K > 512 0.66 - 0.94 (0.79);  17 - 32 0.73 - 1.6 (1.05: not there)
+//   17 to 32 rows         (4600 sizes before that) K < 256 and over 128 tiles 1.0 - 1.7;  256 to 767, 129 - 256 tiles 0.9 - 1.15 (0.97:
+//                         not there), more 0.86 - 1.5;  from 768 on, 129 - 256 tiles, one per CU on the deep ring, 0.9 - 1.33, 257 - 512, a
+//                         second round for some of the CUs, 0.75 - 1.15 (not there)
+// With the element-wise epilogue, which the tile kernel has in a form of its own, 0.43 - 0.9 up to 128 tiles and K up to 2048.
+// Both kernels accumulate exactly and share the epilogue: the same bytes either way.
+constexpr int kSmallMaxRows = 128;       // that itexhip_qgemv takes
+constexpr int kSmallMaxAutoRows = 2048;
 static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int out_type, const void* out) {
   if (M <= 16) return true;
-  if (M > kSmallMaxRows) return false;
+  if (M > kSmallMaxAutoRows) return false;
+  if (M > kSmallMaxRows && __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0) return false;
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (tiles > 128 && K >= 64 && (M > 32 || K < 256 || (K < 768) == (tiles > 256)) && e.addend == nullptr) {
-    CanonChain c;
-    const int act = canon_chain(e, &c);
+  CanonChain c;
+  const int act = canon_chain(e, &c);
+  if (e.addend == nullptr && vector_chain(e, act, c, N)) {
     const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
-    if (vector_chain(e, act, c, N) && N * esz % 16 == 0 && aligned(out, 16)) return false;
+    const bool whole_rows = (N * esz) % 16 == 0 && aligned(out, 16);
+    if (M > 512) return tiles <= 16 && K > 512;
+    if (M > kSmallMaxRows) return tiles <= 16 ? K > 256 : tiles <= 32 && K > 512;
+    if (M > 32 && K >= 128 && tiles > 64 && (M <= 64 || K <= 1536)) return false;
+    if (whole_rows ? K >= 64 && tiles > 128 : K >= 128 && tiles > 144)
+      if (M > 32 || K < 256 || (K < 768) == (tiles > 256)) return false;
+  } else if (M > kSmallMaxRows) {
+    return e.addend == nullptr && tiles <= 128 && K <= 2048;
   }
   if (M <= 32) return true;
   if (K * N <= (8LL << 20)) return true;                       // the weight stays in L2: launch-bound either way
@@ -546,8 +560,8 @@ int launch_packed(Path path, const void* a, int a_type, const int8_t* packed_b, 
                   static_cast<long long>(K));
   ITEXHIP_REQUIRE(aligned(a, 16) && aligned(packed_b, 16), "%s: operands must be 16-byte aligned", who);
   ITEXHIP_REQUIRE(a_type != ITEXHIP_QUINT8 || e.colsum, "%s: quint8 activations need colsum", who);
-  if (path == Path::kAuto) path = small_m(M, K, N, e, out_type, out) ? Path::kSmallM : Path::kAny;
   ITEXHIP_REQUIRE(path != Path::kSmallM || M <= kSmallMaxRows, "%s: M must be <= %d", who, kSmallMaxRows);
+  if (path == Path::kAuto) path = small_m(M, K, N, e, out_type, out) ? Path::kSmallM : Path::kAny;
   ITEXHIP_REQUIRE(M * K < (1LL << 31), "%s: activation matrix too large (M * K must be < 2^31)", who);
   const uint32_t a_xor = (a_type == ITEXHIP_QUINT8) ? 0x80808080u : 0u;
   const uint8_t* ap = reinterpret_cast<const uint8_t*>(a);

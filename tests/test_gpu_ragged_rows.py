@@ -1,8 +1,11 @@
 """The tile kernel's vector epilogue on output rows that are no whole 16-byte vectors or start off a 16-byte boundary: every
-result type and tile shape, the last piece of a row in parts.  Against int64 sums and the epilogue's separately rounded fp32
-steps, bit for bit, with the bytes around the result untouched."""
+result type and tile shape, the last piece of a row in parts; and the small-M kernel beyond 128 rows.  Against int64 sums and the
+epilogue's separately rounded fp32 steps, bit for bit, with the bytes around the result untouched."""
 import numpy as np
 import pytest
+
+from oracle import pyoracle as orc
+from tests.test_gpu_matmul import V2_DEQ, V2_REQ_S8, make_acts, make_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +45,23 @@ def test_rows_of_any_length(hip, dev, M, K, N, shape):
             got = out.cpu().numpy()
             assert (got[:off] == 0x5a).all() and (got[off + M * N * esz:] == 0x5a).all()
             np.testing.assert_array_equal(got[off:off + M * N * esz], convert(torch, hip, np.ascontiguousarray(v), T).ravel())
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 70, 272), (140, 33, 1040), (512, 100, 784), (513, 64, 528), (1024, 30, 592), (17, 50, 1600), (64, 200, 3088)])
+def test_small_m_kernel_on_more_rows_and_wavefronts(hip, dev, M, N, K):
+    layer, w, bias = make_layer(hip, dev, K, N, seed=K + N)
+    x, xq, mn, mx = make_acts(M, K, seed=M + K)
+    r = float(np.abs(x @ w + bias).max())
+    for kw in (V2_DEQ, V2_REQ_S8):
+        np.testing.assert_array_equal(layer.run(xq, kw, mn, mx, -r, r, path="fused"), layer.oracle(xq, kw, mn, mx, -r, r))
+        assert hip.last_kernel()[0] == "small_m"
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 256, "tile"), (512, 256, 272, "tile"), (512, 256, 528, "small_m"), (512, 257, 528, "tile"),
+                                          (513, 64, 528, "small_m"), (1024, 65, 528, "tile"), (2049, 32, 528, "tile"), (64, 4096, 128, "small_m"),
+                                          (64, 4160, 128, "tile"), (128, 2112, 1536, "tile"), (128, 2112, 1552, "small_m")])
+def test_line_between_the_kernels(hip, dev, M, N, K, kernel):
+    layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
+    _, xq, mn, mx = make_acts(M, K, seed=M + K)
+    np.testing.assert_array_equal(layer.run(xq, V2_DEQ, mn, mx, path="fused"), layer.oracle(xq, V2_DEQ, mn, mx))
+    assert hip.last_kernel()[0] == kernel
