@@ -82,8 +82,9 @@ __global__ __launch_bounds__(256) void prepack_b_kernel(const int8_t* __restrict
 }
 
 // ------------------------------------------------------------------------------------------------
-// Small-M kernel (bandwidth bound on the weight).  One workgroup owns a strip of 16 * NT output channels and a block
-// of 16 R rows (M <= 16: R = 1, the whole problem's rows; up to 128 rows in blocks of 32, R = 2, whose workgroups
+// Small-M kernel (bandwidth bound on the weight up to 16 rows; beyond, and as a convolution, for launches of few tiles, bound by
+// a chain of round trips to memory).  One workgroup owns a strip of 16 * NT output channels and a block
+// of 16 R rows (M <= 16: R = 1, the whole problem's rows; more rows, and convolutions, in blocks of 32, R = 2, whose workgroups
 // share the strip's weights through one L2) (NT = 2: whole chunks; NT = 1: one half of each chunk, when N alone would not give every CU a
 // workgroup); its wavefronts split K into contiguous runs of chunk pairs (64 k each).  Per chunk pair a
 // wavefront needs NT weight fragments in the operand layout of the 16x16x64 MFMA (lane l: channel l % 16,
@@ -102,8 +103,12 @@ __global__ __launch_bounds__(256) void prepack_b_kernel(const int8_t* __restrict
 // stream, so that no streaming wavefront starts its loads late or stops for arithmetic.  Rows >= M of the
 // activation operand repeat row M - 1; their results are never stored.  Pairs past the end of a wavefront's
 // run are loaded from clamped addresses and not used.
+// CONV: the rows are output positions of a convolution over a multiple of 64 channels, so that a chunk pair lies in one pixel
+// of the window: its offset from the window's origin is the same for the whole wavefront, and a lane adds its row's origin
+// or, where the pixel lies in the padding, reads zeros.
 // ------------------------------------------------------------------------------------------------
 constexpr int kGemvBatch = 4;                 // chunk pairs per batch of the 32-row kernel (2 for up to 16 rows, see UB below)
+static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};  // what a window reads in the padding
 constexpr int kGemvPanelWords = 6 + 32;       // per channel of the strip: 6 parameter words + {scale, bias} of 16 rows
 
 // UB: chunk pairs per batch; two batches of a wavefront are in flight.  2 for up to 16 rows, 4 for the blocks of 32
@@ -111,11 +116,11 @@ constexpr int kGemvPanelWords = 6 + 32;       // per channel of the strip: 6 par
 // and 11.3 -> 11.0 us, M = 1 11.3 -> 10.95 us and unchanged, M = 16 unchanged and 13.0 -> 12.7 us against batches of 4
 // (a form that fetched the 4 rows of a whole batch of 4 pairs in one load of 4 x 256 bytes was no faster and is gone);
 // batches of 1 or 3 are slower everywhere, and with 32 rows batches of 2 lose on long K.
-template <int NT, int OUT_T, int R, int UB = kGemvBatch>
+template <int NT, int OUT_T, int R, int UB = kGemvBatch, bool CONV = false>
 __global__ __launch_bounds__(576) void qgemv_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
                                                      const uint8_t* __restrict__ bp, int M, int K, int N,
-                                                     int KC, int cnt, EpilogueArgs e,
-                                                     void* __restrict__ out) {
+                                                     int KC, int cnt, int work, FastDiv by_row_blocks, EpilogueArgs e,
+                                                     void* __restrict__ out, typename conv_args_of<CONV>::type cv) {
   constexpr int SW = 16 * NT;
   constexpr int U = UB, RING = 2 * UB;  // RING: activation slots of 1 KiB per wavefront and row block
   constexpr int L = U * (NT + R);       // loads per batch
@@ -126,14 +131,17 @@ __global__ __launch_bounds__(576) void qgemv_kernel(const uint8_t* __restrict__ 
   // strips, 4096 -> 14336: 13.0 -> 12.1 us once that wavefront fetched the 16 rows' ranges in one round trip instead of
   // one per table entry - before that it finished last there).
   extern __shared__ __align__(16) uint8_t smem[];  // [waves][RING][R][1 KiB], then the parameter panel [3 or 6][SW]
-  // R = 1 (M <= 16): one workgroup per strip.  R = 2 (M > 16): a workgroup takes 32 rows of a strip - every weight
-  // fragment meets two activation fragments - and the grid is x = 8 * row blocks, y = groups of 8 strips (x runs
-  // fastest in launch order, consecutive workgroup ids go round robin to the 8 XCDs): the row blocks of a strip get
-  // ids 8 apart, so they run at the same time on the same XCD and its L2 fetches the strip's weights once.  The grid
-  // is padded to whole groups of 8 strips.
-  const int strip = R > 1 ? blockIdx.y * 8 + (blockIdx.x & 7) : blockIdx.x;
-  const int m_base = R > 1 ? (blockIdx.x >> 3) * ROWS : 0;
-  if (R > 1 && strip * SW >= N) return;
+  // R = 1 (M <= 16): one workgroup per strip.  R = 2: a workgroup takes 32 rows of a strip - every weight fragment meets
+  // two activation fragments - and consecutive workgroup ids go round robin to the 8 XCDs: each XCD gets a contiguous
+  // range of the `work` pieces, row blocks fastest, so that the row blocks of a strip run at the same time on the same
+  // XCD and its L2 fetches the strip's weights once.  The grid is padded to whole rounds of the XCDs.
+  int strip = blockIdx.x, m_base = 0;
+  if constexpr (R > 1) {
+    const int piece = static_cast<int>(blockIdx.x & 7) * ((work + 7) >> 3) + static_cast<int>(blockIdx.x >> 3);
+    if (piece >= work) return;  // whole workgroup
+    strip = fast_div(piece, by_row_blocks);
+    m_base = (piece - strip * ((M + ROWS - 1) / ROWS)) * ROWS;
+  }
   const int waves = (blockDim.x >> 6) - 1;  // streaming wavefronts; one more resolves the channel parameters
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lrow = lane & 15, lgrp = lane >> 4;  // fragment lane: row / channel, k-group 0..3 of the chunk pair
@@ -148,8 +156,29 @@ __global__ __launch_bounds__(576) void qgemv_kernel(const uint8_t* __restrict__ 
   const int q = lane >> 2;
   const int dpiece = ((lane & 3) ^ ((q >> 2) & 3)) * 16;
   const uint8_t* arow[R];
+  int win_h[R], win_w[R];  // convolution: the window's origin, which may lie in the padding
 #pragma unroll
-  for (int r = 0; r < R; ++r) arow[r] = a + static_cast<int64_t>(min(m_base + 16 * r + q, M - 1)) * K;
+  for (int r = 0; r < R; ++r) {
+    const int m = min(m_base + 16 * r + q, M - 1);
+    if constexpr (CONV) {
+      const int t = fast_div(m, cv.by_out_w), ow = m - t * cv.out_w;
+      const int b = fast_div(t, cv.by_out_h), oh = t - b * cv.out_h;
+      win_h[r] = oh * cv.stride_h - cv.pad_top;
+      win_w[r] = ow * cv.stride_w - cv.pad_left;
+      arow[r] = a + (static_cast<int64_t>(b * cv.in_h + win_h[r]) * cv.in_w + win_w[r]) * cv.in_c + dpiece;
+    } else {
+      arow[r] = a + static_cast<int64_t>(m) * K;
+    }
+  }
+  // convolution (channels a multiple of 64: a chunk pair lies in one pixel of the window): the pair that is loaded next
+  int next = p0, kw = 0, tap_h = 0, tap_w = 0, tap_c = 0;
+  if constexpr (CONV) {
+    const int tap = fast_div(min(p0, KP - 1) * 64, cv.by_in_c), kh = fast_div(tap, cv.by_k_w);
+    tap_c = min(p0, KP - 1) * 64 - tap * cv.in_c;
+    kw = tap - kh * cv.k_w;
+    tap_h = kh * cv.dil_h;
+    tap_w = kw * cv.dil_w;
+  }
   const int klast = K - 16;  // k beyond K meets zero weights: any in-bounds data will do
   uint8_t* const ring = smem + wave * (RING * R * 1024);
   const uint32_t frag_off = static_cast<uint32_t>((4 * lrow + (lgrp ^ ((lrow >> 2) & 3))) * 16);
@@ -171,9 +200,31 @@ __global__ __launch_bounds__(576) void qgemv_kernel(const uint8_t* __restrict__ 
   for (int r = 0; r < R; ++r) aptr[r] = arow[r] + dpiece + static_cast<int64_t>(p0) * 64;
   const int p_full = min(p1, K >> 6);  // pairs below this index lie entirely inside K
   auto issue = [&](int pb, int slot0, v4i (&w)[U][NT]) {
+    if constexpr (CONV) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t off = (static_cast<int64_t>(tap_h) * cv.in_w + tap_w) * cv.in_c + tap_c;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const bool inside = static_cast<unsigned>(win_h[r] + tap_h) < static_cast<unsigned>(cv.in_h) &&
+                              static_cast<unsigned>(win_w[r] + tap_w) < static_cast<unsigned>(cv.in_w);
+          const uint8_t* src = inside ? arow[r] + off : reinterpret_cast<const uint8_t*>(kZeros);
+          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                           (__attribute__((address_space(3))) void*)(ring + ((slot0 + u) * R + r) * 1024), 16, 0, 0);
+        }
+        if (++next < KP) {  // (a pair past the end loads the last one again)
+          tap_c += 64;
+          if (tap_c == cv.in_c) {
+            tap_c = 0;
+            tap_w += cv.dil_w;
+            if (++kw == cv.k_w) { kw = tap_w = 0; tap_h += cv.dil_h; }
+          }
+        }
+      }
+    }
     if (pb + U <= p_full) {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int u = 0; u < (CONV ? 0 : U); ++u)
 #pragma unroll
         for (int r = 0; r < R; ++r)
           // the builtin, not inline assembly: the compiler's own vmcnt bookkeeping for the weight loads must see these
@@ -186,7 +237,7 @@ __global__ __launch_bounds__(576) void qgemv_kernel(const uint8_t* __restrict__ 
           w[u][t] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wptr + u * (2 * kChunkBytes) + t * 256));
     } else {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < (CONV ? 0 : U); ++u) {
         const int p = min(pb + u, KP - 1);
 #pragma unroll
         for (int r = 0; r < R; ++r)
@@ -445,16 +496,20 @@ EpilogueArgs make_args(int a_type, const int32_t* colsum, const float* scales, c
   return e;
 }
 
-inline int gemv_batch(int M) { return M <= 16 ? 2 : kGemvBatch; }  // chunk pairs per batch of the variant that takes M rows
+inline int gemv_batch(bool blocks) { return blocks ? kGemvBatch : 2; }  // chunk pairs per batch, blocks: of 32 rows
 
-template <int NT, int OUT_T>
+template <int NT, int OUT_T, bool CONV>
 int launch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int K, int N, int KC, int waves, int cnt,
-                const EpilogueArgs& e, void* out, hipStream_t st) {
-  // up to 16 rows: batches of 2 chunk pairs; more: blocks of 32 rows, batches of 4
-  const int variant = M > 16 ? 1 : 0;
-  auto kern = variant == 1 ? qgemv_kernel<NT, OUT_T, 2, 4> : qgemv_kernel<NT, OUT_T, 1, 2>;
-  const int R = M > 16 ? 2 : 1;
-  const int ring = 2 * gemv_batch(M);  // KiB per wavefront and row block
+                const EpilogueArgs& e, void* out, hipStream_t st, const typename conv_args_of<CONV>::type& cv) {
+  // up to 16 rows: batches of 2 chunk pairs; more, and convolutions: blocks of 32 rows, batches of 4
+  const bool blocks = CONV || M > 16;
+  const int variant = blocks ? 1 : 0;
+  auto kern = qgemv_kernel<NT, OUT_T, 2, 4, CONV>;
+  if constexpr (!CONV) {
+    if (!blocks) kern = qgemv_kernel<NT, OUT_T, 1, 2>;
+  }
+  const int R = blocks ? 2 : 1;
+  const int ring = 2 * gemv_batch(blocks);  // KiB per wavefront and row block
   // the kernel's table of per-row parameters holds 16 rows
   ITEXHIP_REQUIRE(e.row_min_a == nullptr || M <= 16, "the small-M kernel takes per-row activation ranges for M <= 16 only");
   const size_t lds_max = static_cast<size_t>(8 * ring * 1024) * R + kGemvPanelWords * 16 * NT * 4;
@@ -467,38 +522,50 @@ int launch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int 
   }
   const size_t lds = static_cast<size_t>(waves) * ring * 1024 * R + kGemvPanelWords * 16 * NT * 4;
   const int strips = (N + 16 * NT - 1) / (16 * NT);
-  const int rbs = (M + 31) / 32;  // row blocks of the R = 2 kernel
-  const dim3 grid = M > 16 ? dim3(8 * rbs, (strips + 7) / 8) : dim3(strips);
-  kern<<<grid, 64 * (waves + 1), lds, st>>>(a, a_xor, bp, M, K, N, KC, cnt, e, out);
+  const int row_blocks = blocks ? (M + 31) / 32 : 1, work = strips * row_blocks;
+  kern<<<blocks ? (work + 7) / 8 * 8 : work, 64 * (waves + 1), lds, st>>>(a, a_xor, bp, M, K, N, KC, cnt, work, make_fast_div(row_blocks), e, out, cv);
   return ITEXHIP_OK;
 }
 
-template <int OUT_T>
+template <int OUT_T, bool CONV = false>
 int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, int K, int N,
-                  const EpilogueArgs& e, void* out, hipStream_t st) {
+                  const EpilogueArgs& e, void* out, hipStream_t st, const typename conv_args_of<CONV>::type& cv = {}) {
+  // A strip is finished by one wavefront per 16-channel tile, so never fewer wavefronts than that.
+  // Blocks of 32 rows: a launch takes one round of workgroups if it can, and a CU holds one of 5 to 8 wavefronts (16 KB of rings
+  // each), two of 4, four of 2.  16-channel strips where they are at most one workgroup per CU, 32 otherwise (weight and rows are read
+  // half as often; against two workgroups per CU of 16 channels with a quarter of the wavefronts 0.75 of the time for K > 1024 and 129 to 256
+  // blocks of 32 x 32, 1.0 - 1.15 for a shorter K, not there).  Then as many wavefronts as fit that round, the fewest of the same number of batches
+  // each; in a MatMul with at most one workgroup per CU 8 chunk pairs for each, a shorter launch (all 8 wavefronts 1.06 for K up to 1024, 1.0
+  // beyond; convolutions 0.95 - 1.0).  257 to 512 workgroups: 4 wavefronts over 1 or 2 of twice the pairs 0.73 - 1.09 (0.9);  more: 2
+  // over up to 8 0.75 - 1.04 (0.99).  (4000 sizes.)
+  // Up to 16 rows: 32-channel strips when they give every CU a workgroup, and about 8 chunk pairs for each of up to 8 wavefronts (16 pairs
+  // 0.88 - 1.35 of the time, 1.09 in the middle; 16 x 1024 -> 1024 4.4 -> 5.8 us).  With ranges per row one wavefront of a workgroup
+  // works out a table for every row, and more of the others are in its way: 16 pairs from 9 rows on (0.72 - 1.2 of the time, 0.97; 12 x 4080 ->
+  // 4624 10.3 -> 7.9 us), and from 5 rows on where CUs hold more than one workgroup and K > 1472 (0.79 - 1.0, 0.91); fewer rows or
+  // less K 0.91 - 1.42 (1.09: not there).  Prefer a count that divides K into whole batches.
   const int KC = 2 * ((K + 63) / 64), KP = KC / 2;
-  // 32-channel strips when they give every CU a workgroup, else 16-channel strips; a strip is finished by one
-  // wavefront per 16-channel tile, so never fewer wavefronts than that.  Wavefronts per strip, at most 8: about 8 chunk pairs each,
-  // so that a launch that does not fill the device is a short chain of round trips (500 sizes of up to 128 rows, K and N up to
-  // 14336, every count; against 16 pairs each for 5 to 16 rows and 32 beyond: 0.95 and 0.89 of the time, 1.04 at most: 128 x 1024 -> 1024
-  // 5.2 -> 4.5 us, 16 x 1024 -> 1024 5.8 -> 4.4, 48 x 2992 -> 333 10.8 -> 6.3, 33 x 4096 -> 4096 10.9 -> 8.4); prefer a count that
-  // divides K into whole batches.
-  // (blocks of 32 rows count as workgroups of their own: 14336 -> 4096 at M = 64 28.1 -> 20.0 us with 32-channel strips,
-  // 256 workgroups instead of 512 that read the activations twice as often)
-  const int row_blocks = M > 16 ? (M + 31) / 32 : 1;
-  const int nt = ((N + 31) / 32) * row_blocks >= 256 ? 2 : 1;
-  // From 65 rows on with more than one workgroup per CU: half as many wavefronts with runs four times as long, fewer rings, so that
-  // workgroups share a CU (8 pairs each 1.02 of that, 1.18 at most).
-  const int64_t wgs = static_cast<int64_t>((N + 16 * nt - 1) / (16 * nt)) * row_blocks;
-  const bool paired = M > 64 && wgs > 256;
-  const int per_wave = paired ? 16 : 8;
-  int waves = std::max(nt, std::min(8, (KP + per_wave - 1) / per_wave));
-  for (int w = waves; w >= std::max(nt, waves / 2 + 1); --w)
-    if (KP % (gemv_batch(M) * w) == 0) { waves = w; break; }
-  if (paired) waves = std::max(nt, waves / 2);
+  const bool blocks = CONV || M > 16;
+  const int row_blocks = blocks ? (M + 31) / 32 : 1;
+  auto workgroups = [&](int nt) { return static_cast<int64_t>((N + 16 * nt - 1) / (16 * nt)) * row_blocks; };
+  int nt, waves;
+  if (blocks) {
+    nt = workgroups(1) <= 256 || (!CONV && K <= 1024 && workgroups(2) < 256) ? 1 : 2;
+    const int64_t wgs = workgroups(nt);
+    const int most = wgs <= 256 ? 8 : wgs <= 512 ? 4 : 2;
+    auto batches = [&](int w) { return ((KP + w - 1) / w + kGemvBatch - 1) / kGemvBatch; };
+    waves = most;
+    if (!CONV && (most == 8 || (nt == 1 && KP <= 8))) waves = std::max(nt, std::min(most, (KP + 7) / 8));
+    for (int w = waves - 1; w >= std::max(nt, most / 2 + 1) && batches(w) == batches(waves); --w) waves = w;
+  } else {
+    nt = workgroups(2) >= 256 ? 2 : 1;
+    const int per_wave = e.row_min_a && (M > 8 || (M > 4 && workgroups(nt) > 256 && KP >= 24)) ? 16 : 8;
+    waves = std::max(nt, std::min(8, (KP + per_wave - 1) / per_wave));
+    for (int w = waves; w >= std::max(nt, waves / 2 + 1); --w)
+      if (KP % (2 * w) == 0) { waves = w; break; }
+  }
   const int cnt = (KP + waves - 1) / waves;
-  if (nt == 2) return launch_gemv<2, OUT_T>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st);
-  return launch_gemv<1, OUT_T>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st);
+  if (nt == 2) return launch_gemv<2, OUT_T, CONV>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st, cv);
+  return launch_gemv<1, OUT_T, CONV>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st, cv);
 }
 
 #define ITEXHIP_DISPATCH_OUT(out_type, CALL)                                  \
@@ -515,15 +582,18 @@ enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or th
 
 // Which packed kernel takes a call.  The small-M kernel (a strip of channels x 16 or 32 rows x all of K per workgroup)
 // streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  Small-M / tile kernel, time,
-// with a chain that the tile kernel's vector epilogue finishes (2500 sizes of up to 2048 rows, K up to 4096, 64 x 64 tiles; 400 of them with
-// operands out of the caches, which changes no line):
-//   33 to 128 rows        up to 16 tiles 0.5 - 1.27 (K <= 256 1.03, 257 - 1024 0.9, more 0.69), 17 - 64 0.53 - 1.3 (0.96);  65 - 128 tiles
-//                         K <= 1536, or up to 64 rows, 0.94 - 1.66 (1.2: not there), else 0.79 - 1.4 (1.05), more tiles 1.0 - 2.4.  Rows that
+// with a chain that the tile kernel's vector epilogue finishes (6800 sizes of up to 2048 rows, K up to 4096; a sum is no exception), by
+// 64 x 64 tiles or by 32 x 32 pieces:
+//   33 to 128 rows        up to 16 tiles 0.5 - 1.27 (K <= 256 1.03, 257 - 1024 0.9, more 0.69), 17 - 64 tiles up to 256 pieces K <= 1024
+//                         0.77 - 1.3 (1.0), more 0.59 - 1.0 (0.8);  65 - 128 tiles up to 256 pieces K 513 - 1024 0.84 - 1.11 (0.94), more
+//                         0.59 - 0.99 (0.8), else K <= 1536, or up to 64 rows, 0.9 - 1.5 (1.1: not there), longer 0.8 - 1.3 (1.05), more tiles 1.0 - 2.4.  Rows that
 //                         are no whole 16-byte vectors differ by 0.1 at most; with a K of one step, or K > 1536 and few more than
 //                         128 tiles, either kernel does.
-//   129 to 512 rows       up to 16 tiles K <= 256 0.78 - 1.27 (1.02: not there), 257 - 512 0.92, 513 - 1024 0.82, more 0.66;  17 - 32 tiles
-//                         K > 512 0.58 - 1.03 (0.78);  33 - 64 tiles 0.7 - 1.3 (1.0: not there), more 1.0 - 4
-//   513 to 2048 rows      up to 16 tiles K > 512 0.66 - 0.94 (0.79);  17 - 32 0.73 - 1.6 (1.05: not there)
+//   129 to 512 rows       up to 16 tiles K <= 256 0.78 - 1.27 (1.02: not there), 257 - 512 0.92;  up to 128 pieces K 513 - 1024 0.66 - 1.03
+//                         (0.83), more 0.47 - 0.9 (0.68);  129 - 256 pieces K <= 1024 0.77 - 1.3 (0.97: not there), more 0.60 - 0.98 (0.77);
+//                         more pieces 0.78 - 2
+//   513 to 2048 rows      up to 128 pieces K <= 512 0.83 - 1.27 (not there), 513 - 1024 0.68 - 1.03 (0.83), more 0.47 - 1.08 (0.71);  129 - 256
+//                         K <= 1024 0.72 - 1.4 (0.96: not there), more 0.70 - 1.14 (0.9);  more pieces 0.82 - 2
 //   17 to 32 rows         (4600 sizes before that) K < 256 and over 128 tiles 1.0 - 1.7;  256 to 767, 129 - 256 tiles 0.9 - 1.15 (0.97:
 //                         not there), more 0.86 - 1.5;  from 768 on, 129 - 256 tiles, one per CU on the deep ring, 0.9 - 1.33, 257 - 512, a
 //                         second round for some of the CUs, 0.75 - 1.15 (not there)
@@ -535,19 +605,21 @@ static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int 
   if (M <= 16) return true;
   if (M > kSmallMaxAutoRows) return false;
   if (M > kSmallMaxRows && __atomic_load_n(&g_forced_tile_shape[0], __ATOMIC_RELAXED) >= 0) return false;
-  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), pieces = ((M + 31) / 32) * ((N + 31) / 32);
   CanonChain c;
   const int act = canon_chain(e, &c);
-  if (e.addend == nullptr && vector_chain(e, act, c, N)) {
+  const bool vector = vector_chain(e, act, c, N);
+  if (M > kSmallMaxRows) {
+    if (!vector) return e.addend == nullptr && tiles <= 128 && K <= 2048;
+    if (M <= 512 && tiles <= 16 && K > 256) return true;
+    return pieces <= 128 ? K > 512 : pieces <= 256 && K > 1024;
+  }
+  if (vector && e.addend == nullptr) {
     const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
     const bool whole_rows = (N * esz) % 16 == 0 && aligned(out, 16);
-    if (M > 512) return tiles <= 16 && K > 512;
-    if (M > kSmallMaxRows) return tiles <= 16 ? K > 256 : tiles <= 32 && K > 512;
-    if (M > 32 && K >= 128 && tiles > 64 && (M <= 64 || K <= 1536)) return false;
+    if (M > 32 && K >= 128 && tiles > 64 && (M <= 64 || K <= 1536) && !(pieces <= 256 && K > 512)) return false;
     if (whole_rows ? K >= 64 && tiles > 128 : K >= 128 && tiles > 144)
       if (M > 32 || K < 256 || (K < 768) == (tiles > 256)) return false;
-  } else if (M > kSmallMaxRows) {
-    return e.addend == nullptr && tiles <= 128 && K <= 2048;
   }
   if (M <= 32) return true;
   if (K * N <= (8LL << 20)) return true;                       // the weight stays in L2: launch-bound either way
@@ -696,6 +768,28 @@ extern "C" int itexhip_qconv2d_implicit_ok(const itexhip_conv_geometry* g, const
 }
 
 namespace {
+// Whether the small-M kernel takes a convolution that neither the direct nor the short-K kernel does.  Few 64 x 64 tiles
+// with a long K are a chain of K steps, whose window arithmetic a ring of loads does not hide; here up to 8 wavefronts
+// share the steps.  Time over the tile kernel's, by 32 x 32 pieces of the result (700 shapes: 1 x 1 to 5 x 5 windows, 64 to
+// 1024 channels, strides 1 and 2):
+//   up to 256      K <= 512 0.9 - 1.28 (not there), 576 - 1024 0.73 - 1.03 (0.88), to 2048 0.59 - 0.77 (0.65), to 4096 0.45 - 0.64
+//                  (0.56), more 0.26 - 0.55 (0.40)
+//   257 - 512      K <= 1024 0.86 - 1.28 (not there), to 2048 0.80 - 0.94 (0.87), to 4096 0.61 - 0.81 (0.69), more 0.47 - 0.83 (0.61)
+//   513 - 768      K <= 4096 0.85 - 1.6 (not there), more 0.71 - 1.10 (0.84);  more pieces 0.82 - 2.5: not there
+// 3 x 3, 7 x 7 x 512 -> 512, 1 image 16.9 -> 6.5 us, 8 images 17.3 -> 7.9, 32 images (784 pieces) 17.9 there;
+// 14 x 14 x 256 -> 256, 1 image 10.1 -> 6.1, 8 images 10.5 -> 7.4.
+bool small_conv(int64_t M, int64_t K, int64_t N, const ConvTileArgs& cv, const EpilogueArgs& e) {
+  if (cv.in_c % 64 != 0 || __atomic_load_n(&g_forced_tile_shape[1], __ATOMIC_RELAXED) >= 0) return false;
+  CanonChain c;
+  const int act = canon_chain(e, &c);
+  if (act < 0 || act == 3) return false;  // the tile kernel refuses these chains, and the summands that it has no load for
+  if ((c.flags & (kChainSumFirst | kChainSumLast)) &&
+      (e.addend == nullptr || N % 4 != 0 || !aligned(e.addend, e.addend_type == ITEXHIP_FLOAT ? 16 : 4)))
+    return false;
+  const int64_t pieces = ((M + 31) / 32) * ((N + 31) / 32);
+  return pieces <= 256 ? K > 512 : pieces <= 512 ? K > 1024 : pieces <= 768 && K > 4096;
+}
+
 int qconv2d_impl(const char* who, const void* x, int x_type, const itexhip_conv_geometry* g, const int8_t* packed_filter,
                  const int32_t* colsum, int64_t out_channels, const float* scales, const float* bias,
                  const itexhip_epilogue* ep, const void* addend, int addend_type, int out_type, void* out, void* stream) {
@@ -727,6 +821,19 @@ int qconv2d_impl(const char* who, const void* x, int x_type, const itexhip_conv_
   if (st__ == 0) st__ = try_stream(xp, a_xor, bp, Mi, Ki, Ni, e, out_type, out, hs, &cv);
   if (st__ < 0) return -st__;
   if (st__ > 0) {
+    ITEXHIP_CHECK_LAUNCH(who);
+    return ITEXHIP_OK;
+  }
+  if (small_conv(M, K, N, cv, e)) {
+    note_kernel(kLastSmallM, 0);
+    switch (out_type) {
+      case ITEXHIP_FLOAT: st__ = dispatch_gemv<ITEXHIP_FLOAT, true>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
+      case ITEXHIP_BFLOAT16: st__ = dispatch_gemv<ITEXHIP_BFLOAT16, true>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
+      case ITEXHIP_QINT32: st__ = dispatch_gemv<ITEXHIP_QINT32, true>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
+      case ITEXHIP_QINT8: st__ = dispatch_gemv<ITEXHIP_QINT8, true>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
+      default: st__ = dispatch_gemv<ITEXHIP_QUINT8, true>(xp, a_xor, bp, Mi, Ki, Ni, e, out, hs, cv); break;
+    }
+    if (st__ != ITEXHIP_OK) return st__;
     ITEXHIP_CHECK_LAUNCH(who);
     return ITEXHIP_OK;
   }

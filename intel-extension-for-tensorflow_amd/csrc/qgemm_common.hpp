@@ -415,6 +415,9 @@ struct ConvTileArgs {
   int stride_h, stride_w, dil_h, dil_w, pad_top, pad_left;
   FastDiv by_out_w, by_out_h, by_in_c, by_k_w;  // the kernel's row and window decompositions divide by these
 };
+struct NoConvArgs {};
+template <bool CONV> struct conv_args_of { using type = NoConvArgs; };  // of a kernel that also exists as a convolution
+template <> struct conv_args_of<true> { using type = ConvTileArgs; };
 constexpr int kMaxConvPieces = 1024;  // 16-byte pieces per patch row: 16 KiB of receptive field per output position
 
 }  // namespace itexhip

@@ -88,9 +88,6 @@ inline int xcd_rectangles(int num_m, int num_n, int BM, int BN, int K) {
 // run of 4 or 2 pixels of one window row, which the host admits only where no window touches the padding.  Either way
 // only the source address of an activation load changes: row -> window origin once per kernel, piece -> offset inside
 // the window from a table in LDS.
-struct NoConvArgs {};
-template <bool CONV> struct conv_args_of { using type = NoConvArgs; };
-template <> struct conv_args_of<true> { using type = ConvTileArgs; };
 static __device__ __align__(16) const uint32_t kZeroPiece[4] = {0u, 0u, 0u, 0u};
 
 // amask: 0x80808080 when the activations are unsigned (they are fed as x ^ 0x80), else 0; a scalar
