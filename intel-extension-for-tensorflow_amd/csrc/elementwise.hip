@@ -37,16 +37,17 @@ __device__ __forceinline__ void store_through(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// n4 = number of complete groups of 4 elements; the caller handles the tail.
+// n elements: whole groups of 4, and up to three more that the first workgroup finishes (a launch of their own cost 1.3 to 1.5 us).
 template <int T>
 __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(const f4* __restrict__ x,
-                                                                uint32_t* __restrict__ q, int64_t n4,
+                                                                uint32_t* __restrict__ q, int64_t n,
                                                                 float scale, float addend,
                                                                 const float* __restrict__ dev_params) {
   if (dev_params) {  // {scale, addend} left in device memory by quantize_dynamic_params_kernel
     scale = dev_params[0];
     addend = dev_params[1];
   }
+  const int64_t n4 = n >> 2;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
   int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
 #pragma unroll 1
@@ -55,6 +56,11 @@ __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(const f4* __rest
       const f4 v = __builtin_nontemporal_load(&x[i]);
       store_through(&q[i], quantize4<T>(v, scale, addend));
     }
+  }
+  const int64_t last = n4 * 4 + threadIdx.x;
+  if (blockIdx.x == 0 && last < n) {
+    const float t = reinterpret_cast<const float*>(x)[last] * scale;
+    reinterpret_cast<uint8_t*>(q)[last] = static_cast<uint8_t>(sat_rne<T>(t + addend));
   }
 }
 
@@ -134,8 +140,9 @@ __device__ __forceinline__ float widen(uint32_t w, int byte) {
 
 template <int T>
 __global__ __launch_bounds__(kThreads) void dequantize_vec_kernel(const uint32_t* __restrict__ q,
-                                                                  f4* __restrict__ y, int64_t n4,
+                                                                  f4* __restrict__ y, int64_t n,
                                                                   float scale, float zp) {
+  const int64_t n4 = n >> 2;  // and up to three elements more, as above
   const int64_t base = static_cast<int64_t>(blockIdx.x) * (kThreads * kWidenUnroll) + threadIdx.x;
   uint32_t w[kWidenUnroll];
 #pragma unroll
@@ -157,6 +164,9 @@ __global__ __launch_bounds__(kThreads) void dequantize_vec_kernel(const uint32_t
       __builtin_nontemporal_store(o, &y[i]);
     }
   }
+  const int64_t last = n4 * 4 + threadIdx.x;
+  if (blockIdx.x == 0 && last < n)
+    reinterpret_cast<float*>(y)[last] = (widen<T>(reinterpret_cast<const uint8_t*>(q)[last], 0) - zp) * scale;
 }
 
 template <int T>
@@ -217,13 +227,15 @@ __global__ __launch_bounds__(kThreads) void dequantize_axis_vec_kernel(const uin
 // ------------------------------------------------------------------------------------------------
 // kMode 0: one scale passed by value; 1: depth % 4 == 0, scales read as f4; 2: the same with fewer than 2^31 groups,
 // where the channel group of a lane is found by one 32-bit remainder and then stepped instead of a 64-bit remainder
-// per step (256 channels over 2^28 elements: 199 -> 195 us); n4 = groups of 4
+// per step (256 channels over 2^28 elements: 199 -> 195 us).  n elements: whole groups of 4 and, mode 0, up to three more that the
+// first workgroup finishes.
 template <int T, int kMode>
 __global__ __launch_bounds__(kThreads) void requantize_vec_kernel(const i4* __restrict__ x,
-                                                                  uint32_t* __restrict__ q, int64_t n4,
+                                                                  uint32_t* __restrict__ q, int64_t n,
                                                                   float scale,
                                                                   const float* __restrict__ scales,
                                                                   int64_t depth4) {
+  const int64_t n4 = n >> 2;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
   int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   uint32_t group = 0, group_step = 0;
@@ -246,6 +258,55 @@ __global__ __launch_bounds__(kThreads) void requantize_vec_kernel(const i4* __re
       const float c = static_cast<float>(v.z) * s.z, d = static_cast<float>(v.w) * s.w;
       store_through(&q[i], pack4(sat_rne<T>(a), sat_rne<T>(b), sat_rne<T>(c), sat_rne<T>(d)));
     }
+  }
+  const int64_t last = n4 * 4 + threadIdx.x;
+  if (kMode == 0 && blockIdx.x == 0 && last < n)
+    reinterpret_cast<uint8_t*>(q)[last] = static_cast<uint8_t>(sat_rne<T>(static_cast<float>(reinterpret_cast<const int32_t*>(x)[last]) * scale));
+}
+
+// Any depth (below 2^30) and any address of the scales, n a multiple of the depth and below 2^33: the scales of a group of 4 are
+// neighbours, read together, or the last channels and then the first; up to 3 channels take turns.  Up to three elements beyond the groups
+// are the first workgroup's.  Bound by memory but for the start, whose remainders and scales cost 0.6 us.  An element per thread with a
+// 64-bit remainder each: 85164 x 197 29.7 -> 16.6 us (85164 x 196 15.7), 16777217 x 1 29.7 -> 14.8, 21291 x 197 9.3 -> 5.6.
+template <int T>
+__global__ __launch_bounds__(kThreads) void requantize_any_vec_kernel(const i4* __restrict__ x, uint32_t* __restrict__ q, int64_t n,
+                                                                      const float* __restrict__ scales, uint32_t depth) {
+  typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const int64_t n4 = n >> 2, stride = static_cast<int64_t>(gridDim.x) * kThreads;
+  int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  i4 v{};
+  if (i < n4) v = __builtin_nontemporal_load(&x[i]);  // (one step in flight, as above: both at once 16.7 -> 18.1 us)
+  uint32_t channel = static_cast<uint32_t>(i) % depth * 4 % depth;  // of the group's first element
+  const uint32_t channel_step = static_cast<uint32_t>(stride) % depth * 4 % depth;
+  // seven scales in turn from channel 0 on, or the first three behind whatever four a group reads
+  auto turn = [&](int t) { return scales[depth >= 4 ? max(t - 4, 0) : t % static_cast<int>(depth)]; };
+  f4 first = f4{turn(0), turn(1), turn(2), turn(3)};
+  const f4 then = f4{turn(4), turn(5), turn(6), 0.0f};
+#pragma unroll 1
+  for (int step = 0; step < kNarrowSteps; ++step) {
+    if (i < n4) {
+      uint32_t past = channel;  // scales of the sequence ahead of the group's first
+      if (depth >= 4) {
+        const uint32_t at = min(channel, depth - 4);
+        past = channel - at;
+        first = *reinterpret_cast<const f4_any*>(scales + at);
+      }
+      const bool two = (past & 2) != 0, one = (past & 1) != 0;
+      const float s0 = two ? first.z : first.x, s1 = two ? first.w : first.y, s2 = two ? then.x : first.z;
+      const float s3 = two ? then.y : first.w, s4 = two ? then.z : then.x;
+      const float a = static_cast<float>(v.x) * (one ? s1 : s0), b = static_cast<float>(v.y) * (one ? s2 : s1);
+      const float c = static_cast<float>(v.z) * (one ? s3 : s2), d = static_cast<float>(v.w) * (one ? s4 : s3);
+      store_through(&q[i], pack4(sat_rne<T>(a), sat_rne<T>(b), sat_rne<T>(c), sat_rne<T>(d)));
+      channel += channel_step;
+      if (channel >= depth) channel -= depth;
+    }
+    i += stride;
+    if (step + 1 < kNarrowSteps && i < n4) v = __builtin_nontemporal_load(&x[i]);
+  }
+  const int64_t last = n4 * 4 + threadIdx.x;
+  if (blockIdx.x == 0 && last < n) {
+    const float s = scales[(depth * 4 - static_cast<uint32_t>(n - last)) % depth];
+    reinterpret_cast<uint8_t*>(q)[last] = static_cast<uint8_t>(sat_rne<T>(static_cast<float>(reinterpret_cast<const int32_t*>(x)[last]) * s));
   }
 }
 
@@ -637,12 +698,18 @@ constexpr int64_t kSmallMax = 4 * kSmallThreads * kSmallLoads * 4;   // elements
 
 template <int T>
 __global__ __launch_bounds__(kSmallThreads) void quantize_dynamic_small_kernel(const f4* __restrict__ x4,
-                                                                               uint32_t* __restrict__ q4, int n4,
+                                                                               uint32_t* __restrict__ q4, int n,
                                                                                float* __restrict__ state, int mode,
                                                                                float ensure_minimum_range) {
   __shared__ float red[2 * (kSmallThreads / 64)];
   __shared__ float params[2];
+  const int n4 = n >> 2, last = n4 * 4 + static_cast<int>(threadIdx.x);  // and up to three elements more
   float mn = __builtin_inff(), mx = -__builtin_inff();
+  if (last < n) {
+    const float t = reinterpret_cast<const float*>(x4)[last];
+    mn = fminf(mn, t);  // (a NaN leaves both as they are, as everywhere)
+    mx = fmaxf(mx, t);
+  }
   for (int base = threadIdx.x; base < n4; base += kSmallThreads * kSmallLoads) {
     f4 v[kSmallLoads];
 #pragma unroll
@@ -691,6 +758,10 @@ __global__ __launch_bounds__(kSmallThreads) void quantize_dynamic_small_kernel(c
   const int per = (n4 + gridDim.x - 1) / gridDim.x;
   const int end = min(n4, static_cast<int>(blockIdx.x + 1) * per);
   for (int i = blockIdx.x * per + threadIdx.x; i < end; i += kSmallThreads) q4[i] = quantize4<T>(x4[i], scale, addend);
+  if (blockIdx.x == 0 && last < n) {
+    const float t = reinterpret_cast<const float*>(x4)[last] * scale;
+    reinterpret_cast<uint8_t*>(q4)[last] = static_cast<uint8_t>(sat_rne<T>(t + addend));
+  }
 }
 
 // Per-row (per-token) form: workgroup m reduces row m, derives its parameters and quantizes it; the rows' output
@@ -865,11 +936,11 @@ int launch_quantize(const char* who, const float* x, void* q, int64_t n, int dst
     const unsigned grid = blocks_for(n4, kThreads * kNarrowSteps);
     if (dst_type == ITEXHIP_QINT8)
       quantize_vec_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n4, scale, addend, dev_params);
+          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n, scale, addend, dev_params);
     else
       quantize_vec_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n4, scale, addend, dev_params);
-    done = n4 * 4;
+          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n, scale, addend, dev_params);
+    done = n;
   }
   in_pieces(done, n, [&](int64_t begin, int64_t end) {
     const unsigned grid = blocks_for(end - begin, kThreads);
@@ -906,15 +977,15 @@ extern "C" int itexhip_quantize_dynamic(const float* x, void* q, int64_t n, int 
                   "itexhip_quantize_dynamic: SCALED, MIN_FIRST_CLASSIC, or MIN_FIRST to quint8");
   ITEXHIP_REQUIRE(n > 0, "itexhip_quantize_dynamic: an empty tensor has no range");
   ITEXHIP_REQUIRE(x && q && state && aligned(state, 8), "itexhip_quantize_dynamic: null or unaligned buffer");
-  if (n <= kSmallMax && n % 4 == 0 && aligned(x, 16) && aligned(q, 4)) {
+  if (n <= kSmallMax && n >= 4 && aligned(x, 16) && aligned(q, 4)) {
     const int n4 = static_cast<int>(n / 4);
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(16, (n4 + kSmallThreads - 1) / kSmallThreads));
     if (dst_type == ITEXHIP_QINT8)
       quantize_dynamic_small_kernel<ITEXHIP_QINT8><<<grid, kSmallThreads, 0, as_stream(stream)>>>(
-          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n4, state, mode, ensure_minimum_range);
+          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), static_cast<int>(n), state, mode, ensure_minimum_range);
     else
       quantize_dynamic_small_kernel<ITEXHIP_QUINT8><<<grid, kSmallThreads, 0, as_stream(stream)>>>(
-          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), n4, state, mode, ensure_minimum_range);
+          reinterpret_cast<const f4*>(x), reinterpret_cast<uint32_t*>(q), static_cast<int>(n), state, mode, ensure_minimum_range);
     ITEXHIP_CHECK_LAUNCH("itexhip_quantize_dynamic");
     return ITEXHIP_OK;
   }
@@ -1019,11 +1090,11 @@ extern "C" int itexhip_dequantize(const void* q, float* y, int64_t n, int src_ty
     const unsigned grid = blocks_for(n4, kThreads * kWidenUnroll);
     if (src_type == ITEXHIP_QINT8)
       dequantize_vec_kernel<ITEXHIP_QINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const uint32_t*>(q), reinterpret_cast<f4*>(y), n4, scale, zp);
+          reinterpret_cast<const uint32_t*>(q), reinterpret_cast<f4*>(y), n, scale, zp);
     else
       dequantize_vec_kernel<ITEXHIP_QUINT8><<<grid, kThreads, 0, st>>>(
-          reinterpret_cast<const uint32_t*>(q), reinterpret_cast<f4*>(y), n4, scale, zp);
-    done = n4 * 4;
+          reinterpret_cast<const uint32_t*>(q), reinterpret_cast<f4*>(y), n, scale, zp);
+    done = n;
   }
   in_pieces(done, n, [&](int64_t begin, int64_t end) {
     const unsigned grid = blocks_for(end - begin, kThreads);
@@ -1078,25 +1149,27 @@ extern "C" int itexhip_dequantize_axis(const void* q, float* y, int64_t outer, i
 }
 
 namespace {
+// elements from which on requantize_any_vec_kernel is the faster one: 2097153 x 1 4.3 -> 4.0 us, 7985 x 197 3.8 -> 4.1, 333 x 197 2.6 -> 3.2
+constexpr int64_t kAnyDepthMin = 1 << 21;
 template <int T>
 int requantize_impl(const int32_t* x, void* q, int64_t n, int64_t depth, float scale,
                     const float* scales, hipStream_t st) {
   int64_t done = 0;
   const bool vec_ok = aligned(x, 16) && aligned(q, 4) && n >= 4;
+  const int64_t n4 = n / 4;
+  const unsigned grid = blocks_for(n4, kThreads * kNarrowSteps);
+  const i4* const x4 = reinterpret_cast<const i4*>(x);
+  uint32_t* const q4 = static_cast<uint32_t*>(q);
   if (vec_ok && scales == nullptr) {
-    const int64_t n4 = n / 4;
-    requantize_vec_kernel<T, 0><<<blocks_for(n4, kThreads * kNarrowSteps), kThreads, 0, st>>>(
-        reinterpret_cast<const i4*>(x), reinterpret_cast<uint32_t*>(q), n4, scale, nullptr, 1);
-    done = n4 * 4;
-  } else if (vec_ok && depth % 4 == 0 && aligned(scales, 16)) {
-    const int64_t n4 = n / 4;  // n is a multiple of depth, hence of 4
-    if (n4 < (1LL << 31))
-      requantize_vec_kernel<T, 2><<<blocks_for(n4, kThreads * kNarrowSteps), kThreads, 0, st>>>(
-          reinterpret_cast<const i4*>(x), reinterpret_cast<uint32_t*>(q), n4, 0.f, scales, depth / 4);
-    else
-      requantize_vec_kernel<T, 1><<<blocks_for(n4, kThreads * kNarrowSteps), kThreads, 0, st>>>(
-          reinterpret_cast<const i4*>(x), reinterpret_cast<uint32_t*>(q), n4, 0.f, scales, depth / 4);
-    done = n4 * 4;
+    requantize_vec_kernel<T, 0><<<grid, kThreads, 0, st>>>(x4, q4, n, scale, nullptr, 1);
+    done = n;
+  } else if (vec_ok && depth % 4 == 0 && aligned(scales, 16)) {  // n is a multiple of depth, hence of 4
+    if (n4 < (1LL << 31)) requantize_vec_kernel<T, 2><<<grid, kThreads, 0, st>>>(x4, q4, n, 0.f, scales, depth / 4);
+    else requantize_vec_kernel<T, 1><<<grid, kThreads, 0, st>>>(x4, q4, n, 0.f, scales, depth / 4);
+    done = n;
+  } else if (vec_ok && n >= kAnyDepthMin && n4 < (1LL << 31) && depth < (1LL << 30)) {
+    requantize_any_vec_kernel<T><<<grid, kThreads, 0, st>>>(x4, q4, n, scales, static_cast<uint32_t>(depth));
+    done = n;
   }
   in_pieces(done, n, [&](int64_t begin, int64_t end) {
     requantize_scalar_kernel<T><<<blocks_for(end - begin, kThreads), kThreads, 0, st>>>(
