@@ -56,7 +56,7 @@ const char* itexhip_build_info(void);
 void itexhip_test_force_tile_shape(int matmul_shape, int conv_shape);
 /* Test hook: the kernel that the calling thread's last MatMul, BatchMatMul or Conv2D (not depthwise) was launched on, times
  * 10^8, plus what was chosen within it: 1 small M, 2 tiles (rows * 10^5 + columns * 100 + LDS stages), 3 short K (chunks per group
- * * 100 + 1 if all are held), 4 3 x 3 convolution (tiles per workgroup), 5 unpacked operands (groups per tile), 6 one output per
+ * * 100 + 1 if all are held), 4 3 x 3 convolution (tiles per workgroup), 5 unpacked operands (groups of four wavefronts per tile), 6 one output per
  * thread, 7 bands of 16 rows (parts that a row is cut into), 8 BatchMatMul tiles (rows / 64 * 10 + columns / 64).  0: none yet. */
 int itexhip_test_last_kernel(void);
 

@@ -1,7 +1,7 @@
 // Quantized MatMul on operands as TensorFlow stores them: any K, no alignment, nothing prepacked.  It takes the problems
 // whose K is not a multiple of 16 (the packed kernels move whole 16-byte pieces of an activation row).
 //
-// A workgroup owns a 64 x 64 output tile, whose K is walked in steps of 256: per step every thread fetches 64 bytes of the
+// A workgroup owns a 64 x 64 output tile (32 x 32 where they are few, a kernel of its own below), whose K is walked in steps of 256: per step every thread fetches 64 bytes of the
 // activations and 64 of the weight with 16-byte loads at whatever byte address they fall on (the hardware takes unaligned
 // vector loads; two cache lines instead of one now and then), and puts them k-contiguous into LDS; a [K, N] weight is
 // transposed on the way, 4 (k) x 16 (n) bytes per thread by byte permutes.  The long step is for latency: these problems
@@ -66,12 +66,48 @@ __device__ __forceinline__ v4i keep_bytes(v4i v, int n) {
 // quarters of a 256-byte span in another order.
 __device__ __forceinline__ int w_offset(int n, int k) { return n * kRow + (k ^ (((n >> 4) & 3) << 6)); }
 
+// column 4 c + j of four rows' bytes -> v[j]
+__device__ __forceinline__ void transpose_bytes(const v4i (&rows)[4], int c, uint32_t (&v)[4]) {
+  const uint32_t r0 = rows[0][c], r1 = rows[1][c], r2 = rows[2][c], r3 = rows[3][c];
+  const uint32_t lo01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), hi01 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+  const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+  v[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+  v[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+  v[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+  v[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+
 template <int ALG, int COUNT>
 __device__ __forceinline__ void apply_all(const itexhip_eltwise& elt, float (&v)[COUNT]) {
   itexhip_eltwise e = elt;
   e.alg = ALG;  // known here: apply_eltwise folds to one case
 #pragma unroll
   for (int i = 0; i < COUNT; ++i) v[i] = apply_eltwise(e, v[i]);
+}
+
+// the post-ops on COUNT results; index(i): where result i stands in the output (the summand's element)
+template <int COUNT, typename Index>
+__device__ __forceinline__ void apply_chain(const EpilogueArgs& e, float (&v)[COUNT], Index&& index) {
+  for (int k = 0; k < e.n_eltwise; ++k) {
+    const itexhip_eltwise& elt = e.elt[k];
+    switch (elt.alg) {
+      case ITEXHIP_ELT_SUM:
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i) v[i] = v[i] + elt.alpha * load_addend(e, index(i));
+        break;
+      case ITEXHIP_ELT_RELU: apply_all<ITEXHIP_ELT_RELU>(elt, v); break;
+      case ITEXHIP_ELT_CLIP: apply_all<ITEXHIP_ELT_CLIP>(elt, v); break;
+      case ITEXHIP_ELT_LINEAR: apply_all<ITEXHIP_ELT_LINEAR>(elt, v); break;
+      case ITEXHIP_ELT_GELU_TANH: apply_all<ITEXHIP_ELT_GELU_TANH>(elt, v); break;
+      case ITEXHIP_ELT_GELU_ERF: apply_all<ITEXHIP_ELT_GELU_ERF>(elt, v); break;
+      case ITEXHIP_ELT_ELU: apply_all<ITEXHIP_ELT_ELU>(elt, v); break;
+      case ITEXHIP_ELT_LOGISTIC: apply_all<ITEXHIP_ELT_LOGISTIC>(elt, v); break;
+      case ITEXHIP_ELT_TANH: apply_all<ITEXHIP_ELT_TANH>(elt, v); break;
+      case ITEXHIP_ELT_SWISH: apply_all<ITEXHIP_ELT_SWISH>(elt, v); break;
+      case ITEXHIP_ELT_MISH: apply_all<ITEXHIP_ELT_MISH>(elt, v); break;
+      default: break;
+    }
+  }
 }
 
 // SPLIT groups of four wavefronts share a tile: group g takes the K steps g, g + SPLIT, ... in LDS of its own, so that the
@@ -162,11 +198,8 @@ __global__ __launch_bounds__(256 * SPLIT) void qmatmul_unpacked_kernel(const uin
     } else {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {  // columns nb + 4 c .. + 3: a 4 x 4 byte transpose in two rounds of permutes
-        const uint32_t r0 = fw[0][c], r1 = fw[1][c], r2 = fw[2][c], r3 = fw[3][c];
-        const uint32_t lo01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), hi01 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-        const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-        const uint32_t v[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
-                               __builtin_amdgcn_perm(hi23, hi01, 0x05040100u), __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+        uint32_t v[4];
+        transpose_bytes(fw, c, v);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           *reinterpret_cast<uint32_t*>(ws + w_offset(nb + 4 * c + j, kb * 4)) = v[j];
@@ -259,29 +292,130 @@ __global__ __launch_bounds__(256 * SPLIT) void qmatmul_unpacked_kernel(const uin
     v[i] = static_cast<float>(sum[i] + comp) * scale;  // scale 1.0f when the node has no output scale (exact)
     v[i] = v[i] + bias;
   }
-  for (int k = 0; k < e.n_eltwise; ++k) {
-    const itexhip_eltwise& elt = e.elt[k];
-    switch (elt.alg) {
-      case ITEXHIP_ELT_SUM:
+  apply_chain(e, v, [&](int i) { return static_cast<int64_t>(min(row_of(i), M - 1)) * N + n; });
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-          const int m = min(row_of(i), M - 1);
-          v[i] = v[i] + elt.alpha * load_addend(e, static_cast<int64_t>(m) * N + n);
-        }
-        break;
-      case ITEXHIP_ELT_RELU: apply_all<ITEXHIP_ELT_RELU>(elt, v); break;
-      case ITEXHIP_ELT_CLIP: apply_all<ITEXHIP_ELT_CLIP>(elt, v); break;
-      case ITEXHIP_ELT_LINEAR: apply_all<ITEXHIP_ELT_LINEAR>(elt, v); break;
-      case ITEXHIP_ELT_GELU_TANH: apply_all<ITEXHIP_ELT_GELU_TANH>(elt, v); break;
-      case ITEXHIP_ELT_GELU_ERF: apply_all<ITEXHIP_ELT_GELU_ERF>(elt, v); break;
-      case ITEXHIP_ELT_ELU: apply_all<ITEXHIP_ELT_ELU>(elt, v); break;
-      case ITEXHIP_ELT_LOGISTIC: apply_all<ITEXHIP_ELT_LOGISTIC>(elt, v); break;
-      case ITEXHIP_ELT_TANH: apply_all<ITEXHIP_ELT_TANH>(elt, v); break;
-      case ITEXHIP_ELT_SWISH: apply_all<ITEXHIP_ELT_SWISH>(elt, v); break;
-      case ITEXHIP_ELT_MISH: apply_all<ITEXHIP_ELT_MISH>(elt, v); break;
-      default: break;
+  for (int i = 0; i < kPer; ++i) {
+    const int m = row_of(i);
+    if (m < M) store_output<OUT_T>(out, static_cast<int64_t>(m) * N + n, v[i]);
+  }
+}
+
+// Few tiles and a [K, N] weight: 32 x 32 results per workgroup, whose WAVES wavefronts take 128 k each in turn and share nothing
+// until their accumulators meet in LDS at the end.  The 64 x 64 tiles are bound by their loads there: one at an odd byte address
+// is served a lane per clock however its lanes lie.  So here the activations come straight as MFMA operands, row by lane, and
+// lanes without a row or a column load nothing; the weight is transposed through LDS that belongs to the wavefront, and its
+// column sums are a second product, with ones.  A CU has half the loads to serve, four times as many CUs share them, and up to
+// 128 WAVES k all are in flight at once.  us, 64 x 64 tiles -> these: 10 x 943 x 9 9.7 -> 5.3, 23 x 961 x 364 9.1 -> 5.9, 300 x 511 x 300
+// 7.3 -> 5.9, 200 x 901 x 1000 9.2 -> 7.4, 64 x 4001 x 64 19.3 -> 14.6, 10 x 137 x 28 6.8 -> 4.3.
+constexpr int kFew = 32, kFewK = 128, kFewRow = kFewK + 16;
+template <int OUT_T, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void qmatmul_unpacked_few_kernel(const uint8_t* __restrict__ a, uint32_t a_xor,
+                                                                              const uint8_t* __restrict__ w, int M, int K, int N,
+                                                                              int tiles_n, int tiles, EpilogueArgs e, void* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[WAVES][kFew * kFewRow];  // the wavefront's weight, then its accumulators
+  __shared__ int colsums[WAVES][kFew];
+  static_assert(kFew * kFewRow >= kFew * kFew * 4, "room for the accumulators");
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int l32 = lane & 31, half = lane >> 5;
+  // contiguous runs of tiles for the 8 XCDs, as above
+  const int per_xcd = (tiles + 7) / 8;
+  const int tile = static_cast<int>(blockIdx.x & 7) * per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;  // whole workgroup
+  const int tm = tile / tiles_n;
+  const int m0 = tm * kFew, n0 = (tile - tm * tiles_n) * kFew;
+  const int64_t a_end = static_cast<int64_t>(M) * K, w_end = static_cast<int64_t>(K) * N;
+  const bool want_sums = e.comp_mul != 0 || e.prep.input_mode == ITEXHIP_MIN_FIRST;
+  uint8_t* const ws = lds[wave];
+  const int kb = (lane >> 1) * 4, nb = (lane & 1) * 16;  // [K, N] weight: 4 rows of 16 columns
+  v16i acc, sums;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = sums[i] = 0;
+  v4i fa[4], fw[4];
+  const bool row_here = m0 + l32 < M, column_here = n0 + nb < N;
+  auto a_off = [&](int c, int k0) { return static_cast<int64_t>(m0 + l32) * K + k0 + c * 32 + half * 16; };
+  auto w_off = [&](int c, int k0) { return static_cast<int64_t>(k0 + kb + c) * N + n0 + nb; };
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) fa[c] = fw[c] = v4i{0, 0, 0, 0};
+    if (row_here) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) fa[c] = fetch16(a, a_off(c, k0), a_end);
+    }
+    if (column_here) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) fw[c] = fetch16(w, w_off(c, k0), w_end);
+    }
+  };
+  int k0 = wave * kFewK;
+  if (k0 < K) fetch(k0);
+  const int n = n0 + l32;
+  RawChannel raw = load_raw_channel(e, min(n, N - 1), N);  // travels behind the operands
+  for (; k0 < K; k0 += WAVES * kFewK) {
+    if (k0 + kFewK + 16 > K) {  // pieces past a tensor's end; what lies past K is zero in the weight (see the other kernel)
+      if (m0 + kFew + 16 > M) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fa[c] = settle16(fa[c], a_off(c, k0), a_end);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        fw[c] = settle16(fw[c], w_off(c, k0), w_end);
+        if (k0 + kb + c >= K) fw[c] = v4i{0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t v[4];
+      transpose_bytes(fw, c, v);
+      // (the 16 columns of the other lanes would fall into the same banks: they keep their halves of a row the other way round)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(ws + (nb + 4 * c + j) * kFewRow + (kb ^ (nb << 2))) = v[j];
+    }
+    v4i x[4], y[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      x[c] = fa[c];
+      x[c].x ^= a_xor; x[c].y ^= a_xor; x[c].z ^= a_xor; x[c].w ^= a_xor;
+      y[c] = *reinterpret_cast<const v4i*>(ws + l32 * kFewRow + ((c * 32 + half * 16) ^ ((l32 & 16) << 2)));
+    }
+    if (k0 + WAVES * kFewK < K) fetch(k0 + WAVES * kFewK);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[c], y[c], acc, 0, 0, 0);
+    if (want_sums) {
+      const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) sums = __builtin_amdgcn_mfma_i32_32x32x32_i8(ones, y[c], sums, 0, 0, 0);
     }
   }
+  int* const mine = reinterpret_cast<int*>(ws) + lane;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) mine[i * 64] = acc[i];
+  if (half == 0) colsums[wave][l32] = sums[0];
+  __syncthreads();
+  constexpr int kPer = 16 / WAVES;  // results of a lane that this wavefront finishes, from `first` on
+  const int first = wave * kPer;
+  int sum[kPer];
+  raw.colsum = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) sum[i] = 0;
+#pragma unroll
+  for (int g = 0; g < WAVES; ++g) {
+    raw.colsum += colsums[g][l32];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) sum[i] += reinterpret_cast<const int*>(lds[g])[(first + i) * 64 + lane];
+  }
+  if (n >= N) return;
+  int comp;
+  float scale, bias;
+  finish_channel(e, raw, &comp, &scale, &bias);
+  // accumulator i of a lane: row (i / 4) * 8 + (lane / 32) * 4 + i % 4, column lane % 32
+  auto row_of = [&](int i) { return m0 + half * 4 + ((first + i) >> 2) * 8 + ((first + i) & 3); };
+  float v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    v[i] = static_cast<float>(sum[i] + comp) * scale;
+    v[i] = v[i] + bias;
+  }
+  apply_chain(e, v, [&](int i) { return static_cast<int64_t>(min(row_of(i), M - 1)) * N + n; });
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int m = row_of(i);
@@ -375,6 +509,22 @@ int launch(const uint8_t* a, uint32_t a_xor, const uint8_t* w, int transpose_b, 
   // 200 x 901 x 1000 10.2 / 8.9, 300 x 511 x 300 8.1 / 7.3; 2000 x 301 x 1000 (512 tiles) 9.4 / 13.0.  Two / one over 1500 sizes of
   // one step: [N, K] 0.93 - 1.07 (0.99 in the middle), [K, N] 0.96 - 1.10 (1.02: 3 x 43 x 68 5.6 / 6.1); of more steps 0.81 - 0.99.
   const bool split = tiles <= 256 && (transpose_b || K > kStepK);
+  // 32 x 32 tiles, time over the kernel that took these calls (1400 sizes of up to 4000 rows, columns and k): up to 256 of them 0.35 - 1.0
+  // (0.68 in the middle), 257 - 512 with K <= 512 0.73 - 0.94 (0.78), with more 0.84 - 1.16 (not there), more tiles 1.05 - 2.
+  const int64_t few_n = (N + kFew - 1) / kFew, few = (static_cast<int64_t>(M) + kFew - 1) / kFew * few_n;
+  if (!transpose_b && !forced && (few <= 256 || (few <= 512 && K <= 512))) {
+#define FEW(WAVES)                                                                                                               \
+  note_kernel(kLastUnpacked, WAVES / 4);                                                                                         \
+  qmatmul_unpacked_few_kernel<OUT_T, WAVES><<<static_cast<unsigned>((few + 7) / 8 * 8), 64 * WAVES, 0, st>>>(                     \
+      a, a_xor, w, M, K, N, static_cast<int>(few_n), static_cast<int>(few), e, out)
+    if (K > 4 * kFewK) {
+      FEW(8);
+    } else {
+      FEW(4);
+    }
+#undef FEW
+    return ITEXHIP_OK;
+  }
 #define TILES(S) (transpose_b ? launch_tiles<OUT_T, true, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st) \
                               : launch_tiles<OUT_T, false, S>(grid, a, a_xor, w, M, K, N, tiles_n, tiles, e, out, st))
   return split ? TILES(2) : TILES(1);
