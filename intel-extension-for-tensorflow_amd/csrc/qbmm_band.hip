@@ -388,14 +388,21 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 
 }  // namespace
 
-// Which calls come here, from 3700 products timed on both kernels (attention's two, 1 to 512 tokens, 8 to 4096 matrices; time of the
-// bands over that of the tiles, in the mean).  `large`: the tiles would be those of 128 rows, at least 1024 of them, which compute
-// past the edges of ragged matrices and hold few wavefronts per CU.  Everywhere while four workgroups (P.V: three) share the LDS of a CU;
+// Which calls come here, from 6900 products of these lines timed on both kernels (attention's two, 1 to 512 tokens, 8 to 4096 matrices; time
+// of the bands over that of the tiles, in the middle; of those that come 2 % take over 1.05, at most 1.29).  `large`: the tiles would be those of 128 rows, at least 1024 of them, which compute
+// past the edges of ragged matrices and hold few wavefronts per CU (aligned operands alone).  Everywhere while four workgroups (P.V: three) share the LDS of a CU;
 // above that (wide results) it is 0.98 - 1.4, but for the second line.
 // * y along k (Q.K^T), large: 16-bit results 0.70.
 // * the same, 32-bit results whose rows are no multiple of 64 bytes, which the tiles write in pieces of lines: 0.65 with fused operands,
-//   0.91 without them on rows that are no whole 16-byte vectors (others 1.08); at any size of the images.  Rows of whole 64-byte pieces
-//   up to 27 KB of LDS 0.68 (wider ones 1.10).
+//   0.93 without them on up to 192 columns that are no whole 16-byte vectors a row (others 1.08); at any size of the images.  Rows of
+//   whole 64-byte pieces up to 27 KB of LDS 0.68 (wider ones 1.10).
+// * not where rows are no whole vectors: 16-bit results of up to 64 columns, one tile wide, 0.77 - 1.35 (1.08), or of one k tile and more than
+// * not where few tiles (two for a CU) of at most three k steps make a launch that the staging of more than 64 columns of y is a part of: over
+//   96 columns, 64 with operands, 80 with 32-bit results 0.88 - 1.28 (1.09; 160 x 160 x 128, 12 times 4.4 -> 5.4);  a step more with operands and
+//   an unaligned y of more than 80 columns 1.03 - 1.13;  nor with operands and unaligned rows on 49 to 64 columns, one tile wide, in many
+//   tiles: 16-bit up to three k steps 0.84 - 1.27 (1.05; 107 x 107 x 64, 2085 times 14.6 -> 18.6), 32-bit up to five 0.97 - 1.20 (1.08).
+//   256 rows by up to 128 columns 0.79 - 1.31 (1.27; 315 x 64 x 107, 3881 times 102 -> 133 us);  32-bit results of more than 192 columns without
+//   operands 0.68 - 1.79 (1.21; 339 x 64 x 339, 265 times 32 -> 56), two workgroups or one on a CU that shift and store wide rows.
 // * y transposed on the way (P.V), 16-bit results: large 0.73; K > 128, where a tile's k steps, one round trip each, are most of its
 //   time, 0.84; K > 64 from 256 matrices on 0.92.  Below 0.95 - 1.07.
 // * the same, 32-bit results: K > 192 0.92 (1.00 unaligned to 64 columns), K > 128 aligned 0.9, or up to 32 columns 0.78.  Below
@@ -409,6 +416,15 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
     if (p.binary[b].stride_m != 0) return false;
   const int esz = p.out_type == ITEXHIP_FLOAT ? 4 : 2, ve = 16 / esz, N = static_cast<int>(p.N);
   const bool aligned_operands = mode_x == kAligned && mode_y == kAligned;
+  const bool operands = p.n_binary > 0, wide = esz == 4;
+  if (p.adj_y) {
+    if (!a.whole_rows && (wide ? !operands && N > 192 : N <= 64 || (p.K <= 64 && p.M > 256 && N <= 128))) return false;
+  } else {
+    const int64_t tiles = batch * ((p.M + 63) / 64) * ((N + 63) / 64);
+    if (tiles <= 512 && p.K <= 192 && N > (operands ? 64 : wide ? 80 : 96)) return false;
+    if (operands && !aligned_operands &&
+        (tiles > 2048 ? N > 48 && N <= 64 && p.K <= (wide ? 320 : 192) : !wide && tiles <= 256 && p.K <= 256 && N > 80)) return false;
+  }
   if (p.adj_y ? !large
               : esz == 2 ? !(large || p.K > 128 || (p.K > 64 && batch >= 256))
                          : !(p.K > 192 || (p.K > 128 && (aligned_operands || N <= 32)))) return false;

@@ -38,10 +38,36 @@ def test_many_matrices(hip, dev, M, K, N, t_out):
     import torch
     rng = np.random.default_rng(M * 7 + K + N)
     x, y = rng.integers(-128, 128, (129, 8, M, K)).astype(np.int8), rng.integers(-128, 128, (129, 8, N, K)).astype(np.int8)
+    # (16-bit rows of up to 64 columns that are no whole vectors are the tiles')
+    kernel = ("bmm_tiles", 21) if t_out != orc.FLOAT and N % 8 and N <= 64 else ("bmm_bands", 1)
     check(hip, dev, x, y, adj_y=True, binary=operands(torch, rng, N, t_out, 129), t_out=t_out)
-    assert hip.last_kernel() == ("bmm_bands", 1)
+    assert hip.last_kernel() == kernel
     check(hip, dev, x, y[:, :1], adj_y=True, binary=operands(torch, rng, N, t_out)[:1] if N == 20 else (), t_out=t_out)
-    assert hip.last_kernel() == ("bmm_bands", 1)
+    assert hip.last_kernel() == kernel
+
+
+# both sides of the lines between the bands and the tiles: y along k, then y transposed on the way
+@pytest.mark.parametrize("B,M,K,N,adj_y,t_out,n_ops,kernel", [
+    (1030, 70, 64, 61, True, orc.BFLOAT16, 1, "bmm_tiles"), (1030, 70, 64, 67, True, orc.BFLOAT16, 1, "bmm_bands"),
+    (345, 257, 64, 67, True, orc.HALF, 0, "bmm_tiles"), (345, 256, 64, 67, True, orc.HALF, 0, "bmm_tiles"), (520, 256, 64, 67, True, orc.HALF, 0, "bmm_bands"),
+    (515, 70, 64, 191, True, orc.FLOAT, 0, "bmm_bands"), (515, 70, 64, 193, True, orc.FLOAT, 0, "bmm_tiles"),
+    (515, 70, 64, 193, True, orc.FLOAT, 1, "bmm_bands"),
+    (64, 130, 192, 100, False, orc.BFLOAT16, 0, "bmm_tiles"), (64, 130, 208, 100, False, orc.BFLOAT16, 0, "bmm_bands"),
+    (86, 130, 192, 100, False, orc.BFLOAT16, 0, "bmm_bands"), (64, 130, 192, 96, False, orc.BFLOAT16, 0, "bmm_bands"),
+    (64, 130, 192, 72, False, orc.BFLOAT16, 2, "bmm_tiles"), (64, 130, 192, 80, False, orc.FLOAT, 0, "bmm_bands"),
+    (64, 130, 192, 84, False, orc.FLOAT, 0, "bmm_tiles"),
+    (40, 130, 199, 84, False, orc.HALF, 1, "bmm_tiles"), (43, 130, 199, 84, False, orc.HALF, 1, "bmm_bands"),
+    (2049, 20, 70, 52, False, orc.HALF, 1, "bmm_tiles"), (2048, 20, 70, 52, False, orc.HALF, 1, "bmm_bands"),
+    (2049, 20, 70, 48, False, orc.HALF, 1, "bmm_bands"), (2049, 20, 70, 52, False, orc.HALF, 0, "bmm_bands"),
+    (2049, 20, 199, 52, False, orc.FLOAT, 1, "bmm_tiles"), (2049, 20, 199, 48, False, orc.FLOAT, 1, "bmm_bands")])
+def test_lines_to_the_tiles(hip, dev, B, M, K, N, adj_y, t_out, n_ops, kernel):
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    x = rng.integers(-128, 128, (B, M, K)).astype(np.int8)
+    y = rng.integers(-128, 128, (B, N, K) if adj_y else (B, K, N)).astype(np.int8)
+    ops = [(alg, v.reshape(v.shape[1:] if v.ndim > 1 else v.shape)) for alg, v in operands(torch, rng, N, t_out)][:n_ops]
+    check(hip, dev, x, y, adj_y=adj_y, binary=ops, t_out=t_out)
+    assert hip.last_kernel()[0] == kernel
 
 
 @pytest.mark.parametrize("K,N,parts,t_out", [(64, 288, 2, orc.HALF), (32, 320, 2, orc.BFLOAT16), (200, 160, 2, orc.FLOAT), (193, 144, 2, orc.FLOAT)])
