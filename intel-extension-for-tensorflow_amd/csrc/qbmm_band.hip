@@ -159,8 +159,9 @@ __global__ __launch_bounds__(64 * kBandWaves, 4) void qbmm_band_kernel(const Ban
   };
 #pragma unroll
   for (int b = 0; b < NB; ++b) first[b] = operand(b, t);
-  if constexpr (ADJ_Y) {  // a thread: 16 k of a column; k fastest over the threads
-    const int y_last = N * K - 16, units = a.rows16 * a.k_tiles * 4;
+  if constexpr (ADJ_Y) {  // a thread: 16 k of a column, aligned; k fastest over the threads
+    static_assert(MODE == kAligned, "the rule takes no unaligned operands where y lies along k");
+    const int units = a.rows16 * a.k_tiles * 4;
     for (int u0 = t; u0 < units; u0 += 4 * 64 * kBandWaves) {
       v4i w[4];
       int n[4], k[4];
@@ -170,20 +171,11 @@ __global__ __launch_bounds__(64 * kBandWaves, 4) void qbmm_band_kernel(const Ban
         const int kt = KT == 1 ? 0 : i / a.rows16;
         n[u] = i - kt * a.rows16;
         k[u] = kt * kTile + (t & 3) * 16;
-        const int at = min(n_first + n[u], N - 1) * K + k[u];
-        if constexpr (MODE == kAligned) w[u] = *reinterpret_cast<const v4i*>(y + (k[u] < K ? at : 0));
-        else w[u] = *reinterpret_cast<const v4i_any*>(y + min(at, y_last));
+        w[u] = *reinterpret_cast<const v4i*>(y + (k[u] < K ? min(n_first + n[u], N - 1) * K + k[u] : 0));
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int left = K - k[u];  // bytes of the piece inside the row: the others are zero
-        if constexpr (MODE == kAny) {
-          w[u] = shift_down(w[u], static_cast<uint32_t>(max(min(n_first + n[u], N - 1) * K + k[u] - y_last, 0)) & 15u);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w[u][i] &= left >= 4 * i + 4 ? -1 : left <= 4 * i ? 0 : (1 << (left & 3) * 8) - 1;
-        } else if (left <= 0) {
-          w[u] = v4i{0, 0, 0, 0};
-        }
+        if (k[u] >= K) w[u] = v4i{0, 0, 0, 0};  // (K is a multiple of 16)
         if (u0 + u * (64 * kBandWaves) < units) *reinterpret_cast<v4i*>(lds + (k[u] >> 6) * k_bytes + y_piece<ADJ_Y>(n[u], t & 3)) = w[u];
       }
     }
@@ -366,8 +358,10 @@ void launch_modes(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* 
       device_bit(&raised, true);
     kernel<<<grid, 64 * kBandWaves, lds, st>>>(a, x, y, out);
   };
-  if (al) go(std::integral_constant<int, kAligned>{});
-  else go(std::integral_constant<int, kAny>{});
+  if constexpr (!ADJ_Y) {
+    if (!al) return go(std::integral_constant<int, kAny>{});
+  }
+  go(std::integral_constant<int, kAligned>{});
 }
 template <bool ADJ_Y, int OUT_T>
 void launch_ops(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x, const int8_t* y, char* out, hipStream_t st) {
@@ -416,6 +410,12 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
     if (p.binary[b].stride_m != 0) return false;
   const int esz = p.out_type == ITEXHIP_FLOAT ? 4 : 2, ve = 16 / esz, N = static_cast<int>(p.N);
   const bool aligned_operands = mode_x == kAligned && mode_y == kAligned;
+  if (p.adj_y ? !(large && aligned_operands)
+              : esz == 2 ? !(large || p.K > 128 || (p.K > 64 && batch >= 256))
+                         : !(p.K > 192 || (p.K > 128 && (aligned_operands || N <= 32)))) return false;
+  BandArgs a;
+  a.p = p;
+  a.whole_rows = N * esz % 16 == 0 && aligned(out, 16);
   const bool operands = p.n_binary > 0, wide = esz == 4;
   if (p.adj_y) {
     if (!a.whole_rows && (wide ? !operands && N > 192 : N <= 64 || (p.K <= 64 && p.M > 256 && N <= 128))) return false;
