@@ -1240,13 +1240,22 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       ITEXHIP_REQUIRE(col_blocks <= 65535, "itexhip_minmax_i32_per_channel: depth too large");
       // 16-byte loads: column blocks of one width (400000 x 260: 87 -> 73 us).  Single ints lose by it (100000 x 257: 28 -> 34).
       if (vec) groups = static_cast<int>((depth / per + col_blocks - 1) / col_blocks);
-      // Few rounds of loads: narrow column blocks (128 bytes, single ints 64) whose workgroup takes all rows; the launch that
-      // initialises costs more than what is lost in parallel reads (us, initialised / alone: 256 x 4096 5.0 / 3.0, 200 x 1000 5.0 / 3.3,
-      // 500 x 64 5.1 / 3.6, 1000 x 1000 5.0 / 5.6), and with a workgroup on every other CU some more rows (1024 x 4096 7.1 / 5.7,
-      // 4096 x 4096 14.5 / 13.6, 8192 x 4096 27 / 37: rows 16 KB apart meet in the same channels).
+      // Little to read: narrow column blocks (128 bytes, single ints 64) whose workgroup takes all rows; the launch that initialises
+      // costs more than what is lost in parallel reads (us, initialised / alone: 256 x 4096 5.0 / 3.0, 200 x 1000 5.0 / 3.3,
+      // 500 x 64 5.1 / 3.6, 1000 x 1000 5.0 / 5.6).  Counted in the pieces that a workgroup loads at a time (32 KB, single ints 8):
+      // * rows of whole 128-byte lines: two rounds up to 2048 pieces 0.56 - 0.95 of the time, more to 1.26 (56 x 89888 5.5 / 6.9); with a
+      //   workgroup on every other CU up to 16 rounds, 0.65 - 1.15, in the middle 0.95 (1024 x 4096 7.1 / 5.7, 4096 x 4096 14.5 / 13.6,
+      //   3304 x 5504 16.2 / 14.3, 3397 x 8576 20.3 / 23.5; 8192 x 4096 27 / 37).
+      // * other rows: neighbouring blocks share lines, which come once for each of their XCDs.  Two rounds up to 1024 pieces (single ints
+      //   2048) 0.55 - 1.05, three and four up to 640 0.77 - 1.02; more 0.76 - 2.0 (455 x 21180 9.6 / 12.3, 225 x 21487 6.4 / 9.9,
+      //   59 x 128396 7.2 / 14.5, 3773 x 17784 44 / 69).
+      // (launches of a captured graph; one by one from the host, where a second launch costs 2.5 us, the lone workgroups gain more)
       const int narrow = vec ? 8 : 16;
       const int64_t narrow_blocks = (depth / per + narrow - 1) / narrow, rounds = (rows + kRowUnroll * (kThreads / narrow) - 1) / (kRowUnroll * (kThreads / narrow));
-      const bool alone = !few && narrow_blocks <= 65535 && (rounds <= 2 || (vec && narrow_blocks >= 128 && rounds <= 16));
+      const bool lines = vec && depth % 32 == 0 && aligned(x, 128);
+      const int64_t pieces = rounds * narrow_blocks;
+      const bool alone = !few && narrow_blocks <= 65535 &&
+                         (rounds <= 2 ? pieces <= (lines || !vec ? 2048 : 1024) : vec && narrow_blocks >= 128 && rounds <= 16 && (lines || pieces <= 640));
       if (alone) {
         groups = static_cast<int>(std::min<int64_t>(narrow, depth / per));
         col_blocks = narrow_blocks;
