@@ -391,16 +391,16 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 //   0.93 without them on up to 192 columns that are no whole 16-byte vectors a row (others 1.08); at any size of the images.  Rows of
 //   whole 64-byte pieces up to 27 KB of LDS 0.68 (wider ones 1.10).
 // * not where rows are no whole vectors: 16-bit results of up to 64 columns, one tile wide, 0.77 - 1.35 (1.08), or of one k tile and more than
-// * not where few tiles (two for a CU) of at most three k steps make a launch that the staging of more than 64 columns of y is a part of: over
-//   96 columns, 64 with operands, 80 with 32-bit results 0.88 - 1.28 (1.09; 160 x 160 x 128, 12 times 4.4 -> 5.4);  a step more with operands and
-//   an unaligned y of more than 80 columns 1.03 - 1.13;  nor with operands and unaligned rows on 49 to 64 columns, one tile wide, in many
-//   tiles: 16-bit up to three k steps 0.84 - 1.27 (1.05; 107 x 107 x 64, 2085 times 14.6 -> 18.6), 32-bit up to five 0.97 - 1.20 (1.08).
 //   256 rows by up to 128 columns 0.79 - 1.31 (1.27; 315 x 64 x 107, 3881 times 102 -> 133 us);  32-bit results of more than 192 columns without
 //   operands 0.68 - 1.79 (1.21; 339 x 64 x 339, 265 times 32 -> 56), two workgroups or one on a CU that shift and store wide rows.
 // * y transposed on the way (P.V), 16-bit results: large 0.73; K > 128, where a tile's k steps, one round trip each, are most of its
 //   time, 0.84; K > 64 from 256 matrices on 0.92.  Below 0.95 - 1.07.
 // * the same, 32-bit results: K > 192 0.92 (1.00 unaligned to 64 columns), K > 128 aligned 0.9, or up to 32 columns 0.78.  Below
 //   1.0 - 1.2, large or not.
+// * not where few tiles (two for a CU) of at most three k steps make a launch that the staging of more than 64 columns of y is a part of: over
+//   96 columns, 64 with operands, 80 with 32-bit results 0.88 - 1.28 (1.09; 160 x 160 x 128, 12 times 4.4 -> 5.4);  a step more with operands and
+//   an unaligned y of more than 80 columns 1.03 - 1.13;  nor with operands and unaligned rows on 49 to 64 columns, one tile wide, in many
+//   tiles: 16-bit up to three k steps 0.84 - 1.27 (1.05; 107 x 107 x 64, 2085 times 14.6 -> 18.6), 32-bit up to five 0.97 - 1.20 (1.08).
 // Small launches of Q.K^T stay with the tiles (1.05 - 1.24): this kernel has a way through LDS more.
 bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_y, bool large, const int8_t* x, const int8_t* y, void* out,
                hipStream_t st) {
@@ -425,12 +425,6 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
     if (operands && !aligned_operands &&
         (tiles > 2048 ? N > 48 && N <= 64 && p.K <= (wide ? 320 : 192) : !wide && tiles <= 256 && p.K <= 256 && N > 80)) return false;
   }
-  if (p.adj_y ? !large
-              : esz == 2 ? !(large || p.K > 128 || (p.K > 64 && batch >= 256))
-                         : !(p.K > 192 || (p.K > 128 && (aligned_operands || N <= 32)))) return false;
-  BandArgs a;
-  a.p = p;
-  a.whole_rows = N * esz % 16 == 0 && aligned(out, 16);
   // rows of whole 64-byte pieces are cut into parts of at most 512 bytes, as even as they get (384 columns of fp32: 25.7 us whole,
   // 18.0 in three parts); the pieces of lines that parts of other rows would end in cost more than they give (216 columns of
   // fp32 in two parts 41 us, the tiles 23)
