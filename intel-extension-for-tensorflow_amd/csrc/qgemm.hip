@@ -582,18 +582,19 @@ enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or th
 
 // Which packed kernel takes a call.  The small-M kernel (a strip of channels x 16 or 32 rows x all of K per workgroup)
 // streams the weight once per block of rows; the tile kernel needs enough 64 x 64 tiles to fill the device.  Small-M / tile kernel, time,
-// with a chain that the tile kernel's vector epilogue finishes (6800 sizes of up to 2048 rows, K up to 4096; a sum is no exception), by
-// 64 x 64 tiles or by 32 x 32 pieces:
+// with a chain that the tile kernel's vector epilogue finishes (6800 sizes of up to 2048 rows, K up to 4096), by 64 x 64 tiles
+// or by 32 x 32 pieces:
 //   33 to 128 rows        up to 16 tiles 0.5 - 1.27 (K <= 256 1.03, 257 - 1024 0.9, more 0.69), 17 - 64 tiles up to 256 pieces K <= 1024
 //                         0.77 - 1.3 (1.0), more 0.59 - 1.0 (0.8);  65 - 128 tiles up to 256 pieces K 513 - 1024 0.84 - 1.11 (0.94), more
 //                         0.59 - 0.99 (0.8), else K <= 1536, or up to 64 rows, 0.9 - 1.5 (1.1: not there), longer 0.8 - 1.3 (1.05), more tiles 1.0 - 2.4.  Rows that
 //                         are no whole 16-byte vectors differ by 0.1 at most; with a K of one step, or K > 1536 and few more than
 //                         128 tiles, either kernel does.
-//   129 to 512 rows       up to 16 tiles K <= 256 0.78 - 1.27 (1.02: not there), 257 - 512 0.92;  up to 128 pieces K 513 - 1024 0.66 - 1.03
-//                         (0.83), more 0.47 - 0.9 (0.68);  129 - 256 pieces K <= 1024 0.77 - 1.3 (0.97: not there), more 0.60 - 0.98 (0.77);
-//                         more pieces 0.78 - 2
-//   513 to 2048 rows      up to 128 pieces K <= 512 0.83 - 1.27 (not there), 513 - 1024 0.68 - 1.03 (0.83), more 0.47 - 1.08 (0.71);  129 - 256
-//                         K <= 1024 0.72 - 1.4 (0.96: not there), more 0.70 - 1.14 (0.9);  more pieces 0.82 - 2
+//   129 to 2048 rows      (950 sizes of whole 16-byte rows) up to 128 pieces K <= 512 1.03 - 1.26 (1.18: not there), 513 - 768 0.93 - 1.12
+//                         (1.03: not there; 32-bit rows that are no whole vectors 0.85 - 0.93), 769 - 1024 0.83 - 1.0 (0.94), to 2048 0.70 - 0.97 (0.84), more 0.53 - 0.78 (0.65);  129 - 256
+//                         pieces K <= 1024 0.72 - 1.4 (0.97: not there), to 2048 0.74 - 1.0 (0.87), more 0.60 - 0.89 (0.75);  more pieces 0.78 - 2
+//   the same with a sum   up to 128 pieces K <= 512 1.01 - 1.36 (not there), 513 - 768 0.98 - 1.25 (not there), 769 - 1024 0.87 - 1.09 (1.02),
+//                         to 2048 0.72 - 1.03 (0.9), more 0.61 - 0.87 (0.72);  129 - 256 pieces K <= 1536 0.86 - 1.09 (1.0: not
+//                         there), more 0.75 - 0.95 (0.83)
 //   17 to 32 rows         (4600 sizes before that) K < 256 and over 128 tiles 1.0 - 1.7;  256 to 767, 129 - 256 tiles 0.9 - 1.15 (0.97:
 //                         not there), more 0.86 - 1.5;  from 768 on, 129 - 256 tiles, one per CU on the deep ring, 0.9 - 1.33, 257 - 512, a
 //                         second round for some of the CUs, 0.75 - 1.15 (not there)
@@ -609,14 +610,13 @@ static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int 
   CanonChain c;
   const int act = canon_chain(e, &c);
   const bool vector = vector_chain(e, act, c, N);
+  const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
+  const bool whole_rows = (N * esz) % 16 == 0 && aligned(out, 16);
   if (M > kSmallMaxRows) {
     if (!vector) return e.addend == nullptr && tiles <= 128 && K <= 2048;
-    if (M <= 512 && tiles <= 16 && K > 256) return true;
-    return pieces <= 128 ? K > 512 : pieces <= 256 && K > 1024;
+    return pieces <= 128 ? K > (esz == 4 && !whole_rows ? 512 : 768) : pieces <= 256 && K > (e.addend ? 1536 : 1024);
   }
   if (vector && e.addend == nullptr) {
-    const int esz = out_type == ITEXHIP_QINT8 || out_type == ITEXHIP_QUINT8 ? 1 : is_float16_type(out_type) ? 2 : 4;
-    const bool whole_rows = (N * esz) % 16 == 0 && aligned(out, 16);
     if (M > 32 && K >= 128 && tiles > 64 && (M <= 64 || K <= 1536) && !(pieces <= 256 && K > 512)) return false;
     if (whole_rows ? K >= 64 && tiles > 128 : K >= 128 && tiles > 144)
       if (M > 32 || K < 256 || (K < 768) == (tiles > 256)) return false;

@@ -47,7 +47,7 @@ def test_rows_of_any_length(hip, dev, M, K, N, shape):
             np.testing.assert_array_equal(got[off:off + M * N * esz], convert(torch, hip, np.ascontiguousarray(v), T).ravel())
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 70, 272), (140, 33, 1040), (512, 100, 784), (513, 64, 528), (1024, 30, 592), (17, 50, 1600), (64, 200, 3088),
+@pytest.mark.parametrize("M,N,K", [(129, 70, 784), (140, 33, 1040), (512, 100, 784), (513, 64, 848), (1024, 30, 976), (17, 50, 1600), (64, 200, 3088),
                                    (260, 700, 1040), (2048, 50, 2064), (100, 2040, 1040), (64, 2100, 272)])
 def test_small_m_kernel_on_more_rows_and_wavefronts(hip, dev, M, N, K):
     layer, w, bias = make_layer(hip, dev, K, N, seed=K + N)
@@ -58,9 +58,9 @@ def test_small_m_kernel_on_more_rows_and_wavefronts(hip, dev, M, N, K):
         assert hip.last_kernel()[0] == "small_m"
 
 
-@pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 256, "tile"), (512, 256, 272, "tile"), (512, 256, 528, "small_m"), (512, 257, 528, "tile"),
-                                          (513, 64, 528, "small_m"), (1024, 128, 528, "small_m"), (1024, 129, 528, "tile"), (1024, 256, 1024, "tile"),
-                                          (1024, 256, 1040, "small_m"), (1024, 257, 1040, "tile"), (2049, 32, 528, "tile"), (64, 4096, 128, "small_m"),
+@pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 768, "tile"), (129, 64, 784, "small_m"), (129, 65, 512, "tile"), (129, 65, 528, "small_m"), (512, 256, 768, "tile"), (512, 256, 784, "small_m"),
+                                          (512, 257, 784, "tile"), (1024, 128, 784, "small_m"), (1024, 129, 784, "tile"), (1024, 256, 1024, "tile"),
+                                          (1024, 256, 1040, "small_m"), (1024, 257, 1040, "tile"), (2048, 64, 784, "small_m"), (2049, 32, 784, "tile"), (64, 4096, 128, "small_m"),
                                           (64, 4160, 128, "tile"), (128, 2112, 1536, "tile"), (128, 2112, 1552, "small_m"),
                                           (96, 2112, 512, "tile"), (96, 2112, 528, "small_m")])
 def test_line_between_the_kernels(hip, dev, M, N, K, kernel):

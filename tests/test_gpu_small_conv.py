@@ -95,7 +95,8 @@ def test_line_to_the_tile_kernel(hip, dev, B, hw, C, k, O, kernel):
     assert torch.equal(*got)
 
 
-@pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 1040, "small_m"), (260, 512, 1040, "small_m"), (2048, 60, 528, "small_m"), (513, 512, 1040, "tile")])
+@pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 768, "tile"), (129, 64, 784, "small_m"), (260, 512, 1536, "tile"), (260, 512, 1552, "small_m"),
+                                          (2048, 60, 1040, "small_m"), (513, 512, 1552, "tile")])
 @pytest.mark.parametrize("addend_type", ["float", "quint8"])
 def test_matmul_with_a_sum(hip, dev, M, N, K, kernel, addend_type):
     import torch
