@@ -768,14 +768,19 @@ extern "C" int itexhip_qconv2d_implicit_ok(const itexhip_conv_geometry* g, const
 }
 
 namespace {
+constexpr int64_t kXcdL2 = 4 << 20;
+
 // Whether the small-M kernel takes a convolution that neither the direct nor the short-K kernel does.  Few 64 x 64 tiles
 // with a long K are a chain of K steps, whose window arithmetic a ring of loads does not hide; here up to 8 wavefronts
 // share the steps.  Time over the tile kernel's, by 32 x 32 pieces of the result (700 shapes: 1 x 1 to 5 x 5 windows, 64 to
 // 1024 channels, strides 1 and 2):
-//   up to 256      K <= 512 0.9 - 1.28 (not there), 576 - 1024 0.73 - 1.03 (0.88), to 2048 0.59 - 0.77 (0.65), to 4096 0.45 - 0.64
-//                  (0.56), more 0.26 - 0.55 (0.40)
-//   257 - 512      K <= 1024 0.86 - 1.28 (not there), to 2048 0.80 - 0.94 (0.87), to 4096 0.61 - 0.81 (0.69), more 0.47 - 0.83 (0.61)
-//   513 - 768      K <= 4096 0.85 - 1.6 (not there), more 0.71 - 1.10 (0.84);  more pieces 0.82 - 2.5: not there
+//   up to 256      K <= 512 0.9 - 1.28 (not there), 576 0.88 - 1.01, 640 - 1024 0.73 - 0.95 (0.86), to 2048 0.59 - 0.77 (0.65), to 4096
+//                  0.45 - 0.64 (0.56), more 0.26 - 0.55 (0.40)
+//   257 - 512      K <= 1024 0.86 - 1.28 (not there), to 2048 0.80 - 0.97 (0.87), to 4096 0.61 - 0.81 (0.69), more 0.47 - 0.83 (0.61)
+//   513 - 768      K <= 4096 0.85 - 1.6 (not there), more 0.70 - 0.96 (0.84), but 1.08 - 1.38 where the input that an XCD's pieces read (they
+//                  walk the rows of one 32-channel strip after the other) does not stay in its L2: not there.  More pieces 0.82 - 2.5: not there
+// With a sum, whose summands are read behind the reduction, 576 is 0.95 - 1.11, 1088 and 1152 0.95 - 1.05, and 4160 to 4800 over 512
+// pieces 0.9 - 1.04: not there.
 // 3 x 3, 7 x 7 x 512 -> 512, 1 image 16.9 -> 6.5 us, 8 images 17.3 -> 7.9, 32 images (784 pieces) 17.9 there;
 // 14 x 14 x 256 -> 256, 1 image 10.1 -> 6.1, 8 images 10.5 -> 7.4.
 bool small_conv(int64_t M, int64_t K, int64_t N, const ConvTileArgs& cv, const EpilogueArgs& e) {
@@ -786,8 +791,12 @@ bool small_conv(int64_t M, int64_t K, int64_t N, const ConvTileArgs& cv, const E
   if ((c.flags & (kChainSumFirst | kChainSumLast)) &&
       (e.addend == nullptr || N % 4 != 0 || !aligned(e.addend, e.addend_type == ITEXHIP_FLOAT ? 16 : 4)))
     return false;
-  const int64_t pieces = ((M + 31) / 32) * ((N + 31) / 32);
-  return pieces <= 256 ? K > 512 : pieces <= 512 ? K > 1024 : pieces <= 768 && K > 4096;
+  const int64_t strips = (N + 31) / 32, pieces = ((M + 31) / 32) * strips;
+  const bool sum = e.addend != nullptr;
+  if (pieces <= 256) return K > (sum ? 576 : 512);
+  if (pieces <= 512) return K > (sum ? 1152 : 1024);
+  const int64_t input = M / (static_cast<int64_t>(cv.out_h) * cv.out_w) * cv.in_h * cv.in_w * cv.in_c;
+  return pieces <= 768 && K > (sum ? 4800 : 4096) && input * std::min<int64_t>(strips, 8) <= 8 * kXcdL2;
 }
 
 int qconv2d_impl(const char* who, const void* x, int x_type, const itexhip_conv_geometry* g, const int8_t* packed_filter,

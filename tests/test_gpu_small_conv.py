@@ -68,16 +68,19 @@ def test_convolutions(hip, dev, shape, k, O, stride, dil, pad, out, signed_in):
             hip.qconv2d(*args, T, y)
         else:
             hip.qconv2d_sum(*args, torch.from_numpy(addend).to(dev), addend_type, T, y)
-        assert hip.last_kernel()[0] == "small_m"
+        pieces = -(-M // 32) * -(-O // 32)
+        tile = addend is not None and K <= (576 if pieces <= 256 else 1152 if pieces <= 512 else 4800)
+        assert hip.last_kernel()[0] == ("tile" if tile else "small_m")
         got = y.cpu().numpy()
         assert (got[M * O * esz:] == 0x5a).all()
         np.testing.assert_array_equal(got[:M * O * esz], convert(torch, hip, finish(v0, elts, hip, addend), T).ravel())
 
 
-# up to 256, 512 and 768 blocks of 32 x 32, and the K from which on
+# up to 256, 512 and 768 blocks of 32 x 32, and the K from which on; beyond 512 up to 4 MB of input for each XCD
 @pytest.mark.parametrize("B,hw,C,k,O,kernel", [(1, 16, 512, 1, 1024, "tile"), (1, 16, 576, 1, 1024, "small_m"), (1, 16, 1024, 1, 1040, "tile"),
                                                (1, 16, 1088, 1, 1040, "small_m"), (1, 16, 1088, 1, 2064, "tile"), (1, 16, 4096, 1, 2064, "tile"),
-                                               (1, 16, 4160, 1, 2064, "small_m"), (1, 16, 4160, 1, 3088, "tile"), (1, 5, 592, 1, 64, "tile")])
+                                               (1, 16, 4160, 1, 2064, "small_m"), (1, 16, 4160, 1, 3088, "tile"), (1, 5, 592, 1, 64, "tile"),
+                                               (11, 9, 4480, 1, 576, "small_m"), (12, 9, 4480, 1, 576, "tile")])
 def test_line_to_the_tile_kernel(hip, dev, B, hw, C, k, O, kernel):
     import torch
     g = hip.ConvGeometry(B, hw, hw, C, k, k, hw, hw, 1, 1, 1, 1, 0, 0)
