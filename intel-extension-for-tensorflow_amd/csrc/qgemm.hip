@@ -539,10 +539,14 @@ int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
   // beyond; convolutions 0.95 - 1.0).  257 to 512 workgroups: 4 wavefronts over 1 or 2 of twice the pairs 0.73 - 1.09 (0.9);  more: 2
   // over up to 8 0.75 - 1.04 (0.99).  (4000 sizes.)
   // Up to 16 rows: 32-channel strips when they give every CU a workgroup, and about 8 chunk pairs for each of up to 8 wavefronts (16 pairs
-  // 0.88 - 1.35 of the time, 1.09 in the middle; 16 x 1024 -> 1024 4.4 -> 5.8 us).  With ranges per row one wavefront of a workgroup
-  // works out a table for every row, and more of the others are in its way: 16 pairs from 9 rows on (0.72 - 1.2 of the time, 0.97; 12 x 4080 ->
-  // 4624 10.3 -> 7.9 us), and from 5 rows on where CUs hold more than one workgroup and K > 1472 (0.79 - 1.0, 0.91); fewer rows or
-  // less K 0.91 - 1.42 (1.09: not there).  Prefer a count that divides K into whole batches.
+  // 0.88 - 1.35 of the time, 1.09 in the middle; 16 x 1024 -> 1024 4.4 -> 5.8 us).  Where CUs hold more than one workgroup the wavefronts
+  // of the others hide a longer run, and fewer partial tiles meet at the end: 16 pairs there from 9 rows on for K of 2561 (32-channel strips 2049)
+  // to 5120 (4608), from 5 on for 3073 to as much: 0.84 - 1.1 of the time, 16-channel strips 0.93, others 0.98 in the middle (1500 sizes; 13 x
+  // 4048 -> 6148 8.4 -> 7.6 us); less K 1.0 - 1.2, more 0.95 - 1.09.
+  // With ranges per row one wavefront of a workgroup works out a table for every row, and more of the others are in its way: 16 pairs
+  // from 9 rows on (0.72 - 1.2 of the time, 0.97; 12 x 4080 -> 4624 10.3 -> 7.9 us), and from 5 rows on where CUs hold more than one
+  // workgroup and K > 1024 (0.79 - 1.0, 0.91); fewer rows or less K 0.91 - 1.42 (1.09: not there).  Prefer a count that divides K into whole
+  // batches.
   const int KC = 2 * ((K + 63) / 64), KP = KC / 2;
   const bool blocks = CONV || M > 16;
   const int row_blocks = blocks ? (M + 31) / 32 : 1;
@@ -558,10 +562,17 @@ int dispatch_gemv(const uint8_t* a, uint32_t a_xor, const uint8_t* bp, int M, in
     for (int w = waves - 1; w >= std::max(nt, most / 2 + 1) && batches(w) == batches(waves); --w) waves = w;
   } else {
     nt = workgroups(2) >= 256 ? 2 : 1;
-    const int per_wave = e.row_min_a && (M > 8 || (M > 4 && workgroups(nt) > 256 && KP >= 24)) ? 16 : 8;
-    waves = std::max(nt, std::min(8, (KP + per_wave - 1) / per_wave));
-    for (int w = waves; w >= std::max(nt, waves / 2 + 1); --w)
-      if (KP % (2 * w) == 0) { waves = w; break; }
+    const bool more = workgroups(nt) > 256;
+    const bool longer = e.row_min_a ? M > 8 || (M > 4 && more && KP > 16)
+                                    : more && M > 4 && KP > (M <= 8 ? 48 : nt == 1 ? 40 : 32) && KP <= (nt == 1 ? 80 : 72);
+    auto wavefronts = [&](int pairs) {
+      const int most = std::max(nt, std::min(8, (KP + pairs - 1) / pairs));
+      for (int w = most; w >= std::max(nt, most / 2 + 1); --w)
+        if (KP % (2 * w) == 0) return w;
+      return most;
+    };
+    waves = wavefronts(longer ? 16 : 8);
+    if (longer && !e.row_min_a && waves < 3) waves = wavefronts(8);  // (two of 20 and more: 9 x 2528 -> 7564 6.1 -> 7.2 us)
   }
   const int cnt = (KP + waves - 1) / waves;
   if (nt == 2) return launch_gemv<2, OUT_T, CONV>(a, a_xor, bp, M, K, N, KC, waves, cnt, e, out, st, cv);

@@ -1,5 +1,5 @@
 """The tile kernel's vector epilogue on output rows that are no whole 16-byte vectors or start off a 16-byte boundary: every
-result type and tile shape, the last piece of a row in parts; and the small-M kernel beyond 128 rows.  Against int64 sums and the
+result type and tile shape, the last piece of a row in parts; and the small-M kernel beyond 128 rows, and with longer runs of K.  Against int64 sums and the
 epilogue's separately rounded fp32 steps, bit for bit, with the bytes around the result untouched."""
 import numpy as np
 import pytest
@@ -48,7 +48,8 @@ def test_rows_of_any_length(hip, dev, M, K, N, shape):
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 70, 784), (140, 33, 1040), (512, 100, 784), (513, 64, 848), (1024, 30, 976), (17, 50, 1600), (64, 200, 3088),
-                                   (260, 700, 1040), (2048, 50, 2064), (100, 2040, 1040), (64, 2100, 272)])
+                                   (260, 700, 1040), (2048, 50, 2064), (100, 2040, 1040), (64, 2100, 272),
+                                   (9, 4112, 2576), (16, 4100, 5120), (5, 8208, 3088), (13, 8208, 4608)])
 def test_small_m_kernel_on_more_rows_and_wavefronts(hip, dev, M, N, K):
     layer, w, bias = make_layer(hip, dev, K, N, seed=K + N)
     x, xq, mn, mx = make_acts(M, K, seed=M + K)
