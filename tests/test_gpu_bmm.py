@@ -156,9 +156,10 @@ def test_random_shapes_layouts_and_operands(hip, dev, seed):
 @pytest.mark.parametrize("adj_x,adj_y", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,K,N", [(72, 48, 132), (128, 64, 128), (100, 80, 36), (68, 16, 64)])
 def test_tiles_of_128_rows(hip, dev, adj_x, adj_y, M, K, N):
-    """Calls with at least 1024 tiles of 128 rows, aligned operands and fused operands that do not depend on the row run
-    tiles of 128 x 128 (N > 64) or 128 x 64 outputs, ragged at both edges here; every layout, fp32 without operands,
-    bfloat16 with a scalar Mul and a mask broadcast over the rows, and with a per-row operand the 64 x 64 tiles again."""
+    """Calls with at least 1024 tiles of 128 rows, aligned operands and fused operands that do not depend on the row: tiles
+    of 128 x 128 (N > 64) or 128 x 64 outputs where x is transposed, and for fp32 results here; bands of 16 rows for the bfloat16
+    results of an x that is not.  Ragged at both edges; every layout, fp32 without operands, bfloat16 with a scalar Mul and a mask
+    broadcast over the rows, and with a per-row operand the 64 x 64 tiles."""
     import torch
     rng = np.random.default_rng(M + K + N + adj_x * 2 + adj_y)
     B = (1030,)
@@ -171,6 +172,30 @@ def test_tiles_of_128_rows(hip, dev, adj_x, adj_y, M, K, N):
     if (adj_x, adj_y) == (False, True):
         per_row = rng.standard_normal((1, M, 1)).astype(np.float32)
         check(hip, dev, x, y, adj_x, adj_y, binary=((orc.BIN_ADD, per_row),))
+
+
+@pytest.mark.parametrize("B,M,K,N,adj_y,t_out,tiles", [
+    (1024, 128, 64, 128, True, orc.FLOAT, 22),      # rows of whole 64-byte pieces, an image above 27 KB
+    (1024, 68, 32, 64, False, orc.FLOAT, 21),       # up to 128 k
+    (1024, 65, 128, 36, False, orc.FLOAT, 21),
+    (342, 72, 64, 300, True, orc.BFLOAT16, 22),     # images above 40 KB
+    (342, 66, 48, 300, True, orc.HALF, 22),
+    (1024, 65, 400, 20, False, orc.BFLOAT16, 21),   # more k than bands take
+    (1024, 70, 400, 16, True, orc.HALF, 21)])
+def test_tiles_of_128_rows_beside_the_bands(hip, dev, B, M, K, N, adj_y, t_out, tiles):
+    """x not transposed and beyond the lines of the bands, with a scalar Mul and a mask of the matrix, and without operands."""
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    x = rng.integers(-128, 128, (B, M, K)).astype(np.int8)
+    y = rng.integers(-128, 128, (B, N, K) if adj_y else (B, K, N)).astype(np.int8)
+    binary = [(orc.BIN_MUL, np.float32([0.125])), (orc.BIN_ADD, rng.standard_normal((B, 1, N)).astype(np.float32))]
+    if t_out != orc.FLOAT:
+        binary = [(alg, to16(torch, v, t_out)) for alg, v in binary]
+    check(hip, dev, x, y, False, adj_y, binary=binary, t_out=t_out)
+    assert hip.last_kernel() == ("bmm_tiles", tiles)
+    if adj_y and t_out == orc.FLOAT or K > 384:
+        check(hip, dev, x, y, False, adj_y, t_out=t_out)
+        assert hip.last_kernel() == ("bmm_tiles", tiles)
 
 
 def test_empty_and_invalid(hip, dev):
