@@ -272,10 +272,10 @@ def check_implicit_conv(hip, dev, shape, wshape, strides, dil, lead, signed_in, 
 @pytest.mark.parametrize("position,alpha", [(1, 0.0), (2, 0.0), (1, 0.2), (2, None)])
 def test_sum_post_op_in_conv_and_gemm(hip, dev, t_add, position, alpha, n_out):
     """One sum post-op (y += scale * addend, the addend float / qint8 / quint8) before or after the activation, through
-    itexhip_qconv2d_sum (implicit GEMM), itexhip_qgemm_sum on the patch matrix (tile kernel), on 16 rows of it
-    (the M <= 16 kernel) and in place (output buffer = addend buffer): all equal to the oracle's epilogue on the
-    int32 convolution.  Output channel counts whose rows are 16-byte aligned (48), only 4-byte aligned (44, 100), with
-    whole 32-channel tiles (read as row segments when the addend is 8-bit) and a ragged last one."""
+    itexhip_qconv2d_sum (implicit GEMM), itexhip_qgemm_sum on the patch matrix and on 16 rows of it (the small-M kernel in
+    blocks of 32 and of 16 rows) and in place (output buffer = addend buffer): all equal to the oracle's epilogue on the
+    int32 convolution.  Output channel counts whose rows are 16-byte aligned (48) and only 4-byte aligned (44, 100), with
+    whole 32-channel tiles and a ragged last one."""
     import torch
     from tests.test_oracle_conv import ref_int_conv
     rng = np.random.default_rng(position * 10 + len(t_add))

@@ -47,6 +47,54 @@ def test_rows_of_any_length(hip, dev, M, K, N, shape):
             np.testing.assert_array_equal(got[off:off + M * N * esz], convert(torch, hip, np.ascontiguousarray(v), T).ravel())
 
 
+@pytest.mark.parametrize("N", [44, 100])
+@pytest.mark.parametrize("K,shapes", [(192, (0, 1, 2, 3, 4)), (80, (3, 4))])
+def test_sums_on_rows_of_any_length(hip, dev, N, K, shapes):
+    """8-bit rows of whole words, 32-bit and 16-bit results off a 16-byte boundary: the addend's row segments, the ragged last
+    channels, the sum before and after the activation, and in place."""
+    import torch
+    f, M = np.float32, 260
+    rng = np.random.default_rng(N + K)
+    x, w = rng.integers(0, 256, (M, K)).astype(np.uint8), rng.integers(-128, 128, (K, N)).astype(np.int8)
+    scale, bias = (rng.random(N).astype(f) + f(0.5)) * f(0.003), (rng.standard_normal(N) * 9).astype(f)
+    v0 = (x.astype(np.int64) @ w.astype(np.int64)).astype(f) * scale + bias
+    packed, colsum = torch.empty(hip.qgemm_packed_bytes(K, N), dtype=torch.int8, device=dev), torch.empty(N, dtype=torch.int32, device=dev)
+    hip.qgemm_prepack_b(torch.from_numpy(w).to(dev), False, K, N, packed, colsum)
+    d = [torch.from_numpy(a).to(dev) for a in (x, scale, bias)]
+    addends = {hip.QUINT8: rng.integers(0, 256, (M, N)).astype(np.uint8), hip.QINT8: rng.integers(-128, 128, (M, N)).astype(np.int8),
+               hip.FLOAT: (rng.standard_normal((M, N)) * 30).astype(f)}
+    total, relu = (hip.ELT_SUM, 0.75, 0.0), (hip.ELT_RELU, 0.0, 0.0)
+    for T, off in ((hip.QUINT8, 0), (hip.QINT8, 4), (hip.FLOAT, 4), (hip.BFLOAT16, 2)):
+        esz = {hip.FLOAT: 4, hip.BFLOAT16: 2}.get(T, 1)
+        for t_add, add in addends.items():
+            for elts in ((total, relu), (relu, total)):
+                v = v0
+                for e in elts:
+                    v = v + f(0.75) * add.astype(f) if e is total else np.maximum(v, f(0))
+                want = convert(torch, hip, np.ascontiguousarray(v), T).ravel()
+                ep = hip.Epilogue()
+                ep.n_scales, ep.n_eltwise = N, 2
+                for i, e in enumerate(elts):
+                    ep.elt[i].alg, ep.elt[i].alpha, ep.elt[i].beta = e
+                add_d = torch.from_numpy(add).to(dev)
+                for shape in shapes:
+                    hip.force_tile_shape(matmul=shape)
+                    out = torch.full((M * N * esz + 64,), 0x5a, dtype=torch.uint8, device=dev)
+                    to = out[off:off + M * N * esz]
+                    hip.qgemm_sum(d[0], hip.QUINT8, packed, colsum, M, K, N, d[1], d[2], ep, add_d, t_add, T, to)
+                    # (tiles wider than 128: the vector epilogue has them, the element-wise one does not)
+                    assert hip.last_kernel()[:3] == ("tile", *[(256, 256), (256, 192), (256, 128), (128, 128), (64, 64)][shape])
+                    got = out.cpu().numpy()
+                    assert (got[:off] == 0x5a).all() and (got[off + M * N * esz:] == 0x5a).all()
+                    np.testing.assert_array_equal(got[off:off + M * N * esz], want)
+                    if esz == 1 and t_add != hip.FLOAT:   # the addend is the output's buffer
+                        to.copy_(add_d.view(torch.uint8).ravel())
+                        hip.qgemm_sum(d[0], hip.QUINT8, packed, colsum, M, K, N, d[1], d[2], ep, to, t_add, T, to)
+                        got = out.cpu().numpy()
+                        assert (got[:off] == 0x5a).all() and (got[off + M * N * esz:] == 0x5a).all()
+                        np.testing.assert_array_equal(got[off:off + M * N * esz], want)
+
+
 @pytest.mark.parametrize("M,N,K", [(129, 70, 784), (140, 33, 1040), (512, 100, 784), (513, 64, 848), (1024, 30, 976), (17, 50, 1600), (64, 200, 3088),
                                    (260, 700, 1040), (2048, 50, 2064), (100, 2040, 1040), (64, 2100, 272),
                                    (9, 4112, 2576), (16, 4100, 5120), (5, 8208, 3088), (13, 8208, 4608)])
