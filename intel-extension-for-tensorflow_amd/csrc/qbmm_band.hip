@@ -44,17 +44,6 @@ typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u2_any __attribute__((ext_vector_type(2), aligned(2)));
 
-// 16 bytes of which the last 16 - n belong to the next row: moved down by n (0 .. 15), zeros behind
-__device__ __forceinline__ v4i shift_down(v4i w, uint32_t n) {
-  uint64_t lo = static_cast<uint64_t>(static_cast<uint32_t>(w[1])) << 32 | static_cast<uint32_t>(w[0]);
-  uint64_t hi = static_cast<uint64_t>(static_cast<uint32_t>(w[3])) << 32 | static_cast<uint32_t>(w[2]);
-  if (n & 8) { lo = hi; hi = 0; }
-  const uint32_t bits = (n & 7) * 8;
-  lo = lo >> bits | (hi << 1) << (63 - bits);
-  hi = hi >> bits;
-  return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
-}
-
 // 16 bytes at base + at (wave-uniform base).  Written through for the product that the attention block reads again (streaming stores
 // are faster by themselves, and what reads the result waits longer: 128 x 128 tokens, P.V to bfloat16 + QuantizeV2 8.7 + 5.0 us
 // streaming, 8.6 + 4.3 written through, 9.6 + 4.3 plain) and for 16-bit results; fp32 scores stream.

@@ -88,14 +88,10 @@ __device__ __forceinline__ void settle_tile(int64_t R, int64_t K, int64_t r0, in
     const int left = static_cast<int>(K - k0) - (t & 3) * 16;  // bytes of this piece inside the row
     if (left >= 16) return;
     const uint32_t shift = left > 0 ? 16 - left : 0;           // 1 .. 15
-    uint64_t lo = static_cast<uint64_t>(w[1]) << 32 | w[0], hi = static_cast<uint64_t>(w[3]) << 32 | w[2];
-    if (shift & 8) { lo = hi; hi = 0; }
-    const uint32_t bits = (shift & 7) * 8;
-    lo = lo >> bits | (hi << 1) << (63 - bits);
-    hi = hi >> bits;
-    if (left <= 0) lo = hi = 0;
-    w[0] = static_cast<uint32_t>(lo); w[1] = static_cast<uint32_t>(lo >> 32);
-    w[2] = static_cast<uint32_t>(hi); w[3] = static_cast<uint32_t>(hi >> 32);
+    v4i v = shift_down(v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])}, shift);
+    if (left <= 0) v = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = static_cast<uint32_t>(v[i]);
   } else {
     if (r0 + kTile > R) {
       const int over = static_cast<int>(r0 - (R - 4)) + (t & 15) * 4;  // how far the load was moved back
@@ -109,19 +105,6 @@ __device__ __forceinline__ void settle_tile(int64_t R, int64_t K, int64_t r0, in
         if (k0 + (t >> 4) * 4 + i >= K) w[i] = 0;
     }
   }
-}
-
-// 4 x 4 bytes in two rounds of byte permutes: byte j of the four words -> word j  (v_perm_b32 numbers the bytes of its second
-// operand 0..3 and of its first 4..7)
-__device__ __forceinline__ void transpose_4x4(const uint32_t (&w)[4], uint32_t (&v)[4]) {
-  const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);  // w0.b0 w1.b0 w0.b1 w1.b1
-  const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);  // w0.b2 w1.b2 w0.b3 w1.b3
-  const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
-  const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
-  v[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-  v[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-  v[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-  v[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
 }
 
 template <bool KCONT>

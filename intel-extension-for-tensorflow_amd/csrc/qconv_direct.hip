@@ -35,8 +35,6 @@ struct DirectArgs : DirectGeometry<FastDiv> {
   int comp_mul, n_scales;
 };
 
-static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
-
 // Registers: 126 with 32 channels, four wavefronts per SIMD; 152 with 64 (72 of weight), three; 200 and 224 (144 of weight), two.
 template <int OUT_T, int POST, int C32>
 __global__ __launch_bounds__(256, C32 == 1 ? 4 : C32 == 2 ? 3 : 2) void qconv_direct_kernel(

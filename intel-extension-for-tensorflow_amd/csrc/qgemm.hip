@@ -108,7 +108,6 @@ __global__ __launch_bounds__(256) void prepack_b_kernel(const int8_t* __restrict
 // or, where the pixel lies in the padding, reads zeros.
 // ------------------------------------------------------------------------------------------------
 constexpr int kGemvBatch = 4;                 // chunk pairs per batch of the 32-row kernel (2 for up to 16 rows, see UB below)
-static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};  // what a window reads in the padding
 constexpr int kGemvPanelWords = 6 + 32;       // per channel of the strip: 6 parameter words + {scale, bias} of 16 rows
 
 // UB: chunk pairs per batch; two batches of a wavefront are in flight.  2 for up to 16 rows, 4 for the blocks of 32

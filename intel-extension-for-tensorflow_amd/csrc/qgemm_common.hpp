@@ -13,6 +13,33 @@ namespace itexhip {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
+// 16 bytes moved down by n (0 .. 15), zeros behind: a piece whose first n bytes lie in front of what was asked for
+__device__ __forceinline__ v4i shift_down(v4i w, uint32_t n) {
+  uint64_t lo = static_cast<uint64_t>(static_cast<uint32_t>(w[1])) << 32 | static_cast<uint32_t>(w[0]);
+  uint64_t hi = static_cast<uint64_t>(static_cast<uint32_t>(w[3])) << 32 | static_cast<uint32_t>(w[2]);
+  if (n & 8) { lo = hi; hi = 0; }
+  const uint32_t bits = (n & 7) * 8;
+  lo = lo >> bits | (hi << 1) << (63 - bits);
+  hi = hi >> bits;
+  return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
+}
+
+// 4 x 4 bytes in two rounds of byte permutes: byte j of the four words -> word j  (v_perm_b32 numbers the bytes of its second
+// operand 0..3 and of its first 4..7)
+__device__ __forceinline__ void transpose_4x4(const uint32_t (&w)[4], uint32_t (&v)[4]) {
+  const uint32_t lo01 = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);  // w0.b0 w1.b0 w0.b1 w1.b1
+  const uint32_t hi01 = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);  // w0.b2 w1.b2 w0.b3 w1.b3
+  const uint32_t lo23 = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+  const uint32_t hi23 = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+  v[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+  v[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+  v[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+  v[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+
+// what a convolution's window reads in the padding
+static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
+
 __device__ __forceinline__ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 constexpr int kChunkRows = 32;     // rows (output channels or activation rows) per operand chunk

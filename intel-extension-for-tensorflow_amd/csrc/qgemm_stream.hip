@@ -39,8 +39,6 @@ struct StreamArgs {
   float sum_scale;
 };
 
-static __device__ __align__(16) const uint32_t kZeros[4] = {0u, 0u, 0u, 0u};
-
 // 128 vector registers for four wavefronts per SIMD, without scratch but for groups of 4 with a residual (it costs a launch
 // 1.5 us); up to 26 scalar registers go to lanes of a vector register.
 // HOLD: the K chunks of a tile are exactly GROUP; all are held at once, and each is replaced by the next tile's as soon as its

@@ -88,7 +88,6 @@ inline int xcd_rectangles(int num_m, int num_n, int BM, int BN, int K) {
 // run of 4 or 2 pixels of one window row, which the host admits only where no window touches the padding.  Either way
 // only the source address of an activation load changes: row -> window origin once per kernel, piece -> offset inside
 // the window from a table in LDS.
-static __device__ __align__(16) const uint32_t kZeroPiece[4] = {0u, 0u, 0u, 0u};
 
 // amask: 0x80808080 when the activations are unsigned (they are fed as x ^ 0x80), else 0; a scalar
 // register operand, so the sign flip costs a 4-byte instruction per dword.  KALIGNED: K is a multiple
@@ -212,7 +211,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
         const bool inside = static_cast<unsigned>(ih) < static_cast<unsigned>(cv.in_h) &&
                             static_cast<unsigned>(iw) < static_cast<unsigned>(cv.in_w);
         const uint8_t* src = inside ? a + static_cast<int>(off_a[ci] + static_cast<uint32_t>(piece.y))
-                                    : reinterpret_cast<const uint8_t*>(kZeroPiece);
+                                    : reinterpret_cast<const uint8_t*>(kZeros);
         lds_dma16(src, stage_addr + (wave * A_PER_WAVE + ci) * kChunkBytes);
       } else if constexpr (KALIGNED) {
         lds_dma16(a + static_cast<int64_t>(kt) * 64, off_a[ci], stage_addr + (wave * A_PER_WAVE + ci) * kChunkBytes);

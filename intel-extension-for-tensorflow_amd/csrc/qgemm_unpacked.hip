@@ -41,13 +41,7 @@ __device__ __forceinline__ v4i settle16(v4i v, int64_t off, int64_t end) {
   const int64_t over = off - (end - 16);
   // 0: in place; 16 and more: a piece that lies past the end as a whole, whose bytes are never used
   const uint32_t shift = over > 0 && over < 16 ? static_cast<uint32_t>(over) : 0;
-  uint64_t lo = static_cast<uint64_t>(static_cast<uint32_t>(v[1])) << 32 | static_cast<uint32_t>(v[0]);
-  uint64_t hi = static_cast<uint64_t>(static_cast<uint32_t>(v[3])) << 32 | static_cast<uint32_t>(v[2]);
-  if (shift & 8) { lo = hi; hi = 0; }
-  const uint32_t bits = (shift & 7) * 8;
-  lo = lo >> bits | (hi << 1) << (63 - bits);
-  hi = hi >> bits;
-  return v4i{static_cast<int>(lo), static_cast<int>(lo >> 32), static_cast<int>(hi), static_cast<int>(hi >> 32)};
+  return shift_down(v, shift);
 }
 
 // the first `n` bytes of a piece (n < 16 cuts, n <= 0 clears)
@@ -68,13 +62,9 @@ __device__ __forceinline__ int w_offset(int n, int k) { return n * kRow + (k ^ (
 
 // column 4 c + j of four rows' bytes -> v[j]
 __device__ __forceinline__ void transpose_bytes(const v4i (&rows)[4], int c, uint32_t (&v)[4]) {
-  const uint32_t r0 = rows[0][c], r1 = rows[1][c], r2 = rows[2][c], r3 = rows[3][c];
-  const uint32_t lo01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), hi01 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-  const uint32_t lo23 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), hi23 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-  v[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-  v[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-  v[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-  v[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+  const uint32_t w[4] = {static_cast<uint32_t>(rows[0][c]), static_cast<uint32_t>(rows[1][c]), static_cast<uint32_t>(rows[2][c]),
+                         static_cast<uint32_t>(rows[3][c])};
+  transpose_4x4(w, v);
 }
 
 template <int ALG, int COUNT>
