@@ -1245,9 +1245,10 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       // Little to read: narrow column blocks (128 bytes, single ints 64) whose workgroup takes all rows; the launch that initialises
       // costs more than what is lost in parallel reads (us, initialised / alone: 256 x 4096 5.0 / 3.0, 200 x 1000 5.0 / 3.3,
       // 500 x 64 5.1 / 3.6, 1000 x 1000 5.0 / 5.6).  Counted in the pieces that a workgroup loads at a time (32 KB, single ints 8):
-      // * rows of whole 128-byte lines: two rounds up to 2048 pieces 0.56 - 0.95 of the time, more to 1.26 (56 x 89888 5.5 / 6.9); with a
-      //   workgroup on every other CU up to 16 rounds, 0.65 - 1.15, in the middle 0.95 (1024 x 4096 7.1 / 5.7, 4096 x 4096 14.5 / 13.6,
-      //   3304 x 5504 16.2 / 14.3, 3397 x 8576 20.3 / 23.5; 8192 x 4096 27 / 37).
+      // * rows of whole 128-byte lines: two rounds up to 2048 pieces 0.56 - 0.95 of the time, more to 1.26 (56 x 89888 5.5 / 6.9);  up to 5
+      //   rounds and 2048 pieces 0.54 - 1.0;  up to 16 rounds with a workgroup on every other CU to every one (4096 to 8192 channels) 0.54 -
+      //   1.05 (0.84; 1024 x 4096 4.6 / 3.4, 4096 x 4096 13.8 / 13.0, 4096 x 8192 23.5 / 21.6; 8192 x 4096 27 / 37).  More channels, where some CUs
+      //   read a second block when the others are done, 0.79 - 1.26 (0.96: not there; 3397 x 8576 20.3 / 23.0, 3072 x 32768 67 / 83).
       // * other rows: neighbouring blocks share lines, which come once for each of their XCDs.  Two rounds up to 1024 pieces (single ints
       //   2048) 0.55 - 1.05, three and four up to 640 0.77 - 1.02; more 0.76 - 2.0 (455 x 21180 9.6 / 12.3, 225 x 21487 6.4 / 9.9,
       //   59 x 128396 7.2 / 14.5, 3773 x 17784 44 / 69).
@@ -1257,7 +1258,9 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       const bool lines = vec && depth % 32 == 0 && aligned(x, 128);
       const int64_t pieces = rounds * narrow_blocks;
       const bool alone = !few && narrow_blocks <= 65535 &&
-                         (rounds <= 2 ? pieces <= (lines || !vec ? 2048 : 1024) : vec && narrow_blocks >= 128 && rounds <= 16 && (lines || pieces <= 640));
+                         (rounds <= 2 ? pieces <= (lines || !vec ? 2048 : 1024)
+                                      : vec && narrow_blocks >= 128 && (lines ? (rounds <= 16 && narrow_blocks <= 256) || (rounds <= 5 && pieces <= 2048)
+                                                                              : pieces <= 640));
       if (alone) {
         groups = static_cast<int>(std::min<int64_t>(narrow, depth / per));
         col_blocks = narrow_blocks;
