@@ -372,7 +372,7 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 }  // namespace
 
 // Which calls come here, from 6900 products of these lines timed on both kernels (attention's two, 1 to 512 tokens, 8 to 4096 matrices; time
-// of the bands over that of the tiles, in the middle; of those that come 2 % take over 1.05, at most 1.29).  `large`: the tiles would be those of 128 rows, at least 1024 of them, which compute
+// of the bands over that of the tiles, in the middle; of those that come 2 % take over 1.05, at most 1.29; and 5600 of y transposed with 33 to 128 columns: 4 % over 1.05, at most 1.27).  `large`: the tiles would be those of 128 rows, at least 1024 of them, which compute
 // past the edges of ragged matrices and hold few wavefronts per CU (aligned operands alone).  Everywhere while four workgroups (P.V: three) share the LDS of a CU;
 // above that (wide results) it is 0.98 - 1.4, but for the second line.
 // * y along k (Q.K^T), large: 16-bit results 0.70.
@@ -390,6 +390,11 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 //   96 columns, 64 with operands, 80 with 32-bit results 0.88 - 1.28 (1.09; 160 x 160 x 128, 12 times 4.4 -> 5.4);  a step more with operands and
 //   an unaligned y of more than 80 columns 1.03 - 1.13;  nor with operands and unaligned rows on 49 to 64 columns, one tile wide, in many
 //   tiles: 16-bit up to three k steps 0.84 - 1.27 (1.05; 107 x 107 x 64, 2085 times 14.6 -> 18.6), 32-bit up to five 0.97 - 1.20 (1.08).
+// * not where the matrices are more than the device holds at once, of one tile of rows, a band for each wavefront behind the staging of a long y:
+//   49 to 64 columns, K > 256 (32-bit results 192) 0.87 - 1.47 (1.18; 25 x 280 x 50, 3032 times 17.8 -> 23.3), 33 to 48 columns, K > 320 0.93 - 1.34
+//   (1.05);  of two tiles of rows, 49 to 64 columns and K > 256 where the last round is a small one 0.96 - 1.31 (1.16; 95 x 304 x 50, 890 times 13.4 -> 17.6).
+// * not 16-bit results whose rows are no whole vectors in few tiles: 49 to 64 columns, up to 1024 tiles of at most three k steps 0.91 - 1.21 (1.06), more
+//   columns up to 256 tiles 0.94 - 1.26 (1.09; 102 x 208 x 100, 34 times 5.0 -> 5.9).
 // Small launches of Q.K^T stay with the tiles (1.05 - 1.24): this kernel has a way through LDS more.
 bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_y, bool large, const int8_t* x, const int8_t* y, void* out,
                hipStream_t st) {
@@ -413,6 +418,7 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
     if (tiles <= 512 && p.K <= 192 && N > (operands ? 64 : wide ? 80 : 96)) return false;
     if (operands && !aligned_operands &&
         (tiles > 2048 ? N > 48 && N <= 64 && p.K <= (wide ? 320 : 192) : !wide && tiles <= 256 && p.K <= 256 && N > 80)) return false;
+    if (!wide && !a.whole_rows && N > 48 && ((tiles <= 256 && N > 64) || (tiles <= (N > 64 ? 512 : 1024) && p.K <= 192))) return false;
   }
   // rows of whole 64-byte pieces are cut into parts of at most 512 bytes, as even as they get (384 columns of fp32: 25.7 us whole,
   // 18.0 in three parts); the pieces of lines that parts of other rows would end in cost more than they give (216 columns of
@@ -448,6 +454,8 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
   // as many workgroups as the device holds at once (two to four on a CU), each with some of a matrix's bands: one that starts late
   // costs a round (Q.K^T over 197 tokens, bfloat16: 768 workgroups 12.3 us, 1536 of half as many bands 14.0)
   const int64_t resident = 256 * std::min(4, std::max(1, 160 * 1024 / lds));
+  if (!p.adj_y && N > 32 && N <= 64 && batch > resident &&
+      (p.M <= 64 ? p.K > (N <= 48 ? 320 : wide ? 192 : 256) : p.M <= 128 && N > 48 && p.K > 256 && batch * 10 <= resident * 13)) return false;
   a.batch = static_cast<uint32_t>(batch);
   a.bands = static_cast<int>((p.M + kBand - 1) / kBand);
   const int64_t want = std::min<int64_t>(std::max<int64_t>(1, resident / (batch * a.chunks)), (a.bands + kBandWaves - 1) / kBandWaves);

@@ -24,11 +24,13 @@ def test_products_over_many_k(hip, dev, M, K, N, t_out):
     import torch
     rng = np.random.default_rng(M * 7 + K + N)
     x, y = rng.integers(-128, 128, (2, 3, M, K)).astype(np.int8), rng.integers(-128, 128, (2, 3, K, N)).astype(np.int8)
+    # (few tiles of 16-bit rows that are no whole vectors and over 64 columns are the tiles')
+    kernel = "bmm_tiles" if t_out != orc.FLOAT and (K, N) == (193, 79) else "bmm_bands"
     check(hip, dev, x, y, t_out=t_out)
-    assert hip.last_kernel()[0] == "bmm_bands"
+    assert hip.last_kernel()[0] == kernel
     check(hip, dev, x, y, binary=operands(torch, rng, N, t_out, 2)[::-1], t_out=t_out, x_off=3, y_off=1)
     check(hip, dev, x, y[:1], binary=operands(torch, rng, N, t_out)[1:], t_out=t_out, x_off=16)
-    assert hip.last_kernel()[0] == "bmm_bands"
+    assert hip.last_kernel()[0] == kernel
 
 
 # Q.K^T of at least 1024 tiles of 128 rows: rows of whole vectors and others, one to eleven column tiles, D of one and two k tiles
@@ -59,6 +61,14 @@ def test_many_matrices(hip, dev, M, K, N, t_out):
     (40, 130, 199, 84, False, orc.HALF, 1, "bmm_tiles"), (43, 130, 199, 84, False, orc.HALF, 1, "bmm_bands"),
     (2049, 20, 70, 52, False, orc.HALF, 1, "bmm_tiles"), (2048, 20, 70, 52, False, orc.HALF, 1, "bmm_bands"),
     (2049, 20, 70, 48, False, orc.HALF, 1, "bmm_bands"), (2049, 20, 70, 52, False, orc.HALF, 0, "bmm_bands"),
+    # (what the device holds at once: 1024 workgroups, 768 where the LDS of a CU takes three)
+    (769, 64, 272, 64, False, orc.HALF, 0, "bmm_tiles"), (1025, 64, 256, 64, False, orc.HALF, 0, "bmm_bands"), (768, 64, 272, 64, False, orc.HALF, 0, "bmm_bands"),
+    (998, 65, 272, 64, False, orc.HALF, 0, "bmm_tiles"), (999, 65, 272, 64, False, orc.HALF, 0, "bmm_bands"), (998, 129, 272, 64, False, orc.HALF, 0, "bmm_bands"),
+    (1025, 20, 208, 56, False, orc.FLOAT, 0, "bmm_tiles"), (1025, 20, 192, 64, False, orc.FLOAT, 0, "bmm_bands"),
+    (1025, 20, 321, 40, False, orc.BFLOAT16, 1, "bmm_tiles"), (1025, 20, 320, 40, False, orc.BFLOAT16, 1, "bmm_bands"), (1025, 20, 321, 32, False, orc.BFLOAT16, 1, "bmm_bands"),
+    (340, 130, 191, 50, False, orc.HALF, 0, "bmm_tiles"), (340, 130, 193, 50, False, orc.HALF, 0, "bmm_bands"), (342, 130, 191, 50, False, orc.HALF, 0, "bmm_bands"),
+    (340, 130, 191, 48, False, orc.HALF, 0, "bmm_bands"), (42, 130, 256, 100, False, orc.HALF, 0, "bmm_tiles"),
+    (43, 130, 256, 100, False, orc.HALF, 0, "bmm_bands"), (42, 130, 256, 104, False, orc.HALF, 0, "bmm_bands"), (256, 60, 190, 70, False, orc.BFLOAT16, 0, "bmm_tiles"),
     (2049, 20, 199, 52, False, orc.FLOAT, 1, "bmm_tiles"), (2049, 20, 199, 48, False, orc.FLOAT, 1, "bmm_bands")])
 def test_lines_to_the_tiles(hip, dev, B, M, K, N, adj_y, t_out, n_ops, kernel):
     import torch
@@ -89,7 +99,7 @@ def test_results_at_any_address(hip, dev, t_out, N):
     """A result that starts off a 16-byte boundary, with the elements around it untouched."""
     import torch
     rng = np.random.default_rng(N)
-    x, y = rng.integers(-128, 128, (5, 37, 200)).astype(np.int8), rng.integers(-128, 128, (5, 200, N)).astype(np.int8)
+    x, y = rng.integers(-128, 128, (130, 37, 200)).astype(np.int8), rng.integers(-128, 128, (130, 200, N)).astype(np.int8)
     want = run(hip, dev, x, y, 2.0, 3.0, t_out=t_out)
     xd, yd = torch.from_numpy(x).to(dev), torch.from_numpy(y).to(dev)
     p, _ = hip.bmm_params(x.shape, y.shape, False, False, t_out, float(np.float32(6.0) / np.float32(127 * 127)))
