@@ -1249,8 +1249,8 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       //   rounds and 2048 pieces 0.54 - 1.0;  up to 16 rounds with a workgroup on every other CU to every one (4096 to 8192 channels) 0.54 -
       //   1.05 (0.84; 1024 x 4096 4.6 / 3.4, 4096 x 4096 13.8 / 13.0, 4096 x 8192 23.5 / 21.6; 8192 x 4096 27 / 37).  More channels, where some CUs
       //   read a second block when the others are done, 0.79 - 1.26 (0.96: not there; 3397 x 8576 20.3 / 23.0, 3072 x 32768 67 / 83).
-      // * other rows: neighbouring blocks share lines, which come once for each of their XCDs.  Two rounds up to 1024 pieces (single ints
-      //   2048) 0.55 - 1.05, three and four up to 640 0.77 - 1.02; more 0.76 - 2.0 (455 x 21180 9.6 / 12.3, 225 x 21487 6.4 / 9.9,
+      // * other rows: neighbouring blocks share lines, which come once for each of their XCDs.  Up to four rounds and 640 pieces 0.55 - 1.02,
+      //   two of single ints up to 1536 0.51 - 0.93; more 0.66 - 2.0 (241 x 16058 5.1 / 7.9, 426 x 15732 6.2 / 9.6, 223 x 27804 6.4 / 8.4,
       //   59 x 128396 7.2 / 14.5, 3773 x 17784 44 / 69).
       // (launches of a captured graph; one by one from the host, where a second launch costs 2.5 us, the lone workgroups gain more)
       const int narrow = vec ? 8 : 16;
@@ -1258,7 +1258,7 @@ extern "C" int itexhip_minmax_i32_per_channel(const int32_t* x, int64_t rows, in
       const bool lines = vec && depth % 32 == 0 && aligned(x, 128);
       const int64_t pieces = rounds * narrow_blocks;
       const bool alone = !few && narrow_blocks <= 65535 &&
-                         (rounds <= 2 ? pieces <= (lines || !vec ? 2048 : 1024)
+                         (rounds <= 2 ? pieces <= (lines ? 2048 : vec ? 640 : 1536)
                                       : vec && narrow_blocks >= 128 && (lines ? (rounds <= 16 && narrow_blocks <= 256) || (rounds <= 5 && pieces <= 2048)
                                                                               : pieces <= 640));
       if (alone) {

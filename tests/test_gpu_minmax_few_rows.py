@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,depth", [(1, 5), (8, 300), (9, 3), (9, 8), (17, 2), (255, 17), (256, 33), (257, 15), (511, 36), (512, 64), (513, 4),
                                         (4095, 4096), (4096, 4100), (4097, 4096), (1, 1), (3, 1), (24576, 1), (24575, 1), (24580, 1),
-                                        (1024, 4096), (1025, 4100), (4096, 4096), (4096, 4128), (1025, 6528), (1025, 6560), (1024, 16384), (1024, 16416), (1280, 13088), (1281, 13088), (4096, 8192), (4096, 8224), (536, 4652), (1024, 5120), (1024, 5124), (1024, 5092), (512, 16380),
+                                        (1024, 4096), (1025, 4100), (4096, 4096), (4096, 4128), (1025, 6528), (1025, 6560), (1024, 16384), (1024, 16416), (1280, 13088), (1281, 13088), (4096, 8192), (4096, 8224), (536, 4652), (1024, 5120), (1024, 5124), (1024, 5092), (512, 16380), (512, 10236), (512, 10244), (256, 20476), (256, 20484), (256, 12287), (256, 12289), (128, 24575), (128, 24577),
                                         (512, 16388), (256, 16383), (256, 16385), (20, 65500), (20, 131200)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_range(hip, dev, rows, depth, off):
