@@ -377,8 +377,11 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 // above that (wide results) it is 0.98 - 1.4, but for the second line.
 // * y along k (Q.K^T), large: 16-bit results 0.70.
 // * the same, 32-bit results whose rows are no multiple of 64 bytes, which the tiles write in pieces of lines: 0.65 with fused operands,
-//   0.93 without them on up to 192 columns that are no whole 16-byte vectors a row (others 1.08); at any size of the images.  Rows of
+//   0.91 without them on up to 192 columns that are no whole 16-byte vectors a row (others 1.08); at any size of the images.  Rows of
 //   whole 64-byte pieces up to 27 KB of LDS 0.68 (wider ones 1.10).
+// * of those without operands, up to 224 MB of results (beyond, out of the memory-side cache, 0.36 - 1.3, 0.6), not: rows whose last 32 columns, a tile's
+//   quadrant, are more than half full, K <= 96 0.53 - 1.42 (1.05; 182 x 32 x 182, 1053 times 36 -> 46 us), more than 176 columns 0.64 - 1.49 (1.08); nor,
+//   at two workgroups a CU or one, more than 12 bands in a workgroup 0.43 - 1.42 (1.07), or a small last round 0.9 - 1.35 (1.1).  900 products: 34 over 1.05.
 // * not where rows are no whole vectors: 16-bit results of up to 64 columns, one tile wide, 0.77 - 1.35 (1.08), or of one k tile and more than
 //   256 rows by up to 128 columns 0.79 - 1.31 (1.27; 315 x 64 x 107, 3881 times 102 -> 133 us);  32-bit results of more than 192 columns without
 //   operands 0.68 - 1.79 (1.21; 339 x 64 x 339, 265 times 32 -> 56), two workgroups or one on a CU that shift and store wide rows.
@@ -411,7 +414,10 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
   a.p = p;
   a.whole_rows = N * esz % 16 == 0 && aligned(out, 16);
   const bool operands = p.n_binary > 0, wide = esz == 4;
+  // scores of fp32 without operands on ragged rows, whose tiles go out as fast where the results stay in the memory-side cache
+  const bool bare = p.adj_y && wide && !operands && !a.whole_rows && batch * p.M * N * esz <= 224LL << 20;
   if (p.adj_y) {
+    if (bare && (N - 1) % 32 >= 16 && (p.K <= 96 || N > 176)) return false;
     if (!a.whole_rows && (wide ? !operands && N > 192 : N <= 64 || (p.K <= 64 && p.M > 256 && N <= 128))) return false;
   } else {
     const int64_t tiles = batch * ((p.M + 63) / 64) * ((N + 63) / 64);
@@ -460,6 +466,7 @@ bool qbmm_band(const itexhip_bmm_params& p, int64_t batch, int mode_x, int mode_
   a.bands = static_cast<int>((p.M + kBand - 1) / kBand);
   const int64_t want = std::min<int64_t>(std::max<int64_t>(1, resident / (batch * a.chunks)), (a.bands + kBandWaves - 1) / kBandWaves);
   a.bands_per_part = static_cast<int>((a.bands + want - 1) / want);
+  if (bare && resident <= 512 && (a.bands_per_part > 12 || (batch > resident && batch * 10 < resident * 13))) return false;
   const int jobs = (a.bands + a.bands_per_part - 1) / a.bands_per_part * a.chunks;
   a.xcd_grid = batch % 8 == 0 || batch >= 64 ? 1 : 0;  // whole matrices per XCD: y is read into one L2
   if (jobs > 65535 || (a.xcd_grid ? (batch + 7) / 8 > 65535 : batch > 65535)) return false;

@@ -45,14 +45,17 @@ def test_many_matrices(hip, dev, M, K, N, t_out):
     check(hip, dev, x, y, adj_y=True, binary=operands(torch, rng, N, t_out, 129), t_out=t_out)
     assert hip.last_kernel() == kernel
     check(hip, dev, x, y[:, :1], adj_y=True, binary=operands(torch, rng, N, t_out)[:1] if N == 20 else (), t_out=t_out)
-    assert hip.last_kernel() == kernel
+    # (nor fp32 rows whose last 32 columns are more than half full, without operands)
+    assert hip.last_kernel() == (("bmm_tiles", 21) if t_out == orc.FLOAT and N == 17 else kernel)
 
 
 # both sides of the lines between the bands and the tiles: y along k, then y transposed on the way
 @pytest.mark.parametrize("B,M,K,N,adj_y,t_out,n_ops,kernel", [
     (1030, 70, 64, 61, True, orc.BFLOAT16, 1, "bmm_tiles"), (1030, 70, 64, 67, True, orc.BFLOAT16, 1, "bmm_bands"),
     (345, 257, 64, 67, True, orc.HALF, 0, "bmm_tiles"), (345, 256, 64, 67, True, orc.HALF, 0, "bmm_tiles"), (520, 256, 64, 67, True, orc.HALF, 0, "bmm_bands"),
-    (515, 70, 64, 191, True, orc.FLOAT, 0, "bmm_bands"), (515, 70, 64, 193, True, orc.FLOAT, 0, "bmm_tiles"),
+    (700, 70, 64, 169, True, orc.FLOAT, 0, "bmm_bands"), (515, 70, 64, 169, True, orc.FLOAT, 0, "bmm_tiles"), (515, 70, 64, 193, True, orc.FLOAT, 0, "bmm_tiles"),
+    (300, 192, 64, 169, True, orc.FLOAT, 0, "bmm_bands"), (300, 193, 64, 169, True, orc.FLOAT, 0, "bmm_tiles"), (515, 129, 96, 61, True, orc.FLOAT, 0, "bmm_tiles"),
+    (515, 129, 112, 61, True, orc.FLOAT, 0, "bmm_bands"), (700, 70, 192, 159, True, orc.FLOAT, 0, "bmm_bands"), (515, 70, 192, 179, True, orc.FLOAT, 0, "bmm_tiles"),
     (515, 70, 64, 193, True, orc.FLOAT, 1, "bmm_bands"),
     (64, 130, 192, 100, False, orc.BFLOAT16, 0, "bmm_tiles"), (64, 130, 208, 100, False, orc.BFLOAT16, 0, "bmm_bands"),
     (86, 130, 192, 100, False, orc.BFLOAT16, 0, "bmm_bands"), (64, 130, 192, 96, False, orc.BFLOAT16, 0, "bmm_bands"),
@@ -78,6 +81,21 @@ def test_lines_to_the_tiles(hip, dev, B, M, K, N, adj_y, t_out, n_ops, kernel):
     ops = [(alg, v.reshape(v.shape[1:] if v.ndim > 1 else v.shape)) for alg, v in operands(torch, rng, N, t_out)][:n_ops]
     check(hip, dev, x, y, adj_y=adj_y, binary=ops, t_out=t_out)
     assert hip.last_kernel()[0] == kernel
+
+
+def test_results_beyond_the_memory_side_cache(hip, dev):
+    """fp32 rows without operands: bands for 235 MB, tiles for each half, the same results."""
+    import torch
+    B, M, K, N = 1100, 280, 16, 191
+    x, y = (torch.randint(-128, 128, s, dtype=torch.int8, device=dev) for s in ((B, M, K), (B, N, K)))
+    whole, halves = torch.empty(B, M, N, device=dev), torch.empty(2, B // 2, M, N, device=dev)
+    hip.qbatch_matmul(hip.bmm_params((B, M, K), (B, N, K), False, True, hip.FLOAT, 0.01)[0], x, y, whole)
+    assert hip.last_kernel()[0] == "bmm_bands"
+    p, _ = hip.bmm_params((B // 2, M, K), (B // 2, N, K), False, True, hip.FLOAT, 0.01)
+    for i in range(2):
+        hip.qbatch_matmul(p, x[i * B // 2:], y[i * B // 2:], halves[i])
+        assert hip.last_kernel()[0] == "bmm_tiles"
+    assert torch.equal(whole, halves.view(B, M, N))
 
 
 @pytest.mark.parametrize("K,N,parts,t_out", [(64, 288, 2, orc.HALF), (32, 320, 2, orc.BFLOAT16), (200, 160, 2, orc.FLOAT), (193, 144, 2, orc.FLOAT)])
