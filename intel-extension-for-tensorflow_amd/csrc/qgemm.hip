@@ -596,9 +596,9 @@ enum class Path { kTile, kSmallM, kAny, kAuto };  // kAny: the tile kernel or th
 // or by 32 x 32 pieces:
 //   33 to 128 rows        up to 16 tiles 0.5 - 1.27 (K <= 256 1.03, 257 - 1024 0.9, more 0.69), 17 - 64 tiles up to 256 pieces K <= 1024
 //                         0.77 - 1.3 (1.0), more 0.59 - 1.0 (0.8);  65 - 128 tiles up to 256 pieces K 513 - 1024 0.84 - 1.11 (0.94), more
-//                         0.59 - 0.99 (0.8), else K <= 1536, or up to 64 rows, 0.9 - 1.5 (1.1: not there), longer 0.8 - 1.3 (1.05), more tiles 1.0 - 2.4.  Rows that
-//                         are no whole 16-byte vectors differ by 0.1 at most; with a K of one step, or K > 1536 and few more than
-//                         128 tiles, either kernel does.
+//                         0.59 - 0.99 (0.8), else 0.9 - 1.55 (1.15, K from 8000 on 1.35: not there; 99 x 10032 -> 2066 27.7 / 19.9), more tiles 1.0 - 2.4.  Rows that
+//                         are no whole 16-byte vectors differ by 0.1 at most; with a K of one step and few more than 128 tiles
+//                         either kernel does.
 //   129 to 2048 rows      (950 sizes of whole 16-byte rows) up to 128 pieces K <= 512 1.03 - 1.26 (1.18: not there), 513 - 768 0.93 - 1.12
 //                         (1.03: not there; 32-bit rows that are no whole vectors 0.85 - 0.93), 769 - 1024 0.83 - 1.0 (0.94), to 2048 0.70 - 0.97 (0.84), more 0.53 - 0.78 (0.65);  129 - 256
 //                         pieces K <= 1024 0.72 - 1.4 (0.97: not there), to 2048 0.74 - 1.0 (0.87), more 0.60 - 0.89 (0.75);  more pieces 0.78 - 2
@@ -627,7 +627,7 @@ static bool small_m(int64_t M, int64_t K, int64_t N, const EpilogueArgs& e, int 
     return pieces <= 128 ? K > (esz == 4 && !whole_rows ? 512 : 768) : pieces <= 256 && K > (e.addend ? 1536 : 1024);
   }
   if (vector && e.addend == nullptr) {
-    if (M > 32 && K >= 128 && tiles > 64 && (M <= 64 || K <= 1536) && !(pieces <= 256 && K > 512)) return false;
+    if (M > 32 && K >= 128 && tiles > 64 && !(pieces <= 256 && K > 512)) return false;
     if (whole_rows ? K >= 64 && tiles > 128 : K >= 128 && tiles > 144)
       if (M > 32 || K < 256 || (K < 768) == (tiles > 256)) return false;
   }

@@ -110,7 +110,7 @@ def test_small_m_kernel_on_more_rows_and_wavefronts(hip, dev, M, N, K):
 @pytest.mark.parametrize("M,N,K,kernel", [(129, 64, 768, "tile"), (129, 64, 784, "small_m"), (129, 65, 512, "tile"), (129, 65, 528, "small_m"), (512, 256, 768, "tile"), (512, 256, 784, "small_m"),
                                           (512, 257, 784, "tile"), (1024, 128, 784, "small_m"), (1024, 129, 784, "tile"), (1024, 256, 1024, "tile"),
                                           (1024, 256, 1040, "small_m"), (1024, 257, 1040, "tile"), (2048, 64, 784, "small_m"), (2049, 32, 784, "tile"), (64, 4096, 128, "small_m"),
-                                          (64, 4160, 128, "tile"), (128, 2112, 1536, "tile"), (128, 2112, 1552, "small_m"),
+                                          (64, 4160, 128, "tile"), (128, 2048, 1552, "small_m"), (128, 2112, 1552, "tile"), (65, 2700, 5168, "small_m"), (97, 2080, 5168, "tile"),
                                           (96, 2112, 512, "tile"), (96, 2112, 528, "small_m")])
 def test_line_between_the_kernels(hip, dev, M, N, K, kernel):
     layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)

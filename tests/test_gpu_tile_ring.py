@@ -64,7 +64,7 @@ def test_where_the_shape_changes(hip, dev, M, K, N, tile):
                                           (32, 752, 16448, "tile"), (32, 768, 16448, "small_m"), (32, 768, 16384, "tile"),
                                           (33, 64, 8192, "small_m"), (33, 64, 8256, "tile"), (65, 64, 4096, "small_m"),
                                           (65, 64, 4160, "tile"), (128, 1040, 4160, "tile"), (128, 64, 4161, "small_m"),
-                                          (128, 2032, 4161, "tile"), (128, 2000, 4161, "small_m"),                           # rows of odd length, 8 MB
+                                          (128, 128, 4161, "tile"), (128, 112, 4161, "small_m"), (128, 2000, 4161, "tile"),  # rows of odd length
                                           (129, 64, 64, "tile")])
 def test_line_between_the_small_m_and_the_tile_kernel(hip, dev, M, K, N, kernel):
     layer, _, _ = make_layer(hip, dev, K, N, seed=K + N)
