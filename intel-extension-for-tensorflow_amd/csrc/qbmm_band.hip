@@ -371,10 +371,11 @@ void launch_out(const BandArgs& a, bool al, int lds, dim3 grid, const int8_t* x,
 
 }  // namespace
 
-// Which calls come here, from 6900 products of these lines timed on both kernels (attention's two, 1 to 512 tokens, 8 to 4096 matrices; time
-// of the bands over that of the tiles, in the middle; of those that come 2 % take over 1.05, at most 1.29; and 5600 of y transposed with 33 to 128 columns: 4 % over 1.05, at most 1.27).  `large`: the tiles would be those of 128 rows, at least 1024 of them, which compute
-// past the edges of ragged matrices and hold few wavefronts per CU (aligned operands alone).  Everywhere while four workgroups (P.V: three) share the LDS of a CU;
-// above that (wide results) it is 0.98 - 1.4, but for the second line.
+// Which calls come here, from products timed on both kernels (6900 of attention's two, 1 to 512 tokens, 8 to 4096 matrices, and 5100 around
+// the lines; time of the bands over that of the tiles, in the middle; of those that come 2 and 5 % take over 1.05, at most 1.47).  `large`: the
+// tiles would be those of 128 rows, at least 1024 of them, which compute past the edges of ragged matrices and hold few wavefronts per CU
+// (aligned operands alone).  Everywhere while four workgroups (P.V: three) share the LDS of a CU; above that (wide results) it is 0.98 - 1.4,
+// but for the second line.
 // * y along k (Q.K^T), large: 16-bit results 0.70.
 // * the same, 32-bit results whose rows are no multiple of 64 bytes, which the tiles write in pieces of lines: 0.65 with fused operands,
 //   0.91 without them on up to 192 columns that are no whole 16-byte vectors a row (others 1.08); at any size of the images.  Rows of

@@ -645,7 +645,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void qgemm_tile_kernel(
       } else {
         // Rows of any length and address: pieces wherever they fall (plain stores, L2 puts the lines together; streaming ones 1 - 15 %
         // slower), the last one of a row in parts.  As the element-wise epilogue, a store per value, such rows took (8-bit, us,
-        // element-wise / this): 1034 x 144 -> 1976 45 / 6.1, 592 x 1024 -> 3747 51 / 10.4, 1000 x 512 -> 1004 8.1 / 4.5.
+        // element-wise / this, in a graph): 1034 x 144 -> 1976 45 / 5.7, 592 x 1024 -> 3747 50 / 7.5, 1000 x 512 -> 1004 8.0 / 3.8.
         const int bytes = (N - n_col) * ESZ;
         flush([&](uint8_t* dst, const v4i& v, const uint8_t* src) {
           typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
